@@ -195,7 +195,9 @@ int vs_cuda_spmm_f16_f32out(int m_vec, int vec_length, int k, int n,
  * rows and small problems).  0 = automatic: schedule 1, except that masks of few
  * nonzeros with vec_length <= 4 - which fill a quarter of a matrix-core tile or
  * less - run on the fine-grained kernel of vs_cuda_sddmm_f16 (same function
- * within the fp32-accumulation tolerance, not the same bits).
+ * within the fp32-accumulation tolerance, not the same bits).  Under 0 and 1, and in vs_cuda_sddmm_f16, masks that
+ * keep a good share of large tiles (short vectors, low sparsity) multiply whole tiles and keep the masked outputs
+ * (option "sddmm_tile"): the bits of schedule 1, columns of a row in any order.
  * 3 (the reference's timing-only hardware
  * simulation, whose results are wrong by design) is rejected with
  * hipErrorInvalidValue.
@@ -527,6 +529,8 @@ int vs_wmma_spmm_launch_shape(int batch, int m_vec, int vec_length, int k, int n
  * vector row, 0 = automatic), "sddmm_group" (16-vector groups per wave step of the
  * MFMA SDDMM: 1, 2, 4, 0 = automatic), "sddmm_block_waves" (1..16, 0 = automatic),
  * "sddmm_flat_supers" (super-groups per wave of algorithm 2, 1..16, 0 = automatic),
+ * "sddmm_tile" (SDDMM on dense tiles, k % 8 == 0: 1 = never, 2 = tiles of 64 x 64, 3 = of 128 x 128,
+ * 0 = where it is expected to be faster than gathering rows),
  * "attention_waves" (1..8, 0 = automatic), "attention_chunk" (nonzero vectors per
  * LDS chunk of the one-row-per-workgroup attention kernel, 0 = automatic).
  * Returns 0, or 1 for an unknown name / bad value.

@@ -1,0 +1,85 @@
+"""SDDMM on dense tiles (csrc/sddmm_tile.hip): both tile sizes at the edges of tiles, rows, columns and contraction
+steps, against the C oracle, and bit for bit against the gathering MFMA kernel (same products in the same order)."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import c_oracle as co
+from vectorsparse_amd import _lib, ops
+from vectorsparse_amd import colvec_csr as cv
+from util import assert_parity
+
+pytestmark = pytest.mark.gpu
+
+
+def _shuffled(pat, seed):
+    rng = np.random.default_rng(seed)
+    cols = pat.column_indices.copy()
+    for i in range(pat.m_vec):
+        rng.shuffle(cols[pat.row_offsets[i]:pat.row_offsets[i + 1]])
+    return cv.ColVecCSR(pat.m_vec, pat.n, pat.vec_length, pat.row_offsets, cols)
+
+
+def _pattern(kind, m_vec, n, V):
+    rng = np.random.default_rng(m_vec + n + V)
+    if kind == "shuffled columns":
+        return _shuffled(cv.binomial_pattern(m_vec, n, 0.6, seed=3, vec_length=V), 4)
+    if kind == "repeated columns":   # more nonzeros of one column than a tile has columns
+        lengths = np.where(np.arange(m_vec) % 3 == 0, 300, 5)
+        ro = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+        return cv.ColVecCSR(m_vec, n, V, ro, np.sort(rng.integers(0, 3, ro[-1])).astype(np.int32))
+    if kind == "dense and empty rows":
+        lengths = np.where(np.arange(m_vec) % 2 == 0, n, 0)
+        ro, ci = cv._pattern_from_lengths(rng, m_vec, n, lengths)
+        return cv.ColVecCSR(m_vec, n, V, ro, ci)
+    if kind == "clustered columns":  # far from uniform: the search's first probes are all off; most tiles are empty
+        rows = [np.sort(rng.choice(np.r_[0:17, n - 9:n], 20, replace=False)) for _ in range(m_vec)]
+        ro = (np.arange(m_vec + 1) * 20).astype(np.int32)
+        return cv.ColVecCSR(m_vec, n, V, ro, np.concatenate(rows).astype(np.int32))
+    return cv.binomial_pattern(m_vec, n, 0.7, seed=5, vec_length=V)
+
+
+@pytest.mark.parametrize("tile", [2, 3])
+@pytest.mark.parametrize("V", [1, 2, 4, 8])
+@pytest.mark.parametrize("kind,rows,n,K", [
+    ("uniform", 1, 1, 8), ("uniform", 64, 64, 64), ("uniform", 128, 128, 128), ("uniform", 136, 129, 72),
+    ("uniform", 56, 63, 320), ("uniform", 1048, 300, 40), ("clustered columns", 200, 900, 136),
+    ("dense and empty rows", 72, 200, 264), ("shuffled columns", 96, 200, 96), ("repeated columns", 48, 65, 64)])
+def test_dense_tiles_match_the_oracle_and_the_gathering_kernel(gpu, kind, rows, n, K, V, tile):
+    m_vec = max(1, rows // V)
+    pat = _pattern(kind, m_vec, n, V)
+    A, B = cv.dense_normal(pat.m, K, seed=6), cv.dense_normal(n, K, seed=7)
+    prob = ops.DeviceProblem(pat)
+    Ad, Bd = torch.from_numpy(A).cuda(), torch.from_numpy(B).cuda()
+    ref = co.sddmm_host_ref_f32(pat.m_vec, K, V, pat.row_offsets, pat.column_indices, A, B)
+    for dtype in (torch.float16, torch.float32):
+        pad = torch.full((pat.nnz_vec + 32, V), 7.0, dtype=dtype, device="cuda")
+        got = pad[16:16 + pat.nnz_vec]
+        with _lib.thread_options(sddmm_tile=tile):
+            prob.sddmm(Ad, Bd, out=got, algorithm=1)
+        with _lib.thread_options(sddmm_tile=1):
+            gathered = prob.sddmm(Ad, Bd, out_dtype=dtype, algorithm=1)
+        torch.cuda.synchronize()
+        assert bool((pad[:16] == 7.0).all()) and bool((pad[16 + pat.nnz_vec:] == 7.0).all())
+        assert_parity(got.cpu().numpy().reshape(-1), ref, "%s %s" % (kind, dtype))
+        if kind not in ("shuffled columns", "repeated columns"):   # (nonzeros served one by one add up in another order)
+            assert torch.equal(got, gathered)
+
+
+def test_dense_tiles_batched(gpu):
+    V, heads, n, K = 2, 3, 190, 72
+    mask = cv.binomial_pattern(75, n, 0.6, seed=8, vec_length=V)
+    prob = ops.DeviceProblem(mask)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    A = torch.randn((heads, mask.m, K), device="cuda", generator=g).half()
+    B = torch.randn((heads, n, K), device="cuda", generator=g).half()
+    out = torch.empty((heads, mask.nnz_vec, V), dtype=torch.float16, device="cuda")
+    for tile in (2, 3):
+        with _lib.thread_options(sddmm_tile=tile):
+            ops.sddmm_batched(mask.m_vec, K, n, mask.nnz_vec, prob.row_indices, prob.row_offsets, prob.column_indices, A, B,
+                              out, V)
+        with _lib.thread_options(sddmm_tile=1):
+            one = [prob.sddmm(A[h], B[h], algorithm=1) for h in range(heads)]
+        torch.cuda.synchronize()
+        for h in range(heads):
+            assert torch.equal(out[h], one[h]), "head %d" % h

@@ -124,6 +124,9 @@ sddmm_mfma_kernel(int m_vec, int K, int slots, int waves_per_block, const int *_
             }
         }
     } else {
+        // contractions beyond 256: eight slices of both operands in flight per turn (one at a time is a chain of K / 32
+        // round trips: 2048 x 2304 at 98 %, V = 4, K = 512, 10.3 us)
+        constexpr int TURN = 8;
         const int k_steps = (K + 31) >> 5;
         for (int sg = s; sg < n_super; sg += slots) {
             const int j0 = beg + SUPER * sg;
@@ -135,15 +138,27 @@ sddmm_mfma_kernel(int m_vec, int K, int slots, int waves_per_block, const int *_
                 rhs_row[u] = rhs + (size_t)col_indices[jl < end ? jl : end - 1] * K;
                 acc[u] = float4_t{0.f, 0.f, 0.f, 0.f};
             }
-            for (int kk = 0; kk < k_steps; ++kk) {
-                const half8_t a = to_mfma_order(load_slice16(lhs_row, kk, q, K, a_row_ok), src);
-                uint4_t raw[GRP];
+            for (int kk = 0; kk < k_steps; kk += TURN) {
+                uint4_t a[TURN], raw[GRP][TURN];
 #pragma unroll
-                for (int u = 0; u < GRP; ++u) raw[u] = load_slice16(rhs_row[u], kk, q, K, true);
+                for (int t = 0; t < TURN; ++t) a[t] = load_slice16(lhs_row, kk + t, q, K, a_row_ok);
 #pragma unroll
                 for (int u = 0; u < GRP; ++u)
-                    acc[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, to_mfma_order(raw[u], src), acc[u], 0, 0, 0);
+#pragma unroll
+                    for (int t = 0; t < TURN; ++t) raw[u][t] = load_slice16(rhs_row[u], kk + t, q, K, true);
+#pragma unroll
+                for (int t = 0; t < TURN; ++t) {
+                    const half8_t at = to_mfma_order(a[t], src);
+#pragma unroll
+                    for (int u = 0; u < GRP; ++u)
+                        acc[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(at, to_mfma_order(raw[u][t], src), acc[u], 0, 0, 0);
+                }
             }
+            // The last product's registers that nobody reads (V = 1: three of four) were handed to the code below while the
+            // product was still to land in them, three issue slots behind it across the loop's exit: the columns' number was
+            // overwritten and nothing stored (V = 1, fp32 outputs).  The products have landed after these slots.
+#pragma unroll
+            for (int u = 0; u < GRP; ++u) asm volatile("s_nop 15" : "+v"(acc[u]));
 #pragma unroll
             for (int u = 0; u < GRP; ++u) {
                 const int j = j0 + 16 * u + c;
@@ -373,7 +388,7 @@ static int launch_ks(int m_vec, int k, int nonzeros_vec, const int *row_indices,
     if (k <= 64) return launch_grp<V, 2, OutT>(grp, m_vec, k, nonzeros_vec, row_indices, row_offsets, col_indices, lhs, rhs, out, stream, batch);
     if (k <= 128) return launch_grp<V, 4, OutT>(grp, m_vec, k, nonzeros_vec, row_indices, row_offsets, col_indices, lhs, rhs, out, stream, batch);
     if (k <= 256) return launch_one<V, 8, 1, OutT>(m_vec, k, nonzeros_vec, row_indices, row_offsets, col_indices, lhs, rhs, out, stream, batch);
-    return launch_one<V, 0, 4, OutT>(m_vec, k, nonzeros_vec, row_indices, row_offsets, col_indices, lhs, rhs, out, stream, batch);
+    return launch_one<V, 0, 1, OutT>(m_vec, k, nonzeros_vec, row_indices, row_offsets, col_indices, lhs, rhs, out, stream, batch);
 }
 
 // Waves per vector row.  Waves are independent (no reduction).  A wave that finds no super-group of its own exits
@@ -422,15 +437,21 @@ int launch_sddmm_mfma(int m_vec, int k, int n, int nonzeros_vec, const int *row_
         return launch_sddmm_valu<OutT>(m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices, lhs, rhs, out,
                                        vec_length, stream, batch);
     }
-    // algorithm 0 (automatic): vectors of 1, 2 or 4 rows fill 1/16 to 4/16 of an MFMA tile, and on masks of few
+    if (batch.algorithm != 2 && !batch.row_parts) {
+        const int tile = sddmm_tile_choice(m_vec, k, n, nonzeros_vec, vec_length, batch.count);
+        if (tile > 0)
+            return launch_sddmm_tile<OutT>(tile, m_vec, k, n, row_offsets, col_indices, lhs, rhs, out, vec_length, stream, batch);
+    }
+    // algorithm 0 (automatic): vectors of 1 to 8 rows fill 1/16 to 8/16 of an MFMA tile, and on masks of few
     // nonzeros the fine-grained kernel (dot products on the vector ALU, reduced across lanes with DPP) is ahead:
     // over the M = N = 512..4096, K = 64..256 grid by 5-40 % below these nonzero counts, behind above them.
-    if (batch.algorithm == 0 && vec_length <= 4 && !batch.row_parts) {
+    if (batch.algorithm == 0 && !batch.row_parts) {
         const long long total = (long long)nonzeros_vec * batch.count;
         long long limit = 0;
         if (vec_length == 1) limit = 800000;
         else if (vec_length == 2) limit = k >= 256 ? 200000 : (k >= 128 ? 16000 : 0);
-        else limit = k >= 256 ? 16000 : (k >= 128 ? 8000 : 0);
+        else if (vec_length == 4) limit = k > 256 ? 40000 : (k >= 256 ? 16000 : (k >= 128 ? 8000 : 0));
+        else limit = k > 256 ? 12000 : 0;
         if (total <= limit)
             return launch_sddmm_valu<OutT>(m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices, lhs, rhs, out,
                                            vec_length, stream, batch);

@@ -231,10 +231,12 @@ int launch_sddmm_valu(int m_vec, int k, int n, int nonzeros_vec, const int *row_
                       const int *row_offsets, const int *col_indices, const half_t *lhs,
                       const half_t *rhs, OutT *out, int vec_length, hipStream_t stream, const Batch &batch)
 {
-    (void)n;
     if (m_vec == 0 || nonzeros_vec == 0 || batch.count == 0) return hipSuccess;
     if (batch.count > 65535) return hipErrorNotSupported;
     if (k <= 0) return hipErrorNotSupported;
+    const int tile = sddmm_tile_choice(m_vec, k, n, nonzeros_vec, vec_length, batch.count);
+    if (tile > 0)
+        return launch_sddmm_tile<OutT>(tile, m_vec, k, n, row_offsets, col_indices, lhs, rhs, out, vec_length, stream, batch);
     switch (vec_length) {
     case 1: return launch_shape<1, OutT>(m_vec, k, nonzeros_vec, row_indices, row_offsets, col_indices, lhs, rhs, out, stream, batch);
     case 2: return launch_shape<2, OutT>(m_vec, k, nonzeros_vec, row_indices, row_offsets, col_indices, lhs, rhs, out, stream, batch);

@@ -226,6 +226,7 @@ struct Options {
     int sddmm_slots = 0;
     int sddmm_block_waves = 0;
     int sddmm_group = 0;        // MFMA SDDMM: 16-vector groups per wave step (1, 2, 4), 0 = automatic
+    int sddmm_tile = 0;         // SDDMM on dense tiles: 1 = never, 2 = 64 x 64 tiles, 3 = 128 x 128 tiles, 0 = automatic
     int sddmm_flat_supers = 0;  // flat MFMA SDDMM (algorithm 2): super-groups per wave, 0 = automatic
     int attention_waves = 0;
     int attention_chunk = 0;
@@ -301,6 +302,14 @@ int launch_sddmm_valu(int m_vec, int k, int n, int nonzeros_vec, const int *row_
                       const int *row_offsets, const int *col_indices, const half_t *lhs,
                       const half_t *rhs, OutT *out, int vec_length, hipStream_t stream,
                       const Batch &batch = Batch());
+
+// SDDMM on dense tiles (csrc/sddmm_tile.hip), k % 8 == 0.  sddmm_tile_choice: 0 = the gathering kernels are expected
+// to be faster, else the `shape` for launch_sddmm_tile (1 = tiles of 64 x 64, 2 = of 128 x 128).
+int sddmm_tile_choice(int m_vec, int k, int n, long long nonzeros_vec, int vec_length, int batch);
+template <typename OutT>
+int launch_sddmm_tile(int shape, int m_vec, int k, int n, const int *row_offsets, const int *col_indices,
+                      const half_t *lhs, const half_t *rhs, OutT *out, int vec_length, hipStream_t stream,
+                      const Batch &batch);
 
 // Writes `bytes` zero bytes to each of `batch` buffers `stride_bytes` apart (a kernel, not a memset node, so that
 // callers may capture the call into a HIP graph).

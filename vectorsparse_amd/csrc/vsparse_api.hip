@@ -771,6 +771,9 @@ static int set_option_field(vs::Options &o, const char *name, int value)
         o.spmm_flat_waves = value;
     } else if (std::strcmp(name, "sddmm_slots") == 0) {
         o.sddmm_slots = value;
+    } else if (std::strcmp(name, "sddmm_tile") == 0) {
+        if (value > 3) return VS_ERROR_INVALID_VALUE;
+        o.sddmm_tile = value;
     } else if (std::strcmp(name, "sddmm_flat_supers") == 0) {
         if (value > 16) return VS_ERROR_INVALID_VALUE;
         o.sddmm_flat_supers = value;
