@@ -26,8 +26,8 @@ namespace vs {
 // SOFTMAX: the sparse values are raw scores and the kernel multiplies by softmax_row(scale * values)
 // instead: a pre-pass finds each scalar row's maximum, the staging step turns every score into
 // exp2(s*x - max) (and sums them), and the accumulated tile is divided by the row sum at the end.
-// RAGGED: the dense width is not a multiple of CPL (rows of the dense operand and of the output start at any 2-byte
-// boundary, the last chunk of a row is cut): chunks are fetched and stored half by half.
+// RAGGED: the dense width is not a multiple of CPL: rows of the dense operand and of the output start at any 2-byte
+// boundary and the last chunk of a row is moved back to end with it (load_ragged).
 // S: 32-vector steps a wave keeps in flight at once (1, 2 or 4): its unit of work is a block of S steps whose 8 * S
 // row segments per lane are all requested before the first MFMA.
 // TEAMS: rows ordered by length; only the first team_slots entries of row_indices get the workgroup's waves as a
@@ -115,10 +115,12 @@ spmm_mfma_kernel(int n_cols, int n_tiles, int shape, const int *__restrict__ row
     }
     const int cs = lane & 15;
     const int g = lane >> 4;
-    const int col0 = tile * TN + cs * CPL;
-    const bool col_ok = col0 < n_cols;  // n_cols % CPL == 0 unless RAGGED: a lane's chunk is all in or all out
+    int col0 = tile * TN + cs * CPL;
+    if constexpr (RAGGED) col0 = whole_chunk_column<CPL>(col0, n_cols);
+    const bool col_ok = col0 < n_cols;  // a lane's chunk is all in or all out (RAGGED: unless the width is below CPL)
     const uint32_t col_off = col_ok ? col0 : 0;
-    const int valid = !col_ok ? 0 : (n_cols - col0 < CPL ? n_cols - col0 : CPL);  // RAGGED: halves of the chunk that exist
+    const bool whole = n_cols >= CPL;   // RAGGED
+    const int valid = whole ? CPL : (col_ok ? n_cols - col0 : 0);
 
     int *idx_s = reinterpret_cast<int *>(smem + (size_t)slot_wave * kStage);
     half_t *vec_s = reinterpret_cast<half_t *>(idx_s + kBlock);  // [V][kBlock]
@@ -344,7 +346,7 @@ spmm_mfma_kernel(int n_cols, int n_tiles, int shape, const int *__restrict__ row
         if constexpr (S == 1) {
             spmm_mfma_step<V, CPL, IDX32, RAGGED>(idx_s, vec_s, rhs, n_cols, col_off, cs, g, acc, [&] {
                 if (base + stride < end) fetch(base + stride);
-            }, valid);
+            }, valid, whole);
         } else {
             // A block that the row fills only in part still requests all its steps (the padding repeats one row
             // segment, which stays in the L1): asking for fewer steps behind a uniform branch measured 5 % slower
@@ -408,7 +410,8 @@ spmm_mfma_kernel(int n_cols, int n_tiles, int shape, const int *__restrict__ row
     if (t < V * 16) {
         const int v = t >> 4;
         const int cs2 = t & 15;
-        const int col = tile * TN + cs2 * CPL;
+        int col = tile * TN + cs2 * CPL;
+        if constexpr (RAGGED) col = whole_chunk_column<CPL>(col, n_cols);
         if (col < n_cols) {
             float sum[CPL];
 #pragma unroll
@@ -525,7 +528,7 @@ static int launch_idx(int m_vec, int k, int n, int waves, const int *row_indices
     return (int)hipGetLastError();
 }
 
-// Dense widths that are not a multiple of 4: the half-by-half variant of the 64-column-tile kernel.
+// Dense widths that are not a multiple of 4: the variant of the 64-column-tile kernel without alignment.
 template <int V, typename OutT>
 static int launch_ragged(int m_vec, int k, int waves, const int *row_indices, const int *row_offsets,
                          const int *column_indices, const half_t *values, const half_t *rhs, OutT *out,
@@ -771,7 +774,9 @@ SpmmShape choose_spmm_shape(bool softmax, int m_vec, int vec_length, int k, int 
                 if (waves < for_longest) waves = for_longest;
             }
         } else {
-            const int max_useful = next_pow2(ceil_div(n > 0 ? n : 1, kStep));  // a row holds at most n vectors
+            // a wave takes two steps before another joins, and the rows are taken to hold half of n at most (511 rows x
+            // 147 at 70 %, N = 205, V = 2: four waves 4.2 us, two 3.9 us)
+            const int max_useful = next_pow2(ceil_div(n > 0 ? n : 1, 4 * kStep));
             if (waves > max_useful) waves = max_useful;
             // On a full chip a second wave per row pays from about ten steps per row (see above); the row
             // lengths are unknown here, so they are taken to be a tenth of n (90 % sparsity).

@@ -52,8 +52,8 @@ __device__ __forceinline__ float sum_over_groups(float x)
     return x;
 }
 
-// RAGGED: the dense width is not a multiple of 8 (rows of the dense operand and of the output start at any 2-byte
-// boundary, the last chunk of a row is cut): chunks are fetched and stored half by half.
+// RAGGED: the dense width is not a multiple of 8: rows of the dense operand and of the output start at any 2-byte
+// boundary and the last chunk of a row is moved back to end with it (load_ragged).
 // The second launch bound (waves per SIMD) is there for the launches of short rows: left to itself the compiler takes
 // 86 (V = 1) and 102 (V = 2) registers where 60 and 72 do without a spill, and a launch of short rows - waves that live for
 // one chain of round trips, three in four of them ending at once - then needs two rounds to seat its waves where one
@@ -128,10 +128,12 @@ spmm_valu_kernel(int n_cols, int n_tiles, int n_waves, uint32_t inv_waves, const
     if (wave >= alive_waves) return;
     const int cl = lane % LR;
     const int g = lane / LR;
-    const int col0 = tile * TN + cl * 8;
-    const bool col_ok = col0 < n_cols;  // n_cols % 8 == 0 unless RAGGED
+    int col0 = tile * TN + cl * 8;
+    if constexpr (RAGGED) col0 = whole_chunk_column<8>(col0, n_cols);
+    const bool col_ok = col0 < n_cols;
     const half_t *rhs_col = rhs + (col_ok ? col0 : 0);
-    const int valid = !col_ok ? 0 : (n_cols - col0 < 8 ? n_cols - col0 : 8);  // RAGGED: halves of the chunk that exist
+    const bool whole = n_cols >= 8;  // RAGGED
+    const int valid = whole ? 8 : (col_ok ? n_cols - col0 : 0);
 
     float acc[V][8];
 #pragma unroll
@@ -176,7 +178,7 @@ spmm_valu_kernel(int n_cols, int n_tiles, int n_waves, uint32_t inv_waves, const
         for (int u = 0; u < N; ++u) {
             if constexpr (RAGGED) {
                 RowChunk<8> chunk;
-                load_ragged<8>(chunk, rhs_col + (size_t)col[u] * n_cols, valid);
+                load_ragged<8>(chunk, rhs_col + (size_t)col[u] * n_cols, valid, whole);
                 b[u] = chunk.d;
             } else {
                 b[u] = *reinterpret_cast<const uint4_t *>(rhs_col + (size_t)col[u] * n_cols);
@@ -255,7 +257,8 @@ spmm_valu_kernel(int n_cols, int n_tiles, int n_waves, uint32_t inv_waves, const
     for (int item = threadIdx.x; item < V * LR; item += 64 * alive_waves) {
         const int v = item / LR;
         const int cl2 = item % LR;
-        const int col = tile * TN + cl2 * 8;
+        int col = tile * TN + cl2 * 8;
+        if constexpr (RAGGED) col = whole_chunk_column<8>(col, n_cols);
         if (col >= n_cols) continue;
         float sum[8];
 #pragma unroll
