@@ -19,6 +19,7 @@ SOURCES = ["vsparse_api.hip", "spmm_mfma.hip", "spmm_mfma_flat.hip", "spmm_mfma_
 RETIRED = os.environ.get("VS_RETIRED_VARIANTS") == "1"
 if RETIRED:
     SOURCES.append("spmm_mfma_dma.hip")
+BINDING_PATH = os.path.join(_HERE, "_binding.so")
 PROBE_PATH = os.path.join(_HERE, "libvsprobe.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -43,7 +44,7 @@ def _run(cmd, verbose):
     noise = "is not a recognized feature for this target"
     out = "\n".join(l for l in proc.stdout.splitlines() if noise not in l)
     if proc.returncode != 0:
-        raise RuntimeError("hipcc failed:\n" + out)
+        raise RuntimeError("compilation failed:\n" + out)
     if verbose and out.strip():
         print(out)
 
@@ -70,7 +71,25 @@ def build(verbose=False, jobs=None, incremental=False):
         list(pool.map(lambda c: _run(c, verbose), cmds))
     _run([HIPCC, "--offload-arch=gfx950", "-fPIC", "-shared", "-Wl,--version-script=" + os.path.join(CSRC, "exports.map"),
           "-o", LIB_PATH] + objects, verbose)
+    build_binding(verbose)
     return LIB_PATH
+
+
+def build_binding(verbose=False):
+    """Compile csrc/binding.cpp (the calls of ops.py from Python tensors to the C ABI) to _binding.so: host code only,
+    against the torch of this interpreter, whose libraries are in the process when it is loaded."""
+    import sysconfig
+    import torch
+    from torch.utils import cpp_extension
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
+           "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch.compiled_with_cxx11_abi())]
+    cmd += ["-I" + path for path in cpp_extension.include_paths("cuda") + [sysconfig.get_paths()["include"]]]
+    cmd += [os.path.join(CSRC, "binding.cpp"), "-o", BINDING_PATH, "-L" + _HERE, "-lvsparse", "-Wl,-rpath,$ORIGIN"]
+    cmd += ["-L" + path for path in cpp_extension.library_paths("cuda")[:1]]
+    cmd += ["-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"]
+    _run(cmd, verbose)
+    return BINDING_PATH
 
 
 def build_probe(verbose=False):

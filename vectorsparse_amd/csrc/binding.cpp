@@ -1,0 +1,382 @@
+// The calls a program makes every step, from Python to the C ABI without ctypes: checks the tensors, takes their
+// addresses and the current stream, calls the library.  Every function returns the library's status, or -1 when an
+// argument is not the ordinary one (a raw address, a tensor of another type, a layout or placement the operator does not
+// take, no tensor at all): ops.py then goes its own way, which takes the unusual arguments and words the errors.
+//
+// What it is for: a small SpMM takes 2.4 us on the GPU and 3.3 us of launch in the HIP runtime; the same call took 6.0 us
+// on the host with ctypes (a Python check per operand, 0.24 us each, the current stream 0.34 us, the conversion of eleven
+// arguments 0.6 us), and 15 to 29 us for the attention layer, whose checks index every operand.
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include "../../include/vsparse.h"
+
+namespace {
+
+constexpr long kUnusual = -1;
+
+// Reads positional arguments in order; the first unusual one clears `ok` and everything after it reads as zero.
+struct Reader {
+    PyObject *const *args;
+    Py_ssize_t left;
+    bool ok = true;
+
+    Reader(PyObject *const *a, Py_ssize_t n) : args(a), left(n) {}
+
+    PyObject *next()
+    {
+        if (!ok || left <= 0) {
+            ok = false;
+            return nullptr;
+        }
+        --left;
+        return *args++;
+    }
+    const at::Tensor *tensor()
+    {
+        PyObject *o = next();
+        if (!o || !THPVariable_Check(o)) {
+            ok = false;
+            return nullptr;
+        }
+        const at::Tensor &t = THPVariable_Unpack(o);
+        if (!t.is_cuda() || t.layout() != at::kStrided) {
+            ok = false;
+            return nullptr;
+        }
+        return &t;
+    }
+    int integer()
+    {
+        PyObject *o = next();
+        if (!o || !PyLong_CheckExact(o)) {
+            ok = false;
+            return 0;
+        }
+        int overflow = 0;
+        const long v = PyLong_AsLongAndOverflow(o, &overflow);
+        if (overflow || v < INT32_MIN || v > INT32_MAX) ok = false;
+        return (int)v;
+    }
+    float number()
+    {
+        PyObject *o = next();
+        if (!o || !PyFloat_CheckExact(o)) {
+            ok = false;
+            return 0.f;
+        }
+        return (float)PyFloat_AS_DOUBLE(o);
+    }
+    void *stream()  // None: torch's current stream of the current device
+    {
+        PyObject *o = next();
+        if (o == Py_None) return (void *)c10::hip::getCurrentHIPStream().stream();
+        if (o && PyLong_CheckExact(o)) return PyLong_AsVoidPtr(o);
+        ok = false;
+        return nullptr;
+    }
+    // a contiguous tensor of one type
+    void *operand(at::ScalarType type)
+    {
+        const at::Tensor *t = tensor();
+        if (!t || t->scalar_type() != type || !t->is_contiguous()) {
+            ok = false;
+            return nullptr;
+        }
+        return t->data_ptr();
+    }
+    void *indices() { return operand(at::kInt); }
+    void *halves() { return operand(at::kHalf); }
+    // halves or floats
+    void *output(bool &f32)
+    {
+        const at::Tensor *t = tensor();
+        if (!t || (t->scalar_type() != at::kHalf && t->scalar_type() != at::kFloat) || !t->is_contiguous()) {
+            ok = false;
+            return nullptr;
+        }
+        f32 = t->scalar_type() == at::kFloat;
+        return t->data_ptr();
+    }
+    // [batch, rows, columns] (or two-dimensional: shared), contiguous behind the first dimension; `batch` of one or a
+    // shared operand has no stride
+    void *batched(int batch, long long &stride)
+    {
+        const at::Tensor *t = tensor();
+        stride = 0;
+        if (!t || t->scalar_type() != at::kHalf) {
+            ok = false;
+            return nullptr;
+        }
+        if (t->dim() == 3) {
+            const auto sizes = t->sizes(), strides = t->strides();
+            const bool whole = sizes[1] == 0 || sizes[2] == 0 ||
+                               ((sizes[2] == 1 || strides[2] == 1) && (sizes[1] == 1 || strides[1] == sizes[2]));
+            if (!whole || sizes[0] == 0) ok = false;
+            if (batch != 1) stride = strides[0];
+        } else if (!t->is_contiguous()) {
+            ok = false;
+        }
+        return t->data_ptr();
+    }
+    // bytes of a caller's buffer, or None
+    void *buffer(long long &bytes)
+    {
+        bytes = 0;
+        if (ok && left > 0 && *args == Py_None) {
+            next();
+            return nullptr;
+        }
+        const at::Tensor *t = tensor();
+        if (!t) return nullptr;
+        bytes = (long long)t->numel() * (long long)t->element_size();
+        return t->data_ptr();
+    }
+    bool done() const { return ok && left == 0; }
+};
+
+template <typename Call>
+PyObject *status_of(const Reader &r, Call &&call)
+{
+    if (!r.done()) return PyLong_FromLong(kUnusual);
+    int status;
+    Py_BEGIN_ALLOW_THREADS;
+    status = call();
+    Py_END_ALLOW_THREADS;
+    return PyLong_FromLong(status);
+}
+
+typedef int (*SpmmEntry)(int, int, int, int, const int *, const int *, const int *, const void *, const void *, void *, void *);
+typedef int (*SpmmEntryF32)(int, int, int, int, const int *, const int *, const int *, const void *, const void *, float *, void *);
+
+// (m_vec, vec_length, k, n, row_indices, row_offsets, column_indices, values, rhs, out, stream)
+template <SpmmEntry F16, SpmmEntryF32 F32>
+PyObject *spmm(PyObject *, PyObject *const *args, Py_ssize_t n_args)
+{
+    Reader r(args, n_args);
+    const int m_vec = r.integer(), v = r.integer(), k = r.integer(), n = r.integer();
+    const int *ri = (const int *)r.indices(), *ro = (const int *)r.indices(), *ci = (const int *)r.indices();
+    const void *values = r.halves(), *rhs = r.halves();
+    bool f32 = false;
+    void *out = r.output(f32), *stream = r.stream();
+    return status_of(r, [&] {
+        return f32 ? F32(m_vec, v, k, n, ri, ro, ci, values, rhs, (float *)out, stream)
+                   : F16(m_vec, v, k, n, ri, ro, ci, values, rhs, out, stream);
+    });
+}
+
+// (m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices, lhs, rhs, out, vec_length, stream, algorithm)
+PyObject *wmma_sddmm(PyObject *, PyObject *const *args, Py_ssize_t n_args)
+{
+    Reader r(args, n_args);
+    const int m_vec = r.integer(), k = r.integer(), n = r.integer(), nnz = r.integer();
+    const int *ri = (const int *)r.indices(), *ro = (const int *)r.indices(), *ci = (const int *)r.indices();
+    const void *lhs = r.halves(), *rhs = r.halves();
+    bool f32 = false;
+    void *out = r.output(f32);
+    const int v = r.integer();
+    void *stream = r.stream();
+    const int algorithm = r.integer();
+    return status_of(r, [&] {
+        return f32 ? vs_wmma_sddmm_f16_f32out(m_vec, k, n, nnz, ri, ro, ci, lhs, rhs, (float *)out, v, stream, algorithm)
+                   : vs_wmma_sddmm_f16(m_vec, k, n, nnz, ri, ro, ci, lhs, rhs, out, v, stream, algorithm);
+    });
+}
+
+// (m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices, lhs, rhs, out, vec_length, stream)
+PyObject *cuda_sddmm(PyObject *, PyObject *const *args, Py_ssize_t n_args)
+{
+    Reader r(args, n_args);
+    const int m_vec = r.integer(), k = r.integer(), n = r.integer(), nnz = r.integer();
+    const int *ri = (const int *)r.indices(), *ro = (const int *)r.indices(), *ci = (const int *)r.indices();
+    const void *lhs = r.halves(), *rhs = r.halves();
+    bool f32 = false;
+    void *out = r.output(f32);
+    const int v = r.integer();
+    void *stream = r.stream();
+    return status_of(r, [&] {
+        return f32 ? vs_cuda_sddmm_f16_f32out(m_vec, k, n, nnz, ri, ro, ci, lhs, rhs, (float *)out, v, stream)
+                   : vs_cuda_sddmm_f16(m_vec, k, n, nnz, ri, ro, ci, lhs, rhs, out, v, stream);
+    });
+}
+
+// (batch, m_vec, vec_length, k, n, nonzeros_vec, longest_row_vec, long_rows, row_indices, row_offsets, column_indices, values,
+// rhs, out, stream); MFMA path, long_rows < 0: not known
+PyObject *wmma_spmm_batched(PyObject *, PyObject *const *args, Py_ssize_t n_args)
+{
+    Reader r(args, n_args);
+    const int batch = r.integer(), m_vec = r.integer(), v = r.integer(), k = r.integer(), n = r.integer();
+    const int nnz = r.integer(), longest = r.integer(), long_rows = r.integer();
+    const int *ri = (const int *)r.indices(), *ro = (const int *)r.indices(), *ci = (const int *)r.indices();
+    long long sa, sb, so;
+    const void *values = r.batched(batch, sa), *rhs = r.batched(batch, sb);
+    void *out = r.batched(batch, so), *stream = r.stream();
+    return status_of(r, [&] {
+        return long_rows >= 0
+                   ? vs_wmma_spmm_f16_batched_sorted(batch, m_vec, v, k, n, nnz, longest, long_rows, ri, ro, ci, values, sa, rhs, sb, out, so, stream)
+                   : vs_wmma_spmm_f16_batched(batch, m_vec, v, k, n, nnz, longest, ri, ro, ci, values, sa, rhs, sb, out, so, stream);
+    });
+}
+
+// (batch, m_vec, vec_length, k, n, nonzeros_vec, longest_row_vec, row_indices, row_offsets, column_indices, values, rhs, out,
+// stream); fine-grained path
+PyObject *cuda_spmm_batched(PyObject *, PyObject *const *args, Py_ssize_t n_args)
+{
+    Reader r(args, n_args);
+    const int batch = r.integer(), m_vec = r.integer(), v = r.integer(), k = r.integer(), n = r.integer();
+    const int nnz = r.integer(), longest = r.integer();
+    const int *ri = (const int *)r.indices(), *ro = (const int *)r.indices(), *ci = (const int *)r.indices();
+    long long sa, sb, so;
+    const void *values = r.batched(batch, sa), *rhs = r.batched(batch, sb);
+    void *out = r.batched(batch, so), *stream = r.stream();
+    return status_of(r, [&] {
+        return vs_cuda_spmm_f16_batched(batch, m_vec, v, k, n, nnz, longest, ri, ro, ci, values, sa, rhs, sb, out, so, stream);
+    });
+}
+
+// (batch, m_vec, vec_length, k, n, nonzeros_vec, longest_row_vec, row_indices, row_offsets, column_indices, scores, rhs, out,
+// scale, stream)
+PyObject *spmm_softmax_batched(PyObject *, PyObject *const *args, Py_ssize_t n_args)
+{
+    Reader r(args, n_args);
+    const int batch = r.integer(), m_vec = r.integer(), v = r.integer(), k = r.integer(), n = r.integer();
+    const int nnz = r.integer(), longest = r.integer();
+    const int *ri = (const int *)r.indices(), *ro = (const int *)r.indices(), *ci = (const int *)r.indices();
+    long long sa, sb, so;
+    const void *scores = r.batched(batch, sa), *rhs = r.batched(batch, sb);
+    void *out = r.batched(batch, so);
+    const float scale = r.number();
+    void *stream = r.stream();
+    return status_of(r, [&] {
+        return vs_wmma_spmm_softmax_f16_batched(batch, m_vec, v, k, n, nnz, longest, ri, ro, ci, scores, sa, rhs, sb, out, so, scale, stream);
+    });
+}
+
+// (batch, m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices, lhs, rhs, out, vec_length, stream, algorithm);
+// algorithm < 0: the fine-grained path
+PyObject *sddmm_batched(PyObject *, PyObject *const *args, Py_ssize_t n_args)
+{
+    Reader r(args, n_args);
+    const int batch = r.integer(), m_vec = r.integer(), k = r.integer(), n = r.integer(), nnz = r.integer();
+    const int *ri = (const int *)r.indices(), *ro = (const int *)r.indices(), *ci = (const int *)r.indices();
+    long long sa, sb, so;
+    const void *lhs = r.batched(batch, sa), *rhs = r.batched(batch, sb);
+    void *out = r.batched(batch, so);
+    const int v = r.integer();
+    void *stream = r.stream();
+    const int algorithm = r.integer();
+    return status_of(r, [&] {
+        return algorithm < 0 ? vs_cuda_sddmm_f16_batched(batch, m_vec, k, n, nnz, ri, ro, ci, lhs, sa, rhs, sb, out, so, v, stream)
+                             : vs_wmma_sddmm_f16_batched(batch, m_vec, k, n, nnz, ri, ro, ci, lhs, sa, rhs, sb, out, so, v, stream, algorithm);
+    });
+}
+
+// (batch, m_vec, vec_length, row_indices, row_offsets, values_in, values_out, scale, stream)
+PyObject *sparse_softmax(PyObject *, PyObject *const *args, Py_ssize_t n_args)
+{
+    Reader r(args, n_args);
+    const int batch = r.integer(), m_vec = r.integer(), v = r.integer();
+    const int *ri = (const int *)r.indices(), *ro = (const int *)r.indices();
+    long long si, so;
+    const void *in = r.batched(batch, si);
+    void *out = r.batched(batch, so);
+    const float scale = r.number();
+    void *stream = r.stream();
+    return status_of(r, [&] { return vs_sparse_softmax_f16(batch, m_vec, v, ri, ro, in, si, out, so, scale, stream); });
+}
+
+// (batch, m_vec, vec_length, n, d_qk, d_v, row_indices, row_offsets, col_indices, q, k, v, out, scale, rows_per_workgroup, plan,
+// stream)
+PyObject *sparse_attention(PyObject *, PyObject *const *args, Py_ssize_t n_args)
+{
+    Reader r(args, n_args);
+    const int batch = r.integer(), m_vec = r.integer(), vec = r.integer(), n = r.integer(), d_qk = r.integer(), d_v = r.integer();
+    const int *ri = (const int *)r.indices(), *ro = (const int *)r.indices(), *ci = (const int *)r.indices();
+    long long sq, sk, sv, so, plan_bytes;
+    const void *q = r.batched(batch, sq), *k = r.batched(batch, sk), *v = r.batched(batch, sv);
+    void *out = r.batched(batch, so);
+    const float scale = r.number();
+    const int rows = r.integer();
+    const void *plan = r.buffer(plan_bytes);
+    void *stream = r.stream();
+    return status_of(r, [&] {
+        return vs_sparse_attention_f16(batch, m_vec, vec, n, d_qk, d_v, ri, ro, ci, q, sq, k, sk, v, sv, out, so, scale, rows, plan,
+                                       plan_bytes, stream);
+    });
+}
+
+// (batch, vec_length, k, n, n_slots, slots, n_split, parts_max, nonzeros_vec, longest_part_vec, column_indices, values, rhs, out,
+// workspace, stream)
+PyObject *spmm_row_parts(PyObject *, PyObject *const *args, Py_ssize_t n_args)
+{
+    Reader r(args, n_args);
+    const int batch = r.integer(), vec = r.integer(), k = r.integer(), n = r.integer(), n_slots = r.integer();
+    const int *slots = (const int *)r.indices();
+    const int n_split = r.integer(), parts_max = r.integer(), nnz = r.integer(), longest = r.integer();
+    const int *ci = (const int *)r.indices();
+    long long sa, sb, so, ws_bytes;
+    const void *values = r.batched(batch, sa), *rhs = r.batched(batch, sb);
+    void *out = r.batched(batch, so), *ws = r.buffer(ws_bytes), *stream = r.stream();
+    return status_of(r, [&] {
+        return vs_wmma_spmm_f16_row_parts(batch, vec, k, n, n_slots, slots, n_split, parts_max, nnz, longest, ci, values, sa, rhs, sb,
+                                          out, so, ws, ws_bytes, stream);
+    });
+}
+
+// (batch, k, n, n_slots, slots, nonzeros_vec, col_indices, lhs, rhs, out, vec_length, stream)
+PyObject *sddmm_row_parts(PyObject *, PyObject *const *args, Py_ssize_t n_args)
+{
+    Reader r(args, n_args);
+    const int batch = r.integer(), k = r.integer(), n = r.integer(), n_slots = r.integer();
+    const int *slots = (const int *)r.indices();
+    const int nnz = r.integer();
+    const int *ci = (const int *)r.indices();
+    long long sa, sb, so;
+    const void *lhs = r.batched(batch, sa), *rhs = r.batched(batch, sb);
+    void *out = r.batched(batch, so);
+    const int vec = r.integer();
+    void *stream = r.stream();
+    return status_of(r, [&] {
+        return vs_wmma_sddmm_f16_row_parts(batch, k, n, n_slots, slots, nnz, ci, lhs, sa, rhs, sb, out, so, vec, stream);
+    });
+}
+
+// (batch, vec_length, n_slots, slots, n_split, parts_max, values_in, values_out, scale, workspace, stream)
+PyObject *softmax_row_parts(PyObject *, PyObject *const *args, Py_ssize_t n_args)
+{
+    Reader r(args, n_args);
+    const int batch = r.integer(), vec = r.integer(), n_slots = r.integer();
+    const int *slots = (const int *)r.indices();
+    const int n_split = r.integer(), parts_max = r.integer();
+    long long si, so, ws_bytes;
+    const void *in = r.batched(batch, si);
+    void *out = r.batched(batch, so);
+    const float scale = r.number();
+    void *ws = r.buffer(ws_bytes), *stream = r.stream();
+    return status_of(r, [&] {
+        return vs_sparse_softmax_f16_row_parts(batch, vec, n_slots, slots, n_split, parts_max, in, si, out, so, scale, ws, ws_bytes, stream);
+    });
+}
+
+#define VS_METHOD(name, fn) {name, (PyCFunction)(void (*)(void))(fn), METH_FASTCALL, nullptr}
+PyMethodDef methods[] = {
+    VS_METHOD("wmma_spmm", (&spmm<vs_wmma_spmm_f16, vs_wmma_spmm_f16_f32out>)),
+    VS_METHOD("cuda_spmm", (&spmm<vs_cuda_spmm_f16, vs_cuda_spmm_f16_f32out>)),
+    VS_METHOD("wmma_sddmm", wmma_sddmm),
+    VS_METHOD("cuda_sddmm", cuda_sddmm),
+    VS_METHOD("wmma_spmm_batched", wmma_spmm_batched),
+    VS_METHOD("cuda_spmm_batched", cuda_spmm_batched),
+    VS_METHOD("spmm_softmax_batched", spmm_softmax_batched),
+    VS_METHOD("sddmm_batched", sddmm_batched),
+    VS_METHOD("sparse_softmax", sparse_softmax),
+    VS_METHOD("sparse_attention", sparse_attention),
+    VS_METHOD("spmm_row_parts", spmm_row_parts),
+    VS_METHOD("sddmm_row_parts", sddmm_row_parts),
+    VS_METHOD("softmax_row_parts", softmax_row_parts),
+    {nullptr, nullptr, 0, nullptr}};
+
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_binding", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__binding() { return PyModule_Create(&module); }

@@ -16,6 +16,24 @@ import torch
 from . import _lib
 
 
+class _Unloaded:
+    """Stands for the compiled binding (csrc/binding.cpp) until its first use, which loads it behind the library; a
+    missing file is an error."""
+
+    def __getattr__(self, name):
+        global _native
+        _lib.lib()
+        from . import _binding
+        _native = _binding
+        return getattr(_binding, name)
+
+
+# The operators call `_native` first: it checks the tensors, takes their addresses and the current stream and calls the
+# C ABI in one step.  It answers with the library's status, or with a negative number for arguments that are not the
+# ordinary ones (raw addresses, layouts and types that are refused): those go through the checks of this file.
+_native = _Unloaded()
+
+
 def _ptr(t):
     if t is None:
         return None
@@ -89,6 +107,12 @@ class spmm:
     def wmmaSpmm(m_vec, vec_length, k, n, row_indices, row_offsets, column_indices, values, rhs_matrix,
                  output_matrix, stream=None):
         """MFMA path (reference: tensor-core path, src/wmma_spmm.cu:400-409)."""
+        st = _native.wmma_spmm(m_vec, vec_length, k, n, row_indices, row_offsets, column_indices, values, rhs_matrix,
+                               output_matrix, stream)
+        if st == 0:
+            return output_matrix
+        if st > 0:
+            _lib.check(st, "vs_wmma_spmm_f16")
         return _spmm("vs_wmma_spmm_f16", m_vec, vec_length, k, n, row_indices, row_offsets, column_indices,
                      values, rhs_matrix, output_matrix, stream)
 
@@ -96,6 +120,12 @@ class spmm:
     def cudaSpmm(m_vec, vec_length, k, n, row_indices, row_offsets, column_indices, values, rhs_matrix,
                  output_matrix, stream=None):
         """Fine-grained packed-fp16 VALU path (reference: src/cuda_spmm.cu:316-325)."""
+        st = _native.cuda_spmm(m_vec, vec_length, k, n, row_indices, row_offsets, column_indices, values, rhs_matrix,
+                               output_matrix, stream)
+        if st == 0:
+            return output_matrix
+        if st > 0:
+            _lib.check(st, "vs_cuda_spmm_f16")
         return _spmm("vs_cuda_spmm_f16", m_vec, vec_length, k, n, row_indices, row_offsets, column_indices,
                      values, rhs_matrix, output_matrix, stream)
 
@@ -170,6 +200,12 @@ class sddmm:
     def wmmaSddmm(m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices, lhs_matrix, rhs_matrix,
                   output_values, vec_length, stream=None, algorithm=1):
         """MFMA path (reference: src/wmma_sddmm.cu:3190-3202)."""
+        st = _native.wmma_sddmm(m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices, lhs_matrix,
+                                rhs_matrix, output_values, vec_length, stream, algorithm)
+        if st == 0:
+            return output_values
+        if st > 0:
+            _lib.check(st, "vs_wmma_sddmm_f16")
         return _sddmm("vs_wmma_sddmm_f16", m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices,
                       lhs_matrix, rhs_matrix, output_values, vec_length, stream, algorithm)
 
@@ -177,6 +213,12 @@ class sddmm:
     def cudaSddmm(m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices, lhs_matrix, rhs_matrix,
                   output_values, vec_length, stream=None):
         """Cross-lane dot-product path (reference: src/cuda_sddmm.cu:1295-1331)."""
+        st = _native.cuda_sddmm(m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices, lhs_matrix,
+                                rhs_matrix, output_values, vec_length, stream)
+        if st == 0:
+            return output_values
+        if st > 0:
+            _lib.check(st, "vs_cuda_sddmm_f16")
         return _sddmm("vs_cuda_sddmm_f16", m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices,
                       lhs_matrix, rhs_matrix, output_values, vec_length, stream)
 
@@ -198,6 +240,15 @@ def spmm_batched(m_vec, vec_length, k, n, row_indices, row_offsets, column_indic
     entries are the rows of more than LONG_ROW_VECTORS nonzero vectors (vs_wmma_spmm_f16_batched_sorted).
     """
     batch = output_matrix.shape[0]
+    if kernel == "wmma":
+        st = _native.wmma_spmm_batched(batch, m_vec, vec_length, k, n, nonzeros_vec, longest_row_vec, long_rows, row_indices,
+                                       row_offsets, column_indices, values, rhs_matrix, output_matrix, stream)
+    else:
+        st = _native.cuda_spmm_batched(batch, m_vec, vec_length, k, n, nonzeros_vec, longest_row_vec, row_indices,
+                                       row_offsets, column_indices, values, rhs_matrix, output_matrix, stream)
+    if st >= 0:
+        _lib.check(st, "vs_%s_spmm_f16_batched" % ("wmma" if kernel == "wmma" else "cuda"))
+        return output_matrix
     for t, nm in ((values, "values"), (rhs_matrix, "rhs_matrix"), (output_matrix, "output_matrix")):
         _expect_batched(t, torch.float16, nm)
     entry = "vs_wmma_spmm_f16_batched" if kernel == "wmma" else "vs_cuda_spmm_f16_batched"
@@ -219,6 +270,11 @@ def spmm_softmax_batched(m_vec, vec_length, k, n, row_indices, row_offsets, colu
     if output_matrix.dim() == 2:
         output_matrix = output_matrix.unsqueeze(0)
     batch = output_matrix.shape[0]
+    st = _native.spmm_softmax_batched(batch, m_vec, vec_length, k, n, nonzeros_vec, longest_row_vec, row_indices, row_offsets,
+                                      column_indices, scores, rhs_matrix, output_matrix, float(scale), stream)
+    if st >= 0:
+        _lib.check(st, "vs_wmma_spmm_softmax_f16_batched")
+        return output_matrix
     for t, nm in ((scores, "scores"), (rhs_matrix, "rhs_matrix"), (output_matrix, "output_matrix")):
         _expect_batched(t, torch.float16, nm)
     st = _lib.lib().vs_wmma_spmm_softmax_f16_batched(
@@ -248,6 +304,11 @@ def sparse_attention(m_vec, vec_length, n, row_indices, row_offsets, col_indices
         scale = 1.0 / float(d_qk) ** 0.5
     if out is None:
         out = torch.empty((heads, m, d_v), dtype=torch.float16, device=q.device)
+    st = _native.sparse_attention(heads, m_vec, vec_length, n, d_qk, d_v, row_indices, row_offsets, col_indices, q, k, v, out,
+                                  float(scale), rows_per_workgroup, plan, stream)
+    if st >= 0:
+        _lib.check(st, "vs_sparse_attention_f16")
+        return out
     for t, nm in ((q, "q"), (k, "k"), (v, "v"), (out, "out")):
         _expect_batched(t, torch.float16, nm)
     st = _lib.lib().vs_sparse_attention_f16(heads, m_vec, vec_length, n, d_qk, d_v, _ptr(row_indices),
@@ -267,6 +328,11 @@ def sddmm_batched(m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indic
     lhs_matrix: [batch, m, k], rhs_matrix: [batch, n, k], output_values: [batch, nnz_vec, V], fp16.
     """
     batch = output_values.shape[0]
+    st = _native.sddmm_batched(batch, m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices, lhs_matrix, rhs_matrix,
+                               output_values, vec_length, stream, algorithm if kernel == "wmma" else -1)
+    if st >= 0:
+        _lib.check(st, "vs_%s_sddmm_f16_batched" % ("wmma" if kernel == "wmma" else "cuda"))
+        return output_values
     for t, nm in ((lhs_matrix, "lhs_matrix"), (rhs_matrix, "rhs_matrix"), (output_values, "output_values")):
         _expect_batched(t, torch.float16, nm)
     args = [batch, m_vec, k, n, nonzeros_vec, _ptr(row_indices), _ptr(row_offsets), _ptr(col_indices),
@@ -286,9 +352,13 @@ def sparse_softmax(m_vec, vec_length, row_indices, row_offsets, values_in, value
     """Row-wise softmax(scale * x) over each scalar row's nonzeros, [nnz_vec, V] or [batch, nnz_vec, V]."""
     if values_out is None:
         values_out = torch.empty_like(values_in)
+    batch = values_in.shape[0] if values_in.dim() == 3 else 1
+    st = _native.sparse_softmax(batch, m_vec, vec_length, row_indices, row_offsets, values_in, values_out, float(scale), stream)
+    if st >= 0:
+        _lib.check(st, "vs_sparse_softmax_f16")
+        return values_out
     _expect_batched(values_in, torch.float16, "values_in")
     _expect_batched(values_out, torch.float16, "values_out")
-    batch = values_in.shape[0] if values_in.dim() == 3 else 1
     st = _lib.lib().vs_sparse_softmax_f16(batch, m_vec, vec_length, _ptr(row_indices), _ptr(row_offsets),
                                           _ptr(values_in), _stride(values_in, batch), _ptr(values_out),
                                           _stride(values_out, batch), float(scale), _stream(stream))
@@ -334,6 +404,7 @@ class SparseAttention:
         self.mask = mask
         self._plans = {}
         self._rows = {}
+        self._routes = {}
 
     def _parts_route_fits(self, d_v, heads):
         """The SpMM of the three-operator route on row parts takes less than 2 GiB of partial tiles (the limit of
@@ -341,6 +412,24 @@ class SparseAttention:
         parts = self.prob.row_parts(512)[0]
         return spmm_row_parts_workspace_bytes(self.prob.vec_length, d_v, parts.n_split, parts.parts_max,
                                               batch=heads) < 2 ** 31
+
+    def _route(self, d, d_v, heads):
+        """`forward`'s default on the MFMA path for these head widths and head count (a matter of sizes and of the mask:
+        decided once)."""
+        key = (d, d_v, heads)
+        route = self._routes.get(key)
+        if route is None:
+            p = self.prob
+            if (d % 8 == 0 and d_v % 4 == 0 and p.n * d_v < 2 ** 31 and p.row_parts(0)[0].n_split > 0
+                    and self._parts_route_fits(d_v, heads)):
+                # rows far longer than the rest - global tokens: the three operators on the dispatch list of row
+                # parts (16 heads x 4096, d = 64, a +-32..128 band with 64-256 global tokens: 72-119 us against
+                # 145-160 us in one launch and 280-295 us for SDDMM + softmax-fused SpMM on whole rows)
+                route = "parts"
+            else:
+                route = "layer" if self.union_rows(d, d_v, heads) >= 2 else True
+            self._routes[key] = route
+        return route
 
     def union_rows(self, d_qk, d_v, heads=16):
         """Rows per workgroup for the single-launch kernel with these head widths and head count (cached)."""
@@ -426,40 +515,31 @@ class SparseAttention:
         """
         p = self.prob
         heads, seq, d = q.shape
+        d_v = v.shape[2]
         if scale is None:
             scale = 1.0 / float(d) ** 0.5
+        if out is None:
+            out = torch.empty((heads, seq, d_v), dtype=torch.float16, device=q.device)
+        if fused is None:
+            fused = self._route(d, d_v, heads) if kernel == "wmma" else False
+        if fused == "layer":    # (keeps the scores to itself)
+            return sparse_attention(p.m_vec, p.vec_length, p.n, p.row_indices, p.row_offsets, p.column_indices,
+                                    q, k, v, out=out, scale=scale, stream=stream,
+                                    rows_per_workgroup=self.union_rows(d, d_v, heads), plan=self.plan(d, d_v, heads))
         if scores is None:
             scores = torch.empty((heads, p.nnz_vec, p.vec_length), dtype=torch.float16, device=q.device)
-        if out is None:
-            out = torch.empty((heads, seq, v.shape[2]), dtype=torch.float16, device=q.device)
-        if fused is None:
-            if kernel != "wmma":
-                fused = False
-            elif (d % 8 == 0 and v.shape[2] % 4 == 0 and p.n * v.shape[2] < 2 ** 31 and p.row_parts(0)[0].n_split > 0
-                  and self._parts_route_fits(v.shape[2], heads)):
-                # rows far longer than the rest - global tokens: the three operators on the dispatch list of row
-                # parts (16 heads x 4096, d = 64, a +-32..128 band with 64-256 global tokens: 72-119 us against
-                # 145-160 us in one launch and 280-295 us for SDDMM + softmax-fused SpMM on whole rows)
-                fused = "parts"
-            else:
-                fused = "layer" if self.union_rows(q.shape[2], v.shape[2], heads) >= 2 else True
         if fused == "parts":
             p.sddmm_row_parts(q, k, out=scores, stream=stream)
             p.softmax_row_parts(scores, scale=scale, stream=stream)
             return p.spmm_row_parts(v, out=out, stream=stream, limit_vec=512, values=scores)
-        if fused == "layer":
-            return sparse_attention(p.m_vec, p.vec_length, p.n, p.row_indices, p.row_offsets, p.column_indices,
-                                    q, k, v, out=out, scale=scale, stream=stream,
-                                    rows_per_workgroup=self.union_rows(q.shape[2], v.shape[2], heads),
-                                    plan=self.plan(q.shape[2], v.shape[2], heads))
         sddmm_batched(p.m_vec, d, p.n, p.nnz_vec, p.row_indices, p.row_offsets, p.column_indices, q, k, scores,
                       p.vec_length, kernel=kernel, stream=stream)
         if fused:
-            return spmm_softmax_batched(p.m_vec, p.vec_length, v.shape[2], p.n, p.row_indices, p.row_offsets,
+            return spmm_softmax_batched(p.m_vec, p.vec_length, d_v, p.n, p.row_indices, p.row_offsets,
                                         p.column_indices, scores, v, out, scale, stream=stream,
                                         nonzeros_vec=p.nnz_vec, longest_row_vec=p.longest_row_vec)
         sparse_softmax(p.m_vec, p.vec_length, p.row_indices, p.row_offsets, scores, scores, scale, stream=stream)
-        spmm_batched(p.m_vec, p.vec_length, v.shape[2], p.n, p.row_indices, p.row_offsets, p.column_indices,
+        spmm_batched(p.m_vec, p.vec_length, d_v, p.n, p.row_indices, p.row_offsets, p.column_indices,
                      scores, v, out, kernel=kernel, stream=stream, nonzeros_vec=p.nnz_vec,
                      longest_row_vec=p.longest_row_vec)
         return out
@@ -517,8 +597,13 @@ def spmm_row_parts(vec_length, k, n, parts, slots, nonzeros_vec, column_indices,
     its first use, or None when no row is split.  A leading batch dimension on output_matrix ([batch, m, k]) runs
     that many problems on the shared pattern; values / rhs_matrix with the same leading dimension are per problem,
     without it shared.  Returns output_matrix."""
-    ws_bytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
     batch = output_matrix.shape[0] if output_matrix.dim() == 3 else 1
+    st = _native.spmm_row_parts(batch, vec_length, k, n, parts.n_slots, slots, parts.n_split, parts.parts_max, nonzeros_vec,
+                                parts.longest_part_vec, column_indices, values, rhs_matrix, output_matrix, workspace, stream)
+    if st >= 0:
+        _lib.check(st, "vs_wmma_spmm_f16_row_parts")
+        return output_matrix
+    ws_bytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
     per_problem = lambda t, dims: _stride(t, batch)
     st = _lib.lib().vs_wmma_spmm_f16_row_parts(
         batch, vec_length, k, n, parts.n_slots, _expect(slots, torch.int32, "slots"), parts.n_split, parts.parts_max,
@@ -539,6 +624,11 @@ def sddmm_row_parts(k, n, parts, slots, nonzeros_vec, col_indices, lhs_matrix, r
     mask; lhs_matrix / rhs_matrix with the same leading dimension are per problem, without it shared.  Returns
     output_values."""
     batch = output_values.shape[0] if output_values.dim() == 3 else 1
+    st = _native.sddmm_row_parts(batch, k, n, parts.n_slots, slots, nonzeros_vec, col_indices, lhs_matrix, rhs_matrix,
+                                 output_values, vec_length, stream)
+    if st >= 0:
+        _lib.check(st, "vs_wmma_sddmm_f16_row_parts")
+        return output_values
     per_problem = lambda t, dims: _stride(t, batch)
     st = _lib.lib().vs_wmma_sddmm_f16_row_parts(
         batch, k, n, parts.n_slots, _expect(slots, torch.int32, "slots"), nonzeros_vec,
@@ -559,6 +649,11 @@ def sparse_softmax_row_parts(vec_length, parts, slots, values_in, values_out=Non
     if values_out is None:
         values_out = values_in
     batch = values_in.shape[0] if values_in.dim() == 3 else 1
+    st = _native.softmax_row_parts(batch, vec_length, parts.n_slots, slots, parts.n_split, parts.parts_max, values_in,
+                                   values_out, float(scale), workspace, stream)
+    if st >= 0:
+        _lib.check(st, "vs_sparse_softmax_f16_row_parts")
+        return values_out
     stride = lambda t: _stride(t, batch)
     ws_bytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
     st = _lib.lib().vs_sparse_softmax_f16_row_parts(
@@ -612,6 +707,7 @@ class DeviceProblem:
         self.column_indices = torch.from_numpy(np.ascontiguousarray(pattern.column_indices)).to(device)
         self._workspace = None  # partial tiles of the split-row SpMM, allocated on first use
         self._parts = {}        # limit -> (RowParts, its list on the device, workspace), made on first use
+        self._parts_need = {}
         self.values = None
         if pattern.values is not None:
             self.values = torch.from_numpy(np.ascontiguousarray(pattern.values)).to(device)
@@ -623,6 +719,18 @@ class DeviceProblem:
             slots = torch.from_numpy(parts.slots).to(self.column_indices.device)
             self._parts[limit_vec] = [parts, slots, None, None]   # (+ SpMM workspace, softmax workspace: on first use)
         return self._parts[limit_vec]
+
+    def _row_parts_bytes(self, limit_vec, k, batch):
+        """Workspace of `spmm_row_parts` (k > 0) or `softmax_row_parts` (k = 0), computed once per size."""
+        need = self._parts_need.get((limit_vec, k, batch))
+        if need is None:
+            parts = self.row_parts(limit_vec)[0]
+            if k:
+                need = spmm_row_parts_workspace_bytes(self.vec_length, k, parts.n_split, parts.parts_max, batch=batch)
+            else:
+                need = sparse_softmax_row_parts_workspace_bytes(self.vec_length, parts.n_split, parts.parts_max, batch=batch)
+            self._parts_need[limit_vec, k, batch] = need
+        return need
 
     def spmm_row_parts(self, rhs_matrix, out=None, stream=None, limit_vec=0, values=None):
         """SpMM (MFMA path, fp16 output) with long rows dispatched as several parts; the list and the workspace
@@ -636,7 +744,7 @@ class DeviceProblem:
             out = torch.empty(shape, dtype=torch.float16, device=rhs_matrix.device)
         entry = self.row_parts(limit_vec)
         parts, slots = entry[0], entry[1]
-        need = spmm_row_parts_workspace_bytes(self.vec_length, k, parts.n_split, parts.parts_max, batch=batch)
+        need = self._row_parts_bytes(limit_vec, k, batch)
         if need and (entry[2] is None or entry[2].numel() < need):
             entry[2] = torch.zeros(need, dtype=torch.uint8, device=rhs_matrix.device)
         return spmm_row_parts(self.vec_length, k, self.n, parts, slots, self.nnz_vec, self.column_indices, values,
@@ -648,7 +756,7 @@ class DeviceProblem:
         entry = self.row_parts(limit_vec)
         parts, slots = entry[0], entry[1]
         batch = values_in.shape[0] if values_in.dim() == 3 else 1
-        need = sparse_softmax_row_parts_workspace_bytes(self.vec_length, parts.n_split, parts.parts_max, batch=batch)
+        need = self._row_parts_bytes(limit_vec, 0, batch)
         if need and (entry[3] is None or entry[3].numel() < need):
             entry[3] = torch.empty(need, dtype=torch.uint8, device=values_in.device)
         return sparse_softmax_row_parts(self.vec_length, parts, slots, values_in, values_out, scale,
@@ -672,8 +780,7 @@ class DeviceProblem:
             if kernel == "wmma" and k % 4 == 0 and out.dtype == torch.float16 and self.n * k < 2 ** 31:
                 parts = self.row_parts(0)[0]
                 # (the entry point addresses the partial tiles with 32-bit offsets: less than 2 GiB of them)
-                if parts.n_split > 0 and spmm_row_parts_workspace_bytes(self.vec_length, k, parts.n_split,
-                                                                        parts.parts_max) < 2 ** 31:
+                if parts.n_split > 0 and self._row_parts_bytes(0, k, 1) < 2 ** 31:
                     return self.spmm_row_parts(rhs_matrix, out=out, stream=stream)
             split_rows = False
             row_length_hint = True
