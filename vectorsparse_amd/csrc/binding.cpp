@@ -71,7 +71,11 @@ struct Reader {
     {
         PyObject *o = next();
         if (o == Py_None) return (void *)c10::hip::getCurrentHIPStream().stream();
-        if (o && PyLong_CheckExact(o)) return PyLong_AsVoidPtr(o);
+        if (o && PyLong_CheckExact(o)) {
+            void *const handle = PyLong_AsVoidPtr(o);
+            if (handle || !PyErr_Occurred()) return handle;
+            PyErr_Clear();
+        }
         ok = false;
         return nullptr;
     }
@@ -358,10 +362,24 @@ PyObject *softmax_row_parts(PyObject *, PyObject *const *args, Py_ssize_t n_args
     });
 }
 
-#define VS_METHOD(name, fn) {name, (PyCFunction)(void (*)(void))(fn), METH_FASTCALL, nullptr}
+// Tensors without storage (fake and functional ones, those inside vmap) throw when they are asked for an address, a
+// process without a device when it is asked for a stream; an exception must not leave a C function.  Both are unusual
+// arguments: ops.py meets the same refusal as a Python exception.
+typedef PyObject *(*Method)(PyObject *, PyObject *const *, Py_ssize_t);
+template <Method F>
+PyObject *guarded(PyObject *self, PyObject *const *args, Py_ssize_t n_args) noexcept
+{
+    try {
+        return F(self, args, n_args);
+    } catch (...) {
+        return PyLong_FromLong(kUnusual);
+    }
+}
+
+#define VS_METHOD(name, fn) {name, (PyCFunction)(void (*)(void))(guarded<fn>), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
-    VS_METHOD("wmma_spmm", (&spmm<vs_wmma_spmm_f16, vs_wmma_spmm_f16_f32out>)),
-    VS_METHOD("cuda_spmm", (&spmm<vs_cuda_spmm_f16, vs_cuda_spmm_f16_f32out>)),
+    VS_METHOD("wmma_spmm", (spmm<vs_wmma_spmm_f16, vs_wmma_spmm_f16_f32out>)),
+    VS_METHOD("cuda_spmm", (spmm<vs_cuda_spmm_f16, vs_cuda_spmm_f16_f32out>)),
     VS_METHOD("wmma_sddmm", wmma_sddmm),
     VS_METHOD("cuda_sddmm", cuda_sddmm),
     VS_METHOD("wmma_spmm_batched", wmma_spmm_batched),
