@@ -197,9 +197,9 @@ int vs_cuda_spmm_f16_f32out(int m_vec, int vec_length, int k, int n,
  * less - run on the fine-grained kernel of vs_cuda_sddmm_f16 (same function
  * within the fp32-accumulation tolerance, not the same bits).  Under 0 and 1, and in vs_cuda_sddmm_f16, masks that
  * keep a good share of large tiles (short vectors, low sparsity) multiply whole tiles and keep the masked outputs
- * (option "sddmm_tile"): the bits of schedule 1, columns of a row in any order.
- * 3 (the reference's timing-only hardware
- * simulation, whose results are wrong by design) is rejected with
+ * (option "sddmm_tile"): the bits of schedule 1 for rows of sorted columns; other orders are taken too, within the
+ * fp32-accumulation tolerance, but several times slower than by gathering (option "sddmm_tile" = 1).
+ * 3 (the reference's timing-only hardware simulation, whose results are wrong by design) is rejected with
  * hipErrorInvalidValue.
  * Any k >= 0; the whole of k is contracted (the reference drops k % 64).  k % 8 != 0
  * runs on the scalar-load variant of the fine-grained kernel of vs_cuda_sddmm_f16,
