@@ -1,5 +1,6 @@
 """SDDMM on dense tiles (csrc/sddmm_tile.hip): both tile sizes at the edges of tiles, rows, columns and contraction
-steps, against the C oracle, and bit for bit against the gathering MFMA kernel (same products in the same order)."""
+steps, against the C oracle, and bit for bit against the gathering MFMA kernel (same products in the same order),
+whatever the order of a row's columns."""
 import numpy as np
 import pytest
 import torch
@@ -44,7 +45,8 @@ def _pattern(kind, m_vec, n, V):
 @pytest.mark.parametrize("kind,rows,n,K", [
     ("uniform", 1, 1, 8), ("uniform", 64, 64, 64), ("uniform", 128, 128, 128), ("uniform", 136, 129, 72),
     ("uniform", 56, 63, 320), ("uniform", 1048, 300, 40), ("clustered columns", 200, 900, 136),
-    ("dense and empty rows", 72, 200, 264), ("shuffled columns", 96, 200, 96), ("repeated columns", 48, 65, 64)])
+    ("dense and empty rows", 72, 200, 264), ("shuffled columns", 96, 200, 96), ("shuffled columns", 136, 1500, 264),
+    ("repeated columns", 48, 65, 64)])
 def test_dense_tiles_match_the_oracle_and_the_gathering_kernel(gpu, kind, rows, n, K, V, tile):
     m_vec = max(1, rows // V)
     pat = _pattern(kind, m_vec, n, V)
@@ -62,8 +64,9 @@ def test_dense_tiles_match_the_oracle_and_the_gathering_kernel(gpu, kind, rows, 
         torch.cuda.synchronize()
         assert bool((pad[:16] == 7.0).all()) and bool((pad[16 + pat.nnz_vec:] == 7.0).all())
         assert_parity(got.cpu().numpy().reshape(-1), ref, "%s %s" % (kind, dtype))
-        if kind not in ("shuffled columns", "repeated columns"):   # (nonzeros served one by one add up in another order)
-            assert torch.equal(got, gathered)
+        # Shuffled columns: a nonzero is then written by several tiles (CPU model of the search over 40 rows of 820 of 4096
+        # columns: two in three lie between the bounds of several tiles, 6 % of them of their own and of another one).
+        assert torch.equal(got, gathered)
 
 
 def test_dense_tiles_batched(gpu):

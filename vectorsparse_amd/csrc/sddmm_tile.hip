@@ -12,8 +12,9 @@
 //   3. the tile, converted, to LDS; every lane picks its nonzeros' outputs there and writes them out.
 // Columns need not be sorted: the bound of (row, column) depends on nothing else, the first bound of a row is its
 // first nonzero and the last one its end, so every nonzero lies between the two bounds of at least one tile whatever
-// the order; a nonzero found in a tile that does not hold its column is computed there by itself (slowly: a pattern of
-// shuffled columns runs several times slower than on the gathering kernels).
+// the order - of several, where the bounds of the row do not ascend.  A nonzero found in a tile that does not hold its
+// column is multiplied there by itself, to the same bits, so that it does not matter which of its tiles writes it last.
+// (Slow: with shuffled columns two nonzeros in three lie in several tiles.)
 //
 // What bounds it (4096 x 4096, V = 1, K = 256, 80 %, tiles of 128: 20.2 us): nothing alone - vector ALU 8 us, LDS 6 us, matrix
 // cores 4 us, 224 MB through the L2s 10 us, around a tile's chain of dependent loads (row extent, two probes, columns) of
@@ -335,26 +336,11 @@ sddmm_tile_kernel(int m_vec, int K, int n, int row_blocks, int column_tiles, con
         }
     __syncthreads();
 
-    // A nonzero by itself, from memory: a column that the tile does not hold (unsorted patterns).
-    auto alone = [&](int j, int column) {
-#pragma unroll 1
-        for (int v = 0; v < V; ++v) {
-            const half_t *a = lhs + ((size_t)row * V + v) * K;
-            const half_t *b = rhs + (size_t)column * K;
-            float sum = 0.f;
-#pragma unroll 1
-            for (int l = 0; l < K; l += 8) {
-                const half8_t x = *reinterpret_cast<const half8_t *>(a + l), y = *reinterpret_cast<const half8_t *>(b + l);
-#pragma unroll
-                for (int i = 0; i < 8; ++i) sum += (float)x[i] * (float)y[i];
-            }
-            out[(size_t)j * V + v] = (OutT)sum;
-        }
-    };
     struct __align__(sizeof(OutT) * V) Vec {
         OutT x[V];
     };
     const OutT *const tile_row = tile + row_here * PITCH * V;
+    bool elsewhere = false;   // a nonzero between the bounds whose column the tile does not hold
     for (int base = beg; base < end;) {
 #pragma unroll
         for (int u = 0; u < AHEAD; ++u) {
@@ -377,17 +363,50 @@ sddmm_tile_kernel(int m_vec, int K, int n, int row_blocks, int column_tiles, con
                     for (int i = 0; i < 4; ++i)
                         if (j + i < end) {
                             if (at[i] < (unsigned)TN) out[j + i] = tile_row[at[i]];
-                            else alone(j + i, col[u][i]);
+                            else elsewhere = true;
                         }
                 }
             } else if (j < end) {
                 const unsigned at = (unsigned)(col[u][0] - c0);
                 if (at < (unsigned)TN) *reinterpret_cast<Vec *>(out + (size_t)j * V) = *reinterpret_cast<const Vec *>(tile_row + at * V);
-                else alone(j, col[u][0]);
+                else elsewhere = true;
             }
         }
         base += EACH * LPR * AHEAD;
         if (base < end) fetch_columns(base);
+    }
+
+    // Rows of unsorted columns: the wave multiplies such nonzeros one by one, on the matrix cores and in the same steps of
+    // 32 as the tiles.  Such a nonzero can lie between the bounds of several tiles, its own among them; whichever of them
+    // writes it last, it writes the same bits.
+    if (__builtin_amdgcn_ballot_w64(elsewhere) == 0) return;
+    for (int j = beg + li; __builtin_amdgcn_ballot_w64(j < end) != 0; j += LPR) {
+        const int column = j < end ? col_indices[j] : c0;
+        uint64_t todo = __builtin_amdgcn_ballot_w64((unsigned)(column - c0) >= (unsigned)TN);
+        while (todo != 0) {
+            const int from = __builtin_ctzll(todo);
+            todo &= todo - 1;
+            const int its_row = __builtin_amdgcn_readlane(row, from), its_column = __builtin_amdgcn_readlane(column, from);
+            const int its_j = __builtin_amdgcn_readlane(j, from);
+            // (lanes past the vector's rows repeat one of them; every column of the product is the same)
+            const half_t *const a = lhs + ((size_t)its_row * V + c % V) * K, *const b = rhs + (size_t)its_column * K;
+            float4_t sum = {0.f, 0.f, 0.f, 0.f};
+            for (int k0 = 0; k0 < K; k0 += 32) {
+                const bool there = k0 + 8 * g < K;
+                const int at = there ? k0 + 8 * g : 0;
+                const uint4_t x = *reinterpret_cast<const uint4_t *>(a + at), y = *reinterpret_cast<const uint4_t *>(b + at);
+                const uint4_t zero = {0u, 0u, 0u, 0u};
+                const uint4_t xs = there ? x : zero, ys = there ? y : zero;
+                sum = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, xs), __builtin_bit_cast(half8_t, ys), sum, 0, 0, 0);
+            }
+            // (all four results land before a register of those that are not stored is used again)
+            asm volatile("s_nop 15" : "+v"(sum));
+            if (c == 0) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (4 * g + e < V) out[(size_t)its_j * V + 4 * g + e] = (OutT)sum[e];
+            }
+        }
     }
 }
 
