@@ -195,10 +195,7 @@ int vs_cuda_spmm_f16_f32out(int m_vec, int vec_length, int k, int n,
  * rows and small problems).  0 = automatic: schedule 1, except that masks of few
  * nonzeros with vec_length <= 4 - which fill a quarter of a matrix-core tile or
  * less - run on the fine-grained kernel of vs_cuda_sddmm_f16 (same function
- * within the fp32-accumulation tolerance, not the same bits).  Under 0 and 1, and in vs_cuda_sddmm_f16, masks that
- * keep a good share of large tiles (short vectors, low sparsity) multiply whole tiles and keep the masked outputs
- * (option "sddmm_tile"): the bits of schedule 1 for rows of sorted columns; other orders are taken too, within the
- * fp32-accumulation tolerance, but several times slower than by gathering (option "sddmm_tile" = 1).
+ * within the fp32-accumulation tolerance, not the same bits).
  * 3 (the reference's timing-only hardware simulation, whose results are wrong by design) is rejected with
  * hipErrorInvalidValue.
  * Any k >= 0; the whole of k is contracted (the reference drops k % 64).  k % 8 != 0
@@ -365,6 +362,29 @@ int vs_cuda_sddmm_f16_batched(int batch, int m_vec, int k, int n, int nonzeros_v
                               int vec_length, void *stream);
 
 /*
+ * vs_wmma_sddmm_f16_batched / vs_cuda_sddmm_f16_batched (f32_output = 0) and their fp32-output counterparts (f32_output = 1;
+ * stride_output in floats) for masks whose columns ascend in every row, repeated ones included: `batch` = 1 and zero
+ * strides for a single problem.  Masks that keep a good share of large tiles (short vectors, low sparsity) then multiply
+ * whole tiles on the matrix cores and keep the masked outputs, for k % 8 == 0 and `algorithm` 0 or 1 (option
+ * "sddmm_tile"): the bits of schedule 1.  Otherwise they are the entry points named above.  The order is a hint: columns in
+ * another order give the same bits, several times slower.  No counterpart in the reference, whose kernels gather.
+ */
+int vs_wmma_sddmm_f16_sorted(int batch, int m_vec, int k, int n, int nonzeros_vec,
+                             const int *row_indices, const int *row_offsets,
+                             const int *col_indices,
+                             const void *lhs_matrix, long long stride_lhs,
+                             const void *rhs_matrix, long long stride_rhs,
+                             void *output_values, long long stride_output,
+                             int f32_output, int vec_length, void *stream, int algorithm);
+int vs_cuda_sddmm_f16_sorted(int batch, int m_vec, int k, int n, int nonzeros_vec,
+                             const int *row_indices, const int *row_offsets,
+                             const int *col_indices,
+                             const void *lhs_matrix, long long stride_lhs,
+                             const void *rhs_matrix, long long stride_rhs,
+                             void *output_values, long long stride_output,
+                             int f32_output, int vec_length, void *stream);
+
+/*
  * Row-wise softmax over the nonzeros of each SCALAR row of a column-vector CSR
  * matrix, on the [nnz_vec][vec_length] fp16 value layout SDDMM writes and SpMM
  * reads:  out = softmax_row(scale * in), computed in fp32.  `values_out` may
@@ -529,8 +549,8 @@ int vs_wmma_spmm_launch_shape(int batch, int m_vec, int vec_length, int k, int n
  * vector row, 0 = automatic), "sddmm_group" (16-vector groups per wave step of the
  * MFMA SDDMM: 1, 2, 4, 0 = automatic), "sddmm_block_waves" (1..16, 0 = automatic),
  * "sddmm_flat_supers" (super-groups per wave of algorithm 2, 1..16, 0 = automatic),
- * "sddmm_tile" (SDDMM on dense tiles, k % 8 == 0: 1 = never, 2 = tiles of 64 x 64, 3 = of 128 x 128,
- * 0 = where it is expected to be faster than gathering rows),
+ * "sddmm_tile" (SDDMM on dense tiles, k % 8 == 0, any order of the columns: 1 = never, 2 = tiles of 64 x 64,
+ * 3 = of 128 x 128, 0 = where the columns are known to ascend and tiles are expected to be faster than gathering rows),
  * "attention_waves" (1..8, 0 = automatic), "attention_chunk" (nonzero vectors per
  * LDS chunk of the one-row-per-workgroup attention kernel, 0 = automatic).
  * Returns 0, or 1 for an unknown name / bad value.

@@ -69,6 +69,13 @@ def test_argument_validation_without_launch():
     # algorithm 3 is the reference's timing-only hardware simulation; unknown algorithms launch nothing
     assert L.vs_wmma_sddmm_f16(4, 64, 64, 10, p, p, p, p, p, p, 8, None, 3) == INVALID
     assert L.vs_wmma_sddmm_f16(4, 64, 64, 10, p, p, p, p, p, p, 8, None, -1) == INVALID
+    # (masks of ascending columns: the checks of the batched entry points)
+    sorted_args = (2, 4, 64, 64, 10, p, p, p, p, 512, p, 512, p, 80)
+    assert L.vs_wmma_sddmm_f16_sorted(*sorted_args, 0, 8, None, 3) == INVALID
+    assert L.vs_wmma_sddmm_f16_sorted(*sorted_args, 0, 8, None, -1) == INVALID
+    assert L.vs_wmma_sddmm_f16_sorted(*sorted_args[:9], 516, *sorted_args[10:], 0, 8, None, 1) == INVALID
+    assert L.vs_cuda_sddmm_f16_sorted(*sorted_args, 0, 3, None) == INVALID
+    assert L.vs_cuda_sddmm_f16_sorted(*sorted_args[:12], p + 16, 80, 1, 8, None) == INVALID      # 16 bytes do for fp16 outputs
     # shapes a path cannot take
     # (the reference-shaped entry points take any dense width / contraction length; the split-row schedule needs
     # k % 4 == 0)

@@ -86,3 +86,34 @@ def test_dense_tiles_batched(gpu):
         torch.cuda.synchronize()
         for h in range(heads):
             assert torch.equal(out[h], one[h]), "head %d" % h
+
+
+@pytest.mark.parametrize("kernel", ["wmma", "cuda"])
+def test_the_automatic_route_takes_tiles_only_where_columns_ascend(gpu, kernel):
+    """A mask dense enough for tiles (V = 1, 512 x 1024 at 50 %, K = 256; gathering it takes the fine-grained kernel, whose
+    fp32 bits are not those of the matrix cores): ascending columns known to the caller run on tiles, the same columns
+    without that word, or shuffled ones, are gathered, and a wrong word changes no bit."""
+    mask = cv.binomial_pattern(512, 1024, 0.5, seed=9, vec_length=1)
+    A = torch.from_numpy(cv.dense_normal(mask.m, 256, seed=10)).cuda()
+    B = torch.from_numpy(cv.dense_normal(mask.n, 256, seed=11)).cuda()
+    for pat in (mask, _shuffled(mask, 12)):
+        prob = ops.DeviceProblem(pat)
+        assert prob.columns_sorted == (pat is mask)
+        with _lib.thread_options(sddmm_tile=1):
+            gathered = prob.sddmm(A, B, kernel=kernel, out_dtype=torch.float32)
+            matrix_cores = prob.sddmm(A, B, out_dtype=torch.float32, algorithm=1)
+        assert not torch.equal(gathered, matrix_cores)
+        assert torch.equal(prob.sddmm(A, B, kernel=kernel, out_dtype=torch.float32), matrix_cores if pat is mask else gathered)
+        out = torch.empty_like(gathered)
+        args = (prob.m_vec, 256, prob.n, prob.nnz_vec, prob.row_indices, prob.row_offsets, prob.column_indices, A, B, out, 1)
+        call, extra = (ops.sddmm.wmmaSddmm, dict(algorithm=0)) if kernel == "wmma" else (ops.sddmm.cudaSddmm, {})
+        assert torch.equal(call(*args, **extra), gathered)
+        # (the compiled binding, then the checks of ops.py, which take the stream as an object)
+        for stream in (None, torch.cuda.current_stream()):
+            assert torch.equal(call(*args, stream=stream, columns_sorted=True, **extra), matrix_cores)
+        one = torch.empty((1, prob.nnz_vec, 1), dtype=torch.float16, device="cuda")
+        args = args[:7] + (A[None], B[None], one, 1)
+        for stream in (None, torch.cuda.current_stream()):
+            ops.sddmm_batched(*args, kernel=kernel, stream=stream, columns_sorted=True, **extra)
+            assert torch.equal(one[0], matrix_cores.half())
+        torch.cuda.synchronize()

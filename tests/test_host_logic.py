@@ -370,3 +370,13 @@ def test_row_parts_dispatch_list():
     assert _lib.lib().vs_wmma_spmm_row_parts_workspace_bytes(1, 8, 256, 0, 0) == 0
     assert _lib.lib().vs_wmma_spmm_row_parts_workspace_bytes(1, 8, 256, 3, 4) > 3 * 4 * 8 * 256 * 4
     assert _lib.lib().vs_wmma_spmm_row_parts_workspace_bytes(5, 8, 256, 3, 4) > 5 * 3 * 4 * 8 * 256 * 4
+
+
+def test_columns_that_ascend_are_recognised():
+    ascend = lambda ro, ci: ops.columns_ascend(np.array(ro, np.int32), np.array(ci, np.int32))
+    assert ascend([0], []) and ascend([0, 1], [5]) and ascend([0, 0, 0], [])
+    assert ascend([0, 3, 3, 5], [0, 2, 7, 0, 1])      # falls only where a row starts, an empty row between
+    assert ascend([0, 4], [1, 1, 1, 2])               # repeated columns
+    assert not ascend([0, 3, 5], [0, 7, 2, 0, 1])
+    assert not ascend([0, 2, 5], [0, 7, 1, 0, 2])
+    assert not ascend([0, 5], [4, 3, 2, 1, 0])

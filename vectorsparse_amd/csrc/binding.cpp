@@ -58,6 +58,12 @@ struct Reader {
         if (overflow || v < INT32_MIN || v > INT32_MAX) ok = false;
         return (int)v;
     }
+    bool flag()
+    {
+        PyObject *o = next();
+        if (!o || !PyBool_Check(o)) ok = false;
+        return o == Py_True;
+    }
     float number()
     {
         PyObject *o = next();
@@ -169,7 +175,7 @@ PyObject *spmm(PyObject *, PyObject *const *args, Py_ssize_t n_args)
     });
 }
 
-// (m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices, lhs, rhs, out, vec_length, stream, algorithm)
+// (m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices, lhs, rhs, out, vec_length, stream, algorithm, columns_sorted)
 PyObject *wmma_sddmm(PyObject *, PyObject *const *args, Py_ssize_t n_args)
 {
     Reader r(args, n_args);
@@ -181,13 +187,15 @@ PyObject *wmma_sddmm(PyObject *, PyObject *const *args, Py_ssize_t n_args)
     const int v = r.integer();
     void *stream = r.stream();
     const int algorithm = r.integer();
+    const bool sorted = r.flag();
     return status_of(r, [&] {
+        if (sorted) return vs_wmma_sddmm_f16_sorted(1, m_vec, k, n, nnz, ri, ro, ci, lhs, 0, rhs, 0, out, 0, f32, v, stream, algorithm);
         return f32 ? vs_wmma_sddmm_f16_f32out(m_vec, k, n, nnz, ri, ro, ci, lhs, rhs, (float *)out, v, stream, algorithm)
                    : vs_wmma_sddmm_f16(m_vec, k, n, nnz, ri, ro, ci, lhs, rhs, out, v, stream, algorithm);
     });
 }
 
-// (m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices, lhs, rhs, out, vec_length, stream)
+// (m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices, lhs, rhs, out, vec_length, stream, columns_sorted)
 PyObject *cuda_sddmm(PyObject *, PyObject *const *args, Py_ssize_t n_args)
 {
     Reader r(args, n_args);
@@ -198,7 +206,9 @@ PyObject *cuda_sddmm(PyObject *, PyObject *const *args, Py_ssize_t n_args)
     void *out = r.output(f32);
     const int v = r.integer();
     void *stream = r.stream();
+    const bool sorted = r.flag();
     return status_of(r, [&] {
+        if (sorted) return vs_cuda_sddmm_f16_sorted(1, m_vec, k, n, nnz, ri, ro, ci, lhs, 0, rhs, 0, out, 0, f32, v, stream);
         return f32 ? vs_cuda_sddmm_f16_f32out(m_vec, k, n, nnz, ri, ro, ci, lhs, rhs, (float *)out, v, stream)
                    : vs_cuda_sddmm_f16(m_vec, k, n, nnz, ri, ro, ci, lhs, rhs, out, v, stream);
     });
@@ -256,8 +266,8 @@ PyObject *spmm_softmax_batched(PyObject *, PyObject *const *args, Py_ssize_t n_a
     });
 }
 
-// (batch, m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices, lhs, rhs, out, vec_length, stream, algorithm);
-// algorithm < 0: the fine-grained path
+// (batch, m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices, lhs, rhs, out, vec_length, stream, algorithm,
+// columns_sorted); algorithm < 0: the fine-grained path
 PyObject *sddmm_batched(PyObject *, PyObject *const *args, Py_ssize_t n_args)
 {
     Reader r(args, n_args);
@@ -269,7 +279,11 @@ PyObject *sddmm_batched(PyObject *, PyObject *const *args, Py_ssize_t n_args)
     const int v = r.integer();
     void *stream = r.stream();
     const int algorithm = r.integer();
+    const bool sorted = r.flag();
     return status_of(r, [&] {
+        if (sorted)
+            return algorithm < 0 ? vs_cuda_sddmm_f16_sorted(batch, m_vec, k, n, nnz, ri, ro, ci, lhs, sa, rhs, sb, out, so, 0, v, stream)
+                                 : vs_wmma_sddmm_f16_sorted(batch, m_vec, k, n, nnz, ri, ro, ci, lhs, sa, rhs, sb, out, so, 0, v, stream, algorithm);
         return algorithm < 0 ? vs_cuda_sddmm_f16_batched(batch, m_vec, k, n, nnz, ri, ro, ci, lhs, sa, rhs, sb, out, so, v, stream)
                              : vs_wmma_sddmm_f16_batched(batch, m_vec, k, n, nnz, ri, ro, ci, lhs, sa, rhs, sb, out, so, v, stream, algorithm);
     });

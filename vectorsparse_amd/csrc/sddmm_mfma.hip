@@ -425,7 +425,6 @@ int launch_sddmm_mfma(int m_vec, int k, int n, int nonzeros_vec, const int *row_
                       const int *row_offsets, const int *col_indices, const half_t *lhs,
                       const half_t *rhs, OutT *out, int vec_length, hipStream_t stream, const Batch &batch)
 {
-    (void)n;
     if (m_vec == 0 || nonzeros_vec == 0 || batch.count == 0) return hipSuccess;
     if (batch.count > 65535) return hipErrorNotSupported;
     if (k <= 0) return hipErrorNotSupported;
@@ -438,7 +437,7 @@ int launch_sddmm_mfma(int m_vec, int k, int n, int nonzeros_vec, const int *row_
                                        vec_length, stream, batch);
     }
     if (batch.algorithm != 2 && !batch.row_parts) {
-        const int tile = sddmm_tile_choice(m_vec, k, n, nonzeros_vec, vec_length, batch.count);
+        const int tile = sddmm_tile_choice(m_vec, k, n, nonzeros_vec, vec_length, batch);
         if (tile > 0)
             return launch_sddmm_tile<OutT>(tile, m_vec, k, n, row_offsets, col_indices, lhs, rhs, out, vec_length, stream, batch);
     }

@@ -443,11 +443,15 @@ int launch_tile_shape(bool wide, int m_vec, int k, int n, const int *row_offsets
 // them to the tiles.  4096 x 4096, V = 1, K = 256: 196 / 90 / 50 / 13.4 us gathering at 50 / 80 / 90 / 98 %, 26.7 / 20.2 / 18.9 /
 // 17.9 us on tiles; 2048 x 2304, V = 4, K = 512, 90 %: 16.0 against 12.3 us; 2048 x 2048, V = 8, K = 64: 2.8 against 4.2 us at
 // 90 %, 5.7 against 5.0 us at 50 %.
-int sddmm_tile_choice(int m_vec, int k, int n, long long nonzeros_vec, int vec_length, int batch)
+// Only where the caller vouches for ascending columns: with shuffled ones most nonzeros are multiplied one by one, in
+// several tiles each, which no row length or sparsity makes up for, and sizes do not tell the order.
+int sddmm_tile_choice(int m_vec, int k, int n, long long nonzeros_vec, int vec_length, const Batch &problems)
 {
+    const int batch = problems.count;
     const Options &o = options();
     if (k <= 0 || k % 8 != 0 || n <= 0 || k > (1 << 20) || o.sddmm_tile == 1) return 0;
     if (o.sddmm_tile >= 2) return o.sddmm_tile - 1;
+    if (!problems.sorted_columns) return 0;
     if (o.sddmm_slots || o.sddmm_group || o.sddmm_block_waves) return 0;  // a launch shape of the gathering kernels is asked for
     const double nonzeros = (double)nonzeros_vec * batch, steps = (k + kTileK - 1) / kTileK;
     const double per_mega = vec_length == 1 ? 0.128 : (vec_length == 2 ? 0.145 : (vec_length == 4 ? 0.175 : 0.21));

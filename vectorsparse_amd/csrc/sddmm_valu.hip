@@ -234,7 +234,7 @@ int launch_sddmm_valu(int m_vec, int k, int n, int nonzeros_vec, const int *row_
     if (m_vec == 0 || nonzeros_vec == 0 || batch.count == 0) return hipSuccess;
     if (batch.count > 65535) return hipErrorNotSupported;
     if (k <= 0) return hipErrorNotSupported;
-    const int tile = sddmm_tile_choice(m_vec, k, n, nonzeros_vec, vec_length, batch.count);
+    const int tile = sddmm_tile_choice(m_vec, k, n, nonzeros_vec, vec_length, batch);
     if (tile > 0)
         return launch_sddmm_tile<OutT>(tile, m_vec, k, n, row_offsets, col_indices, lhs, rhs, out, vec_length, stream, batch);
     switch (vec_length) {

@@ -287,6 +287,7 @@ struct Batch {
     int long_rows = -1;        // SpMM, rows ordered by length: leading entries of row_indices with more than 512 vectors
     int algorithm = 0;         // SDDMM on MFMA: 2 = waves split the nonzero range, else (row, slot) per wave
     bool row_parts = false;    // SDDMM on MFMA: row_indices is a dispatch list of row parts, m_vec counts its slots
+    bool sorted_columns = false;  // SDDMM: the columns of every row are known to ascend (a hint)
 };
 
 // Launch shape of the MFMA SpMM (spmm_mfma.hip), chosen on the host.
@@ -328,7 +329,7 @@ int launch_sddmm_valu(int m_vec, int k, int n, int nonzeros_vec, const int *row_
 
 // SDDMM on dense tiles (csrc/sddmm_tile.hip), k % 8 == 0.  sddmm_tile_choice: 0 = the gathering kernels are expected
 // to be faster, else the `shape` for launch_sddmm_tile (1 = tiles of 64 x 64, 2 = of 128 x 128).
-int sddmm_tile_choice(int m_vec, int k, int n, long long nonzeros_vec, int vec_length, int batch);
+int sddmm_tile_choice(int m_vec, int k, int n, long long nonzeros_vec, int vec_length, const Batch &batch);
 template <typename OutT>
 int launch_sddmm_tile(int shape, int m_vec, int k, int n, const int *row_offsets, const int *col_indices,
                       const half_t *lhs, const half_t *rhs, OutT *out, int vec_length, hipStream_t stream,

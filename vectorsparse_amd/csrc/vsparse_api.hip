@@ -89,6 +89,31 @@ int check_sddmm(int m_vec, int k, int n, int nonzeros_vec, const int *row_indice
     return VS_SUCCESS;
 }
 
+bool stride_ok(long long stride, long long multiple) { return stride >= 0 && stride % multiple == 0; }
+
+template <typename OutT>
+int sddmm_batch(bool mfma, const vs::Batch &batch, int m_vec, int k, int n, int nonzeros_vec, const int *row_indices,
+                       const int *row_offsets, const int *col_indices, const void *lhs_matrix, const void *rhs_matrix,
+                       void *output_values, int vec_length, void *stream)
+{
+    if (batch.count < 0 || (mfma && (batch.algorithm < 0 || batch.algorithm > 2))) return VS_ERROR_INVALID_VALUE;
+    int st = check_sddmm(m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices, lhs_matrix, rhs_matrix,
+                         output_values, vec_length, sizeof(OutT));
+    if (st != VS_SUCCESS) return st;
+    if (k == 0 && m_vec > 0) {
+        if (!stride_ok(batch.stride_out, vec_length)) return VS_ERROR_INVALID_VALUE;
+        return sddmm_zero_outputs(output_values, nonzeros_vec, vec_length, sizeof(OutT), batch.count, batch.stride_out,
+                                  static_cast<hipStream_t>(stream));
+    }
+    const long long in_mult = (mfma || k % 8 == 0) ? 8 : 1;
+    if (!stride_ok(batch.stride_a, in_mult) || !stride_ok(batch.stride_b, in_mult) || !stride_ok(batch.stride_out, vec_length))
+        return VS_ERROR_INVALID_VALUE;
+    const auto launch = mfma ? vs::launch_sddmm_mfma<OutT> : vs::launch_sddmm_valu<OutT>;
+    return launch(m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices, static_cast<const half_t *>(lhs_matrix),
+                  static_cast<const half_t *>(rhs_matrix), static_cast<OutT *>(output_values), vec_length,
+                  static_cast<hipStream_t>(stream), batch);
+}
+
 }  // namespace
 
 // the library is compiled with hidden visibility: what follows is its whole exported surface
@@ -328,8 +353,6 @@ static vs::Batch make_batch(int batch, long long a, long long b, long long out, 
 }
 
 // Strides keep every problem's operand as aligned as the first one.
-static bool stride_ok(long long stride, long long multiple) { return stride >= 0 && stride % multiple == 0; }
-
 int vs_wmma_spmm_f16_batched(int batch, int m_vec, int vec_length, int k, int n, int nonzeros_vec,
                              int longest_row_vec, const int *row_indices,
                              const int *row_offsets, const int *column_indices, const void *values,
@@ -409,23 +432,10 @@ int vs_wmma_sddmm_f16_batched(int batch, int m_vec, int k, int n, int nonzeros_v
                               void *output_values, long long stride_output, int vec_length, void *stream,
                               int algorithm)
 {
-    if (batch < 0 || algorithm < 0 || algorithm > 2) return VS_ERROR_INVALID_VALUE;
-    int st = check_sddmm(m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices, lhs_matrix, rhs_matrix,
-                         output_values, vec_length, sizeof(half_t));
-    if (st != VS_SUCCESS) return st;
-    if (k == 0 && m_vec > 0) {
-        if (!stride_ok(stride_output, vec_length)) return VS_ERROR_INVALID_VALUE;
-        return sddmm_zero_outputs(output_values, nonzeros_vec, vec_length, sizeof(half_t), batch, stride_output, static_cast<hipStream_t>(stream));
-    }
-    if (!stride_ok(stride_lhs, 8) || !stride_ok(stride_rhs, 8) || !stride_ok(stride_output, vec_length))
-        return VS_ERROR_INVALID_VALUE;
     vs::Batch many = make_batch(batch, stride_lhs, stride_rhs, stride_output);
     many.algorithm = algorithm;
-    return vs::launch_sddmm_mfma<half_t>(m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices,
-                                         static_cast<const half_t *>(lhs_matrix),
-                                         static_cast<const half_t *>(rhs_matrix),
-                                         static_cast<half_t *>(output_values), vec_length,
-                                         static_cast<hipStream_t>(stream), many);
+    return sddmm_batch<half_t>(true, many, m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices, lhs_matrix,
+                               rhs_matrix, output_values, vec_length, stream);
 }
 
 int vs_cuda_sddmm_f16_batched(int batch, int m_vec, int k, int n, int nonzeros_vec, const int *row_indices,
@@ -433,23 +443,34 @@ int vs_cuda_sddmm_f16_batched(int batch, int m_vec, int k, int n, int nonzeros_v
                               long long stride_lhs, const void *rhs_matrix, long long stride_rhs,
                               void *output_values, long long stride_output, int vec_length, void *stream)
 {
-    if (batch < 0) return VS_ERROR_INVALID_VALUE;
-    int st = check_sddmm(m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices, lhs_matrix, rhs_matrix,
-                         output_values, vec_length, sizeof(half_t));
-    if (st != VS_SUCCESS) return st;
-    if (k == 0 && m_vec > 0) {
-        if (!stride_ok(stride_output, vec_length)) return VS_ERROR_INVALID_VALUE;
-        return sddmm_zero_outputs(output_values, nonzeros_vec, vec_length, sizeof(half_t), batch, stride_output, static_cast<hipStream_t>(stream));
-    }
-    const long long in_mult = (k % 8 == 0) ? 8 : 1;
-    if (!stride_ok(stride_lhs, in_mult) || !stride_ok(stride_rhs, in_mult) || !stride_ok(stride_output, vec_length))
-        return VS_ERROR_INVALID_VALUE;
-    return vs::launch_sddmm_valu<half_t>(m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices,
-                                         static_cast<const half_t *>(lhs_matrix),
-                                         static_cast<const half_t *>(rhs_matrix),
-                                         static_cast<half_t *>(output_values), vec_length,
-                                         static_cast<hipStream_t>(stream),
-                                         make_batch(batch, stride_lhs, stride_rhs, stride_output));
+    return sddmm_batch<half_t>(false, make_batch(batch, stride_lhs, stride_rhs, stride_output), m_vec, k, n, nonzeros_vec,
+                               row_indices, row_offsets, col_indices, lhs_matrix, rhs_matrix, output_values, vec_length, stream);
+}
+
+int vs_wmma_sddmm_f16_sorted(int batch, int m_vec, int k, int n, int nonzeros_vec, const int *row_indices,
+                             const int *row_offsets, const int *col_indices, const void *lhs_matrix,
+                             long long stride_lhs, const void *rhs_matrix, long long stride_rhs,
+                             void *output_values, long long stride_output, int f32_output, int vec_length,
+                             void *stream, int algorithm)
+{
+    vs::Batch many = make_batch(batch, stride_lhs, stride_rhs, stride_output);
+    many.algorithm = algorithm;
+    many.sorted_columns = true;
+    return (f32_output ? sddmm_batch<float> : sddmm_batch<half_t>)(true, many, m_vec, k, n, nonzeros_vec, row_indices, row_offsets,
+                                                                   col_indices, lhs_matrix, rhs_matrix, output_values, vec_length,
+                                                                   stream);
+}
+
+int vs_cuda_sddmm_f16_sorted(int batch, int m_vec, int k, int n, int nonzeros_vec, const int *row_indices,
+                             const int *row_offsets, const int *col_indices, const void *lhs_matrix,
+                             long long stride_lhs, const void *rhs_matrix, long long stride_rhs,
+                             void *output_values, long long stride_output, int f32_output, int vec_length, void *stream)
+{
+    vs::Batch many = make_batch(batch, stride_lhs, stride_rhs, stride_output);
+    many.sorted_columns = true;
+    return (f32_output ? sddmm_batch<float> : sddmm_batch<half_t>)(false, many, m_vec, k, n, nonzeros_vec, row_indices, row_offsets,
+                                                                   col_indices, lhs_matrix, rhs_matrix, output_values, vec_length,
+                                                                   stream);
 }
 
 int vs_wmma_spmm_softmax_f16_batched(int batch, int m_vec, int vec_length, int k, int n, int nonzeros_vec,

@@ -84,8 +84,18 @@ def _spmm(entry, m_vec, vec_length, k, n, row_indices, row_offsets, column_indic
 
 
 def _sddmm(entry, m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices, lhs_matrix, rhs_matrix,
-           output_values, vec_length, stream, algorithm=None):
+           output_values, vec_length, stream, algorithm=None, columns_sorted=False):
     f32 = isinstance(output_values, torch.Tensor) and output_values.dtype is torch.float32
+    if columns_sorted:
+        args = [1, m_vec, k, n, nonzeros_vec, _expect(row_indices, torch.int32, "row_indices"),
+                _expect(row_offsets, torch.int32, "row_offsets"), _expect(col_indices, torch.int32, "col_indices"),
+                _expect(lhs_matrix, torch.float16, "lhs_matrix"), 0, _expect(rhs_matrix, torch.float16, "rhs_matrix"), 0,
+                _expect(output_values, torch.float32 if f32 else torch.float16, "output_values"), 0, int(f32), vec_length,
+                _stream(stream)]
+        st = getattr(_lib.lib(), entry + "_sorted")(*args, *(() if algorithm is None else (algorithm,)))
+        if st:
+            _lib.check(st, entry + "_sorted")
+        return output_values
     fn = getattr(_lib.lib(), entry + "_f32out" if f32 else entry)
     args = [m_vec, k, n, nonzeros_vec, _expect(row_indices, torch.int32, "row_indices"),
             _expect(row_offsets, torch.int32, "row_offsets"), _expect(col_indices, torch.int32, "col_indices"),
@@ -198,29 +208,30 @@ class sddmm:
 
     @staticmethod
     def wmmaSddmm(m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices, lhs_matrix, rhs_matrix,
-                  output_values, vec_length, stream=None, algorithm=1):
-        """MFMA path (reference: src/wmma_sddmm.cu:3190-3202)."""
+                  output_values, vec_length, stream=None, algorithm=1, columns_sorted=False):
+        """MFMA path (reference: src/wmma_sddmm.cu:3190-3202).  columns_sorted: the columns of every row ascend, which
+        lets dense masks of short vectors run on whole tiles (vs_wmma_sddmm_f16_sorted)."""
         st = _native.wmma_sddmm(m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices, lhs_matrix,
-                                rhs_matrix, output_values, vec_length, stream, algorithm)
+                                rhs_matrix, output_values, vec_length, stream, algorithm, columns_sorted)
         if st == 0:
             return output_values
         if st > 0:
             _lib.check(st, "vs_wmma_sddmm_f16")
         return _sddmm("vs_wmma_sddmm_f16", m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices,
-                      lhs_matrix, rhs_matrix, output_values, vec_length, stream, algorithm)
+                      lhs_matrix, rhs_matrix, output_values, vec_length, stream, algorithm, columns_sorted)
 
     @staticmethod
     def cudaSddmm(m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices, lhs_matrix, rhs_matrix,
-                  output_values, vec_length, stream=None):
-        """Cross-lane dot-product path (reference: src/cuda_sddmm.cu:1295-1331)."""
+                  output_values, vec_length, stream=None, columns_sorted=False):
+        """Cross-lane dot-product path (reference: src/cuda_sddmm.cu:1295-1331).  columns_sorted: as in wmmaSddmm."""
         st = _native.cuda_sddmm(m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices, lhs_matrix,
-                                rhs_matrix, output_values, vec_length, stream)
+                                rhs_matrix, output_values, vec_length, stream, columns_sorted)
         if st == 0:
             return output_values
         if st > 0:
             _lib.check(st, "vs_cuda_sddmm_f16")
         return _sddmm("vs_cuda_sddmm_f16", m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices,
-                      lhs_matrix, rhs_matrix, output_values, vec_length, stream)
+                      lhs_matrix, rhs_matrix, output_values, vec_length, stream, columns_sorted=columns_sorted)
 
 
 def _stride(t, batch):
@@ -322,14 +333,15 @@ def sparse_attention(m_vec, vec_length, n, row_indices, row_offsets, col_indices
 
 
 def sddmm_batched(m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices, lhs_matrix, rhs_matrix,
-                  output_values, vec_length, kernel="wmma", stream=None, algorithm=1):
+                  output_values, vec_length, kernel="wmma", stream=None, algorithm=1, columns_sorted=False):
     """`batch` SDDMMs sharing one mask in one launch.
 
     lhs_matrix: [batch, m, k], rhs_matrix: [batch, n, k], output_values: [batch, nnz_vec, V], fp16.
+    columns_sorted: as in sddmm.wmmaSddmm.
     """
     batch = output_values.shape[0]
     st = _native.sddmm_batched(batch, m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices, lhs_matrix, rhs_matrix,
-                               output_values, vec_length, stream, algorithm if kernel == "wmma" else -1)
+                               output_values, vec_length, stream, algorithm if kernel == "wmma" else -1, columns_sorted)
     if st >= 0:
         _lib.check(st, "vs_%s_sddmm_f16_batched" % ("wmma" if kernel == "wmma" else "cuda"))
         return output_values
@@ -337,12 +349,11 @@ def sddmm_batched(m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indic
         _expect_batched(t, torch.float16, nm)
     args = [batch, m_vec, k, n, nonzeros_vec, _ptr(row_indices), _ptr(row_offsets), _ptr(col_indices),
             _ptr(lhs_matrix), _stride(lhs_matrix, batch), _ptr(rhs_matrix), _stride(rhs_matrix, batch),
-            _ptr(output_values), _stride(output_values, batch), vec_length, _stream(stream)]
+            _ptr(output_values), _stride(output_values, batch)]
+    args += [0, vec_length, _stream(stream)] if columns_sorted else [vec_length, _stream(stream)]
+    entry = "vs_%s_sddmm_f16_%s" % ("wmma" if kernel == "wmma" else "cuda", "sorted" if columns_sorted else "batched")
     if kernel == "wmma":
-        entry = "vs_wmma_sddmm_f16_batched"
         args.append(algorithm)
-    else:
-        entry = "vs_cuda_sddmm_f16_batched"
     _lib.check(getattr(_lib.lib(), entry)(*args), entry)
     return output_values
 
@@ -533,7 +544,7 @@ class SparseAttention:
             p.softmax_row_parts(scores, scale=scale, stream=stream)
             return p.spmm_row_parts(v, out=out, stream=stream, limit_vec=512, values=scores)
         sddmm_batched(p.m_vec, d, p.n, p.nnz_vec, p.row_indices, p.row_offsets, p.column_indices, q, k, scores,
-                      p.vec_length, kernel=kernel, stream=stream)
+                      p.vec_length, kernel=kernel, stream=stream, columns_sorted=p.columns_sorted)
         if fused:
             return spmm_softmax_batched(p.m_vec, p.vec_length, d_v, p.n, p.row_indices, p.row_offsets,
                                         p.column_indices, scores, v, out, scale, stream=stream,
@@ -686,6 +697,13 @@ def split_rows_pays(m_vec, nonzeros_vec, longest_row_vec):
     return longest_row_vec * m_vec >= 25.0 * nonzeros_vec
 
 
+def columns_ascend(row_offsets, column_indices):
+    """Whether the columns of every row ascend (repeated ones included)."""
+    columns = np.asarray(column_indices)
+    falls = np.flatnonzero(columns[1:] < columns[:-1]) + 1
+    return falls.size < len(row_offsets) and bool(np.isin(falls, row_offsets).all())
+
+
 class DeviceProblem:
     """Device-resident operands of one SpMM / SDDMM problem (caller-owned buffers, as in BmFN)."""
 
@@ -705,6 +723,7 @@ class DeviceProblem:
         self.row_indices = torch.from_numpy(swz).to(device)
         self.row_offsets = torch.from_numpy(np.ascontiguousarray(pattern.row_offsets)).to(device)
         self.column_indices = torch.from_numpy(np.ascontiguousarray(pattern.column_indices)).to(device)
+        self.columns_sorted = columns_ascend(pattern.row_offsets, pattern.column_indices)   # (a hint of the SDDMM)
         self._workspace = None  # partial tiles of the split-row SpMM, allocated on first use
         self._parts = {}        # limit -> (RowParts, its list on the device, workspace), made on first use
         self._parts_need = {}
@@ -828,6 +847,7 @@ class DeviceProblem:
         if kernel == "wmma":
             return sddmm.wmmaSddmm(self.m_vec, k, self.n, self.nnz_vec, self.row_indices, self.row_offsets,
                                    self.column_indices, lhs_matrix, rhs_matrix, out, self.vec_length, stream,
-                                   algorithm)
+                                   algorithm, self.columns_sorted)
         return sddmm.cudaSddmm(self.m_vec, k, self.n, self.nnz_vec, self.row_indices, self.row_offsets,
-                               self.column_indices, lhs_matrix, rhs_matrix, out, self.vec_length, stream)
+                               self.column_indices, lhs_matrix, rhs_matrix, out, self.vec_length, stream,
+                               self.columns_sorted)
