@@ -242,6 +242,22 @@ def test_algorithm_2_splits_the_nonzero_range_same_bits(gpu, V):
         assert_parity(got.cpu().numpy().reshape(-1), ref, name)
 
 
+@pytest.mark.parametrize("algorithm", [-2, -1, 3])
+@pytest.mark.parametrize("columns_sorted", [False, True])
+def test_batched_refuses_unknown_algorithms(gpu, algorithm, columns_sorted):
+    mask = cv.binomial_pattern(16, 64, 0.8, seed=1, vec_length=4)
+    prob = ops.DeviceProblem(mask)
+    A = torch.zeros((2, mask.m, 64), dtype=torch.float16, device="cuda")
+    B = torch.zeros((2, 64, 64), dtype=torch.float16, device="cuda")
+    out = torch.full((2, mask.nnz_vec, 4), 7.0, dtype=torch.float16, device="cuda")
+    for stream in (None, torch.cuda.current_stream()):
+        with pytest.raises(_lib.VSparseError):
+            ops.sddmm_batched(mask.m_vec, 64, 64, mask.nnz_vec, prob.row_indices, prob.row_offsets, prob.column_indices, A, B,
+                              out, 4, algorithm=algorithm, stream=stream, columns_sorted=columns_sorted)
+    torch.cuda.synchronize()
+    assert bool((out == 7.0).all())
+
+
 def test_algorithm_2_batched_equals_unbatched(gpu):
     V, heads, n, K = 8, 3, 640, 64
     rng = np.random.default_rng(5)

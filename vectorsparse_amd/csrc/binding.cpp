@@ -266,8 +266,9 @@ PyObject *spmm_softmax_batched(PyObject *, PyObject *const *args, Py_ssize_t n_a
     });
 }
 
-// (batch, m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices, lhs, rhs, out, vec_length, stream, algorithm,
-// columns_sorted); algorithm < 0: the fine-grained path
+// (batch, m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices, lhs, rhs, out, vec_length, stream, columns_sorted)
+// and, MFMA path, (..., algorithm)
+template <bool MFMA>
 PyObject *sddmm_batched(PyObject *, PyObject *const *args, Py_ssize_t n_args)
 {
     Reader r(args, n_args);
@@ -278,14 +279,15 @@ PyObject *sddmm_batched(PyObject *, PyObject *const *args, Py_ssize_t n_args)
     void *out = r.batched(batch, so);
     const int v = r.integer();
     void *stream = r.stream();
-    const int algorithm = r.integer();
     const bool sorted = r.flag();
+    const int algorithm = MFMA ? r.integer() : 0;
     return status_of(r, [&] {
-        if (sorted)
-            return algorithm < 0 ? vs_cuda_sddmm_f16_sorted(batch, m_vec, k, n, nnz, ri, ro, ci, lhs, sa, rhs, sb, out, so, 0, v, stream)
-                                 : vs_wmma_sddmm_f16_sorted(batch, m_vec, k, n, nnz, ri, ro, ci, lhs, sa, rhs, sb, out, so, 0, v, stream, algorithm);
-        return algorithm < 0 ? vs_cuda_sddmm_f16_batched(batch, m_vec, k, n, nnz, ri, ro, ci, lhs, sa, rhs, sb, out, so, v, stream)
-                             : vs_wmma_sddmm_f16_batched(batch, m_vec, k, n, nnz, ri, ro, ci, lhs, sa, rhs, sb, out, so, v, stream, algorithm);
+        if constexpr (MFMA)
+            return sorted ? vs_wmma_sddmm_f16_sorted(batch, m_vec, k, n, nnz, ri, ro, ci, lhs, sa, rhs, sb, out, so, 0, v, stream, algorithm)
+                          : vs_wmma_sddmm_f16_batched(batch, m_vec, k, n, nnz, ri, ro, ci, lhs, sa, rhs, sb, out, so, v, stream, algorithm);
+        else
+            return sorted ? vs_cuda_sddmm_f16_sorted(batch, m_vec, k, n, nnz, ri, ro, ci, lhs, sa, rhs, sb, out, so, 0, v, stream)
+                          : vs_cuda_sddmm_f16_batched(batch, m_vec, k, n, nnz, ri, ro, ci, lhs, sa, rhs, sb, out, so, v, stream);
     });
 }
 
@@ -399,7 +401,8 @@ PyMethodDef methods[] = {
     VS_METHOD("wmma_spmm_batched", wmma_spmm_batched),
     VS_METHOD("cuda_spmm_batched", cuda_spmm_batched),
     VS_METHOD("spmm_softmax_batched", spmm_softmax_batched),
-    VS_METHOD("sddmm_batched", sddmm_batched),
+    VS_METHOD("wmma_sddmm_batched", sddmm_batched<true>),
+    VS_METHOD("cuda_sddmm_batched", sddmm_batched<false>),
     VS_METHOD("sparse_softmax", sparse_softmax),
     VS_METHOD("sparse_attention", sparse_attention),
     VS_METHOD("spmm_row_parts", spmm_row_parts),

@@ -340,8 +340,12 @@ def sddmm_batched(m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indic
     columns_sorted: as in sddmm.wmmaSddmm.
     """
     batch = output_values.shape[0]
-    st = _native.sddmm_batched(batch, m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices, lhs_matrix, rhs_matrix,
-                               output_values, vec_length, stream, algorithm if kernel == "wmma" else -1, columns_sorted)
+    if kernel == "wmma":
+        st = _native.wmma_sddmm_batched(batch, m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices, lhs_matrix,
+                                        rhs_matrix, output_values, vec_length, stream, columns_sorted, algorithm)
+    else:
+        st = _native.cuda_sddmm_batched(batch, m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices, lhs_matrix,
+                                        rhs_matrix, output_values, vec_length, stream, columns_sorted)
     if st >= 0:
         _lib.check(st, "vs_%s_sddmm_f16_batched" % ("wmma" if kernel == "wmma" else "cuda"))
         return output_values
