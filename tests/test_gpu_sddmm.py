@@ -258,6 +258,32 @@ def test_batched_refuses_unknown_algorithms(gpu, algorithm, columns_sorted):
     assert bool((out == 7.0).all())
 
 
+@pytest.mark.parametrize("V", [1, 2, 4, 8])
+@pytest.mark.parametrize("K", [264, 288, 320, 352, 384, 416, 448, 480, 512, 544, 1000])
+def test_long_contractions_in_turns_of_any_length(gpu, K, V):
+    """K > 256: one, two or four groups of vectors per wave with turns of eight, four slices or one, the last turn shorter
+    (K = 288 ... 544: every remainder of both; 264, 1000: a cut slice); rows shorter and longer than a group, an empty one."""
+    rng = np.random.default_rng(K + V)
+    lengths = np.array([1, 15, 16, 17, 0, 70, 200, 33])
+    ro, ci = cv._pattern_from_lengths(rng, 8, 210, lengths)
+    mask = cv.ColVecCSR(8, 210, V, ro, ci)
+    A, B = cv.dense_normal(mask.m, K, seed=1), cv.dense_normal(210, K, seed=2)
+    ref = co.sddmm_host_ref_f32(8, K, V, ro, ci, A, B)
+    prob = ops.DeviceProblem(mask)
+    Ad, Bd = torch.from_numpy(A).cuda(), torch.from_numpy(B).cuda()
+    for dtype in (torch.float16, torch.float32):
+        outs = []
+        for group in (1, 2, 4):
+            pad = torch.full((mask.nnz_vec + 32, V), 7.0, dtype=dtype, device="cuda")
+            outs.append(pad[16:16 + mask.nnz_vec])
+            with _lib.thread_options(sddmm_group=group, sddmm_tile=1):
+                prob.sddmm(Ad, Bd, out=outs[-1], algorithm=1)
+            torch.cuda.synchronize()
+            assert bool((pad[:16] == 7.0).all()) and bool((pad[16 + mask.nnz_vec:] == 7.0).all())
+        assert_parity(outs[0].cpu().numpy().reshape(-1), ref, "K%d V%d" % (K, V))
+        assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+
+
 def test_algorithm_2_batched_equals_unbatched(gpu):
     V, heads, n, K = 8, 3, 640, 64
     rng = np.random.default_rng(5)

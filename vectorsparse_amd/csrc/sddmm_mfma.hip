@@ -124,9 +124,11 @@ sddmm_mfma_kernel(int m_vec, int K, int slots, int waves_per_block, const int *_
             }
         }
     } else {
-        // contractions beyond 256: eight slices of both operands in flight per turn (one at a time is a chain of K / 32
-        // round trips: 2048 x 2304 at 98 %, V = 4, K = 512, 10.3 us)
-        constexpr int TURN = 8;
+        // Contractions beyond 256: a turn requests TURN slices of both operands for its GRP groups of vectors, the last
+        // turn about as many as still cover the rest of K (sddmm_group: when which).  More slices per turn shorten a wave's chain of
+        // round trips, more groups share a slice of lhs and its four ds_bpermute: TURN = 8 takes 8 of those per group and
+        // slice, GRP = 4 takes 5.
+        constexpr int TURN = GRP == 1 ? 8 : (GRP == 2 ? 4 : 1);
         const int k_steps = (K + 31) >> 5;
         for (int sg = s; sg < n_super; sg += slots) {
             const int j0 = beg + SUPER * sg;
@@ -138,21 +140,42 @@ sddmm_mfma_kernel(int m_vec, int K, int slots, int waves_per_block, const int *_
                 rhs_row[u] = rhs + (size_t)col_indices[jl < end ? jl : end - 1] * K;
                 acc[u] = float4_t{0.f, 0.f, 0.f, 0.f};
             }
-            for (int kk = 0; kk < k_steps; kk += TURN) {
-                uint4_t a[TURN], raw[GRP][TURN];
+            auto turn = [&](auto slices, int kk) {
+                constexpr int N = decltype(slices)::value;
+                uint4_t a[N], raw[GRP][N];
 #pragma unroll
-                for (int t = 0; t < TURN; ++t) a[t] = load_slice16(lhs_row, kk + t, q, K, a_row_ok);
+                for (int t = 0; t < N; ++t) a[t] = load_slice16(lhs_row, kk + t, q, K, a_row_ok);
 #pragma unroll
                 for (int u = 0; u < GRP; ++u)
 #pragma unroll
-                    for (int t = 0; t < TURN; ++t) raw[u][t] = load_slice16(rhs_row[u], kk + t, q, K, true);
+                    for (int t = 0; t < N; ++t) raw[u][t] = load_slice16(rhs_row[u], kk + t, q, K, true);
 #pragma unroll
-                for (int t = 0; t < TURN; ++t) {
+                for (int t = 0; t < N; ++t) {
                     const half8_t at = to_mfma_order(a[t], src);
 #pragma unroll
                     for (int u = 0; u < GRP; ++u)
                         acc[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(at, to_mfma_order(raw[u][t], src), acc[u], 0, 0, 0);
                 }
+            };
+            if constexpr (TURN == 1) {
+                // (lhs first: its permutation is what the first product waits for)
+                for (int kk = 0; kk < k_steps; ++kk) {
+                    const half8_t a = to_mfma_order(load_slice16(lhs_row, kk, q, K, a_row_ok), src);
+                    uint4_t raw[GRP];
+#pragma unroll
+                    for (int u = 0; u < GRP; ++u) raw[u] = load_slice16(rhs_row[u], kk, q, K, true);
+#pragma unroll
+                    for (int u = 0; u < GRP; ++u)
+                        acc[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, to_mfma_order(raw[u], src), acc[u], 0, 0, 0);
+                }
+            } else {
+                int kk = 0;
+                for (; kk + TURN <= k_steps; kk += TURN) turn(std::integral_constant<int, TURN>{}, kk);
+                const int rest = k_steps - kk;
+                if (TURN > 4 && rest > 4) turn(std::integral_constant<int, TURN>{}, kk);
+                else if (rest > 2) turn(std::integral_constant<int, 4>{}, kk);
+                else if (rest > 1) turn(std::integral_constant<int, 2>{}, kk);
+                else if (rest > 0) turn(std::integral_constant<int, 1>{}, kk);
             }
             // The last product's registers that nobody reads (V = 1: three of four) were handed to the code below while the
             // product was still to land in them, three issue slots behind it across the loop's exit: the columns' number was
@@ -358,8 +381,14 @@ static int launch_one(int m_vec, int k, int nonzeros_vec, const int *row_indices
 static int sddmm_group(int k, long long nonzeros_vec)
 {
     const int forced = options().sddmm_group;
-    int grp = k <= 64 ? 4 : (k <= 128 ? 2 : 1);
+    int grp = k <= 64 || k > 256 ? 4 : (k <= 128 ? 2 : 1);
     if (forced == 1 || forced == 2 || forced == 4) return forced < grp ? forced : grp;
+    // K > 256, 819 masks (256 to 4096 rows, 50 to 98 %, K = 264 to 1024, every V), microseconds with one / two / four groups:
+    // V = 8, 512 x 512 at 90 %, K = 512 4.7 / 5.8 / 10.8; V = 4, 2048 x 2304 at 98 %, K = 512 6.5 / 6.8 / 10.8; V = 1, 512 x 512
+    // at 80 %, K = 264 6.8 / 4.9 / 5.4; V = 8, 4096 x 4096 at 95 %, K = 320 9.4 / 9.6 / 7.9.  Against four groups throughout
+    // the choice takes 0.81 of the time in the mean (worst 1.14), against one group throughout 0.93 (worst 1.23), against the
+    // fastest of the three 1.07: above 98304 two groups can be faster (by up to 1.4) or slower (by up to 1.3).
+    if (k > 256) return nonzeros_vec < 24000 ? 1 : (nonzeros_vec < 98304 ? 2 : 4);
     while (grp > 1 && nonzeros_vec / (16 * grp) < 4096) grp >>= 1;
     return grp;
 }
@@ -388,7 +417,7 @@ static int launch_ks(int m_vec, int k, int nonzeros_vec, const int *row_indices,
     if (k <= 64) return launch_grp<V, 2, OutT>(grp, m_vec, k, nonzeros_vec, row_indices, row_offsets, col_indices, lhs, rhs, out, stream, batch);
     if (k <= 128) return launch_grp<V, 4, OutT>(grp, m_vec, k, nonzeros_vec, row_indices, row_offsets, col_indices, lhs, rhs, out, stream, batch);
     if (k <= 256) return launch_one<V, 8, 1, OutT>(m_vec, k, nonzeros_vec, row_indices, row_offsets, col_indices, lhs, rhs, out, stream, batch);
-    return launch_one<V, 0, 1, OutT>(m_vec, k, nonzeros_vec, row_indices, row_offsets, col_indices, lhs, rhs, out, stream, batch);
+    return launch_grp<V, 0, OutT>(grp, m_vec, k, nonzeros_vec, row_indices, row_offsets, col_indices, lhs, rhs, out, stream, batch);
 }
 
 // Waves per vector row.  Waves are independent (no reduction).  A wave that finds no super-group of its own exits
@@ -443,14 +472,17 @@ int launch_sddmm_mfma(int m_vec, int k, int n, int nonzeros_vec, const int *row_
     }
     // algorithm 0 (automatic): vectors of 1 to 8 rows fill 1/16 to 8/16 of an MFMA tile, and on masks of few
     // nonzeros the fine-grained kernel (dot products on the vector ALU, reduced across lanes with DPP) is ahead:
-    // over the M = N = 512..4096, K = 64..256 grid by 5-40 % below these nonzero counts, behind above them.
+    // over the M = N = 512..4096, K = 64..256 grid by 5-40 % below these nonzero counts, behind above them.  Beyond K = 256
+    // (410 masks of 256 to 4096 rows, V = 4 and 8, K = 264 to 1024) the matrix cores throughout take 1.17 and 1.11 of the faster
+    // one's time, the vector ALU throughout 1.21 and 1.42, these limits 1.01 (V = 8, 2048 x 2304 at 98 %, K = 1024: 12.8 us on the
+    // vector ALU, 9.9 us on the matrix cores; 512 x 512 at 95 %: 3.6 against 7.5 us).
     if (batch.algorithm == 0 && !batch.row_parts) {
         const long long total = (long long)nonzeros_vec * batch.count;
         long long limit = 0;
         if (vec_length == 1) limit = 800000;
         else if (vec_length == 2) limit = k >= 256 ? 200000 : (k >= 128 ? 16000 : 0);
-        else if (vec_length == 4) limit = k > 256 ? 40000 : (k >= 256 ? 16000 : (k >= 128 ? 8000 : 0));
-        else limit = k > 256 ? 12000 : 0;
+        else if (vec_length == 4) limit = k > 512 ? 16000 : (k > 256 ? 40000 : (k >= 256 ? 16000 : (k >= 128 ? 8000 : 0)));
+        else limit = k > 256 ? 4000 : 0;
         if (total <= limit)
             return launch_sddmm_valu<OutT>(m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices, lhs, rhs, out,
                                            vec_length, stream, batch);
