@@ -380,3 +380,11 @@ def test_columns_that_ascend_are_recognised():
     assert not ascend([0, 3, 5], [0, 7, 2, 0, 1])
     assert not ascend([0, 2, 5], [0, 7, 1, 0, 2])
     assert not ascend([0, 5], [4, 3, 2, 1, 0])
+
+
+@pytest.mark.parametrize("n,waves", [(16, 1), (32, 1), (33, 2), (64, 2), (128, 2), (147, 2), (192, 2), (193, 4), (256, 4), (384, 4), (385, 8), (512, 8)])
+def test_waves_of_short_rows_of_unknown_length(n, waves):
+    """Small grids that ask for as many waves as a row can use, row lengths unknown: a wave per 96 columns, two at least
+    where there are two steps of 32 (a wave per 128 columns: up to 20 % slower on rows that hold half of n)."""
+    for V in (1, 2, 4, 8):
+        assert ops.spmm_launch_shape(64 // V, V, 205, n)["waves"] == waves
