@@ -1,10 +1,13 @@
-"""Arguments the compiled binding (csrc/binding.cpp) does not take: they reach the checks of ops.py and end as Python
-exceptions, never as a C++ exception that leaves a C function."""
+"""Arguments the compiled binding (csrc/binding.cpp) does not take: it answers with a negative status, they reach the
+checks of ops.py and end as Python exceptions, never as a C++ exception that leaves a C function."""
 import pytest
 import torch
 from torch._subclasses.fake_tensor import FakeTensorMode
 
-from vectorsparse_amd import ops
+from vectorsparse_amd import _lib, ops
+
+ENTRIES = {"wmmaSpmm": "wmma_spmm", "cudaSpmm": "cuda_spmm", "wmmaSddmm": "wmma_sddmm", "cudaSddmm": "cuda_sddmm",
+           "sddmm_batched": "wmma_sddmm_batched", "sparse_softmax": "sparse_softmax", "spmm_batched": "wmma_spmm_batched"}
 
 
 def _operands(device):
@@ -28,15 +31,49 @@ def _calls(device):
     }
 
 
-@pytest.mark.parametrize("name", sorted(_calls("cpu")))
-def test_tensors_without_storage_raise(name):
+class _Recorder:
+    """The compiled binding, with every answer noted."""
+
+    def __init__(self):
+        _lib.lib()
+        from vectorsparse_amd import _binding
+        self.binding, self.answers = _binding, []
+
+    def __getattr__(self, name):
+        def call(*args):
+            self.answers.append((name, getattr(self.binding, name)(*args)))
+            return self.answers[-1][1]
+        return call
+
+
+@pytest.fixture
+def recorder(monkeypatch):
+    r = _Recorder()
+    monkeypatch.setattr(ops, "_native", r)
+    return r
+
+
+@pytest.mark.parametrize("name", sorted(ENTRIES))
+def test_tensors_without_storage_raise(name, recorder):
     with FakeTensorMode():
         call = _calls("cuda")[name]
-        with pytest.raises(Exception):
+        with pytest.raises((RuntimeError, ValueError)):
             call()
+    assert recorder.answers == [(ENTRIES[name], -1)]
 
 
-@pytest.mark.parametrize("name", ["wmmaSpmm", "cudaSpmm", "wmmaSddmm", "cudaSddmm"])
-def test_host_tensors_raise(name):
-    with pytest.raises(Exception):
+@pytest.mark.parametrize("name", sorted(ENTRIES))
+def test_host_tensors_raise(name, recorder):
+    with pytest.raises(ValueError, match="device memory"):
         _calls("cpu")[name]()
+    assert recorder.answers == [(ENTRIES[name], -1)]
+
+
+def test_wrong_argument_counts_and_types_are_unusual_not_fatal():
+    binding = _Recorder().binding
+    for name in dir(binding):
+        if not name.startswith("_"):
+            assert getattr(binding, name)() == -1
+            assert getattr(binding, name)(*range(17)) == -1
+            assert getattr(binding, name)(*([None] * 12)) == -1
+            assert getattr(binding, name)(1 << 80, "x", 2.5) == -1

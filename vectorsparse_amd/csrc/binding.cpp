@@ -129,6 +129,14 @@ struct Reader {
         }
         return t->data_ptr();
     }
+    // batched, of an operand that is written: no two problems may share an element
+    void *batched_output(int batch, long long &stride)
+    {
+        const at::Tensor *t = ok && left > 0 && THPVariable_Check(*args) ? &THPVariable_Unpack(*args) : nullptr;
+        void *const p = batched(batch, stride);
+        if (ok && batch != 1 && t->dim() == 3 && stride < (long long)t->size(1) * t->size(2)) ok = false;
+        return p;
+    }
     // bytes of a caller's buffer, or None
     void *buffer(long long &bytes)
     {
@@ -336,7 +344,7 @@ PyObject *spmm_row_parts(PyObject *, PyObject *const *args, Py_ssize_t n_args)
     const int *ci = (const int *)r.indices();
     long long sa, sb, so, ws_bytes;
     const void *values = r.batched(batch, sa), *rhs = r.batched(batch, sb);
-    void *out = r.batched(batch, so), *ws = r.buffer(ws_bytes), *stream = r.stream();
+    void *out = r.batched_output(batch, so), *ws = r.buffer(ws_bytes), *stream = r.stream();
     return status_of(r, [&] {
         return vs_wmma_spmm_f16_row_parts(batch, vec, k, n, n_slots, slots, n_split, parts_max, nnz, longest, ci, values, sa, rhs, sb,
                                           out, so, ws, ws_bytes, stream);
@@ -353,7 +361,7 @@ PyObject *sddmm_row_parts(PyObject *, PyObject *const *args, Py_ssize_t n_args)
     const int *ci = (const int *)r.indices();
     long long sa, sb, so;
     const void *lhs = r.batched(batch, sa), *rhs = r.batched(batch, sb);
-    void *out = r.batched(batch, so);
+    void *out = r.batched_output(batch, so);
     const int vec = r.integer();
     void *stream = r.stream();
     return status_of(r, [&] {
@@ -370,7 +378,7 @@ PyObject *softmax_row_parts(PyObject *, PyObject *const *args, Py_ssize_t n_args
     const int n_split = r.integer(), parts_max = r.integer();
     long long si, so, ws_bytes;
     const void *in = r.batched(batch, si);
-    void *out = r.batched(batch, so);
+    void *out = r.batched_output(batch, so);
     const float scale = r.number();
     void *ws = r.buffer(ws_bytes), *stream = r.stream();
     return status_of(r, [&] {

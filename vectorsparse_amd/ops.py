@@ -391,6 +391,18 @@ def _expect_batched(t, dtype, name):
         raise ValueError("%s must be contiguous in its trailing dimensions" % name)
 
 
+def _row_parts_operand(t, name, written=False):
+    """Checks of an fp16 operand [rows, columns] or [batch, rows, columns] of the row-part operators; its address (raw
+    addresses pass).  Problems may lie any distance apart, those that are written not on top of each other."""
+    if t is None or type(t) is int:
+        return t
+    batched = t.dim() == 3 and t.shape[0] > 0
+    _expect(t[0] if batched else t, torch.float16, name)
+    if written and batched and t.shape[0] > 1 and t.stride(0) < t.shape[1] * t.shape[2]:
+        raise ValueError("%s: the problems of a batch must not overlap" % name)
+    return t.data_ptr()
+
+
 def sparse_attention_plan(m_vec, vec_length, n, d_qk, d_v, rows_per_workgroup, row_offsets, col_indices, stream=None):
     """Analyse a fixed mask once for the union-gather kernel: returns the plan (a device byte tensor) that
     `sparse_attention(..., rows_per_workgroup=..., plan=...)` reads instead of rebuilding it per launch."""
@@ -623,9 +635,9 @@ def spmm_row_parts(vec_length, k, n, parts, slots, nonzeros_vec, column_indices,
     st = _lib.lib().vs_wmma_spmm_f16_row_parts(
         batch, vec_length, k, n, parts.n_slots, _expect(slots, torch.int32, "slots"), parts.n_split, parts.parts_max,
         nonzeros_vec, parts.longest_part_vec, _expect(column_indices, torch.int32, "column_indices"),
-        _expect(values, torch.float16, "values"), per_problem(values, 2),
-        _expect(rhs_matrix, torch.float16, "rhs_matrix"), per_problem(rhs_matrix, 2),
-        _expect(output_matrix, torch.float16, "output_matrix"), per_problem(output_matrix, 2), _ptr(workspace), ws_bytes,
+        _row_parts_operand(values, "values"), per_problem(values, 2),
+        _row_parts_operand(rhs_matrix, "rhs_matrix"), per_problem(rhs_matrix, 2),
+        _row_parts_operand(output_matrix, "output_matrix", written=True), per_problem(output_matrix, 2), _ptr(workspace), ws_bytes,
         _stream(stream))
     if st:
         _lib.check(st, "vs_wmma_spmm_f16_row_parts")
@@ -647,9 +659,9 @@ def sddmm_row_parts(k, n, parts, slots, nonzeros_vec, col_indices, lhs_matrix, r
     per_problem = lambda t, dims: _stride(t, batch)
     st = _lib.lib().vs_wmma_sddmm_f16_row_parts(
         batch, k, n, parts.n_slots, _expect(slots, torch.int32, "slots"), nonzeros_vec,
-        _expect(col_indices, torch.int32, "col_indices"), _expect(lhs_matrix, torch.float16, "lhs_matrix"),
-        per_problem(lhs_matrix, 2), _expect(rhs_matrix, torch.float16, "rhs_matrix"), per_problem(rhs_matrix, 2),
-        _expect(output_values, torch.float16, "output_values"), per_problem(output_values, 2), vec_length, _stream(stream))
+        _expect(col_indices, torch.int32, "col_indices"), _row_parts_operand(lhs_matrix, "lhs_matrix"),
+        per_problem(lhs_matrix, 2), _row_parts_operand(rhs_matrix, "rhs_matrix"), per_problem(rhs_matrix, 2),
+        _row_parts_operand(output_values, "output_values", written=True), per_problem(output_values, 2), vec_length, _stream(stream))
     if st:
         _lib.check(st, "vs_wmma_sddmm_f16_row_parts")
     return output_values
@@ -673,8 +685,8 @@ def sparse_softmax_row_parts(vec_length, parts, slots, values_in, values_out=Non
     ws_bytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
     st = _lib.lib().vs_sparse_softmax_f16_row_parts(
         batch, vec_length, parts.n_slots, _expect(slots, torch.int32, "slots"), parts.n_split, parts.parts_max,
-        _expect(values_in, torch.float16, "values_in"), stride(values_in),
-        _expect(values_out, torch.float16, "values_out"), stride(values_out), float(scale), _ptr(workspace), ws_bytes,
+        _row_parts_operand(values_in, "values_in"), stride(values_in),
+        _row_parts_operand(values_out, "values_out", written=True), stride(values_out), float(scale), _ptr(workspace), ws_bytes,
         _stream(stream))
     if st:
         _lib.check(st, "vs_sparse_softmax_f16_row_parts")
