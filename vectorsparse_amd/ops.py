@@ -715,9 +715,10 @@ def split_rows_pays(m_vec, nonzeros_vec, longest_row_vec):
 
 def columns_ascend(row_offsets, column_indices):
     """Whether the columns of every row ascend (repeated ones included)."""
-    columns = np.asarray(column_indices)
-    falls = np.flatnonzero(columns[1:] < columns[:-1]) + 1
-    return falls.size < len(row_offsets) and bool(np.isin(falls, row_offsets).all())
+    columns, starts = np.asarray(column_indices), np.asarray(row_offsets)
+    falls = columns[1:] < columns[:-1]
+    falls[starts[(starts > 0) & (starts < columns.size)] - 1] = False
+    return not falls.any()
 
 
 class DeviceProblem:
