@@ -92,7 +92,8 @@ def test_dense_tiles_batched(gpu):
 def test_the_automatic_route_takes_tiles_only_where_columns_ascend(gpu, kernel):
     """A mask dense enough for tiles (V = 1, 512 x 1024 at 50 %, K = 256; gathering it takes the fine-grained kernel, whose
     fp32 bits are not those of the matrix cores): ascending columns known to the caller run on tiles, the same columns
-    without that word, or shuffled ones, are gathered, and a wrong word changes no bit."""
+    without that word, or shuffled ones, are gathered, and a wrong word changes no bit.  At 98 % gathering is expected to be
+    faster whatever the order."""
     mask = cv.binomial_pattern(512, 1024, 0.5, seed=9, vec_length=1)
     A = torch.from_numpy(cv.dense_normal(mask.m, 256, seed=10)).cuda()
     B = torch.from_numpy(cv.dense_normal(mask.n, 256, seed=11)).cuda()
@@ -117,3 +118,11 @@ def test_the_automatic_route_takes_tiles_only_where_columns_ascend(gpu, kernel):
             ops.sddmm_batched(*args, kernel=kernel, stream=stream, columns_sorted=True, **extra)
             assert torch.equal(one[0], matrix_cores.half())
         torch.cuda.synchronize()
+    sparse = cv.binomial_pattern(512, 1024, 0.98, seed=9, vec_length=1)
+    prob = ops.DeviceProblem(sparse)
+    assert prob.columns_sorted
+    with _lib.thread_options(sddmm_tile=1):
+        gathered = prob.sddmm(A, B, kernel=kernel, out_dtype=torch.float32)
+    with _lib.thread_options(sddmm_tile=2):
+        tiles = prob.sddmm(A, B, kernel=kernel, out_dtype=torch.float32)
+    assert torch.equal(prob.sddmm(A, B, kernel=kernel, out_dtype=torch.float32), gathered) and not torch.equal(gathered, tiles)

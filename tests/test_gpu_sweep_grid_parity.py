@@ -7,7 +7,7 @@ import pytest
 import torch
 
 from oracle import c_oracle as co
-from vectorsparse_amd import ops, sweep
+from vectorsparse_amd import _lib, ops, sweep
 from vectorsparse_amd import colvec_csr as cv
 from util import assert_parity
 
@@ -61,10 +61,12 @@ def test_every_sddmm_point_of_the_grid(gpu, M, V):
             pat = sweep.sddmm_grid_pattern(M, s, V)
             ref = co.sddmm_host_ref_f32(pat.m_vec, K, V, pat.row_offsets, pat.column_indices, A, B)
             prob = ops.DeviceProblem(pat, sort=True)
-            for kernel in ("wmma", "cuda"):
+            # the automatic route (dense tiles on about a third of the points) and both gathering kernels
+            for kernel, options in (("wmma", {}), ("wmma", dict(sddmm_tile=1)), ("cuda", dict(sddmm_tile=1))):
                 out = torch.full((pat.nnz_vec, V), float("nan"), dtype=torch.float16, device="cuda")
-                prob.sddmm(Ad, Bd, kernel=kernel, out=out)
-                assert_parity(out.cpu().numpy().reshape(-1), ref, "sddmm M%d K%d s%g V%d %s" % (M, K, s, V, kernel))
+                with _lib.thread_options(**options):
+                    prob.sddmm(Ad, Bd, kernel=kernel, out=out)
+                assert_parity(out.cpu().numpy().reshape(-1), ref, "sddmm M%d K%d s%g V%d %s %s" % (M, K, s, V, kernel, options))
                 ok, rel = sweep.verify_sddmm(pat, A, B, out.cpu().numpy())
                 assert ok and rel <= 1e-2
             points += 1
