@@ -98,7 +98,8 @@ def kernel_source_tag(*names):
 
 
 SPMM_SOURCES = ("spmm_mfma.hip", "spmm_mfma_step.hpp", "vs_common.hpp")
-SDDMM_SOURCES = ("sddmm_mfma.hip", "vs_common.hpp")
+# (sddmm_tile.hip decides whether a mask is gathered at all)
+SDDMM_SOURCES = ("sddmm_mfma.hip", "sddmm_tile.hip", "vs_common.hpp")
 
 
 def measured_traffic(path, sources):
@@ -169,7 +170,7 @@ def cpu_baseline(pat, B, n_dense, flops, budget_s=12.0):
     }
 
 
-PMC_MODES = ["spmm", "spmm_largest", "spmm_slab_50", "spmm_slab_90", "spmm_valu_v1", "sddmm_valu_v1", "sddmm_k128", "spmm_dma", "spmm_split_rows", "spmm_row_parts", "sddmm", "attention",
+PMC_MODES = ["spmm", "spmm_largest", "spmm_slab_50", "spmm_slab_90", "spmm_valu_v1", "spmm_ragged", "sddmm_valu_v1", "sddmm_tile", "sddmm_k128", "spmm_dma", "spmm_split_rows", "spmm_row_parts", "sddmm", "attention",
              "attention_window"]
 
 
@@ -451,11 +452,35 @@ def main():
             vmask = fine_grained_sddmm_mask(cv)
             vsprob = ops.DeviceProblem(vmask)
             vsout = torch.empty((vmask.nnz_vec, 1), dtype=torch.float16, device="cuda")
-            for _ in range(10):
-                vsprob.sddmm(lhs, rhs, kernel="cuda", out=vsout)
+            with _lib.thread_options(sddmm_tile=1):
+                for _ in range(10):
+                    vsprob.sddmm(lhs, rhs, kernel="cuda", out=vsout)
             info["algorithmic_bytes"] = sddmm_algorithmic_bytes(vmask, 64)
             info["nonzero_vectors"] = int(vmask.nnz_vec)
             info["kernel_source_tag"] = kernel_source_tag("sddmm_valu.hip", "vs_common.hpp")
+        elif args.pmc == "sddmm_tile":
+            # the SDDMM on dense tiles: 4096 x 4096 at 80 %, V = 1, K = 256
+            tmask = cv.binomial_pattern(4096, 4096, 0.8, seed=31, vec_length=1)
+            tprob = ops.DeviceProblem(tmask)
+            tlhs = torch.from_numpy(cv.dense_normal(4096, 256, seed=32)).cuda()
+            trhs = torch.from_numpy(cv.dense_normal(4096, 256, seed=33)).cuda()
+            tout = torch.empty((tmask.nnz_vec, 1), dtype=torch.float16, device="cuda")
+            for _ in range(10):
+                tprob.sddmm(tlhs, trhs, kernel="wmma", out=tout)
+            info["algorithmic_bytes"] = sddmm_algorithmic_bytes(tmask, 256)
+            info["nonzero_vectors"] = int(tmask.nnz_vec)
+            info["kernel_source_tag"] = kernel_source_tag("sddmm_tile.hip", "vs_common.hpp")
+        elif args.pmc == "spmm_ragged":
+            # a dense width that is a multiple of nothing: 1022 x 147 at 70 %, V = 2, N = 205, fp32 outputs
+            rpat = cv.random_values(cv.binomial_pattern(511, 147, 0.7, seed=34, vec_length=2), seed=35)
+            rprob = ops.DeviceProblem(rpat)
+            rBd = torch.from_numpy(cv.dense_uniform(147, 205, seed=36)).cuda()
+            rout = torch.empty((rpat.m, 205), dtype=torch.float32, device="cuda")
+            for _ in range(10):
+                rprob.spmm(rBd, kernel="wmma", out=rout)
+            info["algorithmic_bytes"] = spmm_algorithmic_bytes(rpat, 205) + 2 * rpat.m * 205   # (fp32 outputs)
+            info["nonzero_vectors"] = int(rpat.nnz_vec)
+            info["kernel_source_tag"] = kernel_source_tag(*SPMM_SOURCES)
         elif args.pmc == "sddmm_k128":
             lhs128 = torch.from_numpy(cv.dense_normal(2048, 128, seed=15)).cuda()
             rhs128 = torch.from_numpy(cv.dense_normal(2048, 128, seed=25)).cuda()
@@ -666,8 +691,10 @@ def main():
     vmask = fine_grained_sddmm_mask(cv)
     vsprob = ops.DeviceProblem(vmask)
     vsout = torch.empty((vmask.nnz_vec, 1), dtype=torch.float16, device="cuda")
-    _, v1_sddmm_valu_ms = time_graph(torch, lambda: vsprob.sddmm(lhs, rhs, kernel="cuda", out=vsout), fine_steps, 3)
-    _, v1_sddmm_mfma_ms = time_graph(torch, lambda: vsprob.sddmm(lhs, rhs, kernel="wmma", out=vsout, algorithm=1), fine_steps, 3)
+    with _lib.thread_options(sddmm_tile=1):     # (both gathering kernels; the automatic choice multiplies whole tiles here)
+        _, v1_sddmm_valu_ms = time_graph(torch, lambda: vsprob.sddmm(lhs, rhs, kernel="cuda", out=vsout), fine_steps, 3)
+        _, v1_sddmm_mfma_ms = time_graph(torch, lambda: vsprob.sddmm(lhs, rhs, kernel="wmma", out=vsout, algorithm=1), fine_steps, 3)
+    _, v1_sddmm_tile_ms = time_graph(torch, lambda: vsprob.sddmm(lhs, rhs, kernel="wmma", out=vsout), fine_steps, 3)
     v1_sddmm_bytes, v1_sddmm_flops = sddmm_algorithmic_bytes(vmask, 64), 2.0 * vmask.nnz * 64
 
     # ---- config 4's other three points (K = 128, and 95 % sparsity)
@@ -780,7 +807,9 @@ def main():
                                       tflops=v1_sddmm_flops / (v1_sddmm_valu_ms * 1e-3) * 1e-12),
                     "wmma_path": dict(hbm(v1_sddmm_bytes, v1_sddmm_mfma_ms, kernel="sddmm_mfma_kernel<V=1>"),
                                       tflops=v1_sddmm_flops / (v1_sddmm_mfma_ms * 1e-3) * 1e-12),
-                    "cuda_over_wmma": v1_sddmm_mfma_ms / v1_sddmm_valu_ms},
+                    "cuda_over_wmma": v1_sddmm_mfma_ms / v1_sddmm_valu_ms,
+                    "automatic": dict(hbm(v1_sddmm_bytes, v1_sddmm_tile_ms, kernel="sddmm_tile_kernel<V=1>"),
+                                      tflops=v1_sddmm_flops / (v1_sddmm_tile_ms * 1e-3) * 1e-12)},
                 "spmm_config2": dict(hbm(alg_bytes, valu_spmm_ms, kernel="spmm_valu_kernel<V=8>"),
                                      tflops=flops / (valu_spmm_ms * 1e-3) * 1e-12, speedup_vs_dense_gemm=dense_ms / valu_spmm_ms),
                 "sddmm_config4_k64": dict(hbm(sddmm_bytes, valu_sddmm_ms, kernel="sddmm_valu_kernel<V=8>"),
