@@ -367,7 +367,7 @@ int vs_cuda_sddmm_f16_batched(int batch, int m_vec, int k, int n, int nonzeros_v
  * strides for a single problem.  Masks that keep a good share of large tiles (short vectors, low sparsity) then multiply
  * whole tiles on the matrix cores and keep the masked outputs, for k % 8 == 0 and `algorithm` 0 or 1 (option
  * "sddmm_tile"): the bits of schedule 1.  Otherwise they are the entry points named above.  The order is a hint: columns in
- * another order give the same bits, several times slower.  No counterpart in the reference, whose kernels gather.
+ * another order give the same bits, an order of magnitude slower.  No counterpart in the reference, whose kernels gather.
  */
 int vs_wmma_sddmm_f16_sorted(int batch, int m_vec, int k, int n, int nonzeros_vec,
                              const int *row_indices, const int *row_offsets,

@@ -14,7 +14,8 @@
 // first nonzero and the last one its end, so every nonzero lies between the two bounds of at least one tile whatever
 // the order - of several, where the bounds of the row do not ascend.  A nonzero found in a tile that does not hold its
 // column is multiplied there by itself, to the same bits, so that it does not matter which of its tiles writes it last.
-// (Slow: with shuffled columns two nonzeros in three lie in several tiles.)
+// (Slow: with shuffled columns two nonzeros in three lie in several tiles; 4096 x 4096, V = 1, K = 256, 80 %:
+// 1130 us against 19 us sorted and 87 us gathered.)
 //
 // What bounds it (4096 x 4096, V = 1, K = 256, 80 %, tiles of 128: 20.2 us): nothing alone - vector ALU 8 us, LDS 6 us, matrix
 // cores 4 us, 224 MB through the L2s 10 us, around a tile's chain of dependent loads (row extent, two probes, columns) of
@@ -376,20 +377,26 @@ sddmm_tile_kernel(int m_vec, int K, int n, int row_blocks, int column_tiles, con
         if (base < end) fetch_columns(base);
     }
 
-    // Rows of unsorted columns: the wave multiplies such nonzeros one by one, on the matrix cores and in the same steps of
-    // 32 as the tiles.  Such a nonzero can lie between the bounds of several tiles, its own among them; whichever of them
-    // writes it last, it writes the same bits.
+    // Rows of unsorted columns: the wave multiplies such nonzeros 16 / V at a time, each with its own rows of both operands
+    // (the results wanted are the product's diagonal), on the matrix cores and in the same steps of 32 as the tiles.  Such
+    // a nonzero can lie between the bounds of several tiles, its own among them; whichever of them writes it last, it
+    // writes the same bits.
     if (__builtin_amdgcn_ballot_w64(elsewhere) == 0) return;
+    constexpr int AT_ONCE = 16 / V;
     for (int j = beg + li; __builtin_amdgcn_ballot_w64(j < end) != 0; j += LPR) {
         const int column = j < end ? col_indices[j] : c0;
-        uint64_t todo = __builtin_amdgcn_ballot_w64((unsigned)(column - c0) >= (unsigned)TN);
-        while (todo != 0) {
-            const int from = __builtin_ctzll(todo);
-            todo &= todo - 1;
-            const int its_row = __builtin_amdgcn_readlane(row, from), its_column = __builtin_amdgcn_readlane(column, from);
-            const int its_j = __builtin_amdgcn_readlane(j, from);
-            // (lanes past the vector's rows repeat one of them; every column of the product is the same)
-            const half_t *const a = lhs + ((size_t)its_row * V + c % V) * K, *const b = rhs + (size_t)its_column * K;
+        const bool mine = (unsigned)(column - c0) >= (unsigned)TN;
+        const uint64_t some_lanes = __builtin_amdgcn_ballot_w64(mine);
+        const int rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(some_lanes >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)some_lanes, 0));
+        for (int first = 0, left = __builtin_popcountll(some_lanes); left > 0; first += AT_ONCE, left -= AT_ONCE) {
+            // lane i < AT_ONCE gets nonzero `first + i` (the last lane takes what is not wanted)
+            const int to = 4 * (mine && rank >= first && rank < first + AT_ONCE ? rank - first : 63);
+            const int rows = __builtin_amdgcn_ds_permute(to, row), columns = __builtin_amdgcn_ds_permute(to, column);
+            const int places = __builtin_amdgcn_ds_permute(to, j);
+            const int its_row = __builtin_amdgcn_ds_bpermute(4 * (c / V), rows), its_column = __builtin_amdgcn_ds_bpermute(4 * c, columns);
+            const int its_place = __builtin_amdgcn_ds_bpermute(4 * c, places);
+            const half_t *const a = lhs + ((size_t)(c / V < left ? its_row : rb * ROWS) * V + c % V) * K;
+            const half_t *const b = rhs + (size_t)(c < AT_ONCE && c < left ? its_column : c0) * K;
             float4_t sum = {0.f, 0.f, 0.f, 0.f};
             for (int k0 = 0; k0 < K; k0 += 32) {
                 const bool there = k0 + 8 * g < K;
@@ -401,11 +408,9 @@ sddmm_tile_kernel(int m_vec, int K, int n, int row_blocks, int column_tiles, con
             }
             // (all four results land before a register of those that are not stored is used again)
             asm volatile("s_nop 15" : "+v"(sum));
-            if (c == 0) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (4 * g + e < V) out[(size_t)its_j * V + 4 * g + e] = (OutT)sum[e];
-            }
+            for (int e = 0; e < 4; ++e)
+                if (c < left && (4 * g + e) / V == c) out[(size_t)its_place * V + (4 * g + e) % V] = (OutT)sum[e];
         }
     }
 }
@@ -439,10 +444,13 @@ int launch_tile_shape(bool wide, int m_vec, int k, int n, const int *row_offsets
 // L2s the longer the vectors (a MB of gathered rows in 0.064 us at V = 1, 0.1 us at V = 8, whose waves hold fewer of them).
 // Tiles: up to 512 tiles of 64 x 64 all run at once and a launch costs one tile's chain (search, product, sampling); larger
 // problems take tiles of 128 x 128 (half the operand traffic), a quarter of a thousand at a time, 0.7 us per 64 of K; the
-// masked outputs come on top.  Over the 600 problems the rule is 0.3 % off always taking the faster side and leaves 30 % of
-// them to the tiles.  4096 x 4096, V = 1, K = 256: 196 / 90 / 50 / 13.4 us gathering at 50 / 80 / 90 / 98 %, 26.7 / 20.2 / 18.9 /
-// 17.9 us on tiles; 2048 x 2304, V = 4, K = 512, 90 %: 16.0 against 12.3 us; 2048 x 2048, V = 8, K = 64: 2.8 against 4.2 us at
-// 90 %, 5.7 against 5.0 us at 50 %.
+// masked outputs come on top.  Over 1400 problems of the same ranges the rule is 0.6 % off always taking the faster side; it
+// sends 213 of them to the tiles and is wrong by more than 3 % on eight (by 11 % at most: either side's estimate is
+// good to about that).  A line that spares those eight (0.80 for 0.92) gathers others that tiles serve up to 1.6 times faster.
+// 4096 x 4096, V = 1, K = 256: 190 / 80 / 43 / 11.4 us gathering at 50 / 80 / 90 / 98 %, 26.1 / 18.9 / 17.5 / 16.2 us on tiles;
+// 2048 x 2304, V = 4, K = 512: 14.7 against 11.2 us at 90 %, 4.7 against 10.7 us at 98 %; 2048 x 2048, V = 8, K = 64: 2.5 against
+// 3.8 us at 90 %, 5.0 against 4.6 us at 50 %; at the line, 2048 x 2048, V = 1, K = 64: 8.3 / 5.1 / 3.6 against 5.8 / 5.4 / 5.1 us
+// at 80 / 90 / 95 % (tiles at 80 and 90 %).
 // Only where the caller vouches for ascending columns: with shuffled ones most nonzeros are multiplied one by one, in
 // several tiles each, which no row length or sparsity makes up for, and sizes do not tell the order.
 int sddmm_tile_choice(int m_vec, int k, int n, long long nonzeros_vec, int vec_length, const Batch &problems)
