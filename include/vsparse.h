@@ -62,7 +62,8 @@ const char *vs_status_string(int status);
  * Requirements: `values` aligned to 2*vec_length bytes, `rhs_matrix` and
  * `output_matrix` aligned to 16 bytes.  Any k >= 1 (the reference assumes
  * k % 64 == 0 and reads / writes past the operands otherwise, src/wmma_spmm.cu:362);
- * k % 4 != 0 takes a slower kernel that moves the dense operands half by half.
+ * k % 4 != 0 takes a slower kernel that assumes no alignment of the rows of the
+ * dense operands.
  */
 int vs_wmma_spmm_f16(int m_vec, int vec_length, int k, int n,
                      const int *row_indices, const int *row_offsets,
@@ -163,7 +164,7 @@ int vs_wmma_spmm_f16_slab(int m_vec, int vec_length, int k, int n,
  * that rounding is deliberately not reproduced because it alone breaks the
  * 1e-2 relative-error contract against the host loop.
  * vec_length in {1, 2, 4, 8}.  Same alignment rules; any k >= 1 (k % 8 != 0 takes a
- * slower kernel that moves the dense operands half by half).
+ * slower kernel that assumes no alignment of the rows of the dense operands).
  * Against vs_wmma_spmm_f16 on the same problems (one MI355X, k = 256, geometric means over 42 shapes per sparsity):
  * at vec_length 1 level with it - 3 % behind at 80 %, 1 % at 90 %, 2 % ahead at 95 %, 8 % ahead at 98 % - because
  * every nonzero of such a pattern brings in its own row of the dense operand and both kernels then run at the rate
@@ -194,8 +195,10 @@ int vs_cuda_spmm_f16_f32out(int m_vec, int vec_length, int k, int n,
  * lengths may be arbitrarily skewed, row_indices is not used; slower on short
  * rows and small problems).  0 = automatic: schedule 1, except that masks of few
  * nonzeros with vec_length <= 4 - which fill a quarter of a matrix-core tile or
- * less - run on the fine-grained kernel of vs_cuda_sddmm_f16 (same function
- * within the fp32-accumulation tolerance, not the same bits).
+ * less - and, for k > 256, with vec_length 8 run on the fine-grained kernel of
+ * vs_cuda_sddmm_f16 (same function within the fp32-accumulation tolerance, not the
+ * same bits).  For masks whose columns ascend in every row, vs_wmma_sddmm_f16_sorted
+ * can be several times faster.
  * 3 (the reference's timing-only hardware simulation, whose results are wrong by design) is rejected with
  * hipErrorInvalidValue.
  * Any k >= 0; the whole of k is contracted (the reference drops k % 64).  k % 8 != 0

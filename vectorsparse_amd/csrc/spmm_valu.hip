@@ -386,7 +386,7 @@ static int launch_lr(int m_vec, int k, int waves, const int *row_indices, const 
                      const int *column_indices, const half_t *values, const half_t *rhs, OutT *out,
                      hipStream_t stream, const Batch &batch)
 {
-    if (k % 8 != 0)  // any dense width: the half-by-half variant, 16 lanes (128 columns) per tile
+    if (k % 8 != 0)  // any dense width: the variant without alignment, 16 lanes (128 columns) per tile
         return launch_one<V, 16, OutT, true>(m_vec, k, waves, row_indices, row_offsets, column_indices, values, rhs, out, stream, batch);
     const int lr = valu_tile_lanes(m_vec, k, batch.count);
     if (lr == 8) return launch_one<V, 8, OutT>(m_vec, k, waves, row_indices, row_offsets, column_indices, values, rhs, out, stream, batch);

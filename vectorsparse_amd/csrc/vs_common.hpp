@@ -298,7 +298,7 @@ struct SpmmShape {
     int blocks_per_wave = 1;   // blocks of a row a wave takes before another wave of the workgroup joins in
     int team_slots = -1;       // >= 0: only that many leading entries of row_indices get the workgroup as a team
     bool pipelined = false;    // waves keep steps of successive blocks of a row in flight (two-step blocks only)
-    bool ragged = false;       // dense width not a multiple of 4: the half-by-half variant
+    bool ragged = false;       // dense width not a multiple of 4: the variant without alignment
     bool dma = false;          // the variant that gathers through LDS-DMA loads (option spmm_gather = 2)
 };
 SpmmShape choose_spmm_shape(bool softmax, int m_vec, int vec_length, int k, int n, const Batch &batch);

@@ -851,7 +851,9 @@ class DeviceProblem:
               algorithm=None):
         """SDDMM on the mask.  algorithm (MFMA path): 1 = a wave per (row, slot), 2 = waves split the nonzero
         range (robust to skewed row lengths), 0 = the library's choice between 1 and the fine-grained kernel (small
-        masks of short vectors); None picks 2 for large, heavily skewed masks, else 0."""
+        masks of short vectors); None picks rows in parts or 2 for large, heavily skewed masks, else 0.  0, 1 and the
+        fine-grained path run masks dense enough for it on whole tiles where the pattern's columns ascend
+        (columns_sorted, found once from the pattern on the host)."""
         k = lhs_matrix.shape[1]
         if out is None:
             out = torch.empty((self.nnz_vec, self.vec_length), dtype=out_dtype, device=lhs_matrix.device)
