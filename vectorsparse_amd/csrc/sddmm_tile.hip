@@ -17,8 +17,8 @@
 // (Slow: with shuffled columns two nonzeros in three lie in several tiles; 4096 x 4096, V = 1, K = 256, 80 %:
 // 1130 us against 19 us sorted and 87 us gathered.)
 //
-// What bounds it (4096 x 4096, V = 1, K = 256, 80 %, tiles of 128: 20.2 us): nothing alone - vector ALU 8 us, LDS 6 us, matrix
-// cores 4 us, 224 MB through the L2s 10 us, around a tile's chain of dependent loads (row extent, two probes, columns) of
+// What bounds it (4096 x 4096, V = 1, K = 256, 80 %, tiles of 128: 18.9 us): nothing alone - vector ALU 8 us, LDS 6 us, matrix
+// cores 3 us, 225 MB through the L2s 10 us, around a tile's chain of dependent loads (row extent, two probes, columns) of
 // about 3 us that two workgroups of eight waves per CU hide from each other.  A flat list of the tile's nonzeros over all
 // threads instead of 4 V lanes per vector row (a scan and an owner per nonzero in LDS) took 34 us, one step of operands in
 // flight instead of two 22.5 us.
