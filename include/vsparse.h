@@ -282,6 +282,25 @@ int vs_wmma_spmm_f16_batched_sorted(int batch, int m_vec, int vec_length, int k,
                                     void *output_matrix, long long stride_output, void *stream);
 
 /*
+ * vs_wmma_spmm_f16 / vs_cuda_spmm_f16 (row_length_hints = 0) or, with row_length_hints = 1, vs_wmma_spmm_f16_batched_sorted
+ * (long_rows < 0: vs_wmma_spmm_f16_batched) / vs_cuda_spmm_f16_batched for one problem, for patterns whose columns ascend
+ * strictly in every row; nonzeros_vec and longest_row_vec are the pattern's.  Patterns that keep a good share of a block of
+ * rows are then multiplied as dense tiles on the matrix cores (k % 4 == 0; option "spmm_tile"), every row of rhs_matrix read
+ * once per block of rows instead of once per nonzero: the same function within the fp32-accumulation tolerance, infinities
+ * and NaNs of the operands included, not the same bits.  Otherwise they are the entry points named above.  Order and
+ * counts are hints: a wrong one costs time, never correctness (row_indices must be a permutation, as everywhere).  No
+ * counterpart in the reference, whose kernels gather (src/wmma_spmm.cu:77-90).
+ */
+int vs_wmma_spmm_f16_ascending(int m_vec, int vec_length, int k, int n, int nonzeros_vec, int longest_row_vec,
+                               int long_rows, int row_length_hints,
+                               const int *row_indices, const int *row_offsets, const int *column_indices,
+                               const void *values, const void *rhs_matrix, void *output_matrix, void *stream);
+int vs_cuda_spmm_f16_ascending(int m_vec, int vec_length, int k, int n, int nonzeros_vec, int longest_row_vec,
+                               int row_length_hints,
+                               const int *row_indices, const int *row_offsets, const int *column_indices,
+                               const void *values, const void *rhs_matrix, void *output_matrix, void *stream);
+
+/*
  * Rows in parts: the row swizzle of the reference (SortedRowSwizzle, include/bm_test_utils.h:200-215, which
  * reorders the dispatch of whole rows) taken one step further - a row far longer than the rest is dispatched as
  * several parts, each to a workgroup of its own, so that no workgroup is left walking one row when the rest of
@@ -552,6 +571,8 @@ int vs_wmma_spmm_launch_shape(int batch, int m_vec, int vec_length, int k, int n
  * vector row, 0 = automatic), "sddmm_group" (16-vector groups per wave step of the
  * MFMA SDDMM: 1, 2, 4, 0 = automatic), "sddmm_block_waves" (1..16, 0 = automatic),
  * "sddmm_flat_supers" (super-groups per wave of algorithm 2, 1..16, 0 = automatic),
+ * "spmm_tile" (SpMM on dense tiles, fp16 outputs, k % 4 == 0, any order of the columns: 1 = never, 2 = tiles of 32 x 64,
+ * 3 = of 64 x 128, 4 = of 128 x 128, 0 = where the columns are known to ascend strictly and tiles are expected to be faster),
  * "sddmm_tile" (SDDMM on dense tiles, k % 8 == 0, any order of the columns: 1 = never, 2 = tiles of 64 x 64,
  * 3 = of 128 x 128, 0 = where the columns are known to ascend and tiles are expected to be faster than gathering rows),
  * "attention_waves" (1..8, 0 = automatic), "attention_chunk" (nonzero vectors per

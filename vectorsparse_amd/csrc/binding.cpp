@@ -183,6 +183,24 @@ PyObject *spmm(PyObject *, PyObject *const *args, Py_ssize_t n_args)
     });
 }
 
+// (fine_grained, m_vec, vec_length, k, n, nonzeros_vec, longest_row_vec, long_rows, row_length_hints, row_indices, row_offsets,
+// column_indices, values, rhs, out, stream), fp16 outputs
+PyObject *spmm_ascending(PyObject *, PyObject *const *args, Py_ssize_t n_args)
+{
+    Reader r(args, n_args);
+    const bool fine_grained = r.flag();
+    const int m_vec = r.integer(), v = r.integer(), k = r.integer(), n = r.integer(), nnz = r.integer(), longest = r.integer();
+    const int long_rows = r.integer();
+    const bool hints = r.flag();
+    const int *ri = (const int *)r.indices(), *ro = (const int *)r.indices(), *ci = (const int *)r.indices();
+    const void *values = r.halves(), *rhs = r.halves();
+    void *out = r.halves(), *stream = r.stream();
+    return status_of(r, [&] {
+        return fine_grained ? vs_cuda_spmm_f16_ascending(m_vec, v, k, n, nnz, longest, hints, ri, ro, ci, values, rhs, out, stream)
+                            : vs_wmma_spmm_f16_ascending(m_vec, v, k, n, nnz, longest, long_rows, hints, ri, ro, ci, values, rhs, out, stream);
+    });
+}
+
 // (m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices, lhs, rhs, out, vec_length, stream, algorithm, columns_sorted)
 PyObject *wmma_sddmm(PyObject *, PyObject *const *args, Py_ssize_t n_args)
 {
@@ -404,6 +422,7 @@ PyObject *guarded(PyObject *self, PyObject *const *args, Py_ssize_t n_args) noex
 PyMethodDef methods[] = {
     VS_METHOD("wmma_spmm", (spmm<vs_wmma_spmm_f16, vs_wmma_spmm_f16_f32out>)),
     VS_METHOD("cuda_spmm", (spmm<vs_cuda_spmm_f16, vs_cuda_spmm_f16_f32out>)),
+    VS_METHOD("spmm_ascending", spmm_ascending),
     VS_METHOD("wmma_sddmm", wmma_sddmm),
     VS_METHOD("cuda_sddmm", cuda_sddmm),
     VS_METHOD("wmma_spmm_batched", wmma_spmm_batched),

@@ -18,6 +18,8 @@
 //     with the sparse vectors as the 16 x 32 A operand (rows v >= V are zero).
 //   The accumulator of lane (cs, g), register e, MFMA c is out[4g + e][tile*TN + cs*CPL + c], i.e.
 //   CPL consecutive outputs per (lane, e): one vector store each.
+#include <type_traits>
+
 #include "spmm_mfma_step.hpp"
 #include "vs_common.hpp"
 
@@ -860,6 +862,10 @@ int launch_spmm_mfma(int m_vec, int vec_length, int k, int n, const int *row_ind
                      const int *row_offsets, const int *column_indices, const half_t *values,
                      const half_t *rhs, OutT *out, hipStream_t stream, const Batch &batch)
 {
+    if constexpr (std::is_same<OutT, half_t>::value) {
+        const int tile = spmm_tile_choice(false, m_vec, k, n, vec_length, batch);
+        if (tile) return launch_spmm_tile(tile, m_vec, vec_length, k, n, row_offsets, column_indices, values, rhs, out, stream, batch);
+    }
     return launch_any<false, OutT>(m_vec, vec_length, k, n, row_indices, row_offsets, column_indices, values, rhs,
                                    out, stream, batch, 1.f);
 }

@@ -402,6 +402,10 @@ int launch_spmm_valu(int m_vec, int vec_length, int k, int n, const int *row_ind
 {
     if (m_vec == 0 || k == 0 || batch.count == 0) return hipSuccess;
     if (batch.count > 65535) return hipErrorNotSupported;
+    if constexpr (std::is_same<OutT, half_t>::value) {
+        const int tile = spmm_tile_choice(true, m_vec, k, n, vec_length, batch);
+        if (tile) return launch_spmm_tile(tile, m_vec, vec_length, k, n, row_offsets, column_indices, values, rhs, out, stream, batch);
+    }
     int waves = options().spmm_waves;
     if (waves <= 0) {
         const int lr = valu_tile_lanes(m_vec, k, batch.count);

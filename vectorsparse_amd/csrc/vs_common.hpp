@@ -251,6 +251,7 @@ struct Options {
     int sddmm_group = 0;        // MFMA SDDMM: 16-vector groups per wave step (1, 2, 4), 0 = automatic
     int sddmm_tile = 0;         // SDDMM on dense tiles: 1 = never, 2 = 64 x 64 tiles, 3 = 128 x 128 tiles, 0 = automatic
     int sddmm_flat_supers = 0;  // flat MFMA SDDMM (algorithm 2): super-groups per wave, 0 = automatic
+    int spmm_tile = 0;          // SpMM on dense tiles: 1 = never, 2 / 3 / 4 = tiles of 32 x 64, 64 x 128, 128 x 128, 0 = automatic
     int attention_waves = 0;
     int attention_chunk = 0;
 };
@@ -287,7 +288,9 @@ struct Batch {
     int long_rows = -1;        // SpMM, rows ordered by length: leading entries of row_indices with more than 512 vectors
     int algorithm = 0;         // SDDMM on MFMA: 2 = waves split the nonzero range, else (row, slot) per wave
     bool row_parts = false;    // SDDMM on MFMA: row_indices is a dispatch list of row parts, m_vec counts its slots
-    bool sorted_columns = false;  // SDDMM: the columns of every row are known to ascend (a hint)
+    bool sorted_columns = false;  // the columns of every row are known to ascend (SpMM: strictly; a hint)
+    int tile_nonzeros_vec = 0;    // SpMM, with sorted_columns: nonzero vectors of the pattern and of its longest row, for the
+    int tile_longest_vec = 0;     // choice of dense tiles alone
 };
 
 // Launch shape of the MFMA SpMM (spmm_mfma.hip), chosen on the host.
@@ -334,6 +337,12 @@ template <typename OutT>
 int launch_sddmm_tile(int shape, int m_vec, int k, int n, const int *row_offsets, const int *col_indices,
                       const half_t *lhs, const half_t *rhs, OutT *out, int vec_length, hipStream_t stream,
                       const Batch &batch);
+
+// SpMM on dense tiles (csrc/spmm_tile.hip), fp16 outputs.  spmm_tile_choice: 0 = the gathering kernels are expected to be
+// faster (or have to take the call), else the `shape` for launch_spmm_tile (1 = tiles of 32 x 64, 2 = 64 x 128, 3 = 128 x 128).
+int spmm_tile_choice(bool fine_grained, int m_vec, int k, int n, int vec_length, const Batch &batch);
+int launch_spmm_tile(int shape, int m_vec, int vec_length, int k, int n, const int *row_offsets, const int *col_indices,
+                     const half_t *values, const half_t *rhs, half_t *out, hipStream_t stream, const Batch &batch);
 
 // Writes `bytes` zero bytes to each of `batch` buffers `stride_bytes` apart (a kernel, not a memset node, so that
 // callers may capture the call into a HIP graph).

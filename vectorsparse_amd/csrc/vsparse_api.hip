@@ -390,6 +390,43 @@ int vs_wmma_spmm_f16_batched_sorted(int batch, int m_vec, int vec_length, int k,
                                                    longest_row_vec, long_rows < 0 ? -1 : long_rows));
 }
 
+static vs::Batch ascending(int nonzeros_vec, int longest_row_vec, int row_length_hints, int long_rows)
+{
+    vs::Batch one = row_length_hints ? make_batch(1, 0, 0, 0, nonzeros_vec, longest_row_vec, long_rows < 0 ? -1 : long_rows) : vs::Batch();
+    one.sorted_columns = nonzeros_vec > 0;
+    one.tile_nonzeros_vec = nonzeros_vec;
+    one.tile_longest_vec = longest_row_vec;
+    return one;
+}
+
+int vs_wmma_spmm_f16_ascending(int m_vec, int vec_length, int k, int n, int nonzeros_vec, int longest_row_vec,
+                               int long_rows, int row_length_hints, const int *row_indices, const int *row_offsets,
+                               const int *column_indices, const void *values, const void *rhs_matrix,
+                               void *output_matrix, void *stream)
+{
+    int st = check_spmm(m_vec, vec_length, k, n, row_indices, row_offsets, column_indices, values, rhs_matrix,
+                        output_matrix, sizeof(half_t));
+    if (st != VS_SUCCESS) return st;
+    return vs::launch_spmm_mfma<half_t>(m_vec, vec_length, k, n, row_indices, row_offsets, column_indices,
+                                        static_cast<const half_t *>(values), static_cast<const half_t *>(rhs_matrix),
+                                        static_cast<half_t *>(output_matrix), static_cast<hipStream_t>(stream),
+                                        ascending(nonzeros_vec, longest_row_vec, row_length_hints, long_rows));
+}
+
+int vs_cuda_spmm_f16_ascending(int m_vec, int vec_length, int k, int n, int nonzeros_vec, int longest_row_vec,
+                               int row_length_hints, const int *row_indices, const int *row_offsets,
+                               const int *column_indices, const void *values, const void *rhs_matrix,
+                               void *output_matrix, void *stream)
+{
+    int st = check_spmm(m_vec, vec_length, k, n, row_indices, row_offsets, column_indices, values, rhs_matrix,
+                        output_matrix, sizeof(half_t));
+    if (st != VS_SUCCESS) return st;
+    return vs::launch_spmm_valu<half_t>(m_vec, vec_length, k, n, row_indices, row_offsets, column_indices,
+                                        static_cast<const half_t *>(values), static_cast<const half_t *>(rhs_matrix),
+                                        static_cast<half_t *>(output_matrix), static_cast<hipStream_t>(stream),
+                                        ascending(nonzeros_vec, longest_row_vec, row_length_hints, -1));
+}
+
 int vs_wmma_spmm_launch_shape(int batch, int m_vec, int vec_length, int k, int n, int nonzeros_vec,
                               int longest_row_vec, int long_rows, int shape[8])
 {
@@ -795,6 +832,9 @@ static int set_option_field(vs::Options &o, const char *name, int value)
     } else if (std::strcmp(name, "sddmm_tile") == 0) {
         if (value > 3) return VS_ERROR_INVALID_VALUE;
         o.sddmm_tile = value;
+    } else if (std::strcmp(name, "spmm_tile") == 0) {
+        if (value > 4) return VS_ERROR_INVALID_VALUE;
+        o.spmm_tile = value;
     } else if (std::strcmp(name, "sddmm_flat_supers") == 0) {
         if (value > 16) return VS_ERROR_INVALID_VALUE;
         o.sddmm_flat_supers = value;

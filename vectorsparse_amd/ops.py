@@ -713,10 +713,10 @@ def split_rows_pays(m_vec, nonzeros_vec, longest_row_vec):
     return longest_row_vec * m_vec >= 25.0 * nonzeros_vec
 
 
-def columns_ascend(row_offsets, column_indices):
-    """Whether the columns of every row ascend (repeated ones included)."""
+def columns_ascend(row_offsets, column_indices, strictly=False):
+    """Whether the columns of every row ascend (repeated ones included, unless `strictly`)."""
     columns, starts = np.asarray(column_indices), np.asarray(row_offsets)
-    falls = columns[1:] < columns[:-1]
+    falls = columns[1:] <= columns[:-1] if strictly else columns[1:] < columns[:-1]
     falls[starts[(starts > 0) & (starts < columns.size)] - 1] = False
     return not falls.any()
 
@@ -740,7 +740,9 @@ class DeviceProblem:
         self.row_indices = torch.from_numpy(swz).to(device)
         self.row_offsets = torch.from_numpy(np.ascontiguousarray(pattern.row_offsets)).to(device)
         self.column_indices = torch.from_numpy(np.ascontiguousarray(pattern.column_indices)).to(device)
-        self.columns_sorted = columns_ascend(pattern.row_offsets, pattern.column_indices)   # (a hint of the SDDMM)
+        # hints: SDDMM and SpMM run dense patterns of ascending columns on whole tiles
+        self.columns_distinct = columns_ascend(pattern.row_offsets, pattern.column_indices, strictly=True)
+        self.columns_sorted = self.columns_distinct or columns_ascend(pattern.row_offsets, pattern.column_indices)
         self._workspace = None  # partial tiles of the split-row SpMM, allocated on first use
         self._parts = {}        # limit -> (RowParts, its list on the device, workspace), made on first use
         self._parts_need = {}
@@ -802,7 +804,8 @@ class DeviceProblem:
              split_rows=False):
         """SpMM through the reference-shaped entry points; with row_length_hint (fp16 output only) through the
         batched entry point with batch = 1, which also takes the pattern's nonzero count and longest row and
-        sizes its workgroups by the real row lengths instead of by n; with split_rows (MFMA path) on the
+        sizes its workgroups by the real row lengths instead of by n; patterns of strictly ascending columns that are dense
+        enough for it (vs_wmma_spmm_f16_ascending, fp16 output) run on whole tiles; with split_rows (MFMA path) on the
         schedule that cuts the nonzero range into equal pieces, with a workspace this object owns.
         split_rows=None chooses from the row lengths: rows in parts (spmm_row_parts) where the pattern has rows
         long enough to be split, else the row-length hints."""
@@ -826,6 +829,14 @@ class DeviceProblem:
                 self._workspace = torch.zeros(max(need, 16), dtype=torch.uint8, device=rhs_matrix.device)
             return spmm_split_rows(self.m_vec, self.vec_length, k, self.n, self.nnz_vec, self.row_offsets,
                                    self.column_indices, self.values, rhs_matrix, out, self._workspace, stream)
+        if self.columns_distinct and out.dtype == torch.float16:
+            st = _native.spmm_ascending(kernel != "wmma", self.m_vec, self.vec_length, k, self.n, self.nnz_vec, self.longest_row_vec,
+                                        self.long_rows, bool(row_length_hint), self.row_indices, self.row_offsets,
+                                        self.column_indices, self.values, rhs_matrix, out, stream)
+            if st >= 0:
+                if st:
+                    _lib.check(st, "vs_%s_spmm_f16%s" % ("wmma" if kernel == "wmma" else "cuda", "_batched" if row_length_hint else ""))
+                return out
         if row_length_hint and out.dtype == torch.float16:
             spmm_batched(self.m_vec, self.vec_length, k, self.n, self.row_indices, self.row_offsets,
                          self.column_indices, self.values, rhs_matrix, out.unsqueeze(0), kernel=kernel, stream=stream,
