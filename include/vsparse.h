@@ -502,6 +502,28 @@ int vs_sparse_attention_plan(int m_vec, int vec_length, int n, int d_qk, int d_v
                              long long plan_bytes, void *stream);
 
 /*
+ * vs_sparse_attention_f16 with workgroups of 128 scalar rows (a row block) for masks in which a few row blocks have far more
+ * distinct columns than the rest (tokens that attend to everything): such a block is streamed by several workgroups, each
+ * taking a range of its sub-rounds of 128 distinct columns, and a second launch adds their partial results up.  A plan of its own (up to
+ * 4096 distinct columns per block; blocks with more take the per-row path) and a list of slots in device memory, 16-byte
+ * aligned: n_slots entries {row block, first sub-round, end of the sub-rounds, partial tile or -1}, then n_merges entries
+ * {row block, first partial tile, number of tiles, 0}.  Every block appears in one slot with first sub-round 0 and tile -1,
+ * or in several that share its sub-rounds (the last one's end may be any large number) with consecutive tiles and a merge
+ * entry.  workspace: 128 * (d_v + 2) floats per partial tile and head, uninitialised.  No counterpart in the reference.
+ */
+long long vs_sparse_attention_split_plan_bytes(int m_vec, int vec_length, int n, int d_qk, int d_v);
+int vs_sparse_attention_split_plan(int m_vec, int vec_length, int n, int d_qk, int d_v,
+                                   const int *row_offsets, const int *col_indices, void *plan,
+                                   long long plan_bytes, void *stream);
+int vs_sparse_attention_f16_split(int batch, int m_vec, int vec_length, int n, int d_qk, int d_v,
+                                  const int *row_offsets, const int *col_indices,
+                                  const void *q, long long stride_q, const void *k, long long stride_k,
+                                  const void *v, long long stride_v, void *out, long long stride_out,
+                                  float scale, const void *plan, long long plan_bytes, const int *slots, int n_slots,
+                                  int n_merges, int n_partials, void *workspace, long long workspace_bytes,
+                                  void *stream);
+
+/*
  * Planning helper for rows_per_workgroup >= 2 of vs_sparse_attention_f16: the number of distinct columns
  * a workgroup can take for this shape (0: shape not supported by the union kernel), and in
  * *rows_used (may be null) the vector rows per workgroup the request is rounded to.  with_plan: nonzero

@@ -1,0 +1,113 @@
+"""Split attention launches (long row blocks streamed by several workgroups): against dense masked attention in float64."""
+import numpy as np
+import pytest
+import torch
+
+from vectorsparse_amd import ops
+from vectorsparse_amd import colvec_csr as cv
+from test_gpu_attention import _check_layer, _dense_attention
+
+pytestmark = pytest.mark.gpu
+
+
+def _mask(kind, seq, V, tokens=24, half_width=40):
+    start = (seq // 2 - 8) // V * V     # the tokens' rows lie in two row blocks
+    rows = []
+    for i in range(seq // V):
+        c = i * V + V // 2
+        cols = np.arange(max(0, c - half_width), min(seq, c + half_width + 1))
+        if kind == "empty rows" and i % 7 == 3:
+            cols = cols[:0]
+        if kind != "band" and start <= i * V < start + tokens:
+            cols = np.arange(seq)
+        elif kind == "global":
+            cols = np.union1d(cols, np.arange(start, start + tokens))
+        rows.append(cols)
+    ro = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    return cv.ColVecCSR(seq // V, seq, V, ro, np.concatenate(rows).astype(np.int32))
+
+
+def _operands(heads, seq, d, d_v, seed=1):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    return [torch.randn((heads, seq, w), device="cuda", generator=g).half() for w in (d, d, d_v)]
+
+
+@pytest.mark.parametrize("V", [1, 2, 4, 8])
+@pytest.mark.parametrize("kind,seq,d,d_v,rounds,scale", [
+    ("global", 520, 64, 64, 1, None), ("global", 776, 32, 64, 2, None), ("global", 520, 128, 32, 3, None),
+    ("global", 640, 64, 128, 1, -0.2), ("empty rows", 520, 64, 64, 2, None), ("empty rows", 264, 16, 24, 1, 0.0),
+    ("band", 520, 64, 64, 1, None), ("global", 1032, 64, 64, 32, None)])
+def test_split_launches_match_dense_attention(gpu, kind, seq, d, d_v, rounds, scale, V):
+    mask = _mask(kind, seq, V)
+    layer = ops.SparseAttention(mask)
+    heads = 2
+    q, k, v = _operands(heads, seq, d, d_v)
+    pad = torch.full((heads, seq + 2, d_v), 7.0, dtype=torch.float16, device="cuda")
+    out = pad[:, 1:-1]
+    layer.forward(q, k, v, out=out, scale=scale, fused=("split", rounds))
+    torch.cuda.synchronize()
+    assert bool((pad[:, 0] == 7.0).all()) and bool((pad[:, -1] == 7.0).all())
+    slots = layer._splits[d, d_v, rounds][0]
+    assert (slots.n_merges > 0) == (rounds < 4 or seq > 4096)
+    ref = _dense_attention(mask, q.cpu().numpy(), k.cpu().numpy(), v.cpu().numpy(), d ** -0.5 if scale is None else scale)
+    _check_layer(out.cpu().numpy(), ref, "%s V%d rounds %d" % (kind, V, rounds))
+
+
+def test_blocks_beyond_the_plan_and_foreign_plans_take_the_per_row_path(gpu):
+    V, heads, d = 8, 1, 32
+    mask = _mask("global", 4352, V)     # blocks of 4352 distinct columns: more than a split plan holds
+    layer = ops.SparseAttention(mask)
+    q, k, v = _operands(heads, 4352, d, d)
+    out = layer.forward(q, k, v, fused=("split", 4))
+    ref = _dense_attention(mask, q.cpu().numpy(), k.cpu().numpy(), v.cpu().numpy(), d ** -0.5)
+    _check_layer(out.cpu().numpy(), ref, "beyond the plan")
+    mask = _mask("global", 520, V)
+    layer = ops.SparseAttention(mask)
+    q, k, v = _operands(heads, 520, d, d)
+    slots, device_slots, plan = layer._split(d, d, 1)
+    out = torch.empty_like(q)
+    ops.sparse_attention_split(layer.prob, slots, device_slots, torch.zeros_like(plan), q, k, v, out, d ** -0.5)
+    ref = _dense_attention(mask, q.cpu().numpy(), k.cpu().numpy(), v.cpu().numpy(), d ** -0.5)
+    _check_layer(out.cpu().numpy(), ref, "a plan of zeros")
+
+
+def test_the_automatic_route_splits_and_replays(gpu):
+    V, heads, seq, d = 1, 4, 1500, 64
+    mask = _mask("global", seq, V, tokens=64)
+    layer = ops.SparseAttention(mask)
+    q, k, v = _operands(heads, seq, d, d)
+    fresh = ops.SparseAttention(mask)
+    route = layer._route(d, d, heads)
+    assert route[0] == "split"
+    assert torch.equal(layer.forward(q, k, v), layer.forward(q, k, v, fused=route))
+    want = layer.forward(q, k, v)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    other = layer.forward(q, k, v, stream=side)
+    side.synchronize()
+    assert torch.equal(other, want)
+    out = torch.empty_like(want)
+    fresh.plan(d, d, heads)     # (makes what the route needs: the first pass can be captured)
+    for one in (layer, fresh):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            one.forward(q, k, v, out=out)
+        for _ in range(3):
+            out.fill_(3.0)
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want)
+
+
+def test_refused_arguments(gpu):
+    mask = _mask("global", 520, 8)
+    layer = ops.SparseAttention(mask)
+    q, k, v = _operands(2, 520, 64, 64)
+    slots, device_slots, plan = layer._split(64, 64, 1)
+    out = torch.empty_like(q)
+    small = torch.empty(slots.n_partials * 2 * 128 * 66 - 1, dtype=torch.float32, device="cuda")
+    for bad_plan, workspace in ((plan[:-16], None), (plan, small)):
+        with pytest.raises(Exception):
+            ops.sparse_attention_split(layer.prob, slots, device_slots, bad_plan, q, k, v, out, 0.125, workspace)
+    with pytest.raises(TypeError):
+        ops.sparse_attention_split(layer.prob, slots, device_slots, plan, q.float(), k, v, out, 0.125)

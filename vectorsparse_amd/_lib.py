@@ -47,6 +47,10 @@ SIGNATURES = {
     "vs_sparse_attention_union_capacity": ([_int] * 6 + [_vp], _int),
     "vs_sparse_attention_plan_bytes": ([_int] * 6, _ll),
     "vs_sparse_attention_plan": ([_int] * 6 + [_vp] * 3 + [_ll, _vp], _int),
+    "vs_sparse_attention_split_plan_bytes": ([_int] * 5, _ll),
+    "vs_sparse_attention_split_plan": ([_int] * 5 + [_vp] * 3 + [_ll, _vp], _int),
+    "vs_sparse_attention_f16_split": ([_int] * 6 + [_vp] * 2 + [_vp, _ll, _vp, _ll, _vp, _ll, _vp, _ll, ctypes.c_float, _vp, _ll, _vp]
+                                      + [_int] * 3 + [_vp, _ll, _vp], _int),
     "vs_sparse_softmax_f16": ([_int] * 3 + [_vp] * 2 + [_vp, _ll, _vp, _ll, ctypes.c_float, _vp], _int),
     "vs_sparse_softmax_row_parts_workspace_bytes": ([_int] * 4, _ll),
     "vs_sparse_softmax_f16_row_parts": ([_int] * 3 + [_vp, _int, _int] + [_vp, _ll, _vp, _ll, ctypes.c_float, _vp, _ll, _vp],

@@ -351,6 +351,27 @@ PyObject *sparse_attention(PyObject *, PyObject *const *args, Py_ssize_t n_args)
     });
 }
 
+// (batch, m_vec, vec_length, n, d_qk, d_v, row_offsets, col_indices, q, k, v, out, scale, plan, slots, n_slots, n_merges,
+// n_partials, workspace, stream)
+PyObject *sparse_attention_split(PyObject *, PyObject *const *args, Py_ssize_t n_args)
+{
+    Reader r(args, n_args);
+    const int batch = r.integer(), m_vec = r.integer(), vec = r.integer(), n = r.integer(), d_qk = r.integer(), d_v = r.integer();
+    const int *ro = (const int *)r.indices(), *ci = (const int *)r.indices();
+    long long sq, sk, sv, so, plan_bytes, bytes;
+    const void *q = r.batched(batch, sq), *k = r.batched(batch, sk), *v = r.batched(batch, sv);
+    void *out = r.batched(batch, so);
+    const float scale = r.number();
+    const void *plan = r.buffer(plan_bytes);
+    const int *slots = (const int *)r.indices();
+    const int n_slots = r.integer(), n_merges = r.integer(), n_partials = r.integer();
+    void *workspace = r.buffer(bytes), *stream = r.stream();
+    return status_of(r, [&] {
+        return vs_sparse_attention_f16_split(batch, m_vec, vec, n, d_qk, d_v, ro, ci, q, sq, k, sk, v, sv, out, so, scale, plan,
+                                             plan_bytes, slots, n_slots, n_merges, n_partials, workspace, bytes, stream);
+    });
+}
+
 // (batch, vec_length, k, n, n_slots, slots, n_split, parts_max, nonzeros_vec, longest_part_vec, column_indices, values, rhs, out,
 // workspace, stream)
 PyObject *spmm_row_parts(PyObject *, PyObject *const *args, Py_ssize_t n_args)
@@ -432,6 +453,7 @@ PyMethodDef methods[] = {
     VS_METHOD("cuda_sddmm_batched", sddmm_batched<false>),
     VS_METHOD("sparse_softmax", sparse_softmax),
     VS_METHOD("sparse_attention", sparse_attention),
+    VS_METHOD("sparse_attention_split", sparse_attention_split),
     VS_METHOD("spmm_row_parts", spmm_row_parts),
     VS_METHOD("sddmm_row_parts", sddmm_row_parts),
     VS_METHOD("softmax_row_parts", softmax_row_parts),

@@ -426,6 +426,15 @@ constexpr int kPlanHeader = 16;
 constexpr int kStreamSteps = 4;
 constexpr int kStreamRanks = 32 * kStreamSteps;
 constexpr int kStreamRounds = 16;
+constexpr int kSplitRounds = 32;   // plans of split launches
+
+// Whether `plan` was made for this mask's sizes and this launch shape (workgroups of eight waves).
+__device__ __forceinline__ bool stream_plan_fits(const int *plan, int m_vec, int vec_length, int n, int rows, int rounds, int stride)
+{
+    return plan[0] == kPlanMagic && plan[1] == m_vec && plan[2] == vec_length && plan[3] == n && plan[4] == rows &&
+           plan[5] == kStreamRanks && plan[6] == stride && plan[7] == (m_vec + rows - 1) / rows && plan[8] == rounds &&
+           plan[9] == kStreamSteps;
+}
 
 __global__ void __launch_bounds__(256)
 sparse_attention_plan_kernel(int m_vec, int vec_length, int n, int rows_per_block, int u_max, int rounds, int steps,
@@ -781,14 +790,20 @@ __device__ __noinline__ void per_row_block_call(int row_first, int row_last, int
                               c, g, col_off);
 }
 
-template <int V, int KS, int CPL>
+//
+// SPLIT: driven by a list of slots {row block, first sub-round, last sub-round + 1, partial tile or -1} instead of a row block
+// per workgroup, so that a block whose union is far longer than the rest (rows that attend to everything) is streamed by
+// several workgroups: a slot with a partial tile leaves its unnormalised sums, row sums and row maxima in the workspace, and
+// sparse_attention_merge_kernel adds them up.
+template <int V, int KS, int CPL, bool SPLIT>
 __global__ void __launch_bounds__(512, union_wide(KS, CPL) ? 2 : 4)
 sparse_attention_stream_kernel(int m_vec, int n, int d_qk, int d_v,
                                const int *__restrict__ row_offsets, const int *__restrict__ col_indices,
                                const int *__restrict__ plan,
                                const half_t *__restrict__ q, const half_t *__restrict__ k,
                                const half_t *__restrict__ v, half_t *__restrict__ out, long long stride_q,
-                               long long stride_k, long long stride_v, long long stride_out, float scale)
+                               long long stride_k, long long stride_v, long long stride_out, float scale,
+                               const int *__restrict__ slots, int n_partials, float *__restrict__ partials)
 {
     q += blockIdx.y * stride_q;
     k += blockIdx.y * stride_k;
@@ -796,6 +811,7 @@ sparse_attention_stream_kernel(int m_vec, int n, int d_qk, int d_v,
     out += blockIdx.y * stride_out;
     constexpr int RPW = 16 / V;
     constexpr int PITCH = 32 * KS + 8;                              // halves between consecutive K rows in LDS
+    constexpr int kRounds = SPLIT ? kSplitRounds : kStreamRounds;
     constexpr int SS = kStreamSteps;
     constexpr int SR = kStreamRanks;
     constexpr int kThreads = 512;
@@ -814,8 +830,16 @@ sparse_attention_stream_kernel(int m_vec, int n, int d_qk, int d_v,
     half_t *kbuf = reinterpret_cast<half_t *>(maskbuf + kRows * SS);  // [SR][PITCH]
     half_t *vbuf = kbuf + SR * PITCH;                                 // [16 * CPL columns][kStreamVPitch]
 
-    int bx = blockIdx.x;
-    if ((gridDim.x & 7) == 0) bx = (bx & 7) * (gridDim.x >> 3) + (bx >> 3);  // a run of row blocks per XCD
+    int bx = blockIdx.x, first_round = 0, end_round = kRounds, partial = -1;
+    if constexpr (SPLIT) {
+        const int4_t slot = reinterpret_cast<const int4_t *>(slots)[blockIdx.x];
+        bx = slot[0];
+        first_round = slot[1];
+        end_round = slot[2];
+        partial = slot[3];
+    } else if ((gridDim.x & 7) == 0) {
+        bx = (bx & 7) * (gridDim.x >> 3) + (bx >> 3);  // a run of row blocks per XCD
+    }
     const int row_first = bx * kRows;
     const int row_last = (row_first + kRows) < m_vec ? (row_first + kRows) : m_vec;
     const int c = lane & 15;
@@ -825,11 +849,9 @@ sparse_attention_stream_kernel(int m_vec, int n, int d_qk, int d_v,
     const bool col_ok = col0 < d_v;
     const int col_off = col_ok ? col0 : 0;
 
-    constexpr int u_cap = kStreamRounds * SR;
-    constexpr int stride = 4 + kStreamRounds * kMaskWords + u_cap;
-    const bool plan_ok = plan[0] == kPlanMagic && plan[1] == m_vec && plan[2] == V && plan[3] == n &&
-                         plan[4] == kRows && plan[5] == SR && plan[6] == stride && plan[7] == (int)gridDim.x &&
-                         plan[8] == kStreamRounds && plan[9] == SS;
+    constexpr int u_cap = kRounds * SR;
+    constexpr int stride = 4 + kRounds * kMaskWords + u_cap;
+    const bool plan_ok = stream_plan_fits(plan, m_vec, V, n, kRows, kRounds, stride);
     const int *rec = plan + kPlanHeader + (size_t)(plan_ok ? bx : 0) * stride;
     const int n_union = plan_ok ? rec[0] : 0x7fffffff;
     // The record, the K rows and the V rows are read through buffer descriptors: a scalar base and one 32-bit byte
@@ -839,7 +861,7 @@ sparse_attention_stream_kernel(int m_vec, int n, int d_qk, int d_v,
     const __amdgpu_buffer_rsrc_t k_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t *>(k), 0, 0x7fffffff, 0x00020000);
     const __amdgpu_buffer_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t *>(v), 0, 0x7fffffff, 0x00020000);
     constexpr unsigned kMasksAt = 4u * 4u;                                        // byte offsets inside the record
-    constexpr unsigned kColsAt = 4u * (4u + kStreamRounds * kMaskWords);
+    constexpr unsigned kColsAt = 4u * (4u + kRounds * kMaskWords);
 
     // What a thread fetches per sub-round: NK slices of K rows (thread t takes slices t, t + 512, ...:
     // consecutive threads read consecutive 16 bytes of a row), NV times the same slice of the V rows of two
@@ -848,7 +870,7 @@ sparse_attention_stream_kernel(int m_vec, int n, int d_qk, int d_v,
     int2_t col_v[NV];
     uint4_t stage_k[NK], stage_v[NV][2];
     unsigned stage_m = 0;
-    // column numbers of sub-round `round` < kStreamRounds (the plan lists 0 past the union: row 0, unused), which
+    // column numbers of sub-round `round` < kRounds (the plan lists 0 past the union: row 0, unused), which
     // do not wait for the union's size
     auto fetch_cols = [&](int round) {
         const unsigned at = kColsAt + 4u * (unsigned)(round * SR);  // (uniform)
@@ -916,20 +938,21 @@ sparse_attention_stream_kernel(int m_vec, int n, int d_qk, int d_v,
         if (tid < kRows * SS) maskbuf[tid] = stage_m;
     };
 
-    fetch_cols(0);  // requested together with the union's size
+    fetch_cols(first_round);  // requested together with the union's size
     if (n_union > u_cap || d_v % 8 != 0) {
+        if (first_round > 0) return;   // (the block's first slot takes all of it)
         per_row_block_call<V, KS, CPL>(row_first, row_last, wave, 8, row_offsets, col_indices, q, k, v, out, d_qk, d_v,
                                        s2, c, g, col_off);
         return;
     }
-    const int n_rounds = (n_union + SR - 1) / SR;
+    const int last_round = (n_union + SR - 1) / SR, n_rounds = end_round < last_round ? end_round : last_round;
     const int q_first = 16 * wave;
     const long long q_global = (long long)row_first * V + q_first;
     const long long q_limit = (long long)row_last * V;
     half8_t qb[KS];
     load_q16<KS>(qb, q, q_global, q_limit, d_qk, c, g);
-    if (n_rounds > 0) fetch_rows(0);
-    if (n_rounds > 1) fetch_cols(1);
+    if (n_rounds > first_round) fetch_rows(first_round);
+    if (n_rounds > first_round + 1) fetch_cols(first_round + 1);
     // The maximum is tracked on raw dot products and masked-out pairs are -inf before the scale is applied, so
     // the scale the exponentials see must be positive: a negative one moves into Q, a zero one becomes Q = 0
     // (every pair of the mask then weighs the same, which is what a zero scale means).
@@ -959,8 +982,8 @@ sparse_attention_stream_kernel(int m_vec, int n, int d_qk, int d_v,
     float4_t lacc = {0.f, 0.f, 0.f, 0.f};
     float mx_run = neg_inf;
 
-    for (int round = 0; round < n_rounds; ++round) {
-        if (round > 0) __syncthreads();  // every wave is done with the previous sub-round's rows and masks
+    for (int round = first_round; round < n_rounds; ++round) {
+        if (round > first_round) __syncthreads();  // every wave is done with the previous sub-round's rows and masks
         commit(round);
         __syncthreads();
         if (round + 1 < n_rounds) fetch_rows(round + 1);  // in flight during the arithmetic below
@@ -1003,7 +1026,7 @@ sparse_attention_stream_kernel(int m_vec, int n, int d_qk, int d_v,
         mx_raw = fmaxf(mx_raw, partner<32>(mx_raw));
         const float mx_new = fmaxf(mx_run, mx_raw);
         const float neg_mx = mx_new == neg_inf ? 0.f : -(mx_new * s2a);
-        if (round > 0) {
+        if (round > first_round) {
             // bring what the earlier sub-rounds accumulated to the new maximum, unless no row's maximum moved
             const float f = mx_new == neg_inf ? 1.f
                             : (mx_run == neg_inf ? 0.f : __builtin_amdgcn_exp2f((mx_run - mx_new) * s2a));
@@ -1038,6 +1061,26 @@ sparse_attention_stream_kernel(int m_vec, int n, int d_qk, int d_v,
             }
         }
     }
+    if constexpr (SPLIT) {
+        if (partial >= 0) {
+            // [128 rows][d_v] sums, [128] row sums, [128] row maxima (of the raw dot products)
+            float *const tile = partials + ((size_t)blockIdx.y * n_partials + partial) * ((size_t)128 * (d_v + 2));
+            float *const sums = tile + (size_t)128 * d_v;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int row = q_first + 4 * g + e;
+                if (col_ok) {
+                    float tmp[CPL];
+#pragma unroll
+                    for (int cc = 0; cc < CPL; ++cc) tmp[cc] = acc[cc][e];
+                    store_converted<float, CPL>(tile + (size_t)row * d_v + col0, tmp);
+                }
+                if (c == 0) sums[row] = lacc[e];
+            }
+            if (g == 0) sums[128 + q_first + c] = mx_run;
+            return;
+        }
+    }
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         const long long row = q_global + 4 * g + e;
@@ -1048,6 +1091,47 @@ sparse_attention_stream_kernel(int m_vec, int n, int d_qk, int d_v,
             for (int cc = 0; cc < CPL; ++cc) tmp[cc] = acc[cc][e] * norm;
             store_converted<half_t, CPL>(out + (size_t)row * d_v + col0, tmp);
         }
+    }
+}
+
+// Adds up the partial tiles of a split row block: merge entry {row block, first partial tile, tiles, -}.  A few hundred KB per
+// head at most, read once: bound by the launch and one round trip (3 us).
+__global__ void __launch_bounds__(512)
+sparse_attention_merge_kernel(int m_vec, int vec_length, int n, int d_v, const int *__restrict__ plan,
+                              const int *__restrict__ merges, int n_partials, const float *__restrict__ partials,
+                              half_t *__restrict__ out, long long stride_out, float scale)
+{
+    const int4_t merge = reinterpret_cast<const int4_t *>(merges)[blockIdx.x];
+    const int rows = 128 / vec_length, mask_words = (rows * kStreamSteps + 3) & ~3;
+    const int stride = 4 + kSplitRounds * (mask_words + kStreamRanks);
+    // (a block that the stream kernel has left to the per-row path is finished)
+    if (!stream_plan_fits(plan, m_vec, vec_length, n, rows, kSplitRounds, stride)) return;
+    if (plan[kPlanHeader + (size_t)merge[0] * stride] > kSplitRounds * kStreamRanks || d_v % 8 != 0) return;
+    const float s2a = scale == 0.f ? 1.f : __builtin_fabsf(scale * kLog2e);
+    const size_t tile = (size_t)128 * (d_v + 2);
+    const float *const first = partials + ((size_t)blockIdx.y * n_partials + merge[1]) * tile;
+    out += blockIdx.y * stride_out;
+    const int chunks = d_v / 4;
+    for (int unit = threadIdx.x + 512 * blockIdx.z; unit < 128 * chunks; unit += 512 * gridDim.z) {
+        const int r = unit / chunks, column = unit % chunks * 4;
+        const long long row = (long long)merge[0] * 128 + r;
+        if (row >= (long long)m_vec * vec_length) continue;
+        float most = -__builtin_inff();
+        for (int i = 0; i < merge[2]; ++i) most = fmaxf(most, first[i * tile + (size_t)128 * d_v + 128 + r]);
+        float4_t sum = {0.f, 0.f, 0.f, 0.f};
+        float weight = 0.f;
+        for (int i = 0; i < merge[2]; ++i) {
+            const float *const part = first + i * tile;
+            const float mx = part[(size_t)128 * d_v + 128 + r];
+            const float f = mx == -__builtin_inff() ? 0.f : __builtin_amdgcn_exp2f((mx - most) * s2a);
+            const float4_t x = *reinterpret_cast<const float4_t *>(part + (size_t)r * d_v + column);
+            weight += f * part[(size_t)128 * d_v + r];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sum[e] += f * x[e];
+        }
+        const float norm = weight > 0.f ? 1.f / weight : 0.f;
+        const float tmp[4] = {sum[0] * norm, sum[1] * norm, sum[2] * norm, sum[3] * norm};
+        store_converted<half_t, 4>(out + (size_t)row * d_v + column, tmp);
     }
 }
 
@@ -1066,7 +1150,7 @@ struct UnionShape {
     size_t plan_lds;  // LDS of the plan kernel for this shape
 };
 
-static bool union_shape(UnionShape &s, int vec_length, int n, int d_qk, int d_v, int rows, bool planned)
+static bool union_shape(UnionShape &s, int vec_length, int n, int d_qk, int d_v, int rows, bool planned, int stream_rounds = kStreamRounds)
 {
     const int rpw = 16 / vec_length;
     s.waves = ceil_div(rows < 1 ? 1 : rows, rpw);
@@ -1080,7 +1164,7 @@ static bool union_shape(UnionShape &s, int vec_length, int n, int d_qk, int d_v,
     const size_t bitmaps = 2 * (size_t)n_words * sizeof(unsigned) + 16 * sizeof(int);  // what build_union adds
     if (s.stream) {
         s.u_max = kStreamRanks;
-        s.rounds = kStreamRounds;
+        s.rounds = stream_rounds;
         s.steps = kStreamSteps;
         const size_t mask = (size_t)union_mask_words(s.rows, s.steps) * sizeof(unsigned);
         // masks of one sub-round, its K rows and its V columns (transposed) side by side
@@ -1121,6 +1205,10 @@ struct UnionLaunch {
     hipStream_t stream;
     const Batch *batch;
     long long stride_v;
+    // split launches (slots != nullptr)
+    const int *slots;
+    int n_slots, n_merges, n_partials;
+    float *partials;
 };
 
 template <int V, int KS, int CPL, bool PLANNED>
@@ -1128,15 +1216,29 @@ static int launch_one(const UnionLaunch &a)
 {
     UnionShape s;
     if (!union_shape(s, V, a.n, a.d_qk, a.d_v, a.rows, PLANNED)) return hipErrorNotSupported;
-    static std::atomic<unsigned long long> lds_allowed{0}, stream_lds_allowed{0};
+    static std::atomic<unsigned long long> lds_allowed{0}, stream_lds_allowed{0}, split_lds_allowed{0};
     const dim3 grid((unsigned)ceil_div(a.m_vec, s.rows), (unsigned)a.batch->count);
+    if (PLANNED && a.slots) {
+        auto kernel = sparse_attention_stream_kernel<V, KS, CPL, true>;
+        const hipError_t attr = allow_large_lds(reinterpret_cast<const void *>(kernel), 160 * 1024, split_lds_allowed);
+        if (attr != hipSuccess) return (int)attr;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)a.n_slots, (unsigned)a.batch->count), dim3(512), s.lds, a.stream, a.m_vec, a.n,
+                           a.d_qk, a.d_v, a.row_offsets, a.col_indices, a.plan, a.q, a.k, a.v, a.out, a.batch->stride_a,
+                           a.batch->stride_b, a.stride_v, a.batch->stride_out, a.scale, a.slots, a.n_partials, a.partials);
+        const hipError_t st = hipGetLastError();
+        if (st != hipSuccess || a.n_merges == 0) return (int)st;
+        hipLaunchKernelGGL(sparse_attention_merge_kernel, dim3((unsigned)a.n_merges, (unsigned)a.batch->count, 4), dim3(512), 0,
+                           a.stream, a.m_vec, V, a.n, a.d_v, a.plan, a.slots + 4 * (size_t)a.n_slots, a.n_partials, a.partials,
+                           a.out, a.batch->stride_out, a.scale);
+        return (int)hipGetLastError();
+    }
     if (PLANNED && s.stream) {
-        auto kernel = sparse_attention_stream_kernel<V, KS, CPL>;
+        auto kernel = sparse_attention_stream_kernel<V, KS, CPL, false>;
         const hipError_t attr = allow_large_lds(reinterpret_cast<const void *>(kernel), 160 * 1024, stream_lds_allowed);
         if (attr != hipSuccess) return (int)attr;
         hipLaunchKernelGGL(kernel, grid, dim3(512), s.lds, a.stream, a.m_vec, a.n, a.d_qk, a.d_v, a.row_offsets,
                            a.col_indices, a.plan, a.q, a.k, a.v, a.out, a.batch->stride_a, a.batch->stride_b,
-                           a.stride_v, a.batch->stride_out, a.scale);
+                           a.stride_v, a.batch->stride_out, a.scale, static_cast<const int *>(nullptr), 0, static_cast<float *>(nullptr));
         return (int)hipGetLastError();
     }
     auto kernel = sparse_attention_union_kernel<V, KS, CPL, PLANNED>;
@@ -1188,22 +1290,22 @@ int sparse_attention_union_capacity(int vec_length, int n, int d_qk, int d_v, in
     return s.rounds * s.u_max;
 }
 
-long long sparse_attention_plan_bytes(int m_vec, int vec_length, int n, int d_qk, int d_v, int rows)
+long long sparse_attention_plan_bytes(int m_vec, int vec_length, int n, int d_qk, int d_v, int rows, bool split)
 {
     UnionShape s;
     if (m_vec < 0 || !union_supported(vec_length, n, d_qk, d_v)) return 0;
-    if (!union_shape(s, vec_length, n, d_qk, d_v, rows, true)) return 0;
+    if (!union_shape(s, vec_length, n, d_qk, d_v, rows, true, split ? kSplitRounds : kStreamRounds)) return 0;
     const long long stride = 4 + s.rounds * ((long long)union_mask_words(s.rows, s.steps) + s.u_max);
     return (long long)sizeof(int) * (kPlanHeader + stride * ceil_div(m_vec, s.rows));
 }
 
 int launch_sparse_attention_plan(int m_vec, int vec_length, int n, int d_qk, int d_v, int rows, const int *row_offsets,
-                                 const int *col_indices, int *plan, long long plan_bytes, hipStream_t stream)
+                                 const int *col_indices, int *plan, long long plan_bytes, hipStream_t stream, bool split)
 {
     UnionShape s;
     if (!union_supported(vec_length, n, d_qk, d_v)) return hipErrorNotSupported;
-    if (!union_shape(s, vec_length, n, d_qk, d_v, rows, true)) return hipErrorNotSupported;
-    const long long need = sparse_attention_plan_bytes(m_vec, vec_length, n, d_qk, d_v, rows);
+    if (!union_shape(s, vec_length, n, d_qk, d_v, rows, true, split ? kSplitRounds : kStreamRounds)) return hipErrorNotSupported;
+    const long long need = sparse_attention_plan_bytes(m_vec, vec_length, n, d_qk, d_v, rows, split);
     if (plan_bytes < need) return hipErrorInvalidValue;
     if (m_vec == 0) return hipSuccess;
     static std::atomic<unsigned long long> lds_allowed{0};
@@ -1224,9 +1326,22 @@ int launch_sparse_attention_union(int m_vec, int vec_length, int n, int d_qk, in
     if (batch.count > 65535) return hipErrorNotSupported;
     if (!union_supported(vec_length, n, d_qk, d_v)) return hipErrorNotSupported;
     const UnionLaunch a = {m_vec, n, d_qk, d_v, rows, row_offsets, col_indices, plan, q, k, v, out,
-                           scale, stream, &batch, stride_v};
+                           scale, stream, &batch, stride_v, nullptr, 0, 0, 0, nullptr};
     if (plan) return launch_v<true>(vec_length, a);
     return launch_v<false>(vec_length, a);
+}
+
+int launch_sparse_attention_split(int m_vec, int vec_length, int n, int d_qk, int d_v, const int *row_offsets,
+                                  const int *col_indices, const int *plan, const int *slots, int n_slots, int n_merges,
+                                  int n_partials, float *partials, const half_t *q, const half_t *k, const half_t *v,
+                                  half_t *out, float scale, hipStream_t stream, const Batch &batch, long long stride_v)
+{
+    if (m_vec == 0 || batch.count == 0 || d_v == 0 || n_slots == 0) return hipSuccess;
+    if (batch.count > 65535 || n_merges > 65535) return hipErrorNotSupported;
+    if (!union_supported(vec_length, n, d_qk, d_v)) return hipErrorNotSupported;
+    const UnionLaunch a = {m_vec, n, d_qk, d_v, 128 / vec_length, row_offsets, col_indices, plan, q, k, v, out,
+                           scale, stream, &batch, stride_v, slots, n_slots, n_merges, n_partials, partials};
+    return launch_v<true>(vec_length, a);
 }
 
 }  // namespace vs

@@ -419,9 +419,15 @@ int launch_sparse_attention_union(int m_vec, int vec_length, int n, int d_qk, in
                                   const int *col_indices, const int *plan, const half_t *q, const half_t *k,
                                   const half_t *v, half_t *out, float scale, hipStream_t stream, const Batch &batch,
                                   long long stride_v);
-long long sparse_attention_plan_bytes(int m_vec, int vec_length, int n, int d_qk, int d_v, int rows);
+// Split launches of the streamed kernel: `slots` = [n_slots][4] {row block, first sub-round, end, partial tile or -1}, then
+// [n_merges][4] {row block, first partial tile, tiles, 0}, in device memory; `partials`: 128 x (d_v + 2) floats per tile and head.
+int launch_sparse_attention_split(int m_vec, int vec_length, int n, int d_qk, int d_v, const int *row_offsets,
+                                  const int *col_indices, const int *plan, const int *slots, int n_slots, int n_merges,
+                                  int n_partials, float *partials, const half_t *q, const half_t *k, const half_t *v,
+                                  half_t *out, float scale, hipStream_t stream, const Batch &batch, long long stride_v);
+long long sparse_attention_plan_bytes(int m_vec, int vec_length, int n, int d_qk, int d_v, int rows, bool split = false);
 int launch_sparse_attention_plan(int m_vec, int vec_length, int n, int d_qk, int d_v, int rows, const int *row_offsets,
-                                 const int *col_indices, int *plan, long long plan_bytes, hipStream_t stream);
+                                 const int *col_indices, int *plan, long long plan_bytes, hipStream_t stream, bool split = false);
 int sparse_attention_union_capacity(int vec_length, int n, int d_qk, int d_v, int rows, bool with_plan, int *rows_used);
 int launch_sparse_softmax(int m_vec, int vec_length, const int *row_indices, const int *row_offsets,
                           const half_t *values_in, half_t *values_out, float scale, hipStream_t stream,

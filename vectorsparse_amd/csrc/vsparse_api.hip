@@ -563,6 +563,48 @@ int vs_sparse_attention_f16(int batch, int m_vec, int vec_length, int n, int d_q
                                        stride_v);
 }
 
+long long vs_sparse_attention_split_plan_bytes(int m_vec, int vec_length, int n, int d_qk, int d_v)
+{
+    if (m_vec < 0 || n < 0 || !vec_ok(vec_length)) return 0;
+    return vs::sparse_attention_plan_bytes(m_vec, vec_length, n, d_qk, d_v, 128 / vec_length, true);
+}
+
+int vs_sparse_attention_split_plan(int m_vec, int vec_length, int n, int d_qk, int d_v, const int *row_offsets,
+                                   const int *col_indices, void *plan, long long plan_bytes, void *stream)
+{
+    if (m_vec < 0 || n < 0 || !vec_ok(vec_length)) return VS_ERROR_INVALID_VALUE;
+    if (!plan || !aligned(plan, 16) || (m_vec > 0 && !row_offsets)) return VS_ERROR_INVALID_VALUE;
+    return vs::launch_sparse_attention_plan(m_vec, vec_length, n, d_qk, d_v, 128 / vec_length, row_offsets, col_indices,
+                                            static_cast<int *>(plan), plan_bytes, static_cast<hipStream_t>(stream), true);
+}
+
+int vs_sparse_attention_f16_split(int batch, int m_vec, int vec_length, int n, int d_qk, int d_v, const int *row_offsets,
+                                  const int *col_indices, const void *q, long long stride_q, const void *k,
+                                  long long stride_k, const void *v, long long stride_v, void *out, long long stride_out,
+                                  float scale, const void *plan, long long plan_bytes, const int *slots, int n_slots,
+                                  int n_merges, int n_partials, void *workspace, long long workspace_bytes, void *stream)
+{
+    if (batch < 0 || m_vec < 0 || n < 0 || !vec_ok(vec_length) || d_qk <= 0 || d_v <= 0) return VS_ERROR_INVALID_VALUE;
+    if (n_slots < 0 || n_merges < 0 || n_partials < 0) return VS_ERROR_INVALID_VALUE;
+    // (the kernels read the plan at offsets that follow from this launch's shape before they know whether it is theirs)
+    const long long need = vs::sparse_attention_plan_bytes(m_vec, vec_length, n, d_qk, d_v, 128 / vec_length, true);
+    if (need <= 0) return VS_ERROR_NOT_SUPPORTED;
+    if (!plan || !aligned(plan, 16) || plan_bytes < need) return VS_ERROR_INVALID_VALUE;
+    if (batch == 0 || m_vec == 0 || n_slots == 0) return VS_SUCCESS;
+    if (!row_offsets || !q || !out || !slots || !aligned(slots, 16) || (n > 0 && (!k || !v))) return VS_ERROR_INVALID_VALUE;
+    if (!aligned(q, 16) || !aligned(k, 16) || !aligned(v, 16) || !aligned(out, 16)) return VS_ERROR_INVALID_VALUE;
+    if (!stride_ok(stride_q, 8) || !stride_ok(stride_k, 8) || !stride_ok(stride_v, 8) || !stride_ok(stride_out, 8))
+        return VS_ERROR_INVALID_VALUE;
+    if (workspace_bytes < 4LL * 128 * (d_v + 2) * n_partials * batch) return VS_ERROR_INVALID_VALUE;
+    if (n_partials > 0 && (!workspace || !aligned(workspace, 16))) return VS_ERROR_INVALID_VALUE;
+    return vs::launch_sparse_attention_split(m_vec, vec_length, n, d_qk, d_v, row_offsets, col_indices, static_cast<const int *>(plan),
+                                             slots, n_slots, n_merges, n_partials, static_cast<float *>(workspace),
+                                             static_cast<const half_t *>(q), static_cast<const half_t *>(k),
+                                             static_cast<const half_t *>(v), static_cast<half_t *>(out), scale,
+                                             static_cast<hipStream_t>(stream), make_batch(batch, stride_q, stride_k, stride_out),
+                                             stride_v);
+}
+
 long long vs_sparse_attention_plan_bytes(int m_vec, int vec_length, int n, int d_qk, int d_v, int rows_per_workgroup)
 {
     if (m_vec < 0 || n < 0 || !vec_ok(vec_length) || rows_per_workgroup < 2 || rows_per_workgroup > 128) return 0;

@@ -416,6 +416,75 @@ def sparse_attention_plan(m_vec, vec_length, n, d_qk, d_v, rows_per_workgroup, r
     return plan
 
 
+def distinct_columns(mask, rows):
+    """Distinct columns of every block of `rows` vector rows."""
+    sizes = []
+    for first in range(0, mask.m_vec, rows):
+        held = np.zeros(mask.n, dtype=bool)
+        held[mask.column_indices[mask.row_offsets[first]:mask.row_offsets[min(first + rows, mask.m_vec)]]] = True
+        sizes.append(int(np.count_nonzero(held)))
+    return sizes
+
+
+class AttentionSlots:
+    """The slots of `vs_sparse_attention_f16_split` for a mask, given the distinct columns of its blocks of 128 scalar rows:
+    blocks of more than `rounds` sub-rounds of 128 columns are cut into that many each.  Host array `slots`
+    (int32 [n_slots + n_merges][4], longest first), and the counts the entry point takes."""
+
+    def __init__(self, unions, rounds):
+        whole, parts, merges = [], [], []
+        for block, size in enumerate(unions):
+            needed = -(-size // 128)
+            if needed <= rounds:
+                whole.append((needed, (block, 0, 1 << 20, -1)))
+                continue
+            count = -(-needed // rounds)
+            cuts = [i * needed // count for i in range(count)] + [1 << 20]   # (even shares)
+            merges.append((block, len(parts), count, 0))
+            parts += [(block, cuts[i], cuts[i + 1], len(parts) + i) for i in range(count)]
+        whole = [slot for _, slot in sorted(whole, key=lambda w: -w[0])]
+        self.n_slots, self.n_merges, self.n_partials = len(whole) + len(parts), len(merges), len(parts)
+        self.slots = np.array(parts + whole + merges, dtype=np.int32).reshape(-1, 4)
+
+
+def sparse_attention_split(prob, slots, device_slots, plan, q, k, v, out, scale, workspace=None, stream=None):
+    """Fixed-mask attention with long row blocks streamed by several workgroups (vs_sparse_attention_f16_split).  prob: the
+    mask's DeviceProblem, slots: an AttentionSlots, device_slots: its list on the device, plan: from
+    `sparse_attention_split_plan`; q, k, v, out [heads, rows, width]; workspace: a float32 tensor of at least
+    n_partials * heads * 128 * (d_v + 2) elements (made for the call when None)."""
+    heads, _, d = q.shape
+    d_v = v.shape[2]
+    if workspace is None and slots.n_partials:
+        workspace = torch.empty(slots.n_partials * heads * 128 * (d_v + 2), dtype=torch.float32, device=q.device)
+        if stream is not None:
+            workspace.record_stream(stream if isinstance(stream, torch.cuda.Stream) else torch.cuda.ExternalStream(int(stream)))
+    st = _native.sparse_attention_split(heads, prob.m_vec, prob.vec_length, prob.n, d, d_v, prob.row_offsets, prob.column_indices,
+                                        q, k, v, out, float(scale), plan, device_slots, slots.n_slots, slots.n_merges,
+                                        slots.n_partials, workspace, stream)
+    if st < 0:
+        for t, nm in ((q, "q"), (k, "k"), (v, "v"), (out, "out")):
+            _expect_batched(t, torch.float16, nm)
+        st = _lib.lib().vs_sparse_attention_f16_split(
+            heads, prob.m_vec, prob.vec_length, prob.n, d, d_v, _ptr(prob.row_offsets), _ptr(prob.column_indices), _ptr(q),
+            _stride(q, heads), _ptr(k), _stride(k, heads), _ptr(v), _stride(v, heads), _ptr(out), _stride(out, heads), float(scale),
+            _ptr(plan), plan.numel() * plan.element_size(), _ptr(device_slots), slots.n_slots, slots.n_merges, slots.n_partials,
+            _ptr(workspace), 0 if workspace is None else workspace.numel() * workspace.element_size(), _stream(stream))
+    _lib.check(st, "vs_sparse_attention_f16_split")
+    return out
+
+
+def sparse_attention_split_plan(m_vec, vec_length, n, d_qk, d_v, row_offsets, col_indices, stream=None):
+    """The plan of `sparse_attention_split` for a mask (a device byte tensor), as `sparse_attention_plan`."""
+    size = _lib.lib().vs_sparse_attention_split_plan_bytes(m_vec, vec_length, n, d_qk, d_v)
+    if size <= 0:
+        raise _lib.VSparseError("vs_sparse_attention_split_plan_bytes: shape not supported by the streamed kernel")
+    plan = torch.empty(size, dtype=torch.uint8, device=row_offsets.device)
+    st = _lib.lib().vs_sparse_attention_split_plan(m_vec, vec_length, n, d_qk, d_v, _ptr(row_offsets), _ptr(col_indices),
+                                                   _ptr(plan), size, _stream(stream))
+    _lib.check(st, "vs_sparse_attention_split_plan")
+    return plan
+
+
 class SparseAttention:
     """One fixed-mask sparse attention layer: SDDMM (QK^T on the mask) -> row softmax -> SpMM (P V).
 
@@ -432,6 +501,24 @@ class SparseAttention:
         self._plans = {}
         self._rows = {}
         self._routes = {}
+        self._splits = {}       # (d, d_v, rounds) -> (AttentionSlots, its list on the device, plan)
+        self._unions = None     # distinct columns of every block of 128 scalar rows
+
+    def _block_unions(self):
+        if self._unions is None:
+            self._unions = distinct_columns(self.mask, 128 // self.mask.vec_length)
+        return self._unions
+
+    def _split(self, d, d_v, rounds):
+        """Slots and plan of the split launch with at most `rounds` sub-rounds per workgroup, made once."""
+        key = (d, d_v, rounds)
+        if key not in self._splits:
+            p = self.prob
+            slots = AttentionSlots(self._block_unions(), rounds)
+            plan = sparse_attention_split_plan(p.m_vec, p.vec_length, p.n, d, d_v, p.row_offsets, p.column_indices)
+            torch.cuda.current_stream().synchronize()   # (calls on any stream may read it from here on)
+            self._splits[key] = (slots, torch.from_numpy(slots.slots).to(p.row_offsets.device), plan)
+        return self._splits[key]
 
     def _parts_route_fits(self, d_v, heads):
         """The SpMM of the three-operator route on row parts takes less than 2 GiB of partial tiles (the limit of
@@ -456,18 +543,83 @@ class SparseAttention:
             else:
                 route = "layer" if self.union_rows(d, d_v, heads) >= 2 else True
             self._routes[key] = route
-        return route
+            self._routes[key] = self._split_route(d, d_v, heads, route) or route
+        return self._routes[key]
+
+    # Microseconds per layer by route, fitted on MI355X to 19000 masks (1..16 heads x 512..4096, band with and without global
+    # tokens, random, every V; head widths to 32, 64 and 128).  Streamed workgroups: launch, per sub-round of the longest one,
+    # launch under load, per workgroup and per sub-round in 512ths, merge, per tile of the longest merge (good to 5-7 %).
+    _STREAM_US = ((3.47, 2.06, 5.15, 2.13, 4.21, 2.9, 0.5), (3.41, 2.47, 5.86, 4.21, 4.87, 3.12, 0.49),
+                  (4.1, 3.64, 6.0, 10.63, 10.22, 3.98, 1.01))
+    # The three operators on row parts: launches, per thousand vector rows of 16 heads, per thousand nonzero vectors of 16 heads
+    # by vector length (7 %).
+    _PARTS_US = ((16.0, 14.0, {1: 0.176, 2: 0.207, 4: 0.276, 8: 0.466}), (16.4, 16.0, {1: 0.223, 2: 0.251, 4: 0.327, 8: 0.523}),
+                 (16.9, 23.7, {1: 0.327, 2: 0.37, 4: 0.463, 8: 0.712}))
+    # The two launches: the same, then per thousand nonzero vectors of the longest row, and the share of the shorter of the
+    # two that is not hidden (13-17 %).
+    _TWO_US = ((6.6, 9.0, {1: 0.16, 2: 0.194, 4: 0.219, 8: 0.314}, 8.2, 1.95), (6.7, 12.5, {1: 0.172, 2: 0.21, 4: 0.272, 8: 0.409}, 8.3, 1.58),
+               (6.7, 20.9, {1: 0.235, 2: 0.326, 4: 0.432, 8: 0.701}, 9.2, 1.52))
+
+    @staticmethod
+    def _stream_us(unions, heads, width_class, rounds):
+        """Estimate of the streamed kernel with at most `rounds` sub-rounds per workgroup."""
+        first, per_round, loaded, per_group, per_part, merge, per_tile = SparseAttention._STREAM_US[width_class]
+        needed = [-(-u // 128) for u in unions]
+        counts = [max(1, -(-n // rounds)) for n in needed]
+        alone = first + per_round * max(-(-n // c) for n, c in zip(needed, counts))
+        busy = loaded + (per_group * sum(counts) + per_part * sum(needed)) * heads / 512.0
+        time = max(alone, busy) + 0.15 * min(alone, busy)
+        return time + (merge + per_tile * max(counts) if max(counts) > 1 else 0.0)
+
+    def _split_route(self, d, d_v, heads, route):
+        """("split", sub-rounds) where streaming long row blocks by several workgroups is expected to take less than four
+        fifths of `route`, else None.  Over the masks of the fit: chosen for 8300 of 18900, 1.34 times faster in the mean of
+        all (1.39 if the faster side were always taken), ten slower by more than 3 %.  16 heads x 2409, V = 1, a +-139 band
+        with 32 global tokens: 260 us in parts, 30 us; 8 heads x 2048, V = 8, +-64 and 64 tokens: 33 us, 19 us."""
+        p, m = self.prob, self.mask
+        if (m.m_vec == 0 or m.nnz_vec == 0 or d % 8 != 0 or d_v % 8 != 0
+                or _lib.lib().vs_sparse_attention_split_plan_bytes(p.m_vec, p.vec_length, p.n, d, d_v) <= 0):
+            return None
+        unions = self._block_unions()
+        longest = -(-max(unions) // 128)
+        if longest > 32 or longest < 2:     # (a split plan holds 4096 columns of a block)
+            return None
+        c = 0 if max(d, d_v) <= 32 else (1 if max(d, d_v) <= 64 else 2)
+        if route == "parts":
+            launches, per_row, per_nonzero = self._PARTS_US[c]
+            other = launches + (per_row * p.m_vec + per_nonzero[p.vec_length] * p.nnz_vec) * heads / 16e3
+        elif route == "layer":
+            other = self._stream_us(unions, heads, c, longest)
+        else:
+            launches, per_row, per_nonzero, per_longest, hidden = self._TWO_US[c]
+            work = (per_row * p.m_vec + per_nonzero[p.vec_length] * p.nnz_vec) * heads / 16e3
+            row = per_longest * p.longest_row_vec * 1e-3
+            other = launches + max(work, row) + hidden * min(work, row)
+        best, rounds = 0.8 * other, None
+        for r in (1, 2, 3, 4, 6, 8, 12, 16, 32):
+            if r >= longest and rounds is None and route == "layer":
+                break
+            tiles = sum(-(-n // r) for n in (-(-u // 128) for u in unions) if n > r)
+            time = self._stream_us(unions, heads, c, r)
+            if time < best and tiles * heads * 512 * (d_v + 2) <= 2 ** 27:   # (128 MiB of partial tiles)
+                best, rounds = time, r
+            if r >= longest:
+                break
+        return None if rounds is None else ("split", rounds)
 
     def union_rows(self, d_qk, d_v, heads=16):
         """Rows per workgroup for the single-launch kernel with these head widths and head count (cached)."""
         key = (int(d_qk), int(d_v), int(heads))
         if key not in self._rows:
-            self._rows[key] = self._union_rows(self.mask, *key)
+            self._rows[key] = self._union_rows(self.mask, *key, unions=self._block_unions())
         return self._rows[key]
 
     def plan(self, d_qk, d_v, heads=16):
         """Device plan of the union kernel for these head widths (built on first use), or None."""
         rows = self.union_rows(d_qk, d_v, heads)
+        route = self._route(d_qk, d_v, heads)
+        if type(route) is tuple:
+            self._split(d_qk, d_v, route[1])
         if rows < 2:
             return None
         key = (int(d_qk), int(d_v), rows)
@@ -486,7 +638,7 @@ class SparseAttention:
     _TWO_LAUNCH_NS = {8: (19.5, 0.35), 4: (15.6, 0.29), 2: (13.2, 0.25), 1: (12.0, 0.22)}
 
     @staticmethod
-    def _union_rows(mask, d_qk, d_v, heads=16):
+    def _union_rows(mask, d_qk, d_v, heads=16, unions=None):
         """Vector rows per workgroup for the single-launch kernel: workgroups of eight waves (128 scalar rows,
         which stream the union of their columns through LDS) when every block's distinct columns stay within
         the library's capacity for this shape and the cost model above puts the launch below the two-launch
@@ -500,7 +652,6 @@ class SparseAttention:
         kernel that holds the union at once) were slower than eight waves on every mask where both apply
         (+-4 .. +-64 bands: four waves 17.6 .. 27.1 us, eight waves 12.5 .. 15.3 us), so they are left to
         callers that ask for them."""
-        ro, ci = mask.row_offsets, mask.column_indices
         if mask.m_vec == 0 or mask.nnz_vec == 0:
             return 1
         used = ctypes.c_int(0)
@@ -510,8 +661,8 @@ class SparseAttention:
         rows = used.value
         if cap <= 0 or rows != want:
             return 1
-        unions = [np.unique(ci[ro[first]:ro[min(first + rows, mask.m_vec)]]).size
-                  for first in range(0, mask.m_vec, rows)]
+        if unions is None:
+            unions = distinct_columns(mask, rows)
         longest = max(unions)
         if longest > cap:
             return 1
@@ -531,7 +682,8 @@ class SparseAttention:
     def forward(self, q, k, v, scale=None, kernel="wmma", stream=None, scores=None, out=None, fused=None):
         """q, k, v: fp16 [heads, seq, d] on the device.  Returns fp16 [heads, seq, d].
 
-        fused: "parts" runs the three operators on the dispatch list of row parts (masks with rows far longer than
+        fused: ("split", rounds) runs the layer in one launch plus a merge, row blocks of more than `rounds` x 128 distinct columns
+        (rows that attend to everything) streamed by several workgroups; "parts" runs the three operators on the dispatch list of row parts (masks with rows far longer than
         the rest, e.g. global tokens); "layer" runs the whole layer in one launch with scores and probabilities kept in LDS; True
         folds only the softmax into the SpMM launch (two launches, raw scores go through memory); False runs
         the three operators one after the other.  Default on the MFMA path: "layer" when the cost model of
@@ -553,6 +705,8 @@ class SparseAttention:
             return sparse_attention(p.m_vec, p.vec_length, p.n, p.row_indices, p.row_offsets, p.column_indices,
                                     q, k, v, out=out, scale=scale, stream=stream,
                                     rows_per_workgroup=self.union_rows(d, d_v, heads), plan=self.plan(d, d_v, heads))
+        if isinstance(fused, tuple):    # ("split", sub-rounds per workgroup)
+            return sparse_attention_split(p, *self._split(d, d_v, fused[1]), q, k, v, out, scale, stream=stream)
         if scores is None:
             scores = torch.empty((heads, p.nnz_vec, p.vec_length), dtype=torch.float16, device=q.device)
         if fused == "parts":
