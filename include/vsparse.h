@@ -452,6 +452,19 @@ int vs_wmma_spmm_softmax_f16_batched(int batch, int m_vec, int vec_length, int k
                                      float scale, void *stream);
 
 /*
+ * values = softmax_row(scale * values) in place, then  out = values * rhs_matrix: vs_sparse_softmax_f16 followed by
+ * vs_wmma_spmm_f16_batched, the probabilities kept (a training forward needs them), in one launch where a row's output is one
+ * column tile.  Same requirements as vs_wmma_spmm_f16_batched.  No counterpart in the reference (see vs_sparse_softmax_f16).
+ */
+int vs_wmma_softmax_spmm_f16_batched(int batch, int m_vec, int vec_length, int k, int n, int nonzeros_vec,
+                                     int longest_row_vec, const int *row_indices,
+                                     const int *row_offsets, const int *column_indices,
+                                     void *values, long long stride_values,
+                                     const void *rhs_matrix, long long stride_rhs,
+                                     void *output_matrix, long long stride_output,
+                                     float scale, void *stream);
+
+/*
  * One fixed-mask sparse attention layer in a single launch:
  *     out[b] = softmax_row(scale * (q[b] k[b]^T sampled on the mask)) v[b]
  * q: [m_vec*vec_length, d_qk], k: [n, d_qk], v: [n, d_v], out: [m_vec*vec_length, d_v], all fp16
@@ -593,6 +606,8 @@ int vs_wmma_spmm_launch_shape(int batch, int m_vec, int vec_length, int k, int n
  * vector row, 0 = automatic), "sddmm_group" (16-vector groups per wave step of the
  * MFMA SDDMM: 1, 2, 4, 0 = automatic), "sddmm_block_waves" (1..16, 0 = automatic),
  * "sddmm_flat_supers" (super-groups per wave of algorithm 2, 1..16, 0 = automatic),
+ * "softmax_spmm" (softmax and SpMM that keeps the probabilities: 1 = in one launch where a row's output is one column tile,
+ * 2 = in two, 0 = automatic),
  * "spmm_tile" (SpMM on dense tiles, fp16 outputs, k % 4 == 0, any order of the columns: 1 = never, 2 = tiles of 32 x 64,
  * 3 = of 64 x 128, 4 = of 128 x 128, 0 = where the columns are known to ascend strictly and tiles are expected to be faster),
  * "sddmm_tile" (SDDMM on dense tiles, k % 8 == 0, any order of the columns: 1 = never, 2 = tiles of 64 x 64,

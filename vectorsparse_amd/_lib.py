@@ -41,6 +41,8 @@ SIGNATURES = {
     "vs_cuda_sddmm_f16_sorted": ([_int] * 5 + [_vp] * 3 + [_vp, _ll, _vp, _ll, _vp, _ll, _int, _int, _vp], _int),
     "vs_wmma_spmm_softmax_f16_batched": ([_int] * 7 + [_vp] * 3 + [_vp, _ll, _vp, _ll, _vp, _ll, ctypes.c_float, _vp],
                                          _int),
+    "vs_wmma_softmax_spmm_f16_batched": ([_int] * 7 + [_vp] * 3 + [_vp, _ll, _vp, _ll, _vp, _ll, ctypes.c_float, _vp],
+                                         _int),
     "vs_sparse_attention_f16": ([_int] * 6 + [_vp] * 3 + [_vp, _ll, _vp, _ll, _vp, _ll, _vp, _ll, ctypes.c_float, _int,
                                  _vp, _ll, _vp],
                                 _int),

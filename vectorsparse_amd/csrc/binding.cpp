@@ -275,7 +275,8 @@ PyObject *cuda_spmm_batched(PyObject *, PyObject *const *args, Py_ssize_t n_args
 }
 
 // (batch, m_vec, vec_length, k, n, nonzeros_vec, longest_row_vec, row_indices, row_offsets, column_indices, scores, rhs, out,
-// scale, stream)
+// scale, stream); KEPT: the scores become the probabilities
+template <bool KEPT>
 PyObject *spmm_softmax_batched(PyObject *, PyObject *const *args, Py_ssize_t n_args)
 {
     Reader r(args, n_args);
@@ -288,7 +289,10 @@ PyObject *spmm_softmax_batched(PyObject *, PyObject *const *args, Py_ssize_t n_a
     const float scale = r.number();
     void *stream = r.stream();
     return status_of(r, [&] {
-        return vs_wmma_spmm_softmax_f16_batched(batch, m_vec, v, k, n, nnz, longest, ri, ro, ci, scores, sa, rhs, sb, out, so, scale, stream);
+        if constexpr (KEPT)
+            return vs_wmma_softmax_spmm_f16_batched(batch, m_vec, v, k, n, nnz, longest, ri, ro, ci, const_cast<void *>(scores), sa, rhs, sb, out, so, scale, stream);
+        else
+            return vs_wmma_spmm_softmax_f16_batched(batch, m_vec, v, k, n, nnz, longest, ri, ro, ci, scores, sa, rhs, sb, out, so, scale, stream);
     });
 }
 
@@ -448,7 +452,8 @@ PyMethodDef methods[] = {
     VS_METHOD("cuda_sddmm", cuda_sddmm),
     VS_METHOD("wmma_spmm_batched", wmma_spmm_batched),
     VS_METHOD("cuda_spmm_batched", cuda_spmm_batched),
-    VS_METHOD("spmm_softmax_batched", spmm_softmax_batched),
+    VS_METHOD("spmm_softmax_batched", spmm_softmax_batched<false>),
+    VS_METHOD("softmax_spmm_batched", spmm_softmax_batched<true>),
     VS_METHOD("wmma_sddmm_batched", sddmm_batched<true>),
     VS_METHOD("cuda_sddmm_batched", sddmm_batched<false>),
     VS_METHOD("sparse_softmax", sparse_softmax),

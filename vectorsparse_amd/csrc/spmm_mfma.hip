@@ -46,12 +46,16 @@ namespace vs {
 // workgroup counts itself in on the row's arrival counter; the one that arrives last adds the parts in ascending
 // order - same bits whoever it is - writes the row and puts the counter back to zero.  Nobody waits for anybody.
 // How the parts reach the workgroup that adds them: PartMeeting in spmm_mfma_step.hpp.
+// KEEP (with SOFTMAX, one column tile): the probabilities replace the scores in memory.  Every wave of a row first finds the
+// row's maximum and sum over all of its scores - a barrier stands between these reads and the first store - and then
+// multiplies by, and writes back, the rounded probabilities of its own blocks: the numbers of the softmax kernel, one launch and
+// one pass over the values less (8 heads x 2048, V = 4, 95 %, d = 64, SDDMM included: 20.8 -> 17.8 us).
 template <int V, int CPL, bool SOFTMAX, bool IDX32, typename OutT, bool RAGGED = false, int S = 1, bool TEAMS = false,
-          bool PIPE = false, bool PARTS = false>
+          bool PIPE = false, bool PARTS = false, bool KEEP = false>
 __global__ void __launch_bounds__(S * CPL >= 32 ? 256 : (S * CPL >= 16 ? 512 : 1024))
 spmm_mfma_kernel(int n_cols, int n_tiles, int shape, const int *__restrict__ row_indices,
                  const int *__restrict__ row_offsets, const int *__restrict__ column_indices,
-                 const half_t *__restrict__ values, const half_t *__restrict__ rhs,
+                 const half_t *__restrict__ sparse_values, const half_t *__restrict__ rhs,
                  OutT *__restrict__ out, long long stride_values, long long stride_rhs, long long stride_out,
                  float scale, int team_slots, int n_slots,  // (the first sixteen dwords arrive preloaded in registers)
                  int *part_counters, float *part_tiles, int parts_max)
@@ -65,9 +69,15 @@ spmm_mfma_kernel(int n_cols, int n_tiles, int shape, const int *__restrict__ row
     const bool full_grid = (shape >> 16) & 1;
     const bool parts_meet_later = (shape >> 17) & 1;  // PARTS: a second launch adds the parts of split rows
     if (blockIdx.y != 0) {  // batch: shared pattern, per-problem operands (the strides are not loaded for problem 0)
-        values += blockIdx.y * stride_values;
+        sparse_values += blockIdx.y * stride_values;
         rhs += blockIdx.y * stride_rhs;
         out += blockIdx.y * stride_out;
+    }
+    static_assert(!KEEP || (SOFTMAX && !RAGGED && !TEAMS && !PIPE && !PARTS), "probabilities are kept by the softmax-fused operator");
+    const half_t *values = sparse_values;
+    if constexpr (KEEP) {   // read and written: nothing may be assumed of what else points there
+        asm volatile("" : "+s"(values)::"memory");
+        values = (const half_t *)(const __attribute__((address_space(1))) half_t *)values;
     }
     extern __shared__ __align__(16) unsigned char smem[];  // [W] staging slots, then [W][V][TN] partials
     constexpr int TN = 16 * CPL;
@@ -154,7 +164,43 @@ spmm_mfma_kernel(int n_cols, int n_tiles, int shape, const int *__restrict__ row
         row_max[v] = -__builtin_inff();
         row_sum[v] = 0.f;
     }
-    if constexpr (SOFTMAX) {
+    if constexpr (KEEP) {
+        constexpr int H = 4;  // vectors of a lane requested together, and held for the second pass in rows of up to 64 H
+        PackedVector<V> held[H];
+        auto load = [&](int j0) __attribute__((always_inline)) {
+#pragma unroll
+            for (int h = 0; h < H; ++h) {
+                const int j = j0 + 64 * h + lane;
+                held[h].load(values + (size_t)(j < end ? j : end - 1) * V);  // (a repeated vector changes no maximum)
+            }
+        };
+        for (int j0 = beg; j0 < end; j0 += 64 * H) {
+            load(j0);
+#pragma unroll
+            for (int h = 0; h < H; ++h) {
+#pragma unroll
+                for (int v = 0; v < V; ++v) row_max[v] = fmaxf(row_max[v], (float)held[h].at(v) * s2);
+            }
+        }
+#pragma unroll
+        for (int v = 0; v < V; ++v) row_max[v] = wave_max(row_max[v]);
+        for (int j0 = beg; j0 < end; j0 += 64 * H) {
+            if (end - beg > 64 * H) load(j0);
+#pragma unroll
+            for (int h = 0; h < H; ++h) {
+                const bool exists = j0 + 64 * h + lane < end;
+#pragma unroll
+                for (int v = 0; v < V; ++v)
+                    row_sum[v] += exists ? __builtin_amdgcn_exp2f((float)held[h].at(v) * s2 - row_max[v]) : 0.f;
+            }
+        }
+#pragma unroll
+        for (int v = 0; v < V; ++v) row_sum[v] = 1.f / wave_sum(row_sum[v]);
+        if (active > 1) {  // (every score of the row has been read by every wave that reads it whole)
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+        }
+    } else if constexpr (SOFTMAX) {
         for (int j = beg + lane; j < end; j += 64) {
             half_t x[V];
             load_vector<V>(x, values + (size_t)j * V);
@@ -205,16 +251,24 @@ spmm_mfma_kernel(int n_cols, int n_tiles, int shape, const int *__restrict__ row
             const int at = 64 * i + lane;
             if (at < kBlock) {
                 idx_s[at] = next_idx[i];
+                float probability[V];
 #pragma unroll
                 for (int v = 0; v < V; ++v) {
                     half_t staged = next_valid[i] ? next_vec[i].at(v) : (half_t)0.f;
-                    if constexpr (SOFTMAX) {
+                    if constexpr (KEEP) {
+                        const float p = __builtin_amdgcn_exp2f((float)next_vec[i].at(v) * s2 - row_max[v]) * row_sum[v];
+                        probability[v] = p;
+                        staged = next_valid[i] ? (half_t)p : (half_t)0.f;
+                    } else if constexpr (SOFTMAX) {
                         const float p =
                             next_valid[i] ? __builtin_amdgcn_exp2f((float)next_vec[i].at(v) * s2 - row_max[v]) : 0.f;
                         row_sum[v] += p;
                         staged = (half_t)p;
                     }
                     vec_s[v * kBlock + at] = staged;
+                }
+                if constexpr (KEEP) {
+                    if (next_valid[i]) store_converted<half_t, V>(const_cast<half_t *>(values) + (size_t)(base + at) * V, probability);
                 }
             }
         }
@@ -227,7 +281,7 @@ spmm_mfma_kernel(int n_cols, int n_tiles, int shape, const int *__restrict__ row
             const int v = 4 * g + e;
             if (v < V && col_ok) {
                 float norm = 1.f;
-                if constexpr (SOFTMAX) {
+                if constexpr (SOFTMAX && !KEEP) {
                     float total = 1.f;
 #pragma unroll
                     for (int vv = 0; vv < V; ++vv) total = (vv == v) ? row_sum[vv] : total;
@@ -359,7 +413,7 @@ spmm_mfma_kernel(int n_cols, int n_tiles, int shape, const int *__restrict__ row
         }
     }
 
-    if constexpr (SOFTMAX) {
+    if constexpr (SOFTMAX && !KEEP) {
 #pragma unroll
         for (int v = 0; v < V; ++v) row_sum[v] = wave_sum(row_sum[v]);
     }
@@ -399,7 +453,7 @@ spmm_mfma_kernel(int n_cols, int n_tiles, int shape, const int *__restrict__ row
             }
         }
     }
-    if constexpr (SOFTMAX) {
+    if constexpr (SOFTMAX && !KEEP) {
         if (lane < V) {
             float mine_sum = 0.f;
 #pragma unroll
@@ -431,7 +485,7 @@ spmm_mfma_kernel(int n_cols, int n_tiles, int shape, const int *__restrict__ row
                     sum[4 * c4 + 3] += x[3];
                 }
             }
-            if constexpr (SOFTMAX) {
+            if constexpr (SOFTMAX && !KEEP) {
                 float total = 0.f;
                 for (int w = 0; w < active; ++w) total += sums_s[w * V + v];
                 const float norm = end > beg ? 1.f / total : 0.f;
@@ -503,7 +557,8 @@ static int next_pow2(int x)
     return p;
 }
 
-template <int V, int CPL, bool SOFTMAX, bool IDX32, typename OutT, int S = 1, bool TEAMS = false, bool PIPE = false>
+template <int V, int CPL, bool SOFTMAX, bool IDX32, typename OutT, int S = 1, bool TEAMS = false, bool PIPE = false,
+          bool KEEP = false>
 static int launch_idx(int m_vec, int k, int n, int waves, const int *row_indices, const int *row_offsets,
                       const int *column_indices, const half_t *values, const half_t *rhs, OutT *out,
                       hipStream_t stream, const Batch &batch, float scale, int per_wave = 1, int team_slots = -1)
@@ -519,7 +574,7 @@ static int launch_idx(int m_vec, int k, int n, int waves, const int *row_indices
     if (blocks > 0x7fffffffLL) return hipErrorNotSupported;
     const size_t lds = (size_t)waves * S * stage_bytes<V>() +
                        (waves > 1 ? (size_t)waves * V * (TN + 1) * sizeof(float) : 0);
-    auto kernel = spmm_mfma_kernel<V, CPL, SOFTMAX, IDX32, OutT, false, S, TEAMS, PIPE>;
+    auto kernel = spmm_mfma_kernel<V, CPL, SOFTMAX, IDX32, OutT, false, S, TEAMS, PIPE, false, KEEP>;
     static std::atomic<unsigned long long> lds_allowed{0};
     const hipError_t attr = allow_large_lds(reinterpret_cast<const void *>(kernel), 96 * 1024, lds_allowed);
     if (attr != hipSuccess) return (int)attr;
@@ -595,7 +650,7 @@ static int launch_v(const SpmmShape &shape, int vec_length, int m_vec, int k, in
 
 // The launch shape of an MFMA SpMM, chosen on the host from what the entry point knows of the problem (the row
 // lengths only through the hints of the batched entry points) and from the calling thread's options.
-SpmmShape choose_spmm_shape(bool softmax, int m_vec, int vec_length, int k, int n, const Batch &batch)
+SpmmShape choose_spmm_shape(bool softmax, int m_vec, int vec_length, int k, int n, const Batch &batch, bool keep)
 {
     SpmmShape shape;
     constexpr int kTargetBlocks = 256;   // one workgroup per CU at least
@@ -648,7 +703,7 @@ SpmmShape choose_spmm_shape(bool softmax, int m_vec, int vec_length, int k, int 
         // average - 16 requested slots per row that a walk in steps of 32 does not issue.  16 heads x 4096 rows, N = 64,
         // V = 1: rows of 82 / 205 / 410 vectors 62.4 -> 50.0, 120.9 -> 109.8, 208.6 -> 201.1 us; V = 2, 205: 63.2 ->
         // 58.5; V = 4 and 8 are the other way round (rows of 102, V = 4: 11.8 against 12.8 us).
-        if (hinted && vec_length <= 2 && blocks >= 16384 && mean_steps <= 16) in_flight = 1;
+        if (!keep && hinted && vec_length <= 2 && blocks >= 16384 && mean_steps <= 16) in_flight = 1;
         // (rows of unequal length end in half-empty blocks of 128: on log-normal and Pareto lengths four steps in
         // flight were 10-25 % behind two)
 #ifdef VS_RETIRED_VARIANTS
@@ -662,7 +717,12 @@ SpmmShape choose_spmm_shape(bool softmax, int m_vec, int vec_length, int k, int 
     // of vectors of four or eight (16 heads x 4096, d = 64: band + strided mask 37.2 -> 31.0 us, uniform 90 % 44.5 ->
     // 39.2 us; rows of 82 vectors 15.8 -> 16.4 us, V = 1 at 95 % 114 -> 125 us).
     if (softmax && in_flight == 4) in_flight = 2;
-    if (softmax && options().spmm_steps == 0 && (vec_length < 4 || row_steps <= 4)) in_flight = 1;
+    // Where the probabilities are kept they also pay on rows of one to two blocks (SDDMM included, V = 8: rows of 102 vectors
+    // 16.3 -> 14.2 us, of 38 10.0 -> 9.6; V = 4, rows of 59: 14.5 -> 13.7; V = 4, rows of 27: 7.4 -> 7.6) and, with 128-bit
+    // segments or on rows of more than 224, for short vectors (d = 128, V = 1, 388: 388 -> 330 us, V = 2, 296: 42.7 -> 38.9;
+    // d = 64, V = 1, 150: 90.0 -> 94.6; d = 32, V = 1, 346: 54.9 -> 52.1).
+    if (softmax && options().spmm_steps == 0 &&
+        (keep ? mean_steps <= (vec_length >= 4 || cpl == 8 ? 1 : 7) : vec_length < 4 || row_steps <= 4)) in_flight = 1;
     int per_wave = 1;
     int team_slots = -1;
     int waves = options().spmm_waves;
@@ -870,12 +930,70 @@ int launch_spmm_mfma(int m_vec, int vec_length, int k, int n, const int *row_ind
                                    out, stream, batch, 1.f);
 }
 
+// Whether the softmax-fused product may keep the probabilities: the problems' values do not overlap, and it is expected to be
+// faster than two launches.  Every wave of a row reads all of its scores, which rows of up to 512 vectors repay (of 180 masks and
+// head counts, SDDMM included: 1.00 to 1.33 times as fast, 1.15 in the mean); with a few rows of 1024 or 2048 vectors among
+// short ones it was 0.86 to 1.08 times as fast.
+static bool softmax_spmm_fused(int vec_length, int k, int n, const Batch &batch)
+{
+    if (k <= 0 || k % 4 != 0 || k > 128 || (long long)n * k >= (1LL << 31) || options().softmax_spmm == 2) return false;
+    if (batch.count > 1 && (batch.nonzeros_vec < 0 || batch.stride_a < (long long)batch.nonzeros_vec * vec_length)) return false;
+    return options().softmax_spmm == 1 || (batch.nonzeros_vec >= 0 && batch.longest_row_vec >= 0 && batch.longest_row_vec <= 512);
+}
+
 int launch_spmm_softmax_mfma(int m_vec, int vec_length, int k, int n, const int *row_indices,
                              const int *row_offsets, const int *column_indices, const half_t *scores,
                              const half_t *rhs, half_t *out, float scale, hipStream_t stream, const Batch &batch)
 {
     return launch_any<true, half_t>(m_vec, vec_length, k, n, row_indices, row_offsets, column_indices, scores, rhs,
                                     out, stream, batch, scale);
+}
+
+namespace {
+
+template <int V>
+int launch_keep(const SpmmShape &shape, int m_vec, int k, int n, const int *row_indices, const int *row_offsets,
+                const int *column_indices, const half_t *values, const half_t *rhs, half_t *out, hipStream_t stream,
+                const Batch &batch, float scale)
+{
+    const bool two = shape.steps_in_flight >= 2;
+#define VS_SPMM_KEEP(CPL, S)                                                                                          \
+    launch_idx<V, CPL, true, true, half_t, S, false, false, true>(m_vec, k, n, shape.waves, row_indices, row_offsets,     \
+                                                                  column_indices, values, rhs, out, stream, batch, scale, \
+                                                                  S == 1 ? 1 : shape.blocks_per_wave, -1)
+    if (shape.cols_per_lane == 8) return two ? VS_SPMM_KEEP(8, 2) : VS_SPMM_KEEP(8, 1);
+    return two ? VS_SPMM_KEEP(4, 2) : VS_SPMM_KEEP(4, 1);
+#undef VS_SPMM_KEEP
+}
+
+}  // namespace
+
+// values = softmax_row(scale * values), out = values * rhs: one launch where a row's output is one column tile (else the
+// workgroups of a row's tiles would read scores that others replace), the softmax and the product otherwise.
+int launch_softmax_spmm_mfma(int m_vec, int vec_length, int k, int n, const int *row_indices, const int *row_offsets,
+                             const int *column_indices, half_t *values, const half_t *rhs, half_t *out, float scale,
+                             hipStream_t stream, const Batch &batch)
+{
+    if (m_vec == 0 || batch.count == 0) return hipSuccess;
+    if (batch.count > 65535) return hipErrorNotSupported;
+    if (softmax_spmm_fused(vec_length, k, n, batch)) {
+        const SpmmShape shape = choose_spmm_shape(true, m_vec, vec_length, k, n, batch, true);
+        if (!shape.ragged && k <= 16 * shape.cols_per_lane) {
+            switch (vec_length) {
+            case 1: return launch_keep<1>(shape, m_vec, k, n, row_indices, row_offsets, column_indices, values, rhs, out, stream, batch, scale);
+            case 2: return launch_keep<2>(shape, m_vec, k, n, row_indices, row_offsets, column_indices, values, rhs, out, stream, batch, scale);
+            case 4: return launch_keep<4>(shape, m_vec, k, n, row_indices, row_offsets, column_indices, values, rhs, out, stream, batch, scale);
+            case 8: return launch_keep<8>(shape, m_vec, k, n, row_indices, row_offsets, column_indices, values, rhs, out, stream, batch, scale);
+            default: return hipErrorInvalidValue;
+            }
+        }
+    }
+    Batch in_place = batch;
+    in_place.stride_out = batch.stride_a;
+    const int st = launch_sparse_softmax(m_vec, vec_length, row_indices, row_offsets, values, values, scale, stream, in_place);
+    return st != hipSuccess ? st
+                            : launch_spmm_mfma<half_t>(m_vec, vec_length, k, n, row_indices, row_offsets, column_indices, values, rhs,
+                                                       out, stream, batch);
 }
 
 // Rows in parts (the kernel's PARTS variant): `slots` is the dispatch list of vs_spmm_row_parts in device memory,

@@ -251,6 +251,7 @@ struct Options {
     int sddmm_group = 0;        // MFMA SDDMM: 16-vector groups per wave step (1, 2, 4), 0 = automatic
     int sddmm_tile = 0;         // SDDMM on dense tiles: 1 = never, 2 = 64 x 64 tiles, 3 = 128 x 128 tiles, 0 = automatic
     int sddmm_flat_supers = 0;  // flat MFMA SDDMM (algorithm 2): super-groups per wave, 0 = automatic
+    int softmax_spmm = 0;       // softmax and SpMM that keeps the probabilities: 1 = one launch, 2 = two, 0 = automatic
     int spmm_tile = 0;          // SpMM on dense tiles: 1 = never, 2 / 3 / 4 = tiles of 32 x 64, 64 x 128, 128 x 128, 0 = automatic
     int attention_waves = 0;
     int attention_chunk = 0;
@@ -304,7 +305,7 @@ struct SpmmShape {
     bool ragged = false;       // dense width not a multiple of 4: the variant without alignment
     bool dma = false;          // the variant that gathers through LDS-DMA loads (option spmm_gather = 2)
 };
-SpmmShape choose_spmm_shape(bool softmax, int m_vec, int vec_length, int k, int n, const Batch &batch);
+SpmmShape choose_spmm_shape(bool softmax, int m_vec, int vec_length, int k, int n, const Batch &batch, bool keep = false);
 
 // Launchers (one per kernel family); return a hipError_t-valued int.
 template <typename OutT>
@@ -411,6 +412,9 @@ int launch_spmm_softmax_mfma(int m_vec, int vec_length, int k, int n, const int 
                              const int *row_offsets, const int *column_indices, const half_t *scores,
                              const half_t *rhs, half_t *out, float scale, hipStream_t stream,
                              const Batch &batch = Batch());
+int launch_softmax_spmm_mfma(int m_vec, int vec_length, int k, int n, const int *row_indices, const int *row_offsets,
+                             const int *column_indices, half_t *values, const half_t *rhs, half_t *out, float scale,
+                             hipStream_t stream, const Batch &batch);
 int launch_sparse_attention(int m_vec, int vec_length, int d_qk, int d_v, const int *row_indices,
                             const int *row_offsets, const int *col_indices, const half_t *q, const half_t *k,
                             const half_t *v, half_t *out, float scale, hipStream_t stream, const Batch &batch,

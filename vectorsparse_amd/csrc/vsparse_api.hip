@@ -529,6 +529,23 @@ int vs_wmma_spmm_softmax_f16_batched(int batch, int m_vec, int vec_length, int k
                                         make_batch(batch, stride_scores, stride_rhs, stride_output, nonzeros_vec, longest_row_vec));
 }
 
+int vs_wmma_softmax_spmm_f16_batched(int batch, int m_vec, int vec_length, int k, int n, int nonzeros_vec, int longest_row_vec,
+                                     const int *row_indices, const int *row_offsets, const int *column_indices,
+                                     void *values, long long stride_values, const void *rhs_matrix, long long stride_rhs,
+                                     void *output_matrix, long long stride_output, float scale, void *stream)
+{
+    if (batch < 0) return VS_ERROR_INVALID_VALUE;
+    int st = check_spmm(m_vec, vec_length, k, n, row_indices, row_offsets, column_indices, values, rhs_matrix,
+                        output_matrix, sizeof(half_t));
+    if (st != VS_SUCCESS) return st;
+    if (!stride_ok(stride_values, vec_length) || !stride_ok(stride_rhs, 8) || !stride_ok(stride_output, 8))
+        return VS_ERROR_INVALID_VALUE;
+    return vs::launch_softmax_spmm_mfma(m_vec, vec_length, k, n, row_indices, row_offsets, column_indices,
+                                        static_cast<half_t *>(values), static_cast<const half_t *>(rhs_matrix),
+                                        static_cast<half_t *>(output_matrix), scale, static_cast<hipStream_t>(stream),
+                                        make_batch(batch, stride_values, stride_rhs, stride_output, nonzeros_vec, longest_row_vec));
+}
+
 int vs_sparse_attention_f16(int batch, int m_vec, int vec_length, int n, int d_qk, int d_v, const int *row_indices,
                             const int *row_offsets, const int *col_indices, const void *q, long long stride_q,
                             const void *k, long long stride_k, const void *v, long long stride_v, void *out,
@@ -874,6 +891,9 @@ static int set_option_field(vs::Options &o, const char *name, int value)
     } else if (std::strcmp(name, "sddmm_tile") == 0) {
         if (value > 3) return VS_ERROR_INVALID_VALUE;
         o.sddmm_tile = value;
+    } else if (std::strcmp(name, "softmax_spmm") == 0) {
+        if (value < 0 || value > 2) return VS_ERROR_INVALID_VALUE;
+        o.softmax_spmm = value;
     } else if (std::strcmp(name, "spmm_tile") == 0) {
         if (value > 4) return VS_ERROR_INVALID_VALUE;
         o.spmm_tile = value;

@@ -297,6 +297,27 @@ def spmm_softmax_batched(m_vec, vec_length, k, n, row_indices, row_offsets, colu
     return output_matrix
 
 
+def softmax_spmm_batched(m_vec, vec_length, k, n, row_indices, row_offsets, column_indices, values, rhs_matrix,
+                         output_matrix, scale=1.0, stream=None, nonzeros_vec=-1, longest_row_vec=-1):
+    """values[b] = softmax_row(scale * values[b]) in place, then out[b] = values[b] @ rhs_matrix[b]."""
+    if output_matrix.dim() == 2:
+        output_matrix = output_matrix.unsqueeze(0)
+    batch = output_matrix.shape[0]
+    st = _native.softmax_spmm_batched(batch, m_vec, vec_length, k, n, nonzeros_vec, longest_row_vec, row_indices, row_offsets,
+                                      column_indices, values, rhs_matrix, output_matrix, float(scale), stream)
+    if st >= 0:
+        _lib.check(st, "vs_wmma_softmax_spmm_f16_batched")
+        return output_matrix
+    for t, nm in ((values, "values"), (rhs_matrix, "rhs_matrix"), (output_matrix, "output_matrix")):
+        _expect_batched(t, torch.float16, nm)
+    st = _lib.lib().vs_wmma_softmax_spmm_f16_batched(
+        batch, m_vec, vec_length, k, n, int(nonzeros_vec), int(longest_row_vec), _ptr(row_indices), _ptr(row_offsets),
+        _ptr(column_indices), _ptr(values), _stride(values, batch), _ptr(rhs_matrix), _stride(rhs_matrix, batch),
+        _ptr(output_matrix), _stride(output_matrix, batch), float(scale), _stream(stream))
+    _lib.check(st, "vs_wmma_softmax_spmm_f16_batched")
+    return output_matrix
+
+
 def sparse_attention(m_vec, vec_length, n, row_indices, row_offsets, col_indices, q, k, v, out=None, scale=None,
                      stream=None, rows_per_workgroup=0, plan=None):
     """Single-launch fixed-mask attention: out = softmax(scale * mask(q k^T)) v.
@@ -686,7 +707,8 @@ class SparseAttention:
         (rows that attend to everything) streamed by several workgroups; "parts" runs the three operators on the dispatch list of row parts (masks with rows far longer than
         the rest, e.g. global tokens); "layer" runs the whole layer in one launch with scores and probabilities kept in LDS; True
         folds only the softmax into the SpMM launch (two launches, raw scores go through memory); False runs
-        the three operators one after the other.  Default on the MFMA path: "layer" when the cost model of
+        the three operators one after the other and leaves the probabilities in `scores` (on the MFMA path softmax and SpMM share
+        a launch where that is faster).  Default on the MFMA path: "layer" when the cost model of
         `_union_rows` puts the streamed union kernel ahead (banded, blocky, strided and very sparse masks: 1.5-15x
         faster than the alternatives), else True - on masks without shared columns the single launch gathers
         K / V rows per row and is 10-60 % slower than the two launches (16 heads x 4096, uniform random masks,
@@ -717,6 +739,10 @@ class SparseAttention:
                       p.vec_length, kernel=kernel, stream=stream, columns_sorted=p.columns_sorted)
         if fused:
             return spmm_softmax_batched(p.m_vec, p.vec_length, d_v, p.n, p.row_indices, p.row_offsets,
+                                        p.column_indices, scores, v, out, scale, stream=stream,
+                                        nonzeros_vec=p.nnz_vec, longest_row_vec=p.longest_row_vec)
+        if kernel == "wmma":
+            return softmax_spmm_batched(p.m_vec, p.vec_length, d_v, p.n, p.row_indices, p.row_offsets,
                                         p.column_indices, scores, v, out, scale, stream=stream,
                                         nonzeros_vec=p.nnz_vec, longest_row_vec=p.longest_row_vec)
         sparse_softmax(p.m_vec, p.vec_length, p.row_indices, p.row_offsets, scores, scores, scale, stream=stream)
