@@ -134,3 +134,49 @@ def test_the_automatic_route_and_its_replays(gpu):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, tiles["wmma"])
+
+
+def _ascending_but_for(V, n, rows, row, at, kind, tight, rng):
+    """Rows of ascending columns (next to each other, or anywhere) with the given numbers of nonzeros, but for one pair:
+    nonzero `at` of row `row` repeats its predecessor's column, or lies in front of all of the row's others."""
+    cols = []
+    for i, length in enumerate(rows):
+        c = np.arange(4, 4 + length) if tight else np.sort(rng.choice(np.arange(4, n), length, replace=False))
+        if i == row:
+            c[at] = c[at - 1] if kind == "repeated" else 1
+        cols.append(c)
+    ro = np.concatenate([[0], np.cumsum(rows)]).astype(np.int32)
+    return cv.random_values(cv.ColVecCSR(len(rows), n, V, ro, np.concatenate(cols).astype(np.int32)), 5)
+
+
+@pytest.mark.parametrize("tile", [2, 3, 4])
+@pytest.mark.parametrize("V", [1, 2, 4, 8])
+def test_a_single_pair_out_of_order_is_noticed(gpu, V, tile):
+    """One repeated or misplaced column in a pattern that ascends otherwise, at the edges of what a lane fetches, of windows
+    and of the pattern's end: nothing else makes a workgroup go nonzero by nonzero."""
+    threads, tile_rows, each = 256, 32 << (tile - 2), {2: (8, 8, 4, 4), 3: (8, 8, 4, 4), 4: (8, 4, 4, 2)}[tile][V.bit_length() - 1]
+    window = min(64, threads * V // tile_rows) * each
+    rng = np.random.default_rng(10 * V + tile)
+    n, N, missed = 1700, 32, []
+    B = cv.dense_uniform(n, N, seed=6)
+    rhs, exact = torch.from_numpy(B).cuda(), B.astype(np.float64)
+    lengths = sorted({*range(2, 2 * each + 2), window - 1, window, window + 1, window + each + 1, 2 * window, 2 * window + 1, 3 * window + 2})
+    for length in lengths:
+        places = {1, length // 2, length - 1, length - 2, (length - 1) // each * each, window, 2 * window}
+        for at in sorted(p for p in places if 0 < p < length):
+            # the last row, or a row of one nonzero behind it
+            for kind, tight, behind in ((k, t, b) for k in ("repeated", "misplaced") for t in (True, False) for b in ((), (1,))):
+                rows = (3, length) + behind
+                pat = _ascending_but_for(V, n, rows, 1, at, kind, tight, rng)
+                prob = ops.DeviceProblem(pat)
+                assert not prob.columns_distinct
+                with _lib.thread_options(spmm_tile=tile):
+                    got = prob.spmm(rhs).double().cpu().numpy()
+                ro, ci = pat.row_offsets, pat.column_indices
+                values = pat.values.astype(np.float64)
+                want = np.concatenate([values[ro[i]:ro[i + 1]].T @ exact[ci[ro[i]:ro[i + 1]]] for i in range(pat.m_vec)])
+                size = np.concatenate([np.abs(values[ro[i]:ro[i + 1]].T) @ np.abs(exact[ci[ro[i]:ro[i + 1]]]) for i in range(pat.m_vec)])
+                # products of halves are exact in fp32; each of their sums and the result's rounding are not
+                if not (np.abs(got - want) <= length * 2.0 ** -23 * size + 2.0 ** -11 * np.abs(want) + 2.0 ** -24).all():
+                    missed.append((rows, at, kind, tight))
+    assert not missed, (len(missed), missed[:8])

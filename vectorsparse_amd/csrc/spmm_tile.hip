@@ -154,12 +154,19 @@ spmm_tile_kernel(int m_vec, int N, int n, int column_tiles, const int *__restric
         int taken = 0, previous = __builtin_amdgcn_update_dpp(-1, w.col[EACH - 1], 0x138, 0xF, 0xF, false);  // wave_shr:1
         previous = li == 0 ? before : previous;
         if (__builtin_amdgcn_ballot_w64(first > 0 || last < EACH) != 0) {
-            // entries ahead of the lane's own (near the pattern's end) pass as very small ones and are not counted
+            // entries ahead of the lane's own (a run moved back from the pattern's end) pass as very small ones and are not
+            // counted; the first of its own still follows what its predecessor says
+            if (__builtin_amdgcn_ballot_w64(first > 0) != 0) {
+                int own = 0x7fffffff;
+#pragma unroll
+                for (int e = 1; e < EACH; ++e) own = e == first && e < last ? w.col[e] : own;
+                disorder |= __builtin_amdgcn_ballot_w64(own < k0 + KC) & __builtin_amdgcn_ballot_w64(previous >= own);
+                if (first > 0) previous = (int)0x80000000;
+            }
 #pragma unroll
             for (int e = 0; e < EACH; ++e) w.col[e] = e >= last ? 0x7fffffff : (e < first ? (int)0x80000001 + e : w.col[e]);
             taken = first < last ? first : last;
             taken = taken < 0 ? 0 : (taken > EACH ? -EACH : -taken);
-            if (first > 0) previous = (int)0x80000000;
         }
 #pragma unroll
         for (int e = 0; e < EACH; ++e) {
@@ -167,7 +174,7 @@ spmm_tile_kernel(int m_vec, int N, int n, int column_tiles, const int *__restric
             disorder |= passed & __builtin_amdgcn_ballot_w64(previous >= w.col[e]);
             previous = w.col[e];
             taken += w.col[e] < k0 + KC ? 1 : 0;
-            const unsigned rel = (unsigned)(w.col[e] - k0), place = __umul24(rel, (unsigned)PITCH) + place_row;
+            const unsigned rel = (unsigned)w.col[e] - (unsigned)k0, place = __umul24(rel, (unsigned)PITCH) + place_row;
             w.val[e].store(reinterpret_cast<half_t *>(area + (rel < (unsigned)KC ? place : dump)));
         }
         taken = row_sum<LPR>(taken);
