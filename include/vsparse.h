@@ -518,7 +518,8 @@ int vs_sparse_attention_plan(int m_vec, int vec_length, int n, int d_qk, int d_v
  * vs_sparse_attention_f16 with workgroups of 128 scalar rows (a row block) for masks in which a few row blocks have far more
  * distinct columns than the rest (tokens that attend to everything): such a block is streamed by several workgroups, each
  * taking a range of its sub-rounds of 128 distinct columns, and a second launch adds their partial results up.  A plan of its own (up to
- * 4096 distinct columns per block; blocks with more take the per-row path) and a list of slots in device memory, 16-byte
+ * 4096 distinct columns, 32 sub-rounds, per block; a block with more takes the per-row path, all of it in its slot with first
+ * sub-round 0, and needs no other) and a list of slots in device memory, 16-byte
  * aligned: n_slots entries {row block, first sub-round, end of the sub-rounds, partial tile or -1}, then n_merges entries
  * {row block, first partial tile, number of tiles, 0}.  Every block appears in one slot with first sub-round 0 and tile -1,
  * or in several that share its sub-rounds (the last one's end may be any large number) with consecutive tiles and a merge

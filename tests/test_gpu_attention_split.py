@@ -111,3 +111,47 @@ def test_refused_arguments(gpu):
             ops.sparse_attention_split(layer.prob, slots, device_slots, bad_plan, q, k, v, out, 0.125, workspace)
     with pytest.raises(TypeError):
         ops.sparse_attention_split(layer.prob, slots, device_slots, plan, q.float(), k, v, out, 0.125)
+
+
+def _layer_in_float64(mask, q, k, v, scale):
+    """Softmax attention over each row's own columns alone (a repeated column counts as often as it is listed)."""
+    out = np.zeros((q.shape[0], mask.m, v.shape[2]))
+    q, k, v = (x.double().cpu().numpy() for x in (q, k, v))
+    V, ro = mask.vec_length, mask.row_offsets
+    with np.errstate(invalid="ignore"):
+        for h in range(q.shape[0]):
+            for i in range(mask.m_vec):
+                cols = mask.column_indices[ro[i]:ro[i + 1]]
+                if len(cols):
+                    s = (q[h, i * V:(i + 1) * V] @ k[h, cols].T) * scale
+                    p = np.exp(s - s.max(axis=1, keepdims=True))
+                    out[h, i * V:(i + 1) * V] = (p / p.sum(axis=1, keepdims=True)) @ v[h, cols]
+    return out
+
+
+def test_slots_that_start_behind_the_plan_are_left_to_the_first_one(gpu):
+    """Parts of a block of more columns than a plan lists, as a caller of the C entry point may dispatch them: the first takes
+    the per-row path for all of the block, the others read nothing behind its record.  Blocks of 8192 columns, parts that
+    start at sub-rounds 0, 4 .. 60; the last block is among them."""
+    V, seq, d = 8, 8192, 32
+    rows = [np.arange(max(0, i * V - 20), min(seq, i * V + 28)) for i in range(seq // V)]
+    rows[3] = rows[-2] = np.arange(seq)
+    mask = cv.ColVecCSR(seq // V, seq, V, np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32),
+                        np.concatenate(rows).astype(np.int32))
+    layer = ops.SparseAttention(mask)
+    q, k, v = _operands(1, seq, d, d)
+    unions = layer._block_unions()
+    assert unions[0] == unions[-1] == seq and sorted(unions)[-3] < 512
+    listed = ops.AttentionSlots(unions, 4)
+    assert listed.n_partials == listed.n_merges == 0
+    cut = ops.AttentionSlots(unions, 4)
+    cut.slots = np.array([(block, start, start + 4, i * 16 + start // 4) for i, block in enumerate((0, len(unions) - 1)) for start in range(0, 64, 4)]
+                         + [slot for slot in listed.slots.tolist() if slot[0] not in (0, len(unions) - 1)]
+                         + [(0, 0, 16, 0), (len(unions) - 1, 16, 16, 0)], dtype=np.int32)
+    cut.n_slots, cut.n_merges, cut.n_partials = len(cut.slots) - 2, 2, 32
+    plan = layer._split(d, d, 4)[2]
+    ref = _layer_in_float64(mask, q, k, v, d ** -0.5)
+    for slots in (listed, cut):
+        out = torch.full_like(q, 7.0)
+        ops.sparse_attention_split(layer.prob, slots, torch.from_numpy(slots.slots).cuda(), plan, q, k, v, out, d ** -0.5)
+        _check_layer(out.double().cpu().numpy(), ref, "%d partial tiles" % slots.n_partials)

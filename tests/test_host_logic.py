@@ -388,3 +388,29 @@ def test_waves_of_short_rows_of_unknown_length(n, waves):
     where there are two steps of 32 (a wave per 128 columns: up to 20 % slower on rows that hold half of n)."""
     for V in (1, 2, 4, 8):
         assert ops.spmm_launch_shape(64 // V, V, 205, n)["waves"] == waves
+
+
+def test_attention_slots_stay_within_the_plan_and_cover_every_block():
+    rng = np.random.default_rng(4)
+    unions = [0, 1, 128, 129, 4095, 4096, 4097, 8192, 65536] + rng.integers(0, 9000, 40).tolist()
+    for rounds in (1, 2, 3, 4, 7, 8, 16, 31, 32, 100):
+        s = ops.AttentionSlots(unions, rounds)
+        assert s.slots.shape == (s.n_slots + s.n_merges, 4) and s.slots.dtype == np.int32
+        slots, merges = s.slots[:s.n_slots].tolist(), s.slots[s.n_slots:].tolist()
+        assert max(first for _, first, _, _ in slots) < 32      # (a plan's record lists no more sub-rounds)
+        tiles = [tile for *_, tile in slots if tile >= 0]
+        assert sorted(tiles) == list(range(s.n_partials))
+        merged = {block: (first, count) for block, first, count, _ in merges}
+        assert len(merged) == s.n_merges and sum(count for _, count in merged.values()) == s.n_partials
+        for block, size in enumerate(unions):
+            needed = -(-size // 128)
+            mine = sorted(slot[1:] for slot in slots if slot[0] == block)
+            if needed <= rounds or needed > 32:
+                assert len(mine) == 1 and mine[0][0] == 0 and mine[0][1] >= needed and mine[0][2] == -1 and block not in merged
+                continue
+            first, count = merged[block]
+            assert [tile for _, _, tile in mine] == list(range(first, first + count))
+            assert mine[0][0] == 0 and mine[-1][1] >= needed
+            for (a0, a1, _), (b0, _, _) in zip(mine, mine[1:]):
+                assert a1 == b0 and 0 < a1 - a0 <= rounds
+            assert 0 < needed - mine[-1][0] <= rounds

@@ -857,7 +857,7 @@ sparse_attention_stream_kernel(int m_vec, int n, int d_qk, int d_v,
     // The record, the K rows and the V rows are read through buffer descriptors: a scalar base and one 32-bit byte
     // offset per thread and load, where a 64-bit pointer per thread and load used to take the registers that the
     // launch bounds do not leave (n <= 2^20 columns of at most 128 halves: every offset is below 2^28).
-    const __amdgpu_buffer_rsrc_t rec_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<int *>(rec), 0, 0x7fffffff, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rec_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<int *>(rec), 0, 4 * stride, 0x00020000);
     const __amdgpu_buffer_rsrc_t k_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t *>(k), 0, 0x7fffffff, 0x00020000);
     const __amdgpu_buffer_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t *>(v), 0, 0x7fffffff, 0x00020000);
     constexpr unsigned kMasksAt = 4u * 4u;                                        // byte offsets inside the record
@@ -938,7 +938,9 @@ sparse_attention_stream_kernel(int m_vec, int n, int d_qk, int d_v,
         if (tid < kRows * SS) maskbuf[tid] = stage_m;
     };
 
-    fetch_cols(first_round);  // requested together with the union's size
+    // requested together with the union's size (a record ends with sub-round kRounds - 1; slots that start behind it belong to
+    // blocks that take the per-row path)
+    fetch_cols((unsigned)first_round < (unsigned)kRounds ? first_round : 0);
     if (n_union > u_cap || d_v % 8 != 0) {
         if (first_round > 0) return;   // (the block's first slot takes all of it)
         per_row_block_call<V, KS, CPL>(row_first, row_last, wave, 8, row_offsets, col_indices, q, k, v, out, d_qk, d_v,

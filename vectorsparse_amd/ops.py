@@ -449,14 +449,17 @@ def distinct_columns(mask, rows):
 
 class AttentionSlots:
     """The slots of `vs_sparse_attention_f16_split` for a mask, given the distinct columns of its blocks of 128 scalar rows:
-    blocks of more than `rounds` sub-rounds of 128 columns are cut into that many each.  Host array `slots`
+    blocks of more than `rounds` sub-rounds of 128 columns are cut into that many each, but for those of more than a plan
+    lists (PLAN_ROUNDS), which take the per-row path whole.  Host array `slots`
     (int32 [n_slots + n_merges][4], longest first), and the counts the entry point takes."""
+
+    PLAN_ROUNDS = 32    # sub-rounds of a block that a plan of `sparse_attention_split_plan` lists
 
     def __init__(self, unions, rounds):
         whole, parts, merges = [], [], []
         for block, size in enumerate(unions):
             needed = -(-size // 128)
-            if needed <= rounds:
+            if needed <= rounds or needed > self.PLAN_ROUNDS:
                 whole.append((needed, (block, 0, 1 << 20, -1)))
                 continue
             count = -(-needed // rounds)
@@ -603,7 +606,7 @@ class SparseAttention:
             return None
         unions = self._block_unions()
         longest = -(-max(unions) // 128)
-        if longest > 32 or longest < 2:     # (a split plan holds 4096 columns of a block)
+        if longest > AttentionSlots.PLAN_ROUNDS or longest < 2:
             return None
         c = 0 if max(d, d_v) <= 32 else (1 if max(d, d_v) <= 64 else 2)
         if route == "parts":
