@@ -488,7 +488,9 @@ int vs_wmma_softmax_spmm_f16_batched(int batch, int m_vec, int vec_length, int k
  * With a plan, workgroups of eight waves (rows_per_workgroup >= 128 / vec_length) stream their union
  * through LDS 128 columns at a time with the next columns' K / V rows already on their way, keeping the
  * running maximum and sums of flash attention: the fastest path, and one that takes unions of up to 2048
- * columns.  plan_bytes is the size of the plan buffer: it must be at least
+ * columns.  Infinities and NaNs of k and v reach the rows that attend to them and no others; only without
+ * such a plan, with rows_per_workgroup >= 2, may they also reach rows of the same 16 (a masked-out pair is
+ * multiplied by zero there).  plan_bytes is the size of the plan buffer: it must be at least
  * vs_sparse_attention_plan_bytes() for THIS shape (else 1, hipErrorInvalidValue, and no launch), so that the
  * kernels never read past it whatever it holds.  A plan made for another shape is detected and ignored
  * (every workgroup then takes the per-row path: correct, slower).
@@ -523,7 +525,8 @@ int vs_sparse_attention_plan(int m_vec, int vec_length, int n, int d_qk, int d_v
  * aligned: n_slots entries {row block, first sub-round, end of the sub-rounds, partial tile or -1}, then n_merges entries
  * {row block, first partial tile, number of tiles, 0}.  Every block appears in one slot with first sub-round 0 and tile -1,
  * or in several that share its sub-rounds (the last one's end may be any large number) with consecutive tiles and a merge
- * entry.  workspace: 128 * (d_v + 2) floats per partial tile and head, uninitialised.  No counterpart in the reference.
+ * entry.  workspace: 128 * (d_v + 2) floats per partial tile and head, uninitialised.  Infinities and NaNs of k and v reach the
+ * rows that attend to them and no others.  No counterpart in the reference.
  */
 long long vs_sparse_attention_split_plan_bytes(int m_vec, int vec_length, int n, int d_qk, int d_v);
 int vs_sparse_attention_split_plan(int m_vec, int vec_length, int n, int d_qk, int d_v,

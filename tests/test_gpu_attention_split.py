@@ -155,3 +155,45 @@ def test_slots_that_start_behind_the_plan_are_left_to_the_first_one(gpu):
         out = torch.full_like(q, 7.0)
         ops.sparse_attention_split(layer.prob, slots, torch.from_numpy(slots.slots).cuda(), plan, q, k, v, out, d ** -0.5)
         _check_layer(out.double().cpu().numpy(), ref, "%d partial tiles" % slots.n_partials)
+
+
+@pytest.mark.parametrize("V", [1, 2, 4, 8])
+@pytest.mark.parametrize("route,d,d_v,scale", [
+    (("split", 1), 64, 64, None), (("split", 2), 32, 24, -0.2), (("split", 32), 64, 64, None), (("split", 1), 128, 64, 0.0),
+    (("split", 2), 64, 128, None), ("layer", 64, 64, None), ("layer", 128, 128, -0.2), (None, 64, 64, None)])
+def test_infinities_and_nans_reach_the_rows_that_attend_to_them_alone(gpu, route, d, d_v, scale, V):
+    seq, heads, tokens = 776, 2, 24
+    mask = _mask("global", seq, V, tokens=tokens)
+    start = (seq // 2 - 8) // V * V     # (the tokens, see _mask)
+    lonely, ro, ci = 40 // V, mask.row_offsets, mask.column_indices
+    cols = [ci[ro[i]:ro[i + 1]] for i in range(mask.m_vec)]
+    cols[lonely] = np.array([300], dtype=np.int32)      # a row whose only score is -infinity below
+    mask = cv.ColVecCSR(mask.m_vec, seq, V, np.concatenate([[0], np.cumsum([len(c) for c in cols])]).astype(np.int32), np.concatenate(cols))
+    q, k, v = _operands(heads, seq, d, d_v)
+    q[:, :, 0] = q[:, :, 0].abs() + 0.1
+    sign = -1.0 if scale is not None and scale < 0 else 1.0
+    k[0, 100, 0] = sign * np.inf
+    k[0, 150, 1] = -np.inf
+    k[0, 200, 2] = np.nan
+    k[0, 300] = 0.0
+    k[0, 300, 0] = -sign * np.inf
+    v[0, 500, 3] = np.inf
+    v[0, 600, d_v - 1] = np.nan
+    v[1, 640, 0] = -np.inf
+    touched = [100, 150, 200, 300, 500, 600, 640]
+    assert not set(touched) & set(range(start, start + tokens))     # (else every row attends to them)
+    if route == "layer":
+        layer = ops.SparseAttention(mask)
+        out = torch.empty((heads, seq, d_v), dtype=torch.float16, device="cuda")
+        plan = ops.sparse_attention_plan(mask.m_vec, V, seq, d, d_v, 128 // V, layer.prob.row_offsets, layer.prob.column_indices)
+        ops.sparse_attention(mask.m_vec, V, seq, layer.prob.row_indices, layer.prob.row_offsets, layer.prob.column_indices, q, k, v,
+                             out=out, scale=scale, rows_per_workgroup=128 // V, plan=plan)
+    else:
+        out = ops.SparseAttention(mask).forward(q, k, v, scale=scale, fused=route)
+    got = out.double().cpu().numpy()
+    ref = _layer_in_float64(mask, q, k, v, d ** -0.5 if scale is None else scale)
+    finite = np.isfinite(ref)
+    assert np.isnan(ref[0, lonely * V:(lonely + 1) * V]).all() and 0.3 < finite.mean() < 1.0
+    # (a probability that rounds to zero in fp16 makes a NaN of an infinite product, in every route)
+    assert np.array_equal(np.isfinite(got), finite)
+    _check_layer(np.where(finite, got, 0.0), np.where(finite, ref, 0.0), "non-finite K and V, V%d %s" % (V, route))

@@ -173,17 +173,17 @@ __device__ __forceinline__ void accumulate_chunk(float4_t (&acc)[CPL], const hal
     }
 }
 
-// Divide the accumulated tile of a vector row by its softmax sums and store it.
+// Divide the accumulated tile of a vector row by its softmax sums and store its scalar rows [from, to).
 template <int V, int CPL>
 __device__ __forceinline__ void store_row(half_t *out, int row, int d_v, const float4_t (&acc)[CPL], float l_sum,
-                                          bool empty, int c, int g)
+                                          bool empty, int c, int g, int from, int to)
 {
     const int col0 = c * CPL;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         const int vv = 4 * g + e;
         const float le = from_lane(l_sum, vv & 15);  // the sum of scalar row vv lives in the lanes with c = vv
-        if (vv < V && col0 < d_v) {
+        if (vv >= from && vv < to && col0 < d_v) {
             const float norm = empty ? 0.f : 1.f / le;  // an empty row attends to nothing: zeros
             float tmp[CPL];
 #pragma unroll
@@ -257,13 +257,13 @@ __device__ __forceinline__ void scores_step(float4_t (&sacc)[2], const half8_t (
 
 // The per-row path for the vector rows [row_first, row_last) of a workgroup: one vector row per wave at a time
 // with the K / V rows read from global memory by column; no barrier, long rows in chunks with a running
-// maximum and sum.
+// maximum and sum.  Of each vector row the scalar rows [from, to) are stored.
 template <int V, int KS, int CPL>
 __device__ __forceinline__ void per_row_block(int row_first, int row_last, int wave, int n_waves,
                                               const int *__restrict__ row_offsets, const int *__restrict__ col_indices,
                                               const half_t *__restrict__ q, const half_t *__restrict__ k,
                                               const half_t *__restrict__ v, half_t *__restrict__ out, int d_qk, int d_v,
-                                              float s2, int c, int g, int col_off)
+                                              float s2, int c, int g, int col_off, int from = 0, int to = V)
 {
     const RowSource ksrc = {k, d_qk, col_indices};
     const RowSource vsrc = {v, d_v, col_indices};
@@ -292,7 +292,7 @@ __device__ __forceinline__ void per_row_block(int row_first, int row_last, int w
             }
             accumulate_chunk<CPL>(acc, p, vsrc, c0, cend, col_off, g);
         }
-        store_row<V, CPL>(out, row, d_v, acc, l_run, end == beg, c, g);
+        store_row<V, CPL>(out, row, d_v, acc, l_run, end == beg, c, g, from, to);
     }
 }
 
@@ -784,10 +784,10 @@ __device__ __noinline__ void per_row_block_call(int row_first, int row_last, int
                                                 const int *__restrict__ row_offsets, const int *__restrict__ col_indices,
                                                 const half_t *__restrict__ q, const half_t *__restrict__ k,
                                                 const half_t *__restrict__ v, half_t *__restrict__ out, int d_qk,
-                                                int d_v, float s2, int c, int g, int col_off)
+                                                int d_v, float s2, int c, int g, int col_off, int from = 0, int to = V)
 {
     per_row_block<V, KS, CPL>(row_first, row_last, wave, n_waves, row_offsets, col_indices, q, k, v, out, d_qk, d_v, s2,
-                              c, g, col_off);
+                              c, g, col_off, from, to);
 }
 
 //
@@ -1083,41 +1083,81 @@ sparse_attention_stream_kernel(int m_vec, int n, int d_qk, int d_v,
             return;
         }
     }
+    // (the lane's place, made anew: kept across the loop it is what the register allocator parks in scratch memory)
+    int again = tid;
+    asm volatile("" : "+v"(again));
+    const int c_out = again & 15, g_out = (again & 63) >> 4, col_out = c_out * CPL;
+    // A masked-out pair is multiplied like any other: its score starts at -infinity and its probability is zero, and both
+    // make a NaN with an infinity or a NaN of K or V.  A wave that meets one, or a row whose every score is -infinity (its
+    // sum stays zero, its softmax is a NaN), does its rows again with the columns of each row alone.  (Every branch up to the
+    // stores is the whole wave's, and nothing is kept across the call: no register is saved under a part of the lanes.)
+    float total[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-        const long long row = q_global + 4 * g + e;
-        if (row < q_limit && col_ok) {
-            const float norm = lacc[e] > 0.f ? 1.f / lacc[e] : 0.f;  // a row with no column attends to nothing: zeros
-            float tmp[CPL];
+        total[e] = acc[0][e];
 #pragma unroll
-            for (int cc = 0; cc < CPL; ++cc) tmp[cc] = acc[cc][e] * norm;
-            store_converted<half_t, CPL>(out + (size_t)row * d_v + col0, tmp);
+        for (int cc = 1; cc < CPL; ++cc) total[e] += acc[cc][e];
+    }
+    const float whole = (total[0] + total[1]) + (total[2] + total[3]);
+    const float least = fminf(fminf(lacc[0], lacc[1]), fminf(lacc[2], lacc[3]));
+    bool strange = whole != whole;
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(least > 0.f)) != 0ull, 0)) {
+        // (rows without a column, and places past the last row, have no sum either; bit i: scalar row i of the wave has one)
+        const int row = row_first + (q_first + c_out) / V, there = row < row_last ? row : row_last - 1;
+        const unsigned held = (unsigned)__builtin_amdgcn_ballot_w64((row_offsets[there + 1] > row_offsets[there]) & (row < row_last));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) strange |= (bool)((held >> (4 * g_out + e)) & 1u) & !(lacc[e] > 0.f);
+    }
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(strange) != 0ull, 0)) {
+        const int first = row_first + wave * RPW, last = first + RPW < row_last ? first + RPW : row_last;
+        per_row_block_call<V, KS, CPL>(first, last, 0, 1, row_offsets, col_indices, q, k, v, out, d_qk, d_v, scale * kLog2e,
+                                       c_out, g_out, col_out < d_v ? col_out : 0);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const long long row = q_global + 4 * g_out + e;
+            if (row < q_limit && col_out < d_v) {
+                const float norm = lacc[e] > 0.f ? 1.f / lacc[e] : 0.f;  // a row with no column attends to nothing: zeros
+                float tmp[CPL];
+#pragma unroll
+                for (int cc = 0; cc < CPL; ++cc) tmp[cc] = acc[cc][e] * norm;
+                store_converted<half_t, CPL>(out + (size_t)row * d_v + col_out, tmp);
+            }
         }
     }
 }
 
-// Adds up the partial tiles of a split row block: merge entry {row block, first partial tile, tiles, -}.  A few hundred KB per
-// head at most, read once: bound by the launch and one round trip (3 us).
-__global__ void __launch_bounds__(512)
-sparse_attention_merge_kernel(int m_vec, int vec_length, int n, int d_v, const int *__restrict__ plan,
+// Adds up the partial tiles of a split row block: merge entry {row block, first partial tile, tiles, -}; a wave takes four scalar
+// rows, a workgroup a quarter of a block.  A few hundred KB per head at most, read once: bound by the launch and one round trip
+// (3 us).  Sums that are NaNs, or of rows whose every score is -infinity, send the wave's rows to the per-row path, as in the
+// streamed kernel.
+template <int V, int KS, int CPL>
+__global__ void __launch_bounds__(512, union_wide(KS, CPL) ? 2 : 4)
+sparse_attention_merge_kernel(int m_vec, int n, int d_qk, int d_v, const int *__restrict__ row_offsets,
+                              const int *__restrict__ col_indices, const int *__restrict__ plan,
                               const int *__restrict__ merges, int n_partials, const float *__restrict__ partials,
-                              half_t *__restrict__ out, long long stride_out, float scale)
+                              const half_t *__restrict__ q, const half_t *__restrict__ k, const half_t *__restrict__ v,
+                              half_t *__restrict__ out, long long stride_q, long long stride_k, long long stride_v,
+                              long long stride_out, float scale)
 {
+    constexpr int kRows = 128 / V, kMaskWords = (kRows * kStreamSteps + 3) & ~3;
+    constexpr int stride = 4 + kSplitRounds * (kMaskWords + kStreamRanks);
+    constexpr int kShare = 4;   // scalar rows of a wave
     const int4_t merge = reinterpret_cast<const int4_t *>(merges)[blockIdx.x];
-    const int rows = 128 / vec_length, mask_words = (rows * kStreamSteps + 3) & ~3;
-    const int stride = 4 + kSplitRounds * (mask_words + kStreamRanks);
     // (a block that the stream kernel has left to the per-row path is finished)
-    if (!stream_plan_fits(plan, m_vec, vec_length, n, rows, kSplitRounds, stride)) return;
+    if (!stream_plan_fits(plan, m_vec, V, n, kRows, kSplitRounds, stride)) return;
     if (plan[kPlanHeader + (size_t)merge[0] * stride] > kSplitRounds * kStreamRanks || d_v % 8 != 0) return;
     const float s2a = scale == 0.f ? 1.f : __builtin_fabsf(scale * kLog2e);
     const size_t tile = (size_t)128 * (d_v + 2);
     const float *const first = partials + ((size_t)blockIdx.y * n_partials + merge[1]) * tile;
     out += blockIdx.y * stride_out;
-    const int chunks = d_v / 4;
-    for (int unit = threadIdx.x + 512 * blockIdx.z; unit < 128 * chunks; unit += 512 * gridDim.z) {
-        const int r = unit / chunks, column = unit % chunks * 4;
+    const int chunks = d_v / 4, lane = threadIdx.x & 63;
+    const int wave_row = kShare * (8 * blockIdx.z + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6));   // (of the block)
+    bool strange = false;
+    for (int unit = lane; unit < kShare * chunks; unit += 64) {
+        const int r = wave_row + unit / chunks, column = unit % chunks * 4;
         const long long row = (long long)merge[0] * 128 + r;
-        if (row >= (long long)m_vec * vec_length) continue;
+        if (row >= (long long)m_vec * V) break;
         float most = -__builtin_inff();
         for (int i = 0; i < merge[2]; ++i) most = fmaxf(most, first[i * tile + (size_t)128 * d_v + 128 + r]);
         float4_t sum = {0.f, 0.f, 0.f, 0.f};
@@ -1133,8 +1173,19 @@ sparse_attention_merge_kernel(int m_vec, int vec_length, int n, int d_v, const i
         }
         const float norm = weight > 0.f ? 1.f / weight : 0.f;
         const float tmp[4] = {sum[0] * norm, sum[1] * norm, sum[2] * norm, sum[3] * norm};
+        const float whole = (sum[0] + sum[1]) + (sum[2] + sum[3]);
+        strange |= whole != whole;
+        if (!(weight > 0.f)) strange |= row_offsets[row / V] < row_offsets[row / V + 1];
         store_converted<half_t, 4>(out + (size_t)row * d_v + column, tmp);
     }
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(strange) == 0ull, 1)) return;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (the same places are stored again)
+    // its four scalar rows: whole vector rows, or half of one (its other half is the next wave's)
+    const int row_first = merge[0] * kRows + wave_row / V, row_last = row_first + (kShare + V - 1) / V;
+    const int from = wave_row % V, to = V > kShare ? from + kShare : V, c = lane & 15;
+    per_row_block_call<V, KS, CPL>(row_first, row_last < m_vec ? row_last : m_vec, 0, 1, row_offsets, col_indices,
+                                   q + blockIdx.y * stride_q, k + blockIdx.y * stride_k, v + blockIdx.y * stride_v, out, d_qk, d_v,
+                                   scale * kLog2e, c, lane >> 4, c * CPL < d_v ? c * CPL : 0, from, to);
 }
 
 // 32-bit words of one round of row masks of a workgroup: `rows` vector rows x `steps` words, padded to 16 bytes.
@@ -1229,9 +1280,10 @@ static int launch_one(const UnionLaunch &a)
                            a.batch->stride_b, a.stride_v, a.batch->stride_out, a.scale, a.slots, a.n_partials, a.partials);
         const hipError_t st = hipGetLastError();
         if (st != hipSuccess || a.n_merges == 0) return (int)st;
-        hipLaunchKernelGGL(sparse_attention_merge_kernel, dim3((unsigned)a.n_merges, (unsigned)a.batch->count, 4), dim3(512), 0,
-                           a.stream, a.m_vec, V, a.n, a.d_v, a.plan, a.slots + 4 * (size_t)a.n_slots, a.n_partials, a.partials,
-                           a.out, a.batch->stride_out, a.scale);
+        hipLaunchKernelGGL((sparse_attention_merge_kernel<V, KS, CPL>), dim3((unsigned)a.n_merges, (unsigned)a.batch->count, 4),
+                           dim3(512), 0, a.stream, a.m_vec, a.n, a.d_qk, a.d_v, a.row_offsets, a.col_indices, a.plan,
+                           a.slots + 4 * (size_t)a.n_slots, a.n_partials, a.partials, a.q, a.k, a.v, a.out, a.batch->stride_a,
+                           a.batch->stride_b, a.stride_v, a.batch->stride_out, a.scale);
         return (int)hipGetLastError();
     }
     if (PLANNED && s.stream) {
