@@ -490,7 +490,8 @@ int vs_wmma_softmax_spmm_f16_batched(int batch, int m_vec, int vec_length, int k
  * running maximum and sums of flash attention: the fastest path, and one that takes unions of up to 2048
  * columns.  Infinities and NaNs of k and v reach the rows that attend to them and no others; only without
  * such a plan, with rows_per_workgroup >= 2, may they also reach rows of the same 16 (a masked-out pair is
- * multiplied by zero there).  plan_bytes is the size of the plan buffer: it must be at least
+ * multiplied by zero there).  A column that a row lists twice counts twice with rows_per_workgroup 0 or 1, and
+ * once in a union.  plan_bytes is the size of the plan buffer: it must be at least
  * vs_sparse_attention_plan_bytes() for THIS shape (else 1, hipErrorInvalidValue, and no launch), so that the
  * kernels never read past it whatever it holds.  A plan made for another shape is detected and ignored
  * (every workgroup then takes the per-row path: correct, slower).

@@ -197,3 +197,17 @@ def test_infinities_and_nans_reach_the_rows_that_attend_to_them_alone(gpu, route
     # (a probability that rounds to zero in fp16 makes a NaN of an infinite product, in every route)
     assert np.array_equal(np.isfinite(got), finite)
     _check_layer(np.where(finite, got, 0.0), np.where(finite, ref, 0.0), "non-finite K and V, V%d %s" % (V, route))
+
+
+@pytest.mark.parametrize("V", [1, 8])
+def test_the_default_counts_a_repeated_column_as_often_as_it_is_listed(gpu, V):
+    """(the union of a block's columns holds it once)"""
+    heads, seq, d = 4, 1500 // V * V, 64
+    mask = _mask("global", seq, V, tokens=64)
+    assert ops.SparseAttention(mask)._route(d, d, heads)[0] == "split"
+    ro, ci = mask.row_offsets, mask.column_indices.copy()
+    ci[ro[:-1] + 2] = ci[ro[:-1] + 1]
+    mask = cv.ColVecCSR(mask.m_vec, seq, V, ro, ci)
+    q, k, v = _operands(heads, seq, d, d)
+    out = ops.SparseAttention(mask).forward(q, k, v)
+    _check_layer(out.double().cpu().numpy(), _layer_in_float64(mask, q, k, v, d ** -0.5), "repeated columns V%d" % V)

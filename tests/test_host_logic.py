@@ -414,3 +414,12 @@ def test_attention_slots_stay_within_the_plan_and_cover_every_block():
             for (a0, a1, _), (b0, _, _) in zip(mine, mine[1:]):
                 assert a1 == b0 and 0 < a1 - a0 <= rounds
             assert 0 < needed - mine[-1][0] <= rounds
+
+
+def test_repeated_columns_are_found_in_any_order():
+    ro = np.array([0, 3, 3, 6, 8], dtype=np.int32)
+    for cols, repeated in (([0, 1, 2, 2, 1, 0, 0, 5], False), ([0, 1, 0, 0, 1, 2, 0, 5], True), ([2, 1, 0, 5, 4, 3, 7, 7], True),
+                           ([0, 1, 2, 2, 3, 4, 4, 5], False)):
+        assert ops.columns_repeat(ro, np.array(cols, dtype=np.int32)) == repeated
+    assert not ops.columns_repeat(np.zeros(1, dtype=np.int32), np.zeros(0, dtype=np.int32))
+    assert not ops.columns_repeat(np.zeros(5, dtype=np.int32), np.zeros(0, dtype=np.int32))

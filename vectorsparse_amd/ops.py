@@ -527,11 +527,18 @@ class SparseAttention:
         self._routes = {}
         self._splits = {}       # (d, d_v, rounds) -> (AttentionSlots, its list on the device, plan)
         self._unions = None     # distinct columns of every block of 128 scalar rows
+        self._repeats = None
 
     def _block_unions(self):
         if self._unions is None:
             self._unions = distinct_columns(self.mask, 128 // self.mask.vec_length)
         return self._unions
+
+    def _repeats_columns(self):
+        """Whether a row lists a column more than once: gathering it counts it as often, a union of columns once."""
+        if self._repeats is None:
+            self._repeats = not self.prob.columns_distinct and columns_repeat(self.mask.row_offsets, self.mask.column_indices)
+        return self._repeats
 
     def _split(self, d, d_v, rounds):
         """Slots and plan of the split launch with at most `rounds` sub-rounds per workgroup, made once."""
@@ -601,7 +608,7 @@ class SparseAttention:
         all (1.39 if the faster side were always taken), ten slower by more than 3 %.  16 heads x 2409, V = 1, a +-139 band
         with 32 global tokens: 260 us in parts, 30 us; 8 heads x 2048, V = 8, +-64 and 64 tokens: 33 us, 19 us."""
         p, m = self.prob, self.mask
-        if (m.m_vec == 0 or m.nnz_vec == 0 or d % 8 != 0 or d_v % 8 != 0
+        if (m.m_vec == 0 or m.nnz_vec == 0 or d % 8 != 0 or d_v % 8 != 0 or self._repeats_columns()
                 or _lib.lib().vs_sparse_attention_split_plan_bytes(p.m_vec, p.vec_length, p.n, d, d_v) <= 0):
             return None
         unions = self._block_unions()
@@ -902,6 +909,14 @@ def columns_ascend(row_offsets, column_indices, strictly=False):
     falls = columns[1:] <= columns[:-1] if strictly else columns[1:] < columns[:-1]
     falls[starts[(starts > 0) & (starts < columns.size)] - 1] = False
     return not falls.any()
+
+
+def columns_repeat(row_offsets, column_indices):
+    """Whether a row lists a column more than once, in any order."""
+    columns, starts = np.asarray(column_indices, dtype=np.int64), np.asarray(row_offsets)
+    rows = np.repeat(np.arange(starts.size - 1, dtype=np.int64), np.diff(starts))
+    places = np.sort(rows * (columns.max(initial=0) + 1) + columns)
+    return bool((places[1:] == places[:-1]).any())
 
 
 class DeviceProblem:
