@@ -423,3 +423,16 @@ def test_repeated_columns_are_found_in_any_order():
         assert ops.columns_repeat(ro, np.array(cols, dtype=np.int32)) == repeated
     assert not ops.columns_repeat(np.zeros(1, dtype=np.int32), np.zeros(0, dtype=np.int32))
     assert not ops.columns_repeat(np.zeros(5, dtype=np.int32), np.zeros(0, dtype=np.int32))
+
+
+def test_a_layers_route_is_stored_once_and_decided():
+    """(another thread that finds the first choice there would take another route, with other bits)"""
+    layer = ops.SparseAttention(cv.band_strided_pattern(2048, 8, band_half_width=64, stride=64), device="cpu")
+    decide, seen = layer._split_route, []
+
+    def watched(*args):
+        seen.append(dict(layer._routes))
+        return decide(*args) or ("split", 2)
+
+    layer._split_route = watched
+    assert layer._route(64, 64, 4) == layer._route(64, 64, 4) == ("split", 2) and seen == [{}]

@@ -573,9 +573,9 @@ class SparseAttention:
                 route = "parts"
             else:
                 route = "layer" if self.union_rows(d, d_v, heads) >= 2 else True
-            self._routes[key] = route
-            self._routes[key] = self._split_route(d, d_v, heads, route) or route
-        return self._routes[key]
+            # (stored once, decided: another thread may read it at any time)
+            self._routes[key] = route = self._split_route(d, d_v, heads, route) or route
+        return route
 
     # Microseconds per layer by route, fitted on MI355X to 19000 masks (1..16 heads x 512..4096, band with and without global
     # tokens, random, every V; head widths to 32, 64 and 128).  Streamed workgroups: launch, per sub-round of the longest one,
