@@ -211,3 +211,20 @@ def test_the_default_counts_a_repeated_column_as_often_as_it_is_listed(gpu, V):
     q, k, v = _operands(heads, seq, d, d)
     out = ops.SparseAttention(mask).forward(q, k, v)
     _check_layer(out.double().cpu().numpy(), _layer_in_float64(mask, q, k, v, d ** -0.5), "repeated columns V%d" % V)
+
+
+def test_the_default_leaves_the_probabilities_in_a_callers_buffer(gpu):
+    """Masks with global tokens: the default on row parts leaves them there, and a buffer asks for it."""
+    V, heads, seq, d = 1, 4, 1500, 64
+    mask = _mask("global", seq, V, tokens=64)
+    layer = ops.SparseAttention(mask)
+    q, k, v = _operands(heads, seq, d, d)
+    assert layer._route(d, d, heads)[0] == "split"
+    scores = torch.full((heads, mask.nnz_vec, V), 7.0, dtype=torch.float16, device="cuda")
+    out = layer.forward(q, k, v, scores=scores)
+    want = torch.empty_like(scores)
+    assert torch.equal(out, layer.forward(q, k, v, scores=want, fused="parts"))
+    assert torch.equal(scores, want)
+    sums = scores.double().cpu().numpy()[0, :, 0]
+    sums = np.add.reduceat(sums, mask.row_offsets[:-1])
+    assert (np.abs(sums - 1.0) < 2.0 ** -11 * 4).all()

@@ -558,12 +558,12 @@ class SparseAttention:
         return spmm_row_parts_workspace_bytes(self.prob.vec_length, d_v, parts.n_split, parts.parts_max,
                                               batch=heads) < 2 ** 31
 
-    def _route(self, d, d_v, heads):
+    def _route(self, d, d_v, heads, split=True):
         """`forward`'s default on the MFMA path for these head widths and head count (a matter of sizes and of the mask:
-        decided once)."""
+        decided once); without `split`, the best route that is not split."""
         key = (d, d_v, heads)
-        route = self._routes.get(key)
-        if route is None:
+        routes = self._routes.get(key)
+        if routes is None:
             p = self.prob
             if (d % 8 == 0 and d_v % 4 == 0 and p.n * d_v < 2 ** 31 and p.row_parts(0)[0].n_split > 0
                     and self._parts_route_fits(d_v, heads)):
@@ -574,8 +574,8 @@ class SparseAttention:
             else:
                 route = "layer" if self.union_rows(d, d_v, heads) >= 2 else True
             # (stored once, decided: another thread may read it at any time)
-            self._routes[key] = route = self._split_route(d, d_v, heads, route) or route
-        return route
+            self._routes[key] = routes = (route, self._split_route(d, d_v, heads, route) or route)
+        return routes[split]
 
     # Microseconds per layer by route, fitted on MI355X to 19000 masks (1..16 heads x 512..4096, band with and without global
     # tokens, random, every V; head widths to 32, 64 and 128).  Streamed workgroups: launch, per sub-round of the longest one,
@@ -713,6 +713,8 @@ class SparseAttention:
     def forward(self, q, k, v, scale=None, kernel="wmma", stream=None, scores=None, out=None, fused=None):
         """q, k, v: fp16 [heads, seq, d] on the device.  Returns fp16 [heads, seq, d].
 
+        scores: fp16 [heads, nonzeros, V], room for what the operators hand on: "parts" and False leave the probabilities there,
+        True the raw scores; "layer" and "split" have no use for it, and the default is never "split" where it is given.
         fused: ("split", rounds) runs the layer in one launch plus a merge, row blocks of more than `rounds` x 128 distinct columns
         (rows that attend to everything) streamed by several workgroups; "parts" runs the three operators on the dispatch list of row parts (masks with rows far longer than
         the rest, e.g. global tokens); "layer" runs the whole layer in one launch with scores and probabilities kept in LDS; True
@@ -732,7 +734,7 @@ class SparseAttention:
         if out is None:
             out = torch.empty((heads, seq, d_v), dtype=torch.float16, device=q.device)
         if fused is None:
-            fused = self._route(d, d_v, heads) if kernel == "wmma" else False
+            fused = self._route(d, d_v, heads, split=scores is None) if kernel == "wmma" else False
         if fused == "layer":    # (keeps the scores to itself)
             return sparse_attention(p.m_vec, p.vec_length, p.n, p.row_indices, p.row_offsets, p.column_indices,
                                     q, k, v, out=out, scale=scale, stream=stream,
