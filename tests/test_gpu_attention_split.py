@@ -228,3 +228,26 @@ def test_the_default_leaves_the_probabilities_in_a_callers_buffer(gpu):
     sums = scores.double().cpu().numpy()[0, :, 0]
     sums = np.add.reduceat(sums, mask.row_offsets[:-1])
     assert (np.abs(sums - 1.0) < 2.0 ** -11 * 4).all()
+
+
+def test_a_first_pass_inside_a_capture_takes_what_needs_no_preparation(gpu):
+    """A layer that has served another head count, captured at one whose split launch was never planned: the plan cannot be
+    made there, the routes that need none can be captured.  The next eager pass makes it."""
+    V, seq, d = 4, 776, 64
+    layer = ops.SparseAttention(_mask("global", seq, V))
+    assert layer._route(d, d, 4) is True and layer._route(d, d, 8) == ("split", 2)
+    layer.forward(*_operands(4, seq, d, d))
+    q, k, v = _operands(8, seq, d, d)
+    out, scores = torch.empty_like(q), torch.empty((8, layer.prob.nnz_vec, V), dtype=torch.float16, device="cuda")
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        layer.forward(q, k, v, out=out)
+    assert not layer._splits
+    want = layer.forward(q, k, v, scores=scores, fused=True)
+    for _ in range(3):
+        out.fill_(3.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+    split = layer.forward(q, k, v)
+    assert torch.equal(split, layer.forward(q, k, v, fused=("split", 2))) and not torch.equal(split, want)

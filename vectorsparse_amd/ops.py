@@ -646,11 +646,15 @@ class SparseAttention:
         return self._rows[key]
 
     def plan(self, d_qk, d_v, heads=16):
-        """Device plan of the union kernel for these head widths (built on first use), or None."""
-        rows = self.union_rows(d_qk, d_v, heads)
+        """Device plan of the union kernel for these head widths (built on first use), or None.  Also makes what the default
+        needs on a mask whose long row blocks are split, so that its next pass can be captured."""
         route = self._route(d_qk, d_v, heads)
         if type(route) is tuple:
             self._split(d_qk, d_v, route[1])
+        return self._union_plan(d_qk, d_v, heads)
+
+    def _union_plan(self, d_qk, d_v, heads):
+        rows = self.union_rows(d_qk, d_v, heads)
         if rows < 2:
             return None
         key = (int(d_qk), int(d_v), rows)
@@ -735,10 +739,12 @@ class SparseAttention:
             out = torch.empty((heads, seq, d_v), dtype=torch.float16, device=q.device)
         if fused is None:
             fused = self._route(d, d_v, heads, split=scores is None) if kernel == "wmma" else False
+            if type(fused) is tuple and (d, d_v, fused[1]) not in self._splits and torch.cuda.is_current_stream_capturing():
+                fused = self._route(d, d_v, heads, split=False)     # (a split cannot be planned inside a capture)
         if fused == "layer":    # (keeps the scores to itself)
             return sparse_attention(p.m_vec, p.vec_length, p.n, p.row_indices, p.row_offsets, p.column_indices,
                                     q, k, v, out=out, scale=scale, stream=stream,
-                                    rows_per_workgroup=self.union_rows(d, d_v, heads), plan=self.plan(d, d_v, heads))
+                                    rows_per_workgroup=self.union_rows(d, d_v, heads), plan=self._union_plan(d, d_v, heads))
         if isinstance(fused, tuple):    # ("split", sub-rounds per workgroup)
             return sparse_attention_split(p, *self._split(d, d_v, fused[1]), q, k, v, out, scale, stream=stream)
         if scores is None:
