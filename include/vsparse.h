@@ -454,7 +454,9 @@ int vs_wmma_spmm_softmax_f16_batched(int batch, int m_vec, int vec_length, int k
 /*
  * values = softmax_row(scale * values) in place, then  out = values * rhs_matrix: vs_sparse_softmax_f16 followed by
  * vs_wmma_spmm_f16_batched, the probabilities kept (a training forward needs them), in one launch where a row's output is one
- * column tile.  Same requirements as vs_wmma_spmm_f16_batched.  No counterpart in the reference (see vs_sparse_softmax_f16).
+ * column tile.  Same requirements as vs_wmma_spmm_f16_batched, and the problems of a batch have values of their own
+ * (stride_values >= nonzeros_vec * vec_length; else 1, hipErrorInvalidValue).  No counterpart in the reference (see
+ * vs_sparse_softmax_f16).
  */
 int vs_wmma_softmax_spmm_f16_batched(int batch, int m_vec, int vec_length, int k, int n, int nonzeros_vec,
                                      int longest_row_vec, const int *row_indices,

@@ -89,6 +89,18 @@ def test_argument_validation_without_launch():
     assert L.vs_cuda_sddmm_f16(0, 64, 64, 0, None, None, None, None, None, None, 8, None) == OK
 
 
+def test_probabilities_kept_in_place_need_values_of_their_own():
+    """vs_wmma_softmax_spmm_f16_batched writes its values: problems that share them are refused before any launch."""
+    L, p = _lib.lib(), 0x1000
+    call = lambda batch, stride, nnz=10, values=p: L.vs_wmma_softmax_spmm_f16_batched(
+        batch, 4, 8, 64, 64, nnz, 5, p, p, p, values, stride, p, 4096, p, 2048, 1.0, None)
+    for batch in (2, 16):
+        assert call(batch, 0) == call(batch, 72) == call(batch, 8) == 1
+        assert call(batch, 0, nnz=-1) == 1
+    assert call(0, 0) == 0
+    assert call(2, 76) == 1         # (whole vectors, as everywhere)
+
+
 def test_attention_planning_helpers_are_consistent():
     """Host-only planning helpers of the union attention kernel: capacity, row rounding, plan size."""
     L = _lib.lib()

@@ -115,3 +115,27 @@ def test_capture_and_replay(gpu):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(values, want[0]) and torch.equal(out, want[1])
+
+
+def test_problems_that_share_values_are_refused(gpu):
+    """(they are replaced in place: several problems would normalise the same scores)"""
+    V, heads, k = 4, 3, 64
+    pat = _pattern(V, LENGTHS, 9)
+    prob = ops.DeviceProblem(pat, sort=True)
+    scores = torch.randn((heads, pat.nnz_vec, V), device="cuda").half()
+    rhs, out = torch.randn((heads, N, k), device="cuda").half(), torch.empty((heads, pat.m, k), dtype=torch.float16, device="cuda")
+
+    def call(values, out=out):
+        return ops.softmax_spmm_batched(pat.m_vec, V, k, N, prob.row_indices, prob.row_offsets, prob.column_indices, values, rhs[:out.shape[0]],
+                                        out, 0.5, nonzeros_vec=pat.nnz_vec, longest_row_vec=prob.longest_row_vec)
+
+    kept = scores.clone()
+    overlapping = scores.view(-1).as_strided((heads, pat.nnz_vec, V), (8 * V, V, 1))
+    for values in (scores[0], scores[:1], scores[:2], scores[:1].expand(heads, -1, -1), overlapping):
+        with pytest.raises(ValueError, match="values of its own"):
+            call(values)
+    torch.cuda.synchronize()
+    assert torch.equal(scores, kept)
+    one = call(scores[0], out=out[:1]).clone()      # (a single problem may be two-dimensional)
+    scores.copy_(kept)
+    assert torch.equal(call(scores)[:1], one)

@@ -137,6 +137,14 @@ struct Reader {
         if (ok && batch != 1 && t->dim() == 3 && stride < (long long)t->size(1) * t->size(2)) ok = false;
         return p;
     }
+    // batched_output, of an operand that is read first: every problem has one
+    void *batched_in_place(int batch, long long &stride)
+    {
+        const at::Tensor *t = ok && left > 0 && THPVariable_Check(*args) ? &THPVariable_Unpack(*args) : nullptr;
+        void *const p = batched_output(batch, stride);
+        if (ok && batch > 1 && (t->dim() != 3 || t->size(0) < batch)) ok = false;
+        return p;
+    }
     // bytes of a caller's buffer, or None
     void *buffer(long long &bytes)
     {
@@ -284,13 +292,14 @@ PyObject *spmm_softmax_batched(PyObject *, PyObject *const *args, Py_ssize_t n_a
     const int nnz = r.integer(), longest = r.integer();
     const int *ri = (const int *)r.indices(), *ro = (const int *)r.indices(), *ci = (const int *)r.indices();
     long long sa, sb, so;
-    const void *scores = r.batched(batch, sa), *rhs = r.batched(batch, sb);
+    void *scores = KEPT ? r.batched_in_place(batch, sa) : r.batched(batch, sa);
+    const void *rhs = r.batched(batch, sb);
     void *out = r.batched(batch, so);
     const float scale = r.number();
     void *stream = r.stream();
     return status_of(r, [&] {
         if constexpr (KEPT)
-            return vs_wmma_softmax_spmm_f16_batched(batch, m_vec, v, k, n, nnz, longest, ri, ro, ci, const_cast<void *>(scores), sa, rhs, sb, out, so, scale, stream);
+            return vs_wmma_softmax_spmm_f16_batched(batch, m_vec, v, k, n, nnz, longest, ri, ro, ci, scores, sa, rhs, sb, out, so, scale, stream);
         else
             return vs_wmma_spmm_softmax_f16_batched(batch, m_vec, v, k, n, nnz, longest, ri, ro, ci, scores, sa, rhs, sb, out, so, scale, stream);
     });

@@ -540,6 +540,9 @@ int vs_wmma_softmax_spmm_f16_batched(int batch, int m_vec, int vec_length, int k
     if (st != VS_SUCCESS) return st;
     if (!stride_ok(stride_values, vec_length) || !stride_ok(stride_rhs, 8) || !stride_ok(stride_output, 8))
         return VS_ERROR_INVALID_VALUE;
+    // (the values are written: no two problems may share one)
+    const long long own = (long long)(nonzeros_vec < 0 ? (values && n > 0) : nonzeros_vec) * vec_length;
+    if (batch > 1 && m_vec > 0 && stride_values < own) return VS_ERROR_INVALID_VALUE;
     return vs::launch_softmax_spmm_mfma(m_vec, vec_length, k, n, row_indices, row_offsets, column_indices,
                                         static_cast<half_t *>(values), static_cast<const half_t *>(rhs_matrix),
                                         static_cast<half_t *>(output_matrix), scale, static_cast<hipStream_t>(stream),

@@ -299,7 +299,8 @@ def spmm_softmax_batched(m_vec, vec_length, k, n, row_indices, row_offsets, colu
 
 def softmax_spmm_batched(m_vec, vec_length, k, n, row_indices, row_offsets, column_indices, values, rhs_matrix,
                          output_matrix, scale=1.0, stream=None, nonzeros_vec=-1, longest_row_vec=-1):
-    """values[b] = softmax_row(scale * values[b]) in place, then out[b] = values[b] @ rhs_matrix[b]."""
+    """values[b] = softmax_row(scale * values[b]) in place, then out[b] = values[b] @ rhs_matrix[b]; values [batch, nnz_vec, V],
+    a problem's own each."""
     if output_matrix.dim() == 2:
         output_matrix = output_matrix.unsqueeze(0)
     batch = output_matrix.shape[0]
@@ -310,6 +311,8 @@ def softmax_spmm_batched(m_vec, vec_length, k, n, row_indices, row_offsets, colu
         return output_matrix
     for t, nm in ((values, "values"), (rhs_matrix, "rhs_matrix"), (output_matrix, "output_matrix")):
         _expect_batched(t, torch.float16, nm)
+    if batch > 1 and (values.dim() != 3 or values.shape[0] < batch or values.stride(0) < values.shape[1] * values.shape[2]):
+        raise ValueError("values: each problem of a batch needs values of its own")
     st = _lib.lib().vs_wmma_softmax_spmm_f16_batched(
         batch, m_vec, vec_length, k, n, int(nonzeros_vec), int(longest_row_vec), _ptr(row_indices), _ptr(row_offsets),
         _ptr(column_indices), _ptr(values), _stride(values, batch), _ptr(rhs_matrix), _stride(rhs_matrix, batch),
