@@ -251,3 +251,34 @@ def test_a_first_pass_inside_a_capture_takes_what_needs_no_preparation(gpu):
         assert torch.equal(out, want)
     split = layer.forward(q, k, v)
     assert torch.equal(split, layer.forward(q, k, v, fused=("split", 2))) and not torch.equal(split, want)
+
+
+def test_partial_tiles_lie_in_memory_of_the_stream_that_uses_them(gpu):
+    """A pass on one stream gives its partial tiles back while it still runs; a pass on another stream that is not ordered
+    behind it must not get the same memory."""
+    V, heads, seq, d = 8, 2, 776, 64
+    layer = ops.SparseAttention(_mask("global", seq, V))
+    q, k, v = _operands(heads, seq, d, d)
+    want = layer.forward(q, k, v, fused=("split", 1))
+    torch.cuda.synchronize()
+    side, handed = torch.cuda.Stream(), []
+    empty = torch.empty
+
+    def watched(*args, **kwargs):
+        t = empty(*args, **kwargs)
+        if t.dtype == torch.float32:
+            handed.append((torch.cuda.current_stream().cuda_stream, t.data_ptr()))
+        return t
+
+    out = [torch.zeros_like(want) for _ in range(9)]
+    torch.empty = watched
+    try:
+        for i, one in enumerate(out):
+            layer.forward(q, k, v, out=one, fused=("split", 1), stream=(None, side, side.cuda_stream)[i % 3])
+    finally:
+        torch.empty = empty
+    torch.cuda.synchronize()
+    assert all(torch.equal(one, want) for one in out)
+    here, there = torch.cuda.current_stream().cuda_stream, side.cuda_stream
+    assert [stream for stream, _ in handed] == [here, there, there] * 3
+    assert not {p for s, p in handed if s == here} & {p for s, p in handed if s == there}

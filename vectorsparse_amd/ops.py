@@ -8,6 +8,7 @@ addresses; the output dtype of ``output_matrix`` / ``output_values`` (fp16 or
 fp32) picks the overload, as C++ overload resolution does in the reference.
 Every call is asynchronous on ``stream`` (default: torch's current stream).
 """
+import contextlib
 import ctypes
 
 import numpy as np
@@ -55,6 +56,11 @@ def _stream(stream):
     if isinstance(stream, torch.cuda.Stream):
         return stream.cuda_stream
     return int(stream)
+
+
+def _as_stream(stream):
+    """A stream argument (not None) as a torch stream."""
+    return stream if isinstance(stream, torch.cuda.Stream) else torch.cuda.ExternalStream(int(stream))
 
 
 def _expect(t, dtype, name):
@@ -482,9 +488,9 @@ def sparse_attention_split(prob, slots, device_slots, plan, q, k, v, out, scale,
     heads, _, d = q.shape
     d_v = v.shape[2]
     if workspace is None and slots.n_partials:
-        workspace = torch.empty(slots.n_partials * heads * 128 * (d_v + 2), dtype=torch.float32, device=q.device)
-        if stream is not None:
-            workspace.record_stream(stream if isinstance(stream, torch.cuda.Stream) else torch.cuda.ExternalStream(int(stream)))
+        # (memory of the stream it is used on: what another stream has given back may still be in use there)
+        with contextlib.nullcontext() if stream is None else torch.cuda.stream(_as_stream(stream)):
+            workspace = torch.empty(slots.n_partials * heads * 128 * (d_v + 2), dtype=torch.float32, device=q.device)
     st = _native.sparse_attention_split(heads, prob.m_vec, prob.vec_length, prob.n, d, d_v, prob.row_offsets, prob.column_indices,
                                         q, k, v, out, float(scale), plan, device_slots, slots.n_slots, slots.n_merges,
                                         slots.n_partials, workspace, stream)
