@@ -3,7 +3,7 @@ import numpy as np
 import pytest
 import torch
 
-from vectorsparse_amd import ops
+from vectorsparse_amd import _lib, ops
 from vectorsparse_amd import colvec_csr as cv
 from test_gpu_attention import _check_layer, _dense_attention
 
@@ -105,10 +105,13 @@ def test_refused_arguments(gpu):
     q, k, v = _operands(2, 520, 64, 64)
     slots, device_slots, plan = layer._split(64, 64, 1)
     out = torch.empty_like(q)
-    small = torch.empty(slots.n_partials * 2 * 128 * 66 - 1, dtype=torch.float32, device="cuda")
-    for bad_plan, workspace in ((plan[:-16], None), (plan, small)):
-        with pytest.raises(Exception):
+    whole = torch.empty(slots.n_partials * 2 * 128 * 66, dtype=torch.float32, device="cuda")
+    for bad_plan, workspace in ((plan[:-16], None), (plan, whole[:-1])):
+        with pytest.raises(_lib.VSparseError, match=r"vs_sparse_attention_f16_split.*invalid"):
             ops.sparse_attention_split(layer.prob, slots, device_slots, bad_plan, q, k, v, out, 0.125, workspace)
+    # (the same call with all of the plan and exactly the room it needs)
+    ops.sparse_attention_split(layer.prob, slots, device_slots, plan, q, k, v, out, 0.125, whole)
+    assert torch.equal(out, layer.forward(q, k, v, scale=0.125, fused=("split", 1)))
     with pytest.raises(TypeError):
         ops.sparse_attention_split(layer.prob, slots, device_slots, plan, q.float(), k, v, out, 0.125)
 
