@@ -100,6 +100,7 @@ def kernel_source_tag(*names):
 SPMM_SOURCES = ("spmm_mfma.hip", "spmm_mfma_step.hpp", "vs_common.hpp")
 # (sddmm_tile.hip decides whether a mask is gathered at all)
 SDDMM_SOURCES = ("sddmm_mfma.hip", "sddmm_tile.hip", "vs_common.hpp")
+STREAM_SOURCES = ("sparse_attention_union.hip", "vs_common.hpp")
 
 
 def measured_traffic(path, sources):
@@ -171,7 +172,7 @@ def cpu_baseline(pat, B, n_dense, flops, budget_s=12.0):
 
 
 PMC_MODES = ["spmm", "spmm_largest", "spmm_slab_50", "spmm_slab_90", "spmm_valu_v1", "spmm_ragged", "sddmm_valu_v1", "sddmm_tile", "sddmm_k128", "spmm_dma", "spmm_split_rows", "spmm_row_parts", "sddmm", "attention",
-             "attention_window"]
+             "attention_window", "attention_global", "attention_chain", "spmm_tile"]
 
 
 def largest_sweep_point(cv):
@@ -303,6 +304,21 @@ def sweep_v8(torch, cv, ops, iters=30):
             "launches_per_replay": iters, "by_sparsity": buckets}
 
 
+def global_token_mask(cv, np, seq, vec_length, half_width, tokens):
+    """A band with `tokens` tokens in the middle that attend to everything and that everybody attends to."""
+    start, rows = seq // 2 // vec_length * vec_length, []
+    for i in range(seq // vec_length):
+        keep = np.zeros(seq, dtype=bool)
+        centre = i * vec_length + vec_length // 2
+        keep[max(0, centre - half_width):centre + half_width + 1] = True
+        keep[start:start + tokens] = True
+        if start <= i * vec_length < start + tokens:
+            keep[:] = True
+        rows.append(np.flatnonzero(keep).astype(np.int32))
+    offsets = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    return cv.ColVecCSR(seq // vec_length, seq, vec_length, offsets, np.concatenate(rows))
+
+
 def skewed_point(cv, np):
     """Pareto-distributed row lengths (mean about 280 vectors, the longest row dense), 1024 vector rows x 4608."""
     rng = np.random.default_rng(0)
@@ -324,7 +340,8 @@ def main():
                          "(calibration), then ten eager launches of one kernel and nothing else: the headline SpMM "
                          "(config 2), the largest sweep point (2048 x 4608 at 90 %%), the LDS-staged schedule on that shape at 50 %% and 90 %%, config 2 on the LDS-DMA gather "
                          "variant, the split-row SpMM and the SpMM with rows in parts on Pareto-distributed rows, the config-4 SDDMM, the config-5 "
-                         "attention layer with its plan, or that layer with a plain 513-wide window mask")
+                         "attention layer with its plan, that layer with a plain 513-wide window mask, a band with global tokens "
+                         "(the split launch and its merge), an attention layer that keeps its probabilities (SDDMM, then softmax and SpMM in one launch), or the SpMM on dense tiles")
     ap.add_argument("--cold", action="store_true",
                     help="flushed-cache mode for `rocprofv3 --kernel-trace --stats`: ten rounds of (1 GiB fill, ONE launch) "
                          "for each of the config-2 SpMM, the largest sweep point, the config-4 SDDMM, the dense GEMM of "
@@ -470,6 +487,17 @@ def main():
             info["algorithmic_bytes"] = sddmm_algorithmic_bytes(tmask, 256)
             info["nonzero_vectors"] = int(tmask.nnz_vec)
             info["kernel_source_tag"] = kernel_source_tag("sddmm_tile.hip", "vs_common.hpp")
+        elif args.pmc == "spmm_tile":
+            # the SpMM on dense tiles: 4096 x 4096 x 2048 at 80 %, V = 4
+            tpat = cv.random_values(cv.binomial_pattern(1024, 4096, 0.8, seed=37, vec_length=4), seed=38)
+            tprob = ops.DeviceProblem(tpat)
+            tBd = torch.from_numpy(cv.dense_uniform(4096, 2048, seed=39)).cuda()
+            tout = torch.empty((tpat.m, 2048), dtype=torch.float16, device="cuda")
+            for _ in range(10):
+                tprob.spmm(tBd, kernel="wmma", out=tout)
+            info["algorithmic_bytes"] = spmm_algorithmic_bytes(tpat, 2048)
+            info["nonzero_vectors"] = int(tpat.nnz_vec)
+            info["kernel_source_tag"] = kernel_source_tag("spmm_tile.hip", "spmm_mfma_step.hpp", "vs_common.hpp")
         elif args.pmc == "spmm_ragged":
             # a dense width that is a multiple of nothing: 1022 x 147 at 70 %, V = 2, N = 205, fp32 outputs
             rpat = cv.random_values(cv.binomial_pattern(511, 147, 0.7, seed=34, vec_length=2), seed=35)
@@ -513,19 +541,33 @@ def main():
             info["algorithmic_bytes"] = sddmm_algorithmic_bytes(mask, 64)
             info["kernel_source_tag"] = kernel_source_tag(*SDDMM_SOURCES)
         else:
-            heads, seq, dim = 16, 4096, 64
+            heads, seq, dim = (16, 4096, 64) if args.pmc in ("attention", "attention_window") else (8, 2048, 64)
             if args.pmc == "attention_window":
                 amask = cv.band_strided_pattern(seq, 8, band_half_width=256, stride=seq)
+            elif args.pmc == "attention_global":
+                amask = global_token_mask(cv, np, seq, 8, half_width=64, tokens=64)
+            elif args.pmc == "attention_chain":
+                amask = cv.binomial_pattern(seq // 4, seq, 0.95, seed=41, vec_length=4)
             else:
                 amask = cv.band_strided_pattern(seq, 8, band_half_width=128, stride=128)
             layer = ops.SparseAttention(amask)
             gen = torch.Generator(device="cuda").manual_seed(5)
             q, kk_, vv = (torch.randn((heads, seq, dim), device="cuda", generator=gen).half() for _ in range(3))
             ctx = torch.empty((heads, seq, dim), dtype=torch.float16, device="cuda")
+            kept = torch.empty((heads, amask.nnz_vec, amask.vec_length), dtype=torch.float16, device="cuda")
+            layer.plan(dim, dim, heads)
             for _ in range(10):
-                layer.forward(q, kk_, vv, out=ctx)
+                if args.pmc == "attention_chain":
+                    layer.forward(q, kk_, vv, out=ctx, fused=False, scores=kept)
+                else:
+                    layer.forward(q, kk_, vv, out=ctx)
             info["algorithmic_bytes"] = 4 * heads * seq * dim * 2      # q, k, v read once, out written once
-            info["rows_per_workgroup"] = layer.union_rows(dim, dim, heads)
+            if args.pmc == "attention_chain":
+                info["kernel_source_tag"] = kernel_source_tag(*SPMM_SOURCES)
+            else:
+                info["route"] = str(layer._route(dim, dim, heads))
+                info["rows_per_workgroup"] = layer.union_rows(dim, dim, heads)
+                info["kernel_source_tag"] = kernel_source_tag(*STREAM_SOURCES)
             info["nonzero_vectors"] = int(amask.nnz_vec)
         torch.cuda.synchronize()
         print(json.dumps(info))

@@ -1128,8 +1128,9 @@ sparse_attention_stream_kernel(int m_vec, int n, int d_qk, int d_v,
 }
 
 // Adds up the partial tiles of a split row block: merge entry {row block, first partial tile, tiles, -}; a wave takes four scalar
-// rows, a workgroup a quarter of a block.  A few hundred KB per head at most, read once: bound by the launch and one round trip
-// (3 us).  Sums that are NaNs, or of rows whose every score is -infinity, send the wave's rows to the per-row path, as in the
+// rows, a workgroup a quarter of a block.  A few hundred KB per head at most, read once: bound by the launch and a chain of
+// dependent loads (5 us in the trace of back-to-back passes, the streamed launch in front of it 13; 8 heads x 2048, V = 8,
+// +-64 and 64 tokens).  Sums that are NaNs, or of rows whose every score is -infinity, send the wave's rows to the per-row path, as in the
 // streamed kernel.
 template <int V, int KS, int CPL>
 __global__ void __launch_bounds__(512, union_wide(KS, CPL) ? 2 : 4)

@@ -19,9 +19,10 @@
 // that does not follow its predecessor or its chunk, a cursor that does not end with its row) and the workgroup then
 // computes its tile again nonzero by nonzero, with the steps of the gathering kernel.
 //
-// What bounds it (4096 x 4096 x 2048, V = 4, 80 %, tiles of 128 x 128: 73 us, 130 us gathering): of a workgroup's 134 k
-// cycles 48 k go into filling, 60 k into multiplying (the matrix cores are busy for half of all cycles, at a clock that
-// their load lowers to about 2 GHz: the products alone take 44 us), 20 k into barriers.  Small launches wait for rhs: the
+// What bounds it (4096 x 4096 x 2048, V = 4, 80 %, tiles of 128 x 128: 75 us, 130 us gathering): of a workgroup's 134 k
+// cycles 48 k go into filling, 60 k into multiplying, 20 k into barriers.  By the counters the matrix cores are busy for 37 %
+// of the launch at 2.4 GHz (44 % at the 2 GHz or so that their load leaves; the products alone take 44 us), LDS for 38 %, of
+// which 42 % are bank conflicts.  Small launches wait for rhs: the
 // vector memory path takes about 18 cycles per request of 512 bytes.  Measured and not kept, same problem: one operand
 // ahead in LDS and the two waves of a SIMD filling and multiplying in opposite order 71 us (one workgroup per CU, 79 us for
 // half the steps per barrier); waves that only fill beside waves that only multiply 70 us (accumulators in AGPRs, else
@@ -382,7 +383,7 @@ int launch_tile(int shape, int m_vec, int k, int n, const int *row_offsets, cons
 }  // namespace
 
 // Both sides of the choice as microseconds per launch, fitted to 2500 problems (64..4096 rows, 64..4608 columns, widths of
-// 32..2048, 50..95 %, every V; device time, the tiles' estimate good to 8 to 10 %, the gathering kernels' to 16 %).
+// 32..2048, 50..95 %, every V; device time).
 // Gathering: a launch, then a time per nonzero vector and dense column (the fine-grained kernel's grows with V).  Tiles: a
 // launch, then per workgroup and contraction element a share of walking, one of scattering the block's nonzeros and, where a
 // row has more nonzeros in a chunk than two windows hold, one of fetching more; a CU runs one workgroup as fast as it can, a
@@ -390,7 +391,13 @@ int launch_tile(int shape, int m_vec, int k, int n, const int *row_offsets, cons
 // on the MFMA path and for 624 on the fine-grained one: 1.12 and 1.17 times faster in the mean of all 2500, 1.13 and 1.20 being
 // what always taking the faster side would give; six are slower by more than 3 % (9 % at most).  A margin of a tenth would
 // gain half a percent more and make eighteen slower, by up to 17 %.
-// 4096 x 4096 x 2048, V = 4, 80 %: 130 us gathering, 73 us on tiles of 128 x 128; 4096 x 4096 x 512, V = 1, 50 %: 317 against
+// How good the estimates are, over 370 problems drawn again from those ranges and both kernels
+// (profiles/spmm_tile_rule_survey.txt): tiles 12 % high to 7 % low in the mean by shape and size, with spreads of 8 to 18 %.  Gathering: 40 % (MFMA) and
+// 30 % (fine-grained) high below 1e7 nonzero vectors x columns, where tiles are far behind; above 1e8 20 % and 11 % low with a
+// spread of 23 % and 20 %, which errs on the gathering side (the largest problems go either way: 4096 x 4096 x 2048, V = 4,
+// 80 % is put at 163 us and takes 130).  One of the 740 choices is slower by more than 3 %: 12 %, 520 workgroups of 32 x 64 on the
+// 512 places of the chip.  Above 1e8 the choice is 1.48 (MFMA) and 1.59 times faster in the mean, 1.60 and 1.68 with the faster side.
+// 4096 x 4096 x 2048, V = 4, 80 %: 130 us gathering, 75 us on tiles of 128 x 128; 4096 x 4096 x 512, V = 1, 50 %: 317 against
 // 79 us (64 x 128); 2048 x 2304 x 256, V = 2, 50 %: 31 against 18 us (32 x 64); 2048 x 2304 x 512, V = 4, 90 %: 9.1 against
 // 18.5 us; at the line, 2048 x 2304 x 256, V = 1, 90 %: 13.4 (MFMA) and 12.6 us (fine-grained) against 12.9 us.
 // Only where the caller vouches for strictly ascending columns: a row in another order makes its workgroup go nonzero by nonzero.

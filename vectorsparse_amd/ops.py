@@ -522,10 +522,11 @@ class SparseAttention:
     """One fixed-mask sparse attention layer: SDDMM (QK^T on the mask) -> row softmax -> SpMM (P V).
 
     The mask is a column-vector CSR pattern over [seq, seq] shared by all heads.  `forward` runs the layer as
-    one launch (scores and probabilities never leave the chip), as two (SDDMM, then the SpMM with the softmax
-    folded in) or as the three operators, one batched launch each, chained on one stream with no host
-    synchronisation and no re-layout (the SDDMM output layout is the SpMM value layout); by default it
-    picks the faster of the first two for the mask, the head widths and the head count.
+    one launch (scores and probabilities never leave the chip), as one launch and a merge where a few row blocks
+    have far more columns than the rest, as two (SDDMM, then the SpMM with the softmax folded in) or as the
+    operators, on whole rows or on row parts, chained on one stream with no host synchronisation and no re-layout
+    (the SDDMM output layout is the SpMM value layout); by default it picks the one that fitted times put ahead
+    for the mask, the head widths and the head count.
     """
 
     def __init__(self, mask, device="cuda", sort=True):
@@ -588,15 +589,17 @@ class SparseAttention:
 
     # Microseconds per layer by route, fitted on MI355X to 19000 masks (1..16 heads x 512..4096, band with and without global
     # tokens, random, every V; head widths to 32, 64 and 128).  Streamed workgroups: launch, per sub-round of the longest one,
-    # launch under load, per workgroup and per sub-round in 512ths, merge, per tile of the longest merge (good to 5-7 %).
+    # launch under load, per workgroup and per sub-round in 512ths, merge, per tile of the longest merge.  Measured again over
+    # 240 drawn masks (profiles/attention_split_rule_survey.txt) the estimates are high by 6 % (streamed with a merge; spread
+    # 9 %), 21 % (one workgroup per block; 11 %), 7 % (row parts; 9 %) and 19 % (two launches; 11 %).
     _STREAM_US = ((3.47, 2.06, 5.15, 2.13, 4.21, 2.9, 0.5), (3.41, 2.47, 5.86, 4.21, 4.87, 3.12, 0.49),
                   (4.1, 3.64, 6.0, 10.63, 10.22, 3.98, 1.01))
     # The three operators on row parts: launches, per thousand vector rows of 16 heads, per thousand nonzero vectors of 16 heads
-    # by vector length (7 %).
+    # by vector length.
     _PARTS_US = ((16.0, 14.0, {1: 0.176, 2: 0.207, 4: 0.276, 8: 0.466}), (16.4, 16.0, {1: 0.223, 2: 0.251, 4: 0.327, 8: 0.523}),
                  (16.9, 23.7, {1: 0.327, 2: 0.37, 4: 0.463, 8: 0.712}))
     # The two launches: the same, then per thousand nonzero vectors of the longest row, and the share of the shorter of the
-    # two that is not hidden (13-17 %).
+    # two that is not hidden.
     _TWO_US = ((6.6, 9.0, {1: 0.16, 2: 0.194, 4: 0.219, 8: 0.314}, 8.2, 1.95), (6.7, 12.5, {1: 0.172, 2: 0.21, 4: 0.272, 8: 0.409}, 8.3, 1.58),
                (6.7, 20.9, {1: 0.235, 2: 0.326, 4: 0.432, 8: 0.701}, 9.2, 1.52))
 
@@ -614,7 +617,8 @@ class SparseAttention:
     def _split_route(self, d, d_v, heads, route):
         """("split", sub-rounds) where streaming long row blocks by several workgroups is expected to take less than four
         fifths of `route`, else None.  Over the masks of the fit: chosen for 8300 of 18900, 1.34 times faster in the mean of
-        all (1.39 if the faster side were always taken), ten slower by more than 3 %.  16 heads x 2409, V = 1, a +-139 band
+        all (1.39 if the faster side were always taken), ten slower by more than 3 %; of 240 drawn again for 67, 1.83 times
+        faster in their mean, none slower (1.18 over all, 1.20 with the faster side).  16 heads x 2409, V = 1, a +-139 band
         with 32 global tokens: 260 us in parts, 30 us; 8 heads x 2048, V = 8, +-64 and 64 tokens: 33 us, 19 us."""
         p, m = self.prob, self.mask
         if (m.m_vec == 0 or m.nnz_vec == 0 or d % 8 != 0 or d_v % 8 != 0 or self._repeats_columns()
@@ -728,16 +732,18 @@ class SparseAttention:
 
         scores: fp16 [heads, nonzeros, V], room for what the operators hand on: "parts" and False leave the probabilities there,
         True the raw scores; "layer" and "split" have no use for it, and the default is never "split" where it is given.
-        fused: ("split", rounds) runs the layer in one launch plus a merge, row blocks of more than `rounds` x 128 distinct columns
-        (rows that attend to everything) streamed by several workgroups; "parts" runs the three operators on the dispatch list of row parts (masks with rows far longer than
-        the rest, e.g. global tokens); "layer" runs the whole layer in one launch with scores and probabilities kept in LDS; True
+        fused: ("split", rounds) runs the layer in one launch plus a merge, row blocks of more than `rounds` x 128 distinct
+        columns (rows that attend to everything) streamed by several workgroups; "parts" runs the three operators on the
+        dispatch list of row parts; "layer" runs the whole layer in one launch with scores and probabilities kept in LDS; True
         folds only the softmax into the SpMM launch (two launches, raw scores go through memory); False runs
         the three operators one after the other and leaves the probabilities in `scores` (on the MFMA path softmax and SpMM share
-        a launch where that is faster).  Default on the MFMA path: "layer" when the cost model of
-        `_union_rows` puts the streamed union kernel ahead (banded, blocky, strided and very sparse masks: 1.5-15x
-        faster than the alternatives), else True - on masks without shared columns the single launch gathers
-        K / V rows per row and is 10-60 % slower than the two launches (16 heads x 4096, uniform random masks,
-        90-98 % sparse, V = 1..8).
+        a launch where that is faster).  Default on the MFMA path (`_route`): "parts" where the mask has rows far longer than
+        the rest (global tokens); else "layer" when the cost model of `_union_rows` puts the streamed union kernel ahead
+        (banded, blocky, strided and very sparse masks: 1.5-15x faster than the alternatives), else True - on masks without
+        shared columns the single launch gathers K / V rows per row and is 10-60 % slower than the two launches (16 heads x
+        4096, uniform random masks, 90-98 % sparse, V = 1..8).  "split" in place of any of these where `_split_route` expects
+        it to take less than four fifths of the time: no `scores` given, no column twice in a row, and not as a first pass
+        inside a stream capture (`plan` prepares one).  Default on the other path: False.
         """
         p = self.prob
         heads, seq, d = q.shape
