@@ -301,6 +301,21 @@ int vs_cuda_spmm_f16_ascending(int m_vec, int vec_length, int k, int n, int nonz
                                const void *values, const void *rhs_matrix, void *output_matrix, void *stream);
 
 /*
+ * The same operators (fine_grained: the function of vs_cuda_spmm_f16_ascending) with fp16 outputs, in two
+ * launches: the rows packed two of every four neighbouring columns into `workspace`, then a product on the sparse matrix
+ * instructions; what does not fit is added from a list.  For patterns whose columns ascend strictly in every row, k % 8 == 0
+ * (option "spmm_packed"); nonzeros_vec and longest_row_vec are the pattern's.  Order and counts are hints as above.
+ * vs_spmm_packed_workspace_bytes: what the call needs (16-byte aligned, uninitialised, used by one call at a time), 0 where
+ * the entry points above are expected to be faster or have to take the call, and the call returns VS_ERROR_NOT_SUPPORTED.
+ * No counterpart in the reference.
+ */
+long long vs_spmm_packed_workspace_bytes(int fine_grained, int m_vec, int vec_length, int k, int n, int nonzeros_vec,
+                                         int longest_row_vec);
+int vs_spmm_f16_packed(int fine_grained, int m_vec, int vec_length, int k, int n, int nonzeros_vec, int longest_row_vec,
+                       const int *row_offsets, const int *column_indices, const void *values, const void *rhs_matrix,
+                       void *output_matrix, void *workspace, long long workspace_bytes, void *stream);
+
+/*
  * Rows in parts: the row swizzle of the reference (SortedRowSwizzle, include/bm_test_utils.h:200-215, which
  * reorders the dispatch of whole rows) taken one step further - a row far longer than the rest is dispatched as
  * several parts, each to a workgroup of its own, so that no workgroup is left walking one row when the rest of
@@ -617,6 +632,8 @@ int vs_wmma_spmm_launch_shape(int batch, int m_vec, int vec_length, int k, int n
  * 2 = in two, 0 = automatic),
  * "spmm_tile" (SpMM on dense tiles, fp16 outputs, k % 4 == 0, any order of the columns: 1 = never, 2 = tiles of 32 x 64,
  * 3 = of 64 x 128, 4 = of 128 x 128, 0 = where the columns are known to ascend strictly and tiles are expected to be faster),
+ * "spmm_packed" (SpMM on rows packed two of four, k % 8 == 0: 1 = never, 2 = tiles of 256 x 128, 3 = of 128 x 128,
+ * 0 = where expected to be faster),
  * "sddmm_tile" (SDDMM on dense tiles, k % 8 == 0, any order of the columns: 1 = never, 2 = tiles of 64 x 64,
  * 3 = of 128 x 128, 0 = where the columns are known to ascend and tiles are expected to be faster than gathering rows),
  * "attention_waves" (1..8, 0 = automatic), "attention_chunk" (nonzero vectors per

@@ -192,7 +192,8 @@ PyObject *spmm(PyObject *, PyObject *const *args, Py_ssize_t n_args)
 }
 
 // (fine_grained, m_vec, vec_length, k, n, nonzeros_vec, longest_row_vec, long_rows, row_length_hints, row_indices, row_offsets,
-// column_indices, values, rhs, out, stream), fp16 outputs
+// column_indices, values, rhs, out, stream, may_pack), fp16 outputs; -2 - with nothing launched - where spmm_packed is expected to
+// be faster and the caller may make its workspace
 PyObject *spmm_ascending(PyObject *, PyObject *const *args, Py_ssize_t n_args)
 {
     Reader r(args, n_args);
@@ -203,9 +204,26 @@ PyObject *spmm_ascending(PyObject *, PyObject *const *args, Py_ssize_t n_args)
     const int *ri = (const int *)r.indices(), *ro = (const int *)r.indices(), *ci = (const int *)r.indices();
     const void *values = r.halves(), *rhs = r.halves();
     void *out = r.halves(), *stream = r.stream();
+    if (r.flag() && r.done() && vs_spmm_packed_workspace_bytes(fine_grained, m_vec, v, k, n, nnz, longest) > 0) return PyLong_FromLong(-2);
     return status_of(r, [&] {
         return fine_grained ? vs_cuda_spmm_f16_ascending(m_vec, v, k, n, nnz, longest, hints, ri, ro, ci, values, rhs, out, stream)
                             : vs_wmma_spmm_f16_ascending(m_vec, v, k, n, nnz, longest, long_rows, hints, ri, ro, ci, values, rhs, out, stream);
+    });
+}
+
+// (fine_grained, m_vec, vec_length, k, n, nonzeros_vec, longest_row_vec, row_offsets, column_indices, values, rhs, out, workspace, stream)
+PyObject *spmm_packed(PyObject *, PyObject *const *args, Py_ssize_t n_args)
+{
+    Reader r(args, n_args);
+    const bool fine_grained = r.flag();
+    const int m_vec = r.integer(), v = r.integer(), k = r.integer(), n = r.integer(), nnz = r.integer(), longest = r.integer();
+    const int *ro = (const int *)r.indices(), *ci = (const int *)r.indices();
+    const void *values = r.halves(), *rhs = r.halves();
+    void *out = r.halves();
+    long long bytes;
+    void *workspace = r.buffer(bytes), *stream = r.stream();
+    return status_of(r, [&] {
+        return vs_spmm_f16_packed(fine_grained, m_vec, v, k, n, nnz, longest, ro, ci, values, rhs, out, workspace, bytes, stream);
     });
 }
 
@@ -457,6 +475,7 @@ PyMethodDef methods[] = {
     VS_METHOD("wmma_spmm", (spmm<vs_wmma_spmm_f16, vs_wmma_spmm_f16_f32out>)),
     VS_METHOD("cuda_spmm", (spmm<vs_cuda_spmm_f16, vs_cuda_spmm_f16_f32out>)),
     VS_METHOD("spmm_ascending", spmm_ascending),
+    VS_METHOD("spmm_packed", spmm_packed),
     VS_METHOD("wmma_sddmm", wmma_sddmm),
     VS_METHOD("cuda_sddmm", cuda_sddmm),
     VS_METHOD("wmma_spmm_batched", wmma_spmm_batched),

@@ -401,19 +401,18 @@ int launch_tile(int shape, int m_vec, int k, int n, const int *row_offsets, cons
 // 79 us (64 x 128); 2048 x 2304 x 256, V = 2, 50 %: 31 against 18 us (32 x 64); 2048 x 2304 x 512, V = 4, 90 %: 9.1 against
 // 18.5 us; at the line, 2048 x 2304 x 256, V = 1, 90 %: 13.4 (MFMA) and 12.6 us (fine-grained) against 12.9 us.
 // Only where the caller vouches for strictly ascending columns: a row in another order makes its workgroup go nonzero by nonzero.
-int spmm_tile_choice(bool fine_grained, int m_vec, int k, int n, int vec_length, const Batch &batch)
+double spmm_gather_us(bool fine_grained, int vec_length, double nonzeros_vec, int k)
 {
-    const Options &o = options();
-    if (o.spmm_tile == 1 || (o.spmm_tile == 0 && !batch.sorted_columns)) return 0;
-    // (the kernel's offsets into a step's rows of rhs, and into rhs, are 32-bit)
-    if (m_vec <= 0 || k <= 0 || k % 4 != 0 || n <= 0 || (long long)n * k >= (1LL << 30) || k >= (1 << 24) || batch.count < 1 || batch.count > 65535) return 0;
-    if (o.spmm_tile >= 2) return o.spmm_tile - 1;
-    if (o.spmm_waves || o.spmm_cols_per_lane || o.spmm_steps || o.spmm_pipe || o.spmm_gather || o.spmm_teams || o.spmm_blocks_per_wave || o.spmm_guard_waves)
-        return 0;  // a launch shape of the gathering kernels is asked for
     const int v = vec_length == 1 ? 0 : (vec_length == 2 ? 1 : (vec_length == 4 ? 2 : 3));
     static constexpr double kPerMega[2][4] = {{0.088, 0.089, 0.0925, 0.0995}, {0.076, 0.091, 0.134, 0.28}};
-    const double gather = (fine_grained ? 4.7 : 4.0) + kPerMega[fine_grained][v] * 1e-6 * (double)batch.tile_nonzeros_vec * k;
-    const double density = (double)batch.tile_nonzeros_vec / ((double)m_vec * n), longest = (double)batch.tile_longest_vec / n;
+    return (fine_grained ? 4.7 : 4.0) + kPerMega[fine_grained][v] * 1e-6 * nonzeros_vec * k;
+}
+
+// The fastest tile shape where one is expected to be ahead of gathering (0: none), and the time of what is then run.
+static int fastest_tile(bool fine_grained, int m_vec, int k, int n, int vec_length, double nonzeros_vec, int longest_vec, double &us)
+{
+    const double gather = spmm_gather_us(fine_grained, vec_length, nonzeros_vec, k);
+    const double density = nonzeros_vec / ((double)m_vec * n), longest = (double)longest_vec / n;
     struct Shape {
         int rows, columns, chunk;
         double launch, per_block, walk, scatter, more, second;
@@ -436,7 +435,28 @@ int spmm_tile_choice(bool fine_grained, int m_vec, int k, int n, int vec_length,
             best = shape;
         }
     }
+    us = best ? least : gather;
     return best;
+}
+
+double spmm_expected_us(bool fine_grained, int m_vec, int k, int n, int vec_length, int nonzeros_vec, int longest_vec)
+{
+    double us = 0;
+    fastest_tile(fine_grained, m_vec, k, n, vec_length, nonzeros_vec, longest_vec, us);
+    return us;
+}
+
+int spmm_tile_choice(bool fine_grained, int m_vec, int k, int n, int vec_length, const Batch &batch)
+{
+    const Options &o = options();
+    if (o.spmm_tile == 1 || (o.spmm_tile == 0 && !batch.sorted_columns)) return 0;
+    // (the kernel's offsets into a step's rows of rhs, and into rhs, are 32-bit)
+    if (m_vec <= 0 || k <= 0 || k % 4 != 0 || n <= 0 || (long long)n * k >= (1LL << 30) || k >= (1 << 24) || batch.count < 1 || batch.count > 65535) return 0;
+    if (o.spmm_tile >= 2) return o.spmm_tile - 1;
+    if (o.spmm_waves || o.spmm_cols_per_lane || o.spmm_steps || o.spmm_pipe || o.spmm_gather || o.spmm_teams || o.spmm_blocks_per_wave || o.spmm_guard_waves)
+        return 0;  // a launch shape of the gathering kernels is asked for
+    double us;
+    return fastest_tile(fine_grained, m_vec, k, n, vec_length, batch.tile_nonzeros_vec, batch.tile_longest_vec, us);
 }
 
 int launch_spmm_tile(int shape, int m_vec, int vec_length, int k, int n, const int *row_offsets, const int *col_indices,

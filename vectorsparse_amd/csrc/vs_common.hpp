@@ -253,6 +253,7 @@ struct Options {
     int sddmm_flat_supers = 0;  // flat MFMA SDDMM (algorithm 2): super-groups per wave, 0 = automatic
     int softmax_spmm = 0;       // softmax and SpMM that keeps the probabilities: 1 = one launch, 2 = two, 0 = automatic
     int spmm_tile = 0;          // SpMM on dense tiles: 1 = never, 2 / 3 / 4 = tiles of 32 x 64, 64 x 128, 128 x 128, 0 = automatic
+    int spmm_packed = 0;        // SpMM on rows packed two of four: 1 = never, 2 / 3 = tiles of 256 x 128, 128 x 128, 0 = automatic
     int attention_waves = 0;
     int attention_chunk = 0;
 };
@@ -344,6 +345,18 @@ int launch_sddmm_tile(int shape, int m_vec, int k, int n, const int *row_offsets
 int spmm_tile_choice(bool fine_grained, int m_vec, int k, int n, int vec_length, const Batch &batch);
 int launch_spmm_tile(int shape, int m_vec, int vec_length, int k, int n, const int *row_offsets, const int *col_indices,
                      const half_t *values, const half_t *rhs, half_t *out, hipStream_t stream, const Batch &batch);
+
+// What the two kinds of kernels are expected to take (microseconds): gathering, and the one of them that is run.
+double spmm_gather_us(bool fine_grained, int vec_length, double nonzeros_vec, int k);
+double spmm_expected_us(bool fine_grained, int m_vec, int k, int n, int vec_length, int nonzeros_vec, int longest_vec);
+
+// SpMM on rows packed two of four (csrc/spmm_pack.hip), for columns that ascend strictly.  spmm_packed_choice: 0 = other
+// kernels are expected to be faster (or have to take the call), else the `shape` for launch_spmm_packed (1 = tiles of
+// 256 x 128, 2 = 128 x 128), which takes a workspace of spmm_packed_bytes, 16-byte aligned, uninitialised.
+int spmm_packed_choice(bool fine_grained, int m_vec, int k, int n, int vec_length, int nonzeros_vec, int longest_row_vec);
+long long spmm_packed_bytes(int m_vec, int vec_length, int n, int nonzeros_vec);
+int launch_spmm_packed(int shape, int m_vec, int vec_length, int k, int n, int nonzeros_vec, const int *row_offsets,
+                       const int *col_indices, const half_t *values, const half_t *rhs, half_t *out, void *workspace, hipStream_t stream);
 
 // Writes `bytes` zero bytes to each of `batch` buffers `stride_bytes` apart (a kernel, not a memset node, so that
 // callers may capture the call into a HIP graph).

@@ -427,6 +427,31 @@ int vs_cuda_spmm_f16_ascending(int m_vec, int vec_length, int k, int n, int nonz
                                         ascending(nonzeros_vec, longest_row_vec, row_length_hints, -1));
 }
 
+long long vs_spmm_packed_workspace_bytes(int fine_grained, int m_vec, int vec_length, int k, int n, int nonzeros_vec, int longest_row_vec)
+{
+    if (!vec_ok(vec_length)) return 0;
+    const int shape = vs::spmm_packed_choice(fine_grained != 0, m_vec, k, n, vec_length, nonzeros_vec, longest_row_vec);
+    return shape ? vs::spmm_packed_bytes(m_vec, vec_length, n, nonzeros_vec) : 0;
+}
+
+int vs_spmm_f16_packed(int fine_grained, int m_vec, int vec_length, int k, int n, int nonzeros_vec, int longest_row_vec,
+                       const int *row_offsets, const int *column_indices, const void *values, const void *rhs_matrix,
+                       void *output_matrix, void *workspace, long long workspace_bytes, void *stream)
+{
+    int st = check_spmm(m_vec, vec_length, k, n, row_offsets, row_offsets, column_indices, values, rhs_matrix,
+                        output_matrix, sizeof(half_t));
+    if (st != VS_SUCCESS) return st;
+    if (m_vec == 0 || k == 0) return VS_SUCCESS;
+    const int shape = vs::spmm_packed_choice(fine_grained != 0, m_vec, k, n, vec_length, nonzeros_vec, longest_row_vec);
+    if (shape == 0) return VS_ERROR_NOT_SUPPORTED;
+    if (!column_indices || !values || !workspace || !aligned(workspace, 16) ||
+        workspace_bytes < vs::spmm_packed_bytes(m_vec, vec_length, n, nonzeros_vec))
+        return VS_ERROR_INVALID_VALUE;
+    return vs::launch_spmm_packed(shape, m_vec, vec_length, k, n, nonzeros_vec, row_offsets, column_indices,
+                                  static_cast<const half_t *>(values), static_cast<const half_t *>(rhs_matrix),
+                                  static_cast<half_t *>(output_matrix), workspace, static_cast<hipStream_t>(stream));
+}
+
 int vs_wmma_spmm_launch_shape(int batch, int m_vec, int vec_length, int k, int n, int nonzeros_vec,
                               int longest_row_vec, int long_rows, int shape[8])
 {
@@ -900,6 +925,9 @@ static int set_option_field(vs::Options &o, const char *name, int value)
     } else if (std::strcmp(name, "spmm_tile") == 0) {
         if (value > 4) return VS_ERROR_INVALID_VALUE;
         o.spmm_tile = value;
+    } else if (std::strcmp(name, "spmm_packed") == 0) {
+        if (value < 0 || value > 3) return VS_ERROR_INVALID_VALUE;
+        o.spmm_packed = value;
     } else if (std::strcmp(name, "sddmm_flat_supers") == 0) {
         if (value > 16) return VS_ERROR_INVALID_VALUE;
         o.sddmm_flat_supers = value;

@@ -185,6 +185,11 @@ def spmm_split_rows(m_vec, vec_length, k, n, nonzeros_vec, row_offsets, column_i
     return output_matrix
 
 
+def spmm_packed_workspace_bytes(m_vec, vec_length, k, n, nonzeros_vec, longest_row_vec, fine_grained=False):
+    """Workspace of the SpMM on packed rows (vs_spmm_f16_packed); 0 where other kernels are expected to be faster."""
+    return int(_lib.lib().vs_spmm_packed_workspace_bytes(int(fine_grained), m_vec, vec_length, k, n, nonzeros_vec, longest_row_vec))
+
+
 def spmm_slab_workspace_bytes(m_vec, vec_length, k, n):
     """Workspace `spmm_slab` needs for this shape under the current "spmm_slab_parts" option (0: none)."""
     return int(_lib.lib().vs_wmma_spmm_slab_workspace_bytes(m_vec, vec_length, k, n))
@@ -1053,7 +1058,13 @@ class DeviceProblem:
         if self.columns_distinct and out.dtype == torch.float16:
             st = _native.spmm_ascending(kernel != "wmma", self.m_vec, self.vec_length, k, self.n, self.nnz_vec, self.longest_row_vec,
                                         self.long_rows, bool(row_length_hint), self.row_indices, self.row_offsets,
-                                        self.column_indices, self.values, rhs_matrix, out, stream)
+                                        self.column_indices, self.values, rhs_matrix, out, stream, True)
+            if st == -2:
+                st = self._spmm_packed(rhs_matrix, kernel != "wmma", out, stream)
+                if st is None:
+                    st = _native.spmm_ascending(kernel != "wmma", self.m_vec, self.vec_length, k, self.n, self.nnz_vec, self.longest_row_vec,
+                                                self.long_rows, bool(row_length_hint), self.row_indices, self.row_offsets,
+                                                self.column_indices, self.values, rhs_matrix, out, stream, False)
             if st >= 0:
                 if st:
                     _lib.check(st, "vs_%s_spmm_f16%s" % ("wmma" if kernel == "wmma" else "cuda", "_batched" if row_length_hint else ""))
@@ -1066,6 +1077,22 @@ class DeviceProblem:
         fn = spmm.wmmaSpmm if kernel == "wmma" else spmm.cudaSpmm
         return fn(self.m_vec, self.vec_length, k, self.n, self.row_indices, self.row_offsets,
                   self.column_indices, self.values, rhs_matrix, out, stream)
+
+    def _spmm_packed(self, rhs_matrix, fine_grained, out, stream):
+        """vs_spmm_f16_packed with a workspace made for the call, in memory of the stream that uses it; None where there is no
+        room for one, and inside a capture (replays would find the workspace given back to the allocator unless torch itself
+        runs the capture)."""
+        k = rhs_matrix.shape[1]
+        need = spmm_packed_workspace_bytes(self.m_vec, self.vec_length, k, self.n, self.nnz_vec, self.longest_row_vec, fine_grained)
+        with contextlib.nullcontext() if stream is None else torch.cuda.stream(_as_stream(stream)):
+            if torch.cuda.is_current_stream_capturing():
+                return None
+            try:
+                workspace = torch.empty(need, dtype=torch.uint8, device=rhs_matrix.device)
+            except torch.cuda.OutOfMemoryError:
+                return None
+        return _native.spmm_packed(fine_grained, self.m_vec, self.vec_length, k, self.n, self.nnz_vec, self.longest_row_vec, self.row_offsets,
+                                   self.column_indices, self.values, rhs_matrix, out, workspace, stream)
 
     def sddmm_row_parts(self, lhs_matrix, rhs_matrix, out=None, stream=None, limit_vec=256):
         """SDDMM (MFMA path, fp16 output, k % 8 == 0) with long rows of the mask dispatched as several parts.  The
