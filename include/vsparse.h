@@ -482,6 +482,20 @@ int vs_wmma_softmax_spmm_f16_batched(int batch, int m_vec, int vec_length, int k
                                      float scale, void *stream);
 
 /*
+ * A fixed-mask attention layer in one launch, a workgroup per vector row, for d_qk = d_v = 64 or 128:
+ * out[b] = softmax_row(scale * mask(q[b] k[b]^T)) v[b], and, where `probabilities` ([batch][nonzeros_vec][vec_length]) is not null, the
+ * probabilities rounded to fp16, which are what v is multiplied by.  row_indices: a permutation of the vector rows.  Rows of more
+ * than longest_row_vec nonzero vectors are correct, and slow.  q, k, v, out: 16-byte aligned, strides in elements (0: shared inputs)
+ * and multiples of 8; problems that share outputs are refused.  Returns VS_ERROR_NOT_SUPPORTED for other widths, n * d_v >= 2^30,
+ * rows of more than 512 vectors and where two launches (SDDMM, softmax and SpMM) are expected to be faster (option "attention_rows").
+ * No counterpart in the reference.
+ */
+int vs_sparse_attention_rows_f16(int batch, int m_vec, int vec_length, int n, int d_qk, int d_v, int nonzeros_vec, int longest_row_vec,
+                                 const int *row_indices, const int *row_offsets, const int *col_indices, const void *q,
+                                 long long stride_q, const void *k, long long stride_k, const void *v, long long stride_v, void *out,
+                                 long long stride_out, void *probabilities, long long stride_probabilities, float scale, void *stream);
+
+/*
  * One fixed-mask sparse attention layer in a single launch:
  *     out[b] = softmax_row(scale * (q[b] k[b]^T sampled on the mask)) v[b]
  * q: [m_vec*vec_length, d_qk], k: [n, d_qk], v: [n, d_v], out: [m_vec*vec_length, d_v], all fp16
@@ -636,7 +650,8 @@ int vs_wmma_spmm_launch_shape(int batch, int m_vec, int vec_length, int k, int n
  * 0 = where expected to be faster),
  * "sddmm_tile" (SDDMM on dense tiles, k % 8 == 0, any order of the columns: 1 = never, 2 = tiles of 64 x 64,
  * 3 = of 128 x 128, 0 = where the columns are known to ascend and tiles are expected to be faster than gathering rows),
- * "attention_waves" (1..8, 0 = automatic), "attention_chunk" (nonzero vectors per
+ * "attention_rows" (attention with a workgroup per vector row in one launch: 1 = never, 2 .. 5 = with 1, 2, 4 or 8 waves, 0 =
+ * automatic), "attention_waves" (1..8, 0 = automatic), "attention_chunk" (nonzero vectors per
  * LDS chunk of the one-row-per-workgroup attention kernel, 0 = automatic).
  * Returns 0, or 1 for an unknown name / bad value.
  * No counterpart in the reference, whose tile sizes are compile-time constants

@@ -45,6 +45,7 @@ SIGNATURES = {
                                          _int),
     "vs_wmma_softmax_spmm_f16_batched": ([_int] * 7 + [_vp] * 3 + [_vp, _ll, _vp, _ll, _vp, _ll, ctypes.c_float, _vp],
                                          _int),
+    "vs_sparse_attention_rows_f16": ([_int] * 8 + [_vp] * 3 + [_vp, _ll] * 5 + [ctypes.c_float, _vp], _int),
     "vs_sparse_attention_f16": ([_int] * 6 + [_vp] * 3 + [_vp, _ll, _vp, _ll, _vp, _ll, _vp, _ll, ctypes.c_float, _int,
                                  _vp, _ll, _vp],
                                 _int),

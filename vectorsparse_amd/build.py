@@ -11,7 +11,7 @@ CSRC = os.path.join(_HERE, "csrc")
 LIB_PATH = os.path.join(_HERE, "libvsparse.so")
 OBJ_DIR = os.path.join(_HERE, "build")
 SOURCES = ["vsparse_api.hip", "spmm_mfma.hip", "spmm_mfma_flat.hip", "spmm_mfma_slab.hip", "spmm_valu.hip", "spmm_tile.hip", "spmm_pack.hip", "sddmm_mfma.hip", "sddmm_valu.hip", "sddmm_tile.hip",
-           "sparse_softmax.hip", "sparse_attention.hip",
+           "sparse_softmax.hip", "sparse_attention.hip", "sparse_attention_rows.hip",
            "sparse_attention_union.hip"]
 # VS_RETIRED_VARIANTS=1 in the environment also compiles the two SpMM variants that measured slower on every shape
 # and are therefore not part of the default library: the LDS-DMA gather (spmm_mfma_dma.hip, option spmm_gather = 2)

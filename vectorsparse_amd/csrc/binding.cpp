@@ -323,6 +323,27 @@ PyObject *spmm_softmax_batched(PyObject *, PyObject *const *args, Py_ssize_t n_a
     });
 }
 
+// (batch, m_vec, vec_length, n, d_qk, d_v, nonzeros_vec, longest_row_vec, row_indices, row_offsets, col_indices, q, k, v, out,
+// probabilities or None, scale, stream)
+PyObject *sparse_attention_rows(PyObject *, PyObject *const *args, Py_ssize_t n_args)
+{
+    Reader r(args, n_args);
+    const int batch = r.integer(), m_vec = r.integer(), vec = r.integer(), n = r.integer(), d_qk = r.integer(), d_v = r.integer();
+    const int nnz = r.integer(), longest = r.integer();
+    const int *ri = (const int *)r.indices(), *ro = (const int *)r.indices(), *ci = (const int *)r.indices();
+    long long sq, sk, sv, so, sp = 0;
+    const void *q = r.batched(batch, sq), *k = r.batched(batch, sk), *v = r.batched(batch, sv);
+    void *out = r.batched_output(batch, so), *probabilities = nullptr;
+    if (r.ok && r.left > 0 && *r.args == Py_None) r.next();
+    else probabilities = r.batched_in_place(batch, sp);
+    const float scale = r.number();
+    void *stream = r.stream();
+    return status_of(r, [&] {
+        return vs_sparse_attention_rows_f16(batch, m_vec, vec, n, d_qk, d_v, nnz, longest, ri, ro, ci, q, sq, k, sk, v, sv, out, so,
+                                            probabilities, sp, scale, stream);
+    });
+}
+
 // (batch, m_vec, k, n, nonzeros_vec, row_indices, row_offsets, col_indices, lhs, rhs, out, vec_length, stream, columns_sorted)
 // and, MFMA path, (..., algorithm)
 template <bool MFMA>
@@ -486,6 +507,7 @@ PyMethodDef methods[] = {
     VS_METHOD("cuda_sddmm_batched", sddmm_batched<false>),
     VS_METHOD("sparse_softmax", sparse_softmax),
     VS_METHOD("sparse_attention", sparse_attention),
+    VS_METHOD("sparse_attention_rows", sparse_attention_rows),
     VS_METHOD("sparse_attention_split", sparse_attention_split),
     VS_METHOD("spmm_row_parts", spmm_row_parts),
     VS_METHOD("sddmm_row_parts", sddmm_row_parts),

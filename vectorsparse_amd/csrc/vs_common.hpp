@@ -254,6 +254,7 @@ struct Options {
     int softmax_spmm = 0;       // softmax and SpMM that keeps the probabilities: 1 = one launch, 2 = two, 0 = automatic
     int spmm_tile = 0;          // SpMM on dense tiles: 1 = never, 2 / 3 / 4 = tiles of 32 x 64, 64 x 128, 128 x 128, 0 = automatic
     int spmm_packed = 0;        // SpMM on rows packed two of four: 1 = never, 2 / 3 = tiles of 256 x 128, 128 x 128, 0 = automatic
+    int attention_rows = 0;     // attention with a workgroup per vector row in one launch: 1 = never, 2 .. 5 = with 1, 2, 4, 8 waves, 0 = automatic
     int attention_waves = 0;
     int attention_chunk = 0;
 };
@@ -357,6 +358,14 @@ int spmm_packed_choice(bool fine_grained, int m_vec, int k, int n, int vec_lengt
 long long spmm_packed_bytes(int m_vec, int vec_length, int n, int nonzeros_vec);
 int launch_spmm_packed(int shape, int m_vec, int vec_length, int k, int n, int nonzeros_vec, const int *row_offsets,
                        const int *col_indices, const half_t *values, const half_t *rhs, half_t *out, void *workspace, hipStream_t stream);
+
+// A sparse attention layer in one launch, a workgroup per vector row (csrc/sparse_attention_rows.hip); `kept`: the probabilities,
+// where wanted.  attention_rows_waves: 0 = other routes take it, else the waves for launch_attention_rows.
+int attention_rows_waves(bool keep, int heads, int m_vec, int n, int vec_length, int d_qk, int d_v, int nonzeros_vec, int longest_row_vec);
+int launch_attention_rows(int waves, bool keep, int m_vec, int vec_length, int n, int d, const int *row_indices, const int *row_offsets,
+                          const int *col_indices, const half_t *q, const half_t *k, const half_t *v, half_t *out, half_t *kept, float scale,
+                          long long stride_q, long long stride_k, long long stride_v, long long stride_out, long long stride_kept, int heads,
+                          hipStream_t stream);
 
 // Writes `bytes` zero bytes to each of `batch` buffers `stride_bytes` apart (a kernel, not a memset node, so that
 // callers may capture the call into a HIP graph).

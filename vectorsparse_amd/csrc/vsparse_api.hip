@@ -574,6 +574,31 @@ int vs_wmma_softmax_spmm_f16_batched(int batch, int m_vec, int vec_length, int k
                                         make_batch(batch, stride_values, stride_rhs, stride_output, nonzeros_vec, longest_row_vec));
 }
 
+int vs_sparse_attention_rows_f16(int batch, int m_vec, int vec_length, int n, int d_qk, int d_v, int nonzeros_vec, int longest_row_vec,
+                                 const int *row_indices, const int *row_offsets, const int *col_indices, const void *q,
+                                 long long stride_q, const void *k, long long stride_k, const void *v, long long stride_v, void *out,
+                                 long long stride_out, void *probabilities, long long stride_probabilities, float scale, void *stream)
+{
+    if (batch < 0 || m_vec < 0 || n < 0 || nonzeros_vec < 0 || !vec_ok(vec_length)) return VS_ERROR_INVALID_VALUE;
+    if (m_vec == 0 || batch == 0) return VS_SUCCESS;
+    const int waves = vs::attention_rows_waves(probabilities != nullptr, batch, m_vec, n, vec_length, d_qk, d_v, nonzeros_vec, longest_row_vec);
+    if (waves == 0) return VS_ERROR_NOT_SUPPORTED;
+    if (!row_indices || !row_offsets || !col_indices || !q || !k || !v || !out) return VS_ERROR_INVALID_VALUE;
+    if (!aligned(q, 16) || !aligned(k, 16) || !aligned(v, 16) || !aligned(out, 16) || !aligned(probabilities, 2 * (size_t)vec_length))
+        return VS_ERROR_INVALID_VALUE;
+    if (!stride_ok(stride_q, 8) || !stride_ok(stride_k, 8) || !stride_ok(stride_v, 8) || !stride_ok(stride_out, 8) ||
+        !stride_ok(stride_probabilities, vec_length))
+        return VS_ERROR_INVALID_VALUE;
+    // (what is written: no two problems may share an element)
+    if (batch > 1 && (stride_out < (long long)m_vec * vec_length * d_v ||
+                      (probabilities && stride_probabilities < (long long)nonzeros_vec * vec_length)))
+        return VS_ERROR_INVALID_VALUE;
+    return vs::launch_attention_rows(waves, probabilities != nullptr, m_vec, vec_length, n, d_v, row_indices, row_offsets, col_indices,
+                                     static_cast<const half_t *>(q), static_cast<const half_t *>(k), static_cast<const half_t *>(v),
+                                     static_cast<half_t *>(out), static_cast<half_t *>(probabilities), scale, stride_q, stride_k, stride_v,
+                                     stride_out, stride_probabilities, batch, static_cast<hipStream_t>(stream));
+}
+
 int vs_sparse_attention_f16(int batch, int m_vec, int vec_length, int n, int d_qk, int d_v, const int *row_indices,
                             const int *row_offsets, const int *col_indices, const void *q, long long stride_q,
                             const void *k, long long stride_k, const void *v, long long stride_v, void *out,
@@ -937,6 +962,9 @@ static int set_option_field(vs::Options &o, const char *name, int value)
     } else if (std::strcmp(name, "sddmm_block_waves") == 0) {
         if (value > 16) return VS_ERROR_INVALID_VALUE;
         o.sddmm_block_waves = value;
+    } else if (std::strcmp(name, "attention_rows") == 0) {
+        if (value < 0 || value > 5) return VS_ERROR_INVALID_VALUE;
+        o.attention_rows = value;
     } else if (std::strcmp(name, "attention_waves") == 0) {
         if (value > 8) return VS_ERROR_INVALID_VALUE;
         o.attention_waves = value;
