@@ -746,36 +746,30 @@ sparse_attention_union_kernel(int m_vec, int n, int d_qk, int d_v, int u_max,
     }
 }
 
-// Planned launches of eight waves stream the union through LDS in sub-rounds of kStreamRanks ranks, K rows
-// and V columns side by side: the rows, row masks and column numbers of the NEXT sub-round are requested
-// before the current one is computed and parked in registers meanwhile, so after the first sub-round no wave
-// waits for a gather.  A sub-round is short enough to keep its raw scores in registers: the K rows are read
+// Planned launches of eight waves stream the union through LDS in sub-rounds of kStreamRanks ranks, K and V rows side by side, in
+// two buffers: the rows and row masks of the NEXT sub-round are copied there without registers while the current one is
+// computed, a barrier per sub-round.  A sub-round is short enough to keep its raw scores in registers: the K rows are read
 // and multiplied once, not twice.  Maximum and sums run across the sub-rounds as in flash attention, so a
 // workgroup takes unions of up to kStreamRounds * kStreamRanks columns.
 //
-// The kernel is bound by vector-ALU instructions (softmax arithmetic and operand shuffles), so two things
-// are kept out of the waves' inner loop.  The V rows of a sub-round go to LDS transposed, in the order the
-// P V MFMA wants its B operand - the transposition is done once per workgroup while the rows are written, not
-// once per wave while they are read.  And the mask enters the scores as the accumulators' start value (0 or
-// -inf), so neither the maximum nor the exponentials look at it again.
-constexpr int kStreamVPitch = kStreamRanks + 8;  // halves between consecutive V columns in LDS
+// V rows lie in LDS as they are; transposing reads hand the P V MFMA its B operand.  And the mask enters the scores as the
+// accumulators' start value (0 or -inf), so neither the maximum nor the exponentials look at it again.
+//
+// What bounds it (16 heads x 4096, V = 8, width 64, a +-128 band and every 128th column: 17.3 us a pass): vector ALU (half of it the
+// exponentials) and the phases of a wave, one after the other.  Through registers, V transposed on its way to LDS, two barriers per
+// sub-round: 19.1 us; copied, with the start values and maxima as the compiler makes them of selects and fmaxf (three and two
+// instructions instead of two and one): 18.3 us.
 typedef int int2_t __attribute__((ext_vector_type(2)));
 
-// Where rank r of a sub-round sits inside a V column: lane (c, g) multiplies ranks 16u + 4g + e (u < 2,
-// e < 4) of a 32-rank step, which this order puts into 16 consecutive bytes.
-__device__ __forceinline__ int stream_v_slot(int r) { return (r & ~31) | (((r >> 2) & 3) << 3) | (((r >> 4) & 1) << 2) | (r & 3); }
-
-// First rank of pair `pair` (0 .. kStreamRanks / 2) in the order the threads take them: consecutive pairs differ
-// in the bits that choose the 32-bit word inside a 16-byte chunk (e bit 1, then u), so the 32 lanes of a
-// transposed write hit 32 different banks.
-__device__ __forceinline__ int stream_v_pair_rank(int pair)
-{
-    return ((pair & 1) << 1) | (((pair >> 1) & 1) << 4) | (((pair >> 2) & 3) << 2) | ((pair >> 4) << 5);
-}
-
-// Offset in halves of 8-rank chunk `chunk` of V column `col`; chunks are permuted by column so that neither
-// the transposed writes (lanes of a quad: columns 8 apart) nor the reads (lanes: columns CPL apart) collide.
-__device__ __forceinline__ int stream_v_offset(int col, int chunk) { return col * kStreamVPitch + ((chunk ^ ((col >> 3) & 7)) << 3); }
+// A row of K is 4 KS pieces of 16 bytes, piece p of row r at place p ^ stream_k_turn(r): sixteen lanes that read one piece of
+// sixteen rows touch every bank once.  A row of V is CPL pieces of 32 bytes, the same way for transposing reads of eight rows.
+template <int KS>
+__device__ __forceinline__ int stream_k_turn(int r) { return KS == 1 ? (r >> 2) & 3 : (KS == 2 ? (r >> 1) & 7 : r & 15); }
+template <int CPL>
+__device__ __forceinline__ int stream_v_turn(int r) { return CPL == 4 ? (r >> 1) & 3 : r & 7; }
+// (a NaN stays one, which spares the two instructions per operand that would quiet it)
+__device__ __forceinline__ float highest(float x, float y, float z) { return __builtin_elementwise_maximum(__builtin_elementwise_maximum(x, y), z); }
+constexpr int stream_buffer_bytes(int rows, int ks, int cpl) { return rows * kStreamSteps * 4 + kStreamRanks * (64 * ks + 32 * cpl); }
 
 // The per-row path as a function of its own: inlined into the streamed kernel it takes every register the launch
 // bounds leave, and the allocator then parks values of the streamed path in scratch memory around it.
@@ -810,25 +804,21 @@ sparse_attention_stream_kernel(int m_vec, int n, int d_qk, int d_v,
     v += blockIdx.y * stride_v;
     out += blockIdx.y * stride_out;
     constexpr int RPW = 16 / V;
-    constexpr int PITCH = 32 * KS + 8;                              // halves between consecutive K rows in LDS
     constexpr int kRounds = SPLIT ? kSplitRounds : kStreamRounds;
     constexpr int SS = kStreamSteps;
     constexpr int SR = kStreamRanks;
-    constexpr int kThreads = 512;
     constexpr int kRows = 8 * RPW;                                  // vector rows per workgroup
     constexpr int kMaskWords = (kRows * SS + 3) & ~3;               // the plan's words per round: [kRows][SS]
-    constexpr int kShiftK = KS == 1 ? 2 : (KS == 2 ? 3 : 4);        // 4 * KS slices of 8 halves per K row
-    constexpr int kShiftV = CPL == 4 ? 3 : 4;                       // 2 * CPL slices per V row
-    constexpr int NK = (SR << kShiftK) / kThreads;                  // 16-byte slices per thread and sub-round
-    constexpr int NV = ((SR / 2) << kShiftV) / kThreads;            // pairs of V slices (two consecutive ranks)
+    // LDS, twice: [kRows][SS] masks of a sub-round, [SR] rows of K, [SR] rows of V
+    constexpr int kRowK = 64 * KS, kRowV = 32 * CPL, kAtK = kRows * SS * 4, kAtV = kAtK + SR * kRowK, kBuffer = kAtV + SR * kRowV;
+    constexpr int NK = SR * kRowK / 8192, NV = SR * kRowV / 8192;   // requests of 1 KB per wave and sub-round
+    constexpr int kEachK = 1024 / kRowK, kEachV = 1024 / kRowV;     // rows of a request
+    static_assert(kBuffer == stream_buffer_bytes(kRows, KS, CPL) && kAtK % 256 == 0 && kAtK <= 2048, "");
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     extern __shared__ __align__(16) unsigned char smem[];
-    unsigned *maskbuf = reinterpret_cast<unsigned *>(smem);        // [kRows][SS] masks of the sub-round in LDS
-    half_t *kbuf = reinterpret_cast<half_t *>(maskbuf + kRows * SS);  // [SR][PITCH]
-    half_t *vbuf = kbuf + SR * PITCH;                                 // [16 * CPL columns][kStreamVPitch]
 
     int bx = blockIdx.x, first_round = 0, end_round = kRounds, partial = -1;
     if constexpr (SPLIT) {
@@ -855,87 +845,46 @@ sparse_attention_stream_kernel(int m_vec, int n, int d_qk, int d_v,
     const int *rec = plan + kPlanHeader + (size_t)(plan_ok ? bx : 0) * stride;
     const int n_union = plan_ok ? rec[0] : 0x7fffffff;
     // The record, the K rows and the V rows are read through buffer descriptors: a scalar base and one 32-bit byte
-    // offset per thread and load, where a 64-bit pointer per thread and load used to take the registers that the
+    // offset per thread and request, where a 64-bit pointer per thread takes the registers that the
     // launch bounds do not leave (n <= 2^20 columns of at most 128 halves: every offset is below 2^28).
     const __amdgpu_buffer_rsrc_t rec_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<int *>(rec), 0, 4 * stride, 0x00020000);
-    const __amdgpu_buffer_rsrc_t k_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t *>(k), 0, 0x7fffffff, 0x00020000);
-    const __amdgpu_buffer_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t *>(v), 0, 0x7fffffff, 0x00020000);
+    const uint4_t rec_from = buffer_of(rec, 4 * stride), k_from = buffer_of(k, 0x7fffffffu), v_from = buffer_of(v, 0x7fffffffu);
     constexpr unsigned kMasksAt = 4u * 4u;                                        // byte offsets inside the record
     constexpr unsigned kColsAt = 4u * (4u + kRounds * kMaskWords);
+    const unsigned lds = (unsigned)(uintptr_t)(__attribute__((address_space(3))) void *)smem;
 
-    // What a thread fetches per sub-round: NK slices of K rows (thread t takes slices t, t + 512, ...:
-    // consecutive threads read consecutive 16 bytes of a row), NV times the same slice of the V rows of two
-    // consecutive ranks, and one mask word.
-    int col_k[NK];
-    int2_t col_v[NV];
-    uint4_t stage_k[NK], stage_v[NV][2];
-    unsigned stage_m = 0;
+    // a lane's rows of the wave's requests, and their column numbers
+    auto row_k = [&](int i) { return (wave * NK + i) * kEachK + lane / (64 / kEachK); };
+    auto row_v = [&](int i) { return (wave * NV + i) * kEachV + lane / (64 / kEachV); };
+    int col_k[NK], col_v[NV];
     // column numbers of sub-round `round` < kRounds (the plan lists 0 past the union: row 0, unused), which
     // do not wait for the union's size
     auto fetch_cols = [&](int round) {
         const unsigned at = kColsAt + 4u * (unsigned)(round * SR);  // (uniform)
 #pragma unroll
-        for (int i = 0; i < NK; ++i)
-            col_k[i] = (int)__builtin_amdgcn_raw_buffer_load_b32(rec_rsrc, 4u * ((unsigned)(tid + i * kThreads) >> kShiftK), at, 0);
+        for (int i = 0; i < NK; ++i) col_k[i] = (int)__builtin_amdgcn_raw_buffer_load_b32(rec_rsrc, 4u * (unsigned)row_k(i), at, 0);
 #pragma unroll
         for (int i = 0; i < NV; ++i)
-            col_v[i] = __builtin_bit_cast(int2_t, __builtin_amdgcn_raw_buffer_load_b64(
-                rec_rsrc, 4u * (unsigned)stream_v_pair_rank((tid + i * kThreads) >> kShiftV), at, 0));
+            col_v[i] = NK == NV ? col_k[i < NK ? i : 0] : (int)__builtin_amdgcn_raw_buffer_load_b32(rec_rsrc, 4u * (unsigned)row_v(i), at, 0);
     };
-    // Requests only: nothing here reads what the loads return, so the wave goes on to the arithmetic at once.
-    // Slices past the union or past d read the start of a valid row and are replaced by zeros in commit().
-    auto fetch_rows = [&](int round) {  // needs col_k / col_v of the same sub-round
+    // Rows past the union and slices past d are out of the buffer's range, which makes them zeros: the arithmetic never meets
+    // stale bits.
+    auto request_rows = [&](int round) {  // needs col_k / col_v of the same sub-round
+        const unsigned to = lds + (unsigned)((round & 1) * kBuffer);
+        if (wave < kAtK / 256)
+            request_to_lds<4>(to + wave * 256, rec_from, (unsigned)(tid * 4), kMasksAt + 4u * (unsigned)(round * kMaskWords));
 #pragma unroll
         for (int i = 0; i < NK; ++i) {
-            const int sidx = tid + i * kThreads;
-            const int u = round * SR + (sidx >> kShiftK), sl = sidx & ((1 << kShiftK) - 1);
-            const bool real = u < n_union && 8 * sl < d_qk;
-            stage_k[i] = __builtin_amdgcn_raw_buffer_load_b128(k_rsrc, 2u * ((unsigned)col_k[i] * (unsigned)d_qk + (real ? 8u * sl : 0u)), 0, 0);
+            const int row = row_k(i), piece = (lane % (64 / kEachK)) ^ stream_k_turn<KS>(row);
+            const bool real = round * SR + row < n_union && 8 * piece < d_qk;
+            request_to_lds<16>(to + kAtK + (wave * NK + i) * 1024, k_from, real ? 2u * ((unsigned)col_k[i] * (unsigned)d_qk + 8u * piece) : 0x80000000u, 0u);
         }
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
-            const int sidx = tid + i * kThreads;
-            const int u = round * SR + stream_v_pair_rank(sidx >> kShiftV), sl = sidx & ((1 << kShiftV) - 1);
-            const unsigned off = (u < n_union && 8 * sl < d_v) ? 8u * sl : 0u;
-            stage_v[i][0] = __builtin_amdgcn_raw_buffer_load_b128(v_rsrc, 2u * ((unsigned)col_v[i][0] * (unsigned)d_v + off), 0, 0);
-            stage_v[i][1] = __builtin_amdgcn_raw_buffer_load_b128(v_rsrc, 2u * ((unsigned)col_v[i][1] * (unsigned)d_v + off), 0, 0);
+            const int row = row_v(i), place = lane % (64 / kEachV), piece = 2 * ((place >> 1) ^ stream_v_turn<CPL>(row)) + (place & 1);
+            const bool real = round * SR + row < n_union && 8 * piece < d_v;
+            request_to_lds<16>(to + kAtV + (wave * NV + i) * 1024, v_from, real ? 2u * ((unsigned)col_v[i] * (unsigned)d_v + 8u * piece) : 0x80000000u, 0u);
         }
-        if (tid < kRows * SS) {
-            // (the offset is made anew in every sub-round: kept across the loop it is the one value the register
-            // allocator parks in scratch memory, and its reload waits for every gather requested just above)
-            unsigned word = (unsigned)tid;
-            asm volatile("" : "+v"(word));
-            stage_m = __builtin_amdgcn_raw_buffer_load_b32(rec_rsrc, 4u * word, kMasksAt + 4u * (unsigned)(round * kMaskWords), 0);
-        }
-    };
-    // The parked sub-round `round` into LDS; rows past the union and slices past d as zeros, so the arithmetic
-    // never meets stale bits.  V goes in transposed: a thread holds 8 columns of two consecutive ranks and
-    // writes, per column, the two ranks as one 32-bit word.
-    auto commit = [&](int round) {
-        const uint4_t zero = {0u, 0u, 0u, 0u};
-#pragma unroll
-        for (int i = 0; i < NK; ++i) {
-            const int sidx = tid + i * kThreads;
-            const int u = sidx >> kShiftK, sl = sidx & ((1 << kShiftK) - 1);
-            const bool real = round * SR + u < n_union && 8 * sl < d_qk;
-            *reinterpret_cast<uint4_t *>(kbuf + u * PITCH + 8 * sl) = real ? stage_k[i] : zero;
-        }
-#pragma unroll
-        for (int i = 0; i < NV; ++i) {
-            const int sidx = tid + i * kThreads;
-            const int r0 = stream_v_pair_rank(sidx >> kShiftV), sl = sidx & ((1 << kShiftV) - 1);
-            const bool wide_enough = 8 * sl < d_v;
-            const uint4_t first = (wide_enough && round * SR + r0 < n_union) ? stage_v[i][0] : zero;
-            const uint4_t second = (wide_enough && round * SR + r0 + 1 < n_union) ? stage_v[i][1] : zero;
-            const int slot = stream_v_slot(r0);
-            half_t *dst = vbuf + stream_v_offset(8 * sl, slot >> 3) + (slot & 7);  // columns 8 sl .. 8 sl + 7 share their chunk order
-#pragma unroll
-            for (int jj = 0; jj < 4; ++jj) {
-                *reinterpret_cast<uint32_t *>(dst + (2 * jj) * kStreamVPitch) = pack_lo(first[jj], second[jj]);
-                *reinterpret_cast<uint32_t *>(dst + (2 * jj + 1) * kStreamVPitch) = pack_hi(first[jj], second[jj]);
-            }
-        }
-        if (tid < kRows * SS) maskbuf[tid] = stage_m;
     };
 
     // requested together with the union's size (a record ends with sub-round kRounds - 1; slots that start behind it belong to
@@ -953,7 +902,7 @@ sparse_attention_stream_kernel(int m_vec, int n, int d_qk, int d_v,
     const long long q_limit = (long long)row_last * V;
     half8_t qb[KS];
     load_q16<KS>(qb, q, q_global, q_limit, d_qk, c, g);
-    if (n_rounds > first_round) fetch_rows(first_round);
+    if (n_rounds > first_round) request_rows(first_round);
     if (n_rounds > first_round + 1) fetch_cols(first_round + 1);
     // The maximum is tracked on raw dot products and masked-out pairs are -inf before the scale is applied, so
     // the scale the exponentials see must be positive: a negative one moves into Q, a zero one becomes Q = 0
@@ -973,8 +922,11 @@ sparse_attention_stream_kernel(int m_vec, int n, int d_qk, int d_v,
             qb[kk] = __builtin_bit_cast(half8_t, bits);
         }
     }
-    const unsigned *mrow = maskbuf + ((q_first + c) / V) * SS;
-    const half_t *k_lane = kbuf + c * PITCH + 8 * g;
+    const unsigned mask_at = (unsigned)((q_first + c) / V) * SS * 4, v_at = (unsigned)(kAtV + (4 * g + (c >> 2)) * kRowV + 8 * (c & 3));
+    unsigned k_at[KS];
+#pragma unroll
+    for (int kk = 0; kk < KS; ++kk) k_at[kk] = (unsigned)(kAtK + c * kRowK + 16 * ((4 * kk + g) ^ stream_k_turn<KS>(c)));
+    const int v_turn = stream_v_turn<CPL>(4 * g + (c >> 2));
     const float neg_inf = -__builtin_inff();
     constexpr unsigned kLaneBits = 0x000F000Fu;
     const half8_t ones = {1, 1, 1, 1, 1, 1, 1, 1};
@@ -985,11 +937,15 @@ sparse_attention_stream_kernel(int m_vec, int n, int d_qk, int d_v,
     float mx_run = neg_inf;
 
     for (int round = first_round; round < n_rounds; ++round) {
-        if (round > first_round) __syncthreads();  // every wave is done with the previous sub-round's rows and masks
-        commit(round);
-        __syncthreads();
-        if (round + 1 < n_rounds) fetch_rows(round + 1);  // in flight during the arithmetic below
+        // the wave's part of the sub-round has arrived (and the column numbers of the next one), behind the barrier everybody's;
+        // nobody reads the other buffer any more
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (round + 1 < n_rounds) request_rows(round + 1);  // in flight during the arithmetic below
         if (round + 2 < n_rounds) fetch_cols(round + 2);
+        const unsigned char *const buffer = smem + (round & 1) * kBuffer;
+        const unsigned *const mrow = reinterpret_cast<const unsigned *>(buffer + mask_at);
         const int n_here = (n_union - round * SR) < SR ? (n_union - round * SR) : SR;
         const int n_steps = (n_here + 31) >> 5;
 
@@ -1006,19 +962,27 @@ sparse_attention_stream_kernel(int m_vec, int n, int d_qk, int d_v,
                     act |= 1u << t;
                     const unsigned wg = word >> (4 * g);
                     half8_t a[2][KS];
-                    load_k_step<KS, PITCH>(a, k_lane, t);
+#pragma unroll
+                    for (int u = 0; u < 2; ++u)
+#pragma unroll
+                        for (int kk = 0; kk < KS; ++kk) a[u][kk] = *reinterpret_cast<const half8_t *>(buffer + k_at[kk] + (32 * t + 16 * u) * kRowK);
                     if (__builtin_amdgcn_ballot_w64((wg & kLaneBits) != kLaneBits) != 0ull) {
 #pragma unroll
                         for (int u = 0; u < 2; ++u)
 #pragma unroll
-                            for (int e = 0; e < 4; ++e) sacc[t][u][e] = select_bit(wg, 16 * u + e, 0.f, neg_inf);
+                            for (int e = 0; e < 4; ++e) {
+                                // (two instructions: kept apart, or they become a comparison and a select)
+                                int held = __builtin_amdgcn_sbfe((int)wg, 16 * u + e, 1);
+                                asm("" : "+v"(held));
+                                sacc[t][u][e] = __builtin_bit_cast(float, ~held & (int)0xff800000);
+                            }
                     }
 #pragma unroll
                     for (int u = 0; u < 2; ++u) {
 #pragma unroll
                         for (int kk = 0; kk < KS; ++kk)
                             sacc[t][u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[u][kk], qb[kk], sacc[t][u], 0, 0, 0);
-                        mx_raw = fmaxf(fmaxf(mx_raw, fmaxf(sacc[t][u][0], sacc[t][u][1])), fmaxf(sacc[t][u][2], sacc[t][u][3]));
+                        mx_raw = highest(highest(mx_raw, sacc[t][u][0], sacc[t][u][1]), sacc[t][u][2], sacc[t][u][3]);
                     }
                 }
             }
@@ -1056,7 +1020,13 @@ sparse_attention_stream_kernel(int m_vec, int n, int d_qk, int d_v,
                         p[4 * u + e] = (half_t)__builtin_amdgcn_exp2f(__builtin_fmaf(sacc[t][u][e], s2a, neg_mx));
 #pragma unroll
                 for (int cc = 0; cc < CPL; ++cc) {
-                    const half8_t b = *reinterpret_cast<const half8_t *>(vbuf + stream_v_offset(col_off + cc, 4 * t + g));
+                    // columns 16 cc + c of V: ranks 4 g .. 4 g + 3 of either half of the step
+                    typedef short short4_v __attribute__((ext_vector_type(4)));
+                    typedef short short8_v __attribute__((ext_vector_type(8)));
+                    const unsigned char *const at = buffer + v_at + 32 * t * kRowV + 32 * (cc ^ v_turn);
+                    const short4_v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_v *)at);
+                    const short4_v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_v *)(at + 16 * kRowV));
+                    const half8_t b = __builtin_bit_cast(half8_t, (short8_v){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]});
                     acc[cc] = __builtin_amdgcn_mfma_f32_16x16x32_f16(p, b, acc[cc], 0, 0, 0);
                 }
                 lacc = __builtin_amdgcn_mfma_f32_16x16x32_f16(p, ones, lacc, 0, 0, 0);
@@ -1071,12 +1041,9 @@ sparse_attention_stream_kernel(int m_vec, int n, int d_qk, int d_v,
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const int row = q_first + 4 * g + e;
-                if (col_ok) {
-                    float tmp[CPL];
 #pragma unroll
-                    for (int cc = 0; cc < CPL; ++cc) tmp[cc] = acc[cc][e];
-                    store_converted<float, CPL>(tile + (size_t)row * d_v + col0, tmp);
-                }
+                for (int cc = 0; cc < CPL; ++cc)
+                    if (16 * cc + c < d_v) tile[(size_t)row * d_v + 16 * cc + c] = acc[cc][e];
                 if (c == 0) sums[row] = lacc[e];
             }
             if (g == 0) sums[128 + q_first + c] = mx_run;
@@ -1116,12 +1083,11 @@ sparse_attention_stream_kernel(int m_vec, int n, int d_qk, int d_v,
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const long long row = q_global + 4 * g_out + e;
-            if (row < q_limit && col_out < d_v) {
+            if (row < q_limit) {
                 const float norm = lacc[e] > 0.f ? 1.f / lacc[e] : 0.f;  // a row with no column attends to nothing: zeros
-                float tmp[CPL];
 #pragma unroll
-                for (int cc = 0; cc < CPL; ++cc) tmp[cc] = acc[cc][e] * norm;
-                store_converted<half_t, CPL>(out + (size_t)row * d_v + col_out, tmp);
+                for (int cc = 0; cc < CPL; ++cc)
+                    if (16 * cc + c_out < d_v) out[(size_t)row * d_v + 16 * cc + c_out] = (half_t)(acc[cc][e] * norm);
             }
         }
     }
@@ -1221,8 +1187,7 @@ static bool union_shape(UnionShape &s, int vec_length, int n, int d_qk, int d_v,
         s.rounds = stream_rounds;
         s.steps = kStreamSteps;
         const size_t mask = (size_t)union_mask_words(s.rows, s.steps) * sizeof(unsigned);
-        // masks of one sub-round, its K rows and its V columns (transposed) side by side
-        s.lds = mask + (size_t)s.u_max * (32 * ks + 8) * sizeof(half_t) + (size_t)16 * cpl * kStreamVPitch * sizeof(half_t);
+        s.lds = 2 * (size_t)stream_buffer_bytes(s.rows, ks, cpl);
         s.plan_lds = bitmaps + s.rounds * (mask + (size_t)s.u_max * sizeof(int));
         return s.plan_lds <= 160 * 1024;
     }

@@ -266,23 +266,6 @@ struct PackedShape {
     static_assert(TN == 128, "rows of rhs in LDS: eight pieces of 32 bytes");
 };
 
-// One request of a wave, memory to LDS: lane l's SIZE bytes to `to` + SIZE * l.  In asm so that the waits are the kernel's own:
-// behind the builtin the compiler waits for every request before the next transposing read.
-template <int SIZE>
-__device__ __forceinline__ void request_to_lds(unsigned to, const uint4_t &from, unsigned lane_offset, unsigned offset)
-{
-    if constexpr (SIZE == 16)
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(to), "v"(lane_offset), "s"(from), "s"(offset));
-    else
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(to), "v"(lane_offset), "s"(from), "s"(offset));
-}
-
-__device__ __forceinline__ uint4_t buffer_of(const void *base, unsigned bytes)
-{
-    const uint64_t at = reinterpret_cast<uint64_t>(base);
-    return uint4_t{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)at), (uint32_t)__builtin_amdgcn_readfirstlane((int)((at >> 32) & 0xffffu)), bytes, 0x00020000u};
-}
-
 template <int MI, int WM, int WN, int DEPTH>
 __global__ void __launch_bounds__(64 * WM * WN, 2)
 spmm_packed_kernel(int m, int V, int N, int n, int steps, int row_tiles, int column_tiles, const int *__restrict__ row_offsets,

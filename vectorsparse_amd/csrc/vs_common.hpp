@@ -132,6 +132,23 @@ __device__ __forceinline__ uint4_t load_slice16(const half_t *row, int kk, int q
     return take ? x : zero;
 }
 
+// One request of a wave, memory to LDS: lane l's SIZE bytes to `to` + SIZE * l.  In asm so that the waits are the kernel's own:
+// behind the builtin the compiler waits for every request before the next transposing read.
+template <int SIZE>
+__device__ __forceinline__ void request_to_lds(unsigned to, const uint4_t &from, unsigned lane_offset, unsigned offset)
+{
+    if constexpr (SIZE == 16)
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(to), "v"(lane_offset), "s"(from), "s"(offset));
+    else
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(to), "v"(lane_offset), "s"(from), "s"(offset));
+}
+
+__device__ __forceinline__ uint4_t buffer_of(const void *base, unsigned bytes)
+{
+    const uint64_t at = reinterpret_cast<uint64_t>(base);
+    return uint4_t{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)at), (uint32_t)__builtin_amdgcn_readfirstlane((int)((at >> 32) & 0xffffu)), bytes, 0x00020000u};
+}
+
 // All-lane max / sum over the 64 lanes of a wave (every lane must be active).
 __device__ __forceinline__ float wave_max(float x)
 {
