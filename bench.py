@@ -172,7 +172,7 @@ def cpu_baseline(pat, B, n_dense, flops, budget_s=12.0):
 
 
 PMC_MODES = ["spmm", "spmm_largest", "spmm_slab_50", "spmm_slab_90", "spmm_valu_v1", "spmm_ragged", "sddmm_valu_v1", "sddmm_tile", "sddmm_k128", "spmm_dma", "spmm_split_rows", "spmm_row_parts", "sddmm", "attention",
-             "attention_window", "attention_global", "attention_chain", "spmm_tile"]
+             "attention_window", "attention_global", "attention_chain", "attention_rows", "spmm_tile", "spmm_packed"]
 
 
 def largest_sweep_point(cv):
@@ -487,8 +487,10 @@ def main():
             info["algorithmic_bytes"] = sddmm_algorithmic_bytes(tmask, 256)
             info["nonzero_vectors"] = int(tmask.nnz_vec)
             info["kernel_source_tag"] = kernel_source_tag("sddmm_tile.hip", "vs_common.hpp")
-        elif args.pmc == "spmm_tile":
-            # the SpMM on dense tiles: 4096 x 4096 x 2048 at 80 %, V = 4
+        elif args.pmc in ("spmm_tile", "spmm_packed"):
+            # the SpMM on dense tiles and on packed rows: 4096 x 4096 x 2048 at 80 %, V = 4
+            if args.pmc == "spmm_tile":
+                _lib.set_option("spmm_packed", 1)
             tpat = cv.random_values(cv.binomial_pattern(1024, 4096, 0.8, seed=37, vec_length=4), seed=38)
             tprob = ops.DeviceProblem(tpat)
             tBd = torch.from_numpy(cv.dense_uniform(4096, 2048, seed=39)).cuda()
@@ -497,7 +499,8 @@ def main():
                 tprob.spmm(tBd, kernel="wmma", out=tout)
             info["algorithmic_bytes"] = spmm_algorithmic_bytes(tpat, 2048)
             info["nonzero_vectors"] = int(tpat.nnz_vec)
-            info["kernel_source_tag"] = kernel_source_tag("spmm_tile.hip", "spmm_mfma_step.hpp", "vs_common.hpp")
+            info["kernel_source_tag"] = kernel_source_tag("spmm_tile.hip" if args.pmc == "spmm_tile" else "spmm_pack.hip",
+                                                          "spmm_mfma_step.hpp", "vs_common.hpp")
         elif args.pmc == "spmm_ragged":
             # a dense width that is a multiple of nothing: 1022 x 147 at 70 %, V = 2, N = 205, fp32 outputs
             rpat = cv.random_values(cv.binomial_pattern(511, 147, 0.7, seed=34, vec_length=2), seed=35)
@@ -546,8 +549,10 @@ def main():
                 amask = cv.band_strided_pattern(seq, 8, band_half_width=256, stride=seq)
             elif args.pmc == "attention_global":
                 amask = global_token_mask(cv, np, seq, 8, half_width=64, tokens=64)
-            elif args.pmc == "attention_chain":
+            elif args.pmc in ("attention_chain", "attention_rows"):
                 amask = cv.binomial_pattern(seq // 4, seq, 0.95, seed=41, vec_length=4)
+                if args.pmc == "attention_chain":   # (the operators, not the one launch that takes their place)
+                    _lib.set_option("attention_rows", 1)
             else:
                 amask = cv.band_strided_pattern(seq, 8, band_half_width=128, stride=128)
             layer = ops.SparseAttention(amask)
@@ -557,13 +562,15 @@ def main():
             kept = torch.empty((heads, amask.nnz_vec, amask.vec_length), dtype=torch.float16, device="cuda")
             layer.plan(dim, dim, heads)
             for _ in range(10):
-                if args.pmc == "attention_chain":
+                if args.pmc in ("attention_chain", "attention_rows"):
                     layer.forward(q, kk_, vv, out=ctx, fused=False, scores=kept)
                 else:
                     layer.forward(q, kk_, vv, out=ctx)
             info["algorithmic_bytes"] = 4 * heads * seq * dim * 2      # q, k, v read once, out written once
             if args.pmc == "attention_chain":
                 info["kernel_source_tag"] = kernel_source_tag(*SPMM_SOURCES)
+            elif args.pmc == "attention_rows":
+                info["kernel_source_tag"] = kernel_source_tag("sparse_attention_rows.hip", "spmm_mfma_step.hpp", "vs_common.hpp")
             else:
                 info["route"] = str(layer._route(dim, dim, heads))
                 info["rows_per_workgroup"] = layer.union_rows(dim, dim, heads)
