@@ -26,7 +26,8 @@
 // vector memory path takes about 18 cycles per request of 512 bytes.  Measured and not kept, same problem: one operand
 // ahead in LDS and the two waves of a SIMD filling and multiplying in opposite order 71 us (one workgroup per CU, 79 us for
 // half the steps per barrier); waves that only fill beside waves that only multiply 70 us (accumulators in AGPRs, else
-// spills) to 88 us (starts of the chunks scouted ahead); rhs copied to LDS without registers 73 to 83 us.
+// spills) to 88 us (starts of the chunks scouted ahead); rhs copied to LDS without registers 73 to 83 us.  Where a workspace
+// may be had, rows packed two of four (spmm_pack.hip) take 67 us there.
 #include <cmath>
 #include <type_traits>
 

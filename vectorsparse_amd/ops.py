@@ -742,7 +742,8 @@ class SparseAttention:
         dispatch list of row parts; "layer" runs the whole layer in one launch with scores and probabilities kept in LDS; True
         folds only the softmax into the SpMM launch (two launches, raw scores go through memory); False runs
         the three operators one after the other and leaves the probabilities in `scores` (on the MFMA path softmax and SpMM share
-        a launch where that is faster).  Default on the MFMA path (`_route`): "parts" where the mask has rows far longer than
+        a launch where that is faster).  True without `scores` and False on the MFMA path run with a workgroup per vector row in one
+        launch where that is expected to be faster (vs_sparse_attention_rows_f16).  Default on the MFMA path (`_route`): "parts" where the mask has rows far longer than
         the rest (global tokens); else "layer" when the cost model of `_union_rows` puts the streamed union kernel ahead
         (banded, blocky, strided and very sparse masks: 1.5-15x faster than the alternatives), else True - on masks without
         shared columns the single launch gathers K / V rows per row and is 10-60 % slower than the two launches (16 heads x
@@ -1039,7 +1040,8 @@ class DeviceProblem:
         """SpMM through the reference-shaped entry points; with row_length_hint (fp16 output only) through the
         batched entry point with batch = 1, which also takes the pattern's nonzero count and longest row and
         sizes its workgroups by the real row lengths instead of by n; patterns of strictly ascending columns that are dense
-        enough for it (vs_wmma_spmm_f16_ascending, fp16 output) run on whole tiles; with split_rows (MFMA path) on the
+        enough for it (vs_wmma_spmm_f16_ascending, fp16 output) run on whole tiles, large ones on rows packed two of four
+        (vs_spmm_f16_packed, a workspace made for the call; not inside a capture); with split_rows (MFMA path) on the
         schedule that cuts the nonzero range into equal pieces, with a workspace this object owns.
         split_rows=None chooses from the row lengths: rows in parts (spmm_row_parts) where the pattern has rows
         long enough to be split, else the row-length hints."""
