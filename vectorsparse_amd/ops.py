@@ -768,9 +768,10 @@ class SparseAttention:
                                     rows_per_workgroup=self.union_rows(d, d_v, heads), plan=self._union_plan(d, d_v, heads))
         if isinstance(fused, tuple):    # ("split", sub-rounds per workgroup)
             return sparse_attention_split(p, *self._split(d, d_v, fused[1]), q, k, v, out, scale, stream=stream)
-        if kernel == "wmma" and (d == 64 or d == 128) and d == d_v and p.nnz_vec > 0 and (fused is False or (fused is True and scores is None)):
-            # (a row per workgroup, in one launch, where that is expected to be faster: status 801 where it is not.  Of other widths it
-            # has none, and a call that is refused costs 0.4 us of the host: 1 head x 664, V = 4, width 32, 95 %: 12.5 us a pass without it)
+        if kernel == "wmma" and (d == 64 or d == 128) and d == d_v and 0 < p.longest_row_vec <= 512 and (fused is False or (fused is True and scores is None)):
+            # (a row per workgroup, in one launch, where that is expected to be faster: status 801 where it is not.  Other widths and
+            # longer rows are always refused, and a call that is refused costs 0.4 us of the host: 1 head x 664, V = 4, width 32, 95 %:
+            # 12.1 us a pass without it, 12.9 with it)
             if fused is False and scores is None:
                 scores = torch.empty((heads, p.nnz_vec, p.vec_length), dtype=torch.float16, device=q.device)
             st = _native.sparse_attention_rows(heads, p.m_vec, p.vec_length, p.n, d, d_v, p.nnz_vec, p.longest_row_vec, p.row_indices,
