@@ -487,7 +487,8 @@ int vs_wmma_softmax_spmm_f16_batched(int batch, int m_vec, int vec_length, int k
  * probabilities rounded to fp16, which are what v is multiplied by.  row_indices: a permutation of the vector rows.  Rows of more
  * than longest_row_vec nonzero vectors are correct, and slow.  q, k, v, out: 16-byte aligned, strides in elements (0: shared inputs)
  * and multiples of 8; problems that share outputs are refused.  Returns VS_ERROR_NOT_SUPPORTED for other widths, n * d_v >= 2^30,
- * rows of more than 512 vectors and where two launches (SDDMM, softmax and SpMM) are expected to be faster (option "attention_rows").
+ * rows of more than 512 vectors, where out or probabilities share memory with q, k or v (out in the place of q is allowed: the same
+ * address and stride) and where two launches (SDDMM, softmax and SpMM) are expected to be faster (option "attention_rows").
  * No counterpart in the reference.
  */
 int vs_sparse_attention_rows_f16(int batch, int m_vec, int vec_length, int n, int d_qk, int d_v, int nonzeros_vec, int longest_row_vec,

@@ -139,3 +139,28 @@ def test_the_default_route(gpu):
     assert _rows(layer.prob, *narrow, torch.empty_like(narrow[0]), None, 1.0) == 801
     assert _rows(layer.prob, q, k, v, out, None, 1.0, longest=513) == 801
     assert _rows(layer.prob, q, k, v, out[:1].expand(heads, -1, -1), None, 1.0) == -1     # (problems that share outputs)
+
+
+def test_outputs_in_the_place_of_inputs(gpu):
+    """Other workgroups still gather k and v while one writes: an output there takes two launches, as without this kernel; in the place
+    of q it is the same launch, and side by side with the inputs in one tensor too."""
+    V, heads, seq, d = 8, 8, 1024, 64
+    layer = ops.SparseAttention(cv.binomial_pattern(seq // V, seq, 0.96, seed=3, vec_length=V))
+    q, k, v = (torch.randn((heads, seq, d), device="cuda").half() for _ in range(3))
+    kept = torch.empty((heads, layer.prob.nnz_vec, V), dtype=torch.float16, device="cuda")
+    one = layer.forward(q, k, v, fused=True)
+    assert _rows(layer.prob, q, k, v, torch.empty_like(q), None, d ** -0.5) == 0
+    with _lib.thread_options(attention_rows=1):
+        two, operators = layer.forward(q, k, v, fused=True), layer.forward(q, k, v, fused=False, scores=kept)
+    assert not torch.equal(one, two)
+    over = k.clone()
+    assert _rows(layer.prob, q, over, v, over, None, d ** -0.5) == 801
+    assert torch.equal(layer.forward(q, over, v, out=over, fused=True), two)
+    over = k.clone()
+    assert torch.equal(layer.forward(q, over, v, out=over, fused=False, scores=kept), operators)
+    over = q.clone()
+    assert torch.equal(layer.forward(over, k, v, out=over, fused=True), one)
+    room = torch.stack((q, k, v, torch.zeros_like(q)), dim=1)
+    side = [room[:, i] for i in range(4)]
+    assert _rows(layer.prob, *side, None, d ** -0.5) == 0 and torch.equal(side[3], one)
+    assert _rows(layer.prob, side[0], side[1], side[2], room.reshape(heads, 4 * seq, d)[:, 3 * seq - V:4 * seq - V], None, d ** -0.5) == 801

@@ -436,3 +436,22 @@ def test_a_layers_route_is_stored_once_and_decided():
 
     layer._split_route = watched
     assert layer._route(64, 64, 4) == layer._route(64, 64, 4) == ("split", 2) and seen == [{}]
+
+
+def test_attention_rows_refuses_outputs_in_its_inputs():
+    """(addresses alone: every call here is refused before anything is read)"""
+    heads, seq, d, V, nnz = 4, 256, 64, 8, 640
+    q, k, v, out, kept, index = (0x10000000 * i for i in range(1, 7))
+    size = heads * seq * d * 2
+
+    def status(q=q, k=k, v=v, out=out, kept=kept, stride=seq * d, stride_out=seq * d):
+        return _lib.lib().vs_sparse_attention_rows_f16(heads, seq // V, V, seq, d, d, nnz, 30, index, index, index, q, stride, k, stride, v, stride,
+                                                       out, stride_out, kept, nnz * V, 1.0, 0)
+
+    with _lib.thread_options(attention_rows=3):
+        assert status(out=k) == status(out=v) == status(out=k + size - 16) == status(out=v - size + 16) == 801
+        assert status(kept=k) == status(kept=v + 512) == status(kept=q) == 801
+        assert status(out=q, stride_out=2 * seq * d) == status(out=q + 16) == status(out=q, k=q) == 801
+        # in one tensor, [heads, 4, seq, d]: the output over the end of v and its own place
+        wide = dict(q=q, k=q + seq * d * 2, v=q + 2 * seq * d * 2, stride=4 * seq * d, stride_out=4 * seq * d)
+        assert status(out=q + 3 * seq * d * 2 - 1024, **wide) == status(out=q + 3 * seq * d * 2 + 1024, **wide) == 801

@@ -33,9 +33,9 @@ __device__ __forceinline__ void load_row_of_v(RowChunk<CPL> &to, const __amdgpu_
 template <int V, int CPL, int STEPS, int W, bool KEEP>
 __global__ void __launch_bounds__(64 * W, 4)
 attention_rows_kernel(int heads, int n, const int *__restrict__ row_indices, const int *__restrict__ row_offsets,
-                      const int *__restrict__ col_indices, const half_t *__restrict__ q, const half_t *__restrict__ k,
-                      const half_t *__restrict__ v, half_t *__restrict__ out, half_t *__restrict__ kept, long long stride_q,
-                      long long stride_k, long long stride_v, long long stride_out, long long stride_kept, float scale_log2e)
+                      const int *__restrict__ col_indices, const half_t *q /* (out in its place is allowed) */, const half_t *__restrict__ k,
+                      const half_t *__restrict__ v, half_t *out, half_t *__restrict__ kept, long long stride_q, long long stride_k,
+                      long long stride_v, long long stride_out, long long stride_kept, float scale_log2e)
 {
     constexpr int D = 16 * CPL, KK = D / 32;
     __shared__ float stat[2][W][16];

@@ -89,6 +89,25 @@ int check_sddmm(int m_vec, int k, int n, int nonzeros_vec, const int *row_indice
     return VS_SUCCESS;
 }
 
+// The memory of `batch` operands of `elements` halves each, `stride` halves apart.
+struct Extent {
+    uintptr_t begin, end;
+    size_t each, apart;
+    Extent(const void *p, int batch, long long stride, long long elements)
+        : begin(reinterpret_cast<uintptr_t>(p)), each(elements > 0 ? 2 * (size_t)elements : 0), apart(batch > 1 ? 2 * (size_t)stride : 0)
+    {
+        end = begin + (each ? (size_t)(batch - 1) * apart + each : 0);
+    }
+    bool meets(const Extent &other) const
+    {
+        if (!each || !other.each || begin >= other.end || other.begin >= end) return false;
+        if (apart != other.apart || each > apart || other.each > apart) return true;
+        // (the same stride: side by side in every problem)
+        const size_t from = begin <= other.begin ? (other.begin - begin) % apart : (apart - (begin - other.begin) % apart) % apart;
+        return from < each || from + other.each > apart;
+    }
+};
+
 bool stride_ok(long long stride, long long multiple) { return stride >= 0 && stride % multiple == 0; }
 
 template <typename OutT>
@@ -590,9 +609,15 @@ int vs_sparse_attention_rows_f16(int batch, int m_vec, int vec_length, int n, in
         !stride_ok(stride_probabilities, vec_length))
         return VS_ERROR_INVALID_VALUE;
     // (what is written: no two problems may share an element)
-    if (batch > 1 && (stride_out < (long long)m_vec * vec_length * d_v ||
-                      (probabilities && stride_probabilities < (long long)nonzeros_vec * vec_length)))
-        return VS_ERROR_INVALID_VALUE;
+    const long long rows = (long long)m_vec * vec_length, kept = probabilities ? (long long)nonzeros_vec * vec_length : 0;
+    if (batch > 1 && (stride_out < rows * d_v || (probabilities && stride_probabilities < kept))) return VS_ERROR_INVALID_VALUE;
+    // Workgroups read q, k and v while others write: two launches, of which the first has read q and k when the second writes, take
+    // outputs that lie in an input.  The output in the place of q is its own row of q that a workgroup has read when it writes.
+    const Extent inputs[3] = {Extent(q, batch, stride_q, rows * d_qk), Extent(k, batch, stride_k, (long long)n * d_qk), Extent(v, batch, stride_v, (long long)n * d_v)};
+    const Extent outputs[2] = {Extent(out, batch, stride_out, rows * d_v), Extent(probabilities, batch, stride_probabilities, kept)};
+    const bool in_place = out == q && (batch == 1 || stride_out == stride_q);
+    for (int i = 0; i < 3; ++i)
+        if ((outputs[0].meets(inputs[i]) && !(i == 0 && in_place)) || outputs[1].meets(inputs[i])) return VS_ERROR_NOT_SUPPORTED;
     return vs::launch_attention_rows(waves, probabilities != nullptr, m_vec, vec_length, n, d_v, row_indices, row_offsets, col_indices,
                                      static_cast<const half_t *>(q), static_cast<const half_t *>(k), static_cast<const half_t *>(v),
                                      static_cast<half_t *>(out), static_cast<half_t *>(probabilities), scale, stride_q, stride_k, stride_v,
