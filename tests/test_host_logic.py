@@ -2,6 +2,7 @@
 host-only capacity query."""
 import numpy as np
 import pytest
+import torch
 
 from oracle import c_oracle as co
 from vectorsparse_amd import colvec_csr as cv
@@ -455,3 +456,26 @@ def test_attention_rows_refuses_outputs_in_its_inputs():
         # in one tensor, [heads, 4, seq, d]: the output over the end of v and its own place
         wide = dict(q=q, k=q + seq * d * 2, v=q + 2 * seq * d * 2, stride=4 * seq * d, stride_out=4 * seq * d)
         assert status(out=q + 3 * seq * d * 2 - 1024, **wide) == status(out=q + 3 * seq * d * 2 + 1024, **wide) == 801
+
+
+def test_a_failed_launch_of_attention_rows_is_not_taken_for_a_refusal(monkeypatch):
+    layer = ops.SparseAttention(cv.binomial_pattern(32, 256, 0.9, seed=1, vec_length=8), device="cpu")
+    q = torch.zeros((2, 256, 64), dtype=torch.float16)
+    went_on = []
+
+    def status(value):
+        monkeypatch.setattr(ops._native, "sparse_attention_rows", lambda *args: value)
+
+    monkeypatch.setattr(ops, "sddmm_batched", lambda *args, **kw: went_on.append("sddmm"))
+    monkeypatch.setattr(ops, "softmax_spmm_batched", lambda *args, **kw: went_on.append("spmm"))
+    for refused in (801, -1):
+        status(refused)
+        layer.forward(q, q, q, fused=False)
+    assert went_on == ["sddmm", "spmm"] * 2
+    for failed in (1, 2, 700):
+        status(failed)
+        with pytest.raises(_lib.VSparseError):
+            layer.forward(q, q, q, fused=False)
+    status(0)
+    layer.forward(q, q, q, fused=False)
+    assert len(went_on) == 4

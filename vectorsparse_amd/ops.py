@@ -776,7 +776,8 @@ class SparseAttention:
                 scores = torch.empty((heads, p.nnz_vec, p.vec_length), dtype=torch.float16, device=q.device)
             st = _native.sparse_attention_rows(heads, p.m_vec, p.vec_length, p.n, d, d_v, p.nnz_vec, p.longest_row_vec, p.row_indices,
                                                p.row_offsets, p.column_indices, q, k, v, out, scores, float(scale), stream)
-            if st == 0:
+            if st >= 0 and st != 801:   # (unusual arguments, -1, go on to the operators, which say what is wrong with them)
+                _lib.check(st, "vs_sparse_attention_rows_f16")
                 return out
         if scores is None:
             scores = torch.empty((heads, p.nnz_vec, p.vec_length), dtype=torch.float16, device=q.device)
