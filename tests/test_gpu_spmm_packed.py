@@ -181,3 +181,17 @@ def test_what_the_entry_point_refuses(gpu):
         assert call(64, 0, need) == 1 and call(64, workspace.data_ptr(), need - 1) == 1 and call(64, workspace.data_ptr() + 8, need) == 1
     torch.cuda.synchronize()
     assert bool((out == 7.0).all())
+
+
+@pytest.mark.parametrize("shape", [2, 3])
+def test_lists_behind_two_gigabytes(gpu, shape):
+    """2^25 rows: the operands of the last units' lists lie from step 2^21 on, 2^31 bytes into the lists."""
+    V, m_vec, n, dense = 8, 1 << 22, 64, 64
+    ro = np.zeros(m_vec + 1, dtype=np.int32)
+    ro[m_vec - dense + 1:] = n * np.arange(1, dense + 1)
+    pat = cv.random_values(cv.ColVecCSR(m_vec, n, V, ro, np.tile(np.arange(n, dtype=np.int32), dense)), 5)
+    B = cv.dense_uniform(n, 8, seed=6)
+    got = _packed(ops.DeviceProblem(pat), torch.from_numpy(B).cuda(), shape)
+    assert not bool(got[:-dense * V].any())
+    last = cv.ColVecCSR(dense, n, V, n * np.arange(dense + 1, dtype=np.int32), pat.column_indices, pat.values)
+    _check(got[-dense * V:], last, B, "the last rows")

@@ -452,7 +452,9 @@ spmm_packed_kernel(int m, int V, int N, int n, int steps, int row_tiles, int col
     const int col_wave = ct * S::TN + wn * 64;
     if (list_total > 0) {
         const unsigned mine = (unsigned)(wave * S::LIST_DEPTH * S::LIST_STEP);
-        const uint4_t operands_from = buffer_of(lists, 0x7fffffffu);
+        // (from the wave's first list on: those of its units lie within 2^20 + 4 steps, where all lists may take more than 4 GB)
+        const int lists_at = list_first[0];
+        const uint4_t operands_from = buffer_of(lists + (size_t)lists_at * kListBytes, 0x7fffffffu);
         for (bool first_time = true; list_total > 0; first_time = false) {
             if (!first_time) {
                 request_columns();
@@ -476,7 +478,7 @@ spmm_packed_kernel(int m, int V, int N, int n, int steps, int row_tiles, int col
                 const bool there = t < steps_now;
                 const unsigned to = lds + mine + slot * S::LIST_STEP;
                 const int4_t rows = *reinterpret_cast<const int4_t *>(area + my_columns + (unit * S::LIST_AT_ONCE + (there ? t - begin : 0)) * kListColumnBytes + (lane >> 3) * 16);
-                request_to_lds<16>(to + kListed * 128, operands_from, there ? (unsigned)(first + t - begin) * (unsigned)kListBytes + lane * 16 : 0x80000000u, 0u);
+                request_to_lds<16>(to + kListed * 128, operands_from, there ? (unsigned)(first - lists_at + t - begin) * (unsigned)kListBytes + lane * 16 : 0x80000000u, 0u);
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
                     // (pieces of 32 bytes: p of row r at place p ^ (r / 2 % 4))
