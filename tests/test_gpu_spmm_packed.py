@@ -195,3 +195,14 @@ def test_lists_behind_two_gigabytes(gpu, shape):
     assert not bool(got[:-dense * V].any())
     last = cv.ColVecCSR(dense, n, V, n * np.arange(dense + 1, dtype=np.int32), pat.column_indices, pat.values)
     _check(got[-dense * V:], last, B, "the last rows")
+
+
+@pytest.mark.parametrize("shape", [2, 3])
+def test_lists_that_do_not_fit_start_nowhere(gpu, shape):
+    """One nonzero announced: the units behind a row of 2^18 nonzeros would have their lists half a megabyte behind the workspace."""
+    n = 1 << 18
+    lengths = [3] + [0] * 15 + [n] + [0] * 15 + [5] * 32
+    ro = np.cumsum([0] + lengths).astype(np.int32)
+    pat = cv.random_values(cv.ColVecCSR(64, n, 1, ro, np.concatenate([np.arange(size, dtype=np.int32) for size in lengths])), 5)
+    B = cv.dense_uniform(n, 8, seed=6)
+    _check(_packed(ops.DeviceProblem(pat), torch.from_numpy(B).cuda(), shape, nonzeros=1), pat, B, "announced: one nonzero")

@@ -223,7 +223,8 @@ spmm_pack_kernel(int m_vec, int n, int blocks, int steps, int chunk_steps, int c
             put(look(fetch_column(t), t), value);
         }
         __syncthreads();
-        if (first == 0 && tid == 0) units[unit] = UnitInfo{list_first, fits ? list_steps : 0, any_bad || !fits, 0};
+        // (a list that does not fit starts nowhere: the second launch fetches four steps' columns from every list's start)
+        if (first == 0 && tid == 0) units[unit] = UnitInfo{fits ? list_first : 0, fits ? list_steps : 0, any_bad || !fits, 0};
         for (int p = tid; p < here * 64; p += kPackThreads) {
             const long long at = (long long)block * steps + first + (p >> 6);
             *reinterpret_cast<uint4_t *>(packed + (at * kBlockUnits + unit_here) * kUnitBytes + lane * 16) = reinterpret_cast<const uint4_t *>(area)[p];
