@@ -306,9 +306,15 @@ int vs_cuda_spmm_f16_ascending(int m_vec, int vec_length, int k, int n, int nonz
  * instructions; what does not fit is added from a list.  For patterns whose columns ascend strictly in every row, k % 8 == 0
  * (option "spmm_packed"); nonzeros_vec and longest_row_vec are the pattern's.  Order and counts are hints as above.
  * vs_spmm_packed_workspace_bytes: what the call needs (16-byte aligned, uninitialised, used by one call at a time), 0 where
- * the entry points above are expected to be faster or have to take the call, and the call returns VS_ERROR_NOT_SUPPORTED.
+ * the entry points above are expected to be faster or have to take the call; the call returns VS_ERROR_NOT_SUPPORTED where they
+ * would for even rows.  Uneven rows list more: vs_spmm_packed_workspace_bytes expects the worst that nonzeros_vec and longest_row_vec
+ * allow, vs_spmm_packed_workspace_bytes_lists (NULL: the same) what vs_spmm_packed_lists has counted in the host's pattern, the steps
+ * of 32 nonzeros that the fullest 16, 32 and 64 scalar rows list.
  * No counterpart in the reference.
  */
+int vs_spmm_packed_lists(int m_vec, int vec_length, const int *row_offsets, const int *column_indices, int lists[3]);
+long long vs_spmm_packed_workspace_bytes_lists(int fine_grained, int m_vec, int vec_length, int k, int n, int nonzeros_vec,
+                                               int longest_row_vec, const int lists[3]);
 long long vs_spmm_packed_workspace_bytes(int fine_grained, int m_vec, int vec_length, int k, int n, int nonzeros_vec,
                                          int longest_row_vec);
 int vs_spmm_f16_packed(int fine_grained, int m_vec, int vec_length, int k, int n, int nonzeros_vec, int longest_row_vec,

@@ -206,3 +206,18 @@ def test_lists_that_do_not_fit_start_nowhere(gpu, shape):
     pat = cv.random_values(cv.ColVecCSR(64, n, 1, ro, np.concatenate([np.arange(size, dtype=np.int32) for size in lengths])), 5)
     B = cv.dense_uniform(n, 8, seed=6)
     _check(_packed(ops.DeviceProblem(pat), torch.from_numpy(B).cuda(), shape, nonzeros=1), pat, B, "announced: one nonzero")
+
+
+def test_uneven_rows_are_not_packed(gpu):
+    """4096 x 4096 x 1024, V = 2, 90 %: Pareto rows run as if packing were off, with both kernels and both schedules."""
+    rng = np.random.default_rng(3)
+    lengths = np.minimum((rng.pareto(1.5, 2048) + 0.3) * 4096 * 0.1 / 1.9, 4096).astype(np.int64)
+    pat = cv.random_values(cv.ColVecCSR(2048, 4096, 2, *cv._pattern_from_lengths(rng, 2048, 4096, lengths)), 4)
+    prob, B = ops.DeviceProblem(pat), torch.from_numpy(cv.dense_uniform(4096, 1024, seed=5)).cuda()
+    for kernel in ("wmma", "cuda"):
+        for hint in (False, True):
+            got = prob.spmm(B, kernel=kernel, row_length_hint=hint)
+            with _lib.thread_options(spmm_packed=1):
+                assert torch.equal(prob.spmm(B, kernel=kernel, row_length_hint=hint), got)
+            with _lib.thread_options(spmm_packed=2):
+                assert not torch.equal(prob.spmm(B, kernel=kernel, row_length_hint=hint), got)

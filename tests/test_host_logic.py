@@ -479,3 +479,52 @@ def test_a_failed_launch_of_attention_rows_is_not_taken_for_a_refusal(monkeypatc
     status(0)
     layer.forward(q, q, q, fused=False)
     assert len(went_on) == 4
+
+
+def _uneven(kind, m_vec, n, V, density):
+    rng = np.random.default_rng(m_vec + V)
+    if kind == "pareto":
+        lengths = (rng.pareto(1.5, m_vec) + 0.3) * n * density / 1.9
+    elif kind == "a dense row":
+        lengths = rng.binomial(n, density, m_vec)
+        lengths[m_vec // 2] = n
+    else:
+        lengths = np.full(m_vec, n * density)
+    lengths = np.minimum(lengths, n).astype(np.int64)
+    if kind == "clusters":      # each row a run of columns
+        ro = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+        starts = rng.integers(0, n - lengths + 1)
+        return cv.ColVecCSR(m_vec, n, V, ro, np.concatenate([np.arange(s, s + size, dtype=np.int32) for s, size in zip(starts, lengths)]))
+    return cv.ColVecCSR(m_vec, n, V, *cv._pattern_from_lengths(rng, m_vec, n, lengths))
+
+
+@pytest.mark.parametrize("V", [1, 2, 4, 8])
+def test_what_packed_rows_list_is_counted(V):
+    for kind, m_vec, n in (("even", 70, 900), ("a dense row", 33, 1030), ("clusters", 64, 515), ("even", 1, 3), ("even", 5, 8)):
+        pat = _uneven(kind, m_vec, n, V, 0.5)
+        steps = np.zeros(-(-m_vec * V // 64) * 4, dtype=np.int64)       # of 16 rows each
+        for i in range(m_vec):
+            groups = np.bincount(pat.column_indices[pat.row_offsets[i]:pat.row_offsets[i + 1]] // 4)
+            steps[i * V // 16] += np.maximum(groups - 2, 0).sum()
+        steps = -(-steps // 32)
+        want = tuple(int(steps.reshape(-1, units).sum(axis=1).max()) for units in (1, 2, 4))
+        assert ops.spmm_packed_lists(pat) == want, (kind, m_vec)
+        assert ops.DeviceProblem(pat, device="cpu").packed_lists == want
+    assert ops.spmm_packed_lists(cv.ColVecCSR(0, 8, V, np.zeros(1, dtype=np.int32), np.zeros(0, dtype=np.int32))) == (0, 0, 0)
+
+
+@pytest.mark.parametrize("V,n,k,density", [(1, 4096, 2048, 0.1), (2, 4096, 1024, 0.1), (2, 4096, 2048, 0.15), (4, 4096, 2048, 0.2)])
+def test_packed_rows_are_for_rows_of_short_lists(V, n, k, density):
+    """4096 rows: even ones are packed, by the counts and by the lengths alone (1.1 to 1.6 times faster than what runs else), Pareto
+    rows, a dense row among even ones and clustered columns are not (0.3 to 0.96 times as fast)."""
+    m_vec = 4096 // V
+    for kind, packed in (("even", True), ("pareto", False), ("a dense row", False), ("clusters", False)):
+        pat = _uneven(kind, m_vec, n, V, density)
+        longest = int(np.diff(pat.row_offsets).max())
+        need = lambda **lists: ops.spmm_packed_workspace_bytes(m_vec, V, k, n, pat.nnz_vec, longest, **lists)
+        assert (need(lists=ops.spmm_packed_lists(pat)) > 0) == packed, kind
+        if kind != "clusters":      # (the lengths do not show them)
+            assert (need() > 0) == packed, kind
+            assert (_lib.lib().vs_spmm_packed_workspace_bytes(0, m_vec, V, k, n, pat.nnz_vec, longest) > 0) == packed, kind
+        with _lib.thread_options(spmm_packed=2):
+            assert need(lists=ops.spmm_packed_lists(pat)) > 0 and need() > 0

@@ -33,6 +33,8 @@ SIGNATURES = {
     "vs_wmma_spmm_f16_batched_sorted": ([_int] * 8 + [_vp] * 3 + [_vp, _ll, _vp, _ll, _vp, _ll, _vp], _int),
     "vs_wmma_spmm_f16_ascending": ([_int] * 8 + [_vp] * 7, _int),
     "vs_cuda_spmm_f16_ascending": ([_int] * 7 + [_vp] * 7, _int),
+    "vs_spmm_packed_lists": ([_int] * 2 + [_vp] * 3, _int),
+    "vs_spmm_packed_workspace_bytes_lists": ([_int] * 7 + [_vp], _ll),
     "vs_spmm_packed_workspace_bytes": ([_int] * 7, _ll),
     "vs_spmm_f16_packed": ([_int] * 7 + [_vp] * 6 + [_ll, _vp], _int),
     "vs_wmma_spmm_launch_shape": ([_int] * 8 + [_vp], _int),

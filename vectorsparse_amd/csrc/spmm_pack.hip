@@ -23,6 +23,7 @@
 // What a dense product cannot see is put right afterwards, per workgroup, as in spmm_tile.hip: zeros times infinities
 // (noticed as NaN outputs) and columns that do not ascend strictly (noticed while packing) make a workgroup compute its tile
 // again nonzero by nonzero.
+#include <algorithm>
 #include <cmath>
 #include <type_traits>
 
@@ -632,7 +633,15 @@ int launch_packed_shape(int m, int V, int k, int n, const PackedLayout &at, cons
 // line lies 15 % on this side of the others' estimate, which is low where tiles of either kind come in: at the line, 2248 x 2742 x 1488,
 // V = 1, 90 %: 44.3 against 33.7 us; 2672 x 2353 x 1224, V = 8, 80 %: 32.4 against 30.1 us.  Below 25 us the packing is
 // too large a part of it: 1571 x 1116 x 1976, V = 1, 92 %: 20.8 against 22.5 us.
-int spmm_packed_choice(bool fine_grained, int m_vec, int k, int n, int vec_length, int nonzeros_vec, int longest_row_vec)
+//
+// The lists of uneven rows, or of columns in clusters, are many times those of even ones, and a wave goes through those of its units
+// alone: 0.94 us per step of the fullest 64 rows (tiles of 256), 0.5 us of the fullest 32 (of 128), and packing a row beyond what a
+// wave keeps 0.55 us per turn of 64 nonzeros and 0.27 us more for every further pass over it, which its unit's list asks for.  Fitted
+// to 81 problems (4096 x 4096 x 2048 and less, even to Pareto rows) within 4 % (tiles of 256) and 6 %.  Gathering waits for its longest
+// row too: 0.03 us per nonzero vector beyond two mean rows on the fine-grained path, 0.005 us on the matrix cores.  4096 x 4096 x 2048, V = 4, 80 %:
+// 67 us for even rows, 171 us (and 118 us as they run now) for log-normal rows of width 0.5, 364 us (124 us) for Pareto rows.
+int spmm_packed_choice(bool fine_grained, int m_vec, int k, int n, int vec_length, int nonzeros_vec, int longest_row_vec,
+                       const PackedLists *lists)
 {
     const Options &o = options();
     if (o.spmm_packed == 1) return 0;
@@ -642,17 +651,57 @@ int spmm_packed_choice(bool fine_grained, int m_vec, int k, int n, int vec_lengt
     if (o.spmm_packed >= 2) return o.spmm_packed - 1;
     if (o.spmm_tile || o.spmm_waves || o.spmm_cols_per_lane || o.spmm_steps || o.spmm_pipe || o.spmm_gather || o.spmm_teams || o.spmm_blocks_per_wave || o.spmm_guard_waves)
         return 0;  // a launch shape of other kernels is asked for
-    if (spmm_gather_us(fine_grained, vec_length, nonzeros_vec, k) < 25) return 0;
-    const double others = spmm_expected_us(fine_grained, m_vec, k, n, vec_length, nonzeros_vec, longest_row_vec);
+    const double gather = spmm_gather_us(fine_grained, vec_length, nonzeros_vec, k);
+    if (gather < 25) return 0;
+    double others = spmm_expected_us(fine_grained, m_vec, k, n, vec_length, nonzeros_vec, longest_row_vec);
     if (others < 25) return 0;
     const double m = (double)m_vec * vec_length, density = nonzeros_vec / ((double)m_vec * n), steps = 4 * std::ceil(n / 256.0);
     const double unit = (double)kUnitRows / vec_length * n * density;   // nonzero vectors, and those of them that are listed
     const double listed = (double)kUnitRows / vec_length * n / 4 * (4 * density * density * density * (1 - density) + 2 * density * density * density * density);
     const double wide = std::ceil(m / 256) * std::ceil(k / 128.0) / 256, narrow = std::ceil(m / 128) * std::ceil(k / 128.0) / 256;
-    const double wide_us = 11.8 + (0.498 * steps + 0.116 * listed) * std::ceil(wide) + 9.4 * wide + 0.19e-3 * unit;
-    const double narrow_us = 6.6 + (0.417 * steps + 0.043 * listed) * std::ceil(narrow) + 7.1 * narrow + 0.57e-3 * unit;
+    double wide_us = 11.8 + (0.498 * steps + 0.116 * listed) * std::ceil(wide) + 9.4 * wide + 0.19e-3 * unit;
+    double narrow_us = 6.6 + (0.417 * steps + 0.043 * listed) * std::ceil(narrow) + 7.1 * narrow + 0.57e-3 * unit;
+    if (lists) {
+        // (what the fullest of 64 even rows takes: a fourth more than the mean, half a step of padding per unit)
+        const double even = 1.25 * 4 * (listed / kListed + 0.5);
+        const auto turns = [&](double row) { return std::fmax(0.0, std::ceil(row / (64 * vec_length)) - (vec_length <= 2 ? 8 : 4)); };
+        const double more_turns = std::fmax(0.0, turns(longest_row_vec) - turns(1.25 * density * n));
+        const double passes = std::fmax(0.0, std::ceil(lists->rows16 / (vec_length == 1 ? 16.0 : 8.0)) - 1);
+        constexpr double kDoubt = 1.4;   // (the line below is drawn for even rows)
+        const double packing = more_turns * (0.55 + 0.27 * passes);
+        wide_us += kDoubt * (packing + 0.94 * std::fmax(0.0, lists->rows64 - even) * std::ceil(wide));
+        narrow_us += kDoubt * (packing + 0.5 * std::fmax(0.0, lists->rows32 - even / 2) * std::ceil(narrow));
+        if (others >= gather) others += (fine_grained ? 0.03 : 0.005) * std::fmax(0.0, longest_row_vec - 2 * density * n);
+    }
     if (std::fmin(wide_us, narrow_us) > 1.15 * others) return 0;
     return wide_us <= narrow_us ? 1 : 2;
+}
+
+PackedLists spmm_packed_lists(int m_vec, int vec_length, const int *row_offsets, const int *column_indices)
+{
+    const int unit_rows = kUnitRows / vec_length;
+    PackedLists most{0, 0, 0};
+    int two = 0, four = 0;
+    for (int unit = 0; unit * (long long)unit_rows < m_vec; ++unit) {
+        const int first = unit * unit_rows, behind = std::min(first + unit_rows, m_vec);
+        int count = 0;
+        for (int r = first; r < behind; ++r)
+            for (int j = row_offsets[r] + 2; j < row_offsets[r + 1]; ++j) count += ((column_indices[j] ^ column_indices[j - 2]) & ~3) == 0;
+        const int steps = (count + kListed - 1) / kListed;
+        two = (unit & 1 ? two : 0) + steps;
+        four = (unit & 3 ? four : 0) + steps;
+        most = {std::max(most.rows16, steps), std::max(most.rows32, two), std::max(most.rows64, four)};
+    }
+    return most;
+}
+
+PackedLists spmm_packed_lists_bound(int m_vec, int n, int vec_length, int nonzeros_vec, int longest_row_vec)
+{
+    const double mean = nonzeros_vec / ((double)m_vec * n), longest = std::fmin(std::fmax((double)longest_row_vec / n, mean), 1.0);
+    const double row = n / 4 * (4 * longest * longest * longest * (1 - longest) + 2 * longest * longest * longest * longest);
+    const double others = row * (mean > 0 ? mean / longest : 0.0);
+    const auto steps = [&](int rows) { return (int)((row + (rows / vec_length - 1) * others) / kListed + 0.5 * rows / kUnitRows); };
+    return {steps(16), steps(32), steps(64)};
 }
 
 long long spmm_packed_bytes(int m_vec, int vec_length, int n, int nonzeros_vec)

@@ -370,8 +370,17 @@ double spmm_expected_us(bool fine_grained, int m_vec, int k, int n, int vec_leng
 
 // SpMM on rows packed two of four (csrc/spmm_pack.hip), for columns that ascend strictly.  spmm_packed_choice: 0 = other
 // kernels are expected to be faster (or have to take the call), else the `shape` for launch_spmm_packed (1 = tiles of
-// 256 x 128, 2 = 128 x 128), which takes a workspace of spmm_packed_bytes, 16-byte aligned, uninitialised.
-int spmm_packed_choice(bool fine_grained, int m_vec, int k, int n, int vec_length, int nonzeros_vec, int longest_row_vec);
+// 256 x 128, 2 = 128 x 128), which takes a workspace of spmm_packed_bytes, 16-byte aligned, uninitialised.  `lists`: what the
+// pattern's lists take, null: as if its rows were even.
+struct PackedLists {
+    int rows16, rows32, rows64;   // steps of 32 nonzeros, of the fullest 16, 32 and 64 scalar rows
+};
+int spmm_packed_choice(bool fine_grained, int m_vec, int k, int n, int vec_length, int nonzeros_vec, int longest_row_vec, const PackedLists *lists);
+// Host arrays, columns that ascend strictly in every row.
+PackedLists spmm_packed_lists(int m_vec, int vec_length, const int *row_offsets, const int *column_indices);
+// The same of a pattern of which only the longest row is known: the most that rows of random columns take (their number in a row
+// grows faster than the row).
+PackedLists spmm_packed_lists_bound(int m_vec, int n, int vec_length, int nonzeros_vec, int longest_row_vec);
 long long spmm_packed_bytes(int m_vec, int vec_length, int n, int nonzeros_vec);
 int launch_spmm_packed(int shape, int m_vec, int vec_length, int k, int n, int nonzeros_vec, const int *row_offsets,
                        const int *col_indices, const half_t *values, const half_t *rhs, half_t *out, void *workspace, hipStream_t stream);

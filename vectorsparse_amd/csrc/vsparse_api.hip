@@ -446,11 +446,30 @@ int vs_cuda_spmm_f16_ascending(int m_vec, int vec_length, int k, int n, int nonz
                                         ascending(nonzeros_vec, longest_row_vec, row_length_hints, -1));
 }
 
+int vs_spmm_packed_lists(int m_vec, int vec_length, const int *row_offsets, const int *column_indices, int lists[3])
+{
+    if (m_vec < 0 || !vec_ok(vec_length) || !lists || (m_vec > 0 && !row_offsets)) return VS_ERROR_INVALID_VALUE;
+    if (m_vec > 0 && row_offsets[m_vec] > row_offsets[0] && !column_indices) return VS_ERROR_INVALID_VALUE;
+    const vs::PackedLists most = vs::spmm_packed_lists(m_vec, vec_length, row_offsets, column_indices);
+    lists[0] = most.rows16;
+    lists[1] = most.rows32;
+    lists[2] = most.rows64;
+    return VS_SUCCESS;
+}
+
+long long vs_spmm_packed_workspace_bytes_lists(int fine_grained, int m_vec, int vec_length, int k, int n, int nonzeros_vec, int longest_row_vec,
+                                               const int lists[3])
+{
+    if (!vec_ok(vec_length) || m_vec <= 0 || n <= 0 || nonzeros_vec <= 0) return 0;
+    const vs::PackedLists most = lists ? vs::PackedLists{lists[0], lists[1], lists[2]}
+                                       : vs::spmm_packed_lists_bound(m_vec, n, vec_length, nonzeros_vec, longest_row_vec);
+    const int shape = vs::spmm_packed_choice(fine_grained != 0, m_vec, k, n, vec_length, nonzeros_vec, longest_row_vec, &most);
+    return shape ? vs::spmm_packed_bytes(m_vec, vec_length, n, nonzeros_vec) : 0;
+}
+
 long long vs_spmm_packed_workspace_bytes(int fine_grained, int m_vec, int vec_length, int k, int n, int nonzeros_vec, int longest_row_vec)
 {
-    if (!vec_ok(vec_length)) return 0;
-    const int shape = vs::spmm_packed_choice(fine_grained != 0, m_vec, k, n, vec_length, nonzeros_vec, longest_row_vec);
-    return shape ? vs::spmm_packed_bytes(m_vec, vec_length, n, nonzeros_vec) : 0;
+    return vs_spmm_packed_workspace_bytes_lists(fine_grained, m_vec, vec_length, k, n, nonzeros_vec, longest_row_vec, nullptr);
 }
 
 int vs_spmm_f16_packed(int fine_grained, int m_vec, int vec_length, int k, int n, int nonzeros_vec, int longest_row_vec,
@@ -461,7 +480,7 @@ int vs_spmm_f16_packed(int fine_grained, int m_vec, int vec_length, int k, int n
                         output_matrix, sizeof(half_t));
     if (st != VS_SUCCESS) return st;
     if (m_vec == 0 || k == 0) return VS_SUCCESS;
-    const int shape = vs::spmm_packed_choice(fine_grained != 0, m_vec, k, n, vec_length, nonzeros_vec, longest_row_vec);
+    const int shape = vs::spmm_packed_choice(fine_grained != 0, m_vec, k, n, vec_length, nonzeros_vec, longest_row_vec, nullptr);
     if (shape == 0) return VS_ERROR_NOT_SUPPORTED;
     if (!column_indices || !values || !workspace || !aligned(workspace, 16) ||
         workspace_bytes < vs::spmm_packed_bytes(m_vec, vec_length, n, nonzeros_vec))

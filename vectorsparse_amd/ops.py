@@ -185,9 +185,21 @@ def spmm_split_rows(m_vec, vec_length, k, n, nonzeros_vec, row_offsets, column_i
     return output_matrix
 
 
-def spmm_packed_workspace_bytes(m_vec, vec_length, k, n, nonzeros_vec, longest_row_vec, fine_grained=False):
-    """Workspace of the SpMM on packed rows (vs_spmm_f16_packed); 0 where other kernels are expected to be faster."""
-    return int(_lib.lib().vs_spmm_packed_workspace_bytes(int(fine_grained), m_vec, vec_length, k, n, nonzeros_vec, longest_row_vec))
+def spmm_packed_workspace_bytes(m_vec, vec_length, k, n, nonzeros_vec, longest_row_vec, fine_grained=False, lists=None):
+    """Workspace of the SpMM on packed rows (vs_spmm_f16_packed); 0 where other kernels are expected to be faster.  lists:
+    the pattern's `spmm_packed_lists`, None for the worst that the counts allow."""
+    counted = None if lists is None else (ctypes.c_int * 3)(*lists)
+    return int(_lib.lib().vs_spmm_packed_workspace_bytes_lists(int(fine_grained), m_vec, vec_length, k, n, nonzeros_vec, longest_row_vec, counted))
+
+
+def spmm_packed_lists(pattern):
+    """What the SpMM on packed rows lists of a pattern of strictly ascending columns: steps of 32 nonzeros of its fullest
+    16, 32 and 64 scalar rows."""
+    ro = np.ascontiguousarray(pattern.row_offsets, dtype=np.int32)
+    ci = np.ascontiguousarray(pattern.column_indices, dtype=np.int32)
+    counted = (ctypes.c_int * 3)()
+    _lib.check(_lib.lib().vs_spmm_packed_lists(pattern.m_vec, pattern.vec_length, ro.ctypes.data, ci.ctypes.data, counted), "vs_spmm_packed_lists")
+    return tuple(counted)
 
 
 def spmm_slab_workspace_bytes(m_vec, vec_length, k, n):
@@ -981,6 +993,7 @@ class DeviceProblem:
         # hints: SDDMM and SpMM run dense patterns of ascending columns on whole tiles
         self.columns_distinct = columns_ascend(pattern.row_offsets, pattern.column_indices, strictly=True)
         self.columns_sorted = self.columns_distinct or columns_ascend(pattern.row_offsets, pattern.column_indices)
+        self.packed_lists = spmm_packed_lists(pattern) if self.columns_distinct else (0, 0, 0)
         self._workspace = None  # partial tiles of the split-row SpMM, allocated on first use
         self._parts = {}        # limit -> (RowParts, its list on the device, workspace), made on first use
         self._parts_need = {}
@@ -1071,13 +1084,13 @@ class DeviceProblem:
         if self.columns_distinct and out.dtype == torch.float16:
             st = _native.spmm_ascending(kernel != "wmma", self.m_vec, self.vec_length, k, self.n, self.nnz_vec, self.longest_row_vec,
                                         self.long_rows, bool(row_length_hint), self.row_indices, self.row_offsets,
-                                        self.column_indices, self.values, rhs_matrix, out, stream, True)
+                                        self.column_indices, self.values, rhs_matrix, out, stream, True, *self.packed_lists)
             if st == -2:
                 st = self._spmm_packed(rhs_matrix, kernel != "wmma", out, stream)
                 if st is None:
                     st = _native.spmm_ascending(kernel != "wmma", self.m_vec, self.vec_length, k, self.n, self.nnz_vec, self.longest_row_vec,
                                                 self.long_rows, bool(row_length_hint), self.row_indices, self.row_offsets,
-                                                self.column_indices, self.values, rhs_matrix, out, stream, False)
+                                                self.column_indices, self.values, rhs_matrix, out, stream, False, *self.packed_lists)
             if st >= 0:
                 if st:
                     _lib.check(st, "vs_%s_spmm_f16%s" % ("wmma" if kernel == "wmma" else "cuda", "_batched" if row_length_hint else ""))
@@ -1096,7 +1109,7 @@ class DeviceProblem:
         room for one, and inside a capture (replays would find the workspace given back to the allocator unless torch itself
         runs the capture)."""
         k = rhs_matrix.shape[1]
-        need = spmm_packed_workspace_bytes(self.m_vec, self.vec_length, k, self.n, self.nnz_vec, self.longest_row_vec, fine_grained)
+        need = spmm_packed_workspace_bytes(self.m_vec, self.vec_length, k, self.n, self.nnz_vec, self.longest_row_vec, fine_grained, self.packed_lists)
         with contextlib.nullcontext() if stream is None else torch.cuda.stream(_as_stream(stream)):
             if torch.cuda.is_current_stream_capturing():
                 return None
