@@ -528,3 +528,13 @@ def test_packed_rows_are_for_rows_of_short_lists(V, n, k, density):
             assert (_lib.lib().vs_spmm_packed_workspace_bytes(0, m_vec, V, k, n, pat.nnz_vec, longest) > 0) == packed, kind
         with _lib.thread_options(spmm_packed=2):
             assert need(lists=ops.spmm_packed_lists(pat)) > 0 and need() > 0
+
+
+def test_the_workspace_of_packed_rows_has_a_limit():
+    """1 GiB by itself (16384 x 16384 takes 0.36 GB, 65536 x 65536 5.5 GB); callers that ask for the kernel say how much they have."""
+    for size, packed in ((16384, True), (65536, False)):
+        m_vec, k = size // 8, 2048
+        need = lambda: ops.spmm_packed_workspace_bytes(m_vec, 8, k, size, m_vec * size // 10, size // 10 + size // 80, fine_grained=True)
+        assert need() <= 2 ** 30 and (need() > 0) == packed
+        with _lib.thread_options(spmm_packed=2):
+            assert (need() > 2 ** 30) == (not packed)

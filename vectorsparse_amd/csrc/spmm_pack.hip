@@ -640,6 +640,12 @@ int launch_packed_shape(int m, int V, int k, int n, const PackedLayout &at, cons
 // to 81 problems (4096 x 4096 x 2048 and less, even to Pareto rows) within 4 % (tiles of 256) and 6 %.  Gathering waits for its longest
 // row too: 0.03 us per nonzero vector beyond two mean rows on the fine-grained path, 0.005 us on the matrix cores.  4096 x 4096 x 2048, V = 4, 80 %:
 // 67 us for even rows, 171 us (and 118 us as they run now) for log-normal rows of width 0.5, 364 us (124 us) for Pareto rows.
+//
+// The workspace grows with the matrix, whatever its sparsity, and those who call the operators did not ask for one: none beyond
+// 1 GiB, which takes in what gains most (16384 x 16384 x 2048, V = 1, 95 %: 0.54 GB, 1.17 ms as gathered, 0.80 ms packed; 32768 x 16384 x
+// 2048, V = 4, 90 %: 0.85 GB, 1.90 and 1.55 ms; refused: 32768 x 32768 x 1024, V = 8, 90 %: 1.45 GB, 1.82 and 1.59 ms).
+constexpr long long kMostWorkspace = 1LL << 30;
+
 int spmm_packed_choice(bool fine_grained, int m_vec, int k, int n, int vec_length, int nonzeros_vec, int longest_row_vec,
                        const PackedLists *lists)
 {
@@ -652,7 +658,7 @@ int spmm_packed_choice(bool fine_grained, int m_vec, int k, int n, int vec_lengt
     if (o.spmm_tile || o.spmm_waves || o.spmm_cols_per_lane || o.spmm_steps || o.spmm_pipe || o.spmm_gather || o.spmm_teams || o.spmm_blocks_per_wave || o.spmm_guard_waves)
         return 0;  // a launch shape of other kernels is asked for
     const double gather = spmm_gather_us(fine_grained, vec_length, nonzeros_vec, k);
-    if (gather < 25) return 0;
+    if (gather < 25 || spmm_packed_bytes(m_vec, vec_length, n, nonzeros_vec) > kMostWorkspace) return 0;
     double others = spmm_expected_us(fine_grained, m_vec, k, n, vec_length, nonzeros_vec, longest_row_vec);
     if (others < 25) return 0;
     const double m = (double)m_vec * vec_length, density = nonzeros_vec / ((double)m_vec * n), steps = 4 * std::ceil(n / 256.0);
