@@ -538,3 +538,18 @@ def test_the_workspace_of_packed_rows_has_a_limit():
         assert need() <= 2 ** 30 and (need() > 0) == packed
         with _lib.thread_options(spmm_packed=2):
             assert (need() > 2 ** 30) == (not packed)
+
+
+@pytest.mark.parametrize("heads,seq,V,d,mean,keep,taken", [
+    # microseconds as two launches and as one: 17.9 and 14.8, 18.6 and 15.1, 8.3 and 5.4, 33.4 and 25.5, 31.0 and 24.9
+    (8, 2048, 4, 64, 102, False, True), (8, 2048, 4, 64, 102, True, True), (2, 1730, 2, 64, 35, False, True), (16, 4096, 8, 128, 40, False, True),
+    (16, 2600, 8, 64, 160, False, True),
+    # 69.9 and 75.4, 54.9 and 59.1, 39.4 and 48.1, 47.0 and 60.2, 53.9 and 63.2, 45.3 and 49.4
+    (16, 3928, 8, 64, 393, False, False), (16, 3762, 2, 64, 75, False, False), (8, 4096, 2, 128, 40, True, False), (16, 2600, 2, 128, 40, True, False),
+    (16, 4096, 4, 128, 80, False, False), (16, 2600, 1, 64, 40, False, False)])
+def test_attention_rows_is_for_layers_it_is_faster_on(heads, seq, V, d, mean, keep, taken):
+    """(without addresses a call that is taken is an invalid value, before anything is read)"""
+    m_vec = seq // V
+    status = _lib.lib().vs_sparse_attention_rows_f16(heads, m_vec, V, seq, d, d, m_vec * mean, mean + mean // 3, 0, 0, 0, 0, seq * d, 0, seq * d, 0, seq * d,
+                                                     0, seq * d, 16 if keep else 0, m_vec * mean * V, 1.0, 0)
+    assert status == (1 if taken else 801)

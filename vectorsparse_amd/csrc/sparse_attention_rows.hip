@@ -316,12 +316,13 @@ int launch_rows_width(int d, int waves, Args... args)
 
 }  // namespace
 
-// One launch against the two it replaces as microseconds, fitted to 160 masks (bands and random ones, 1..16 heads x 512..4096, head
-// widths of 64 and 128, rows of 13 to 490 nonzero vectors, every V; profiles/attention_rows_rule_survey.txt) to within 7 to 9 %
-// (width 64) and 5 to 12 % (128): one launch costs 2 to 3 us less, and nothing per row beyond its gathers, which come by the same columns;
-// the two gather in wider waves, so that many long rows are theirs.  1.1 to 1.7 times faster where it is taken (16 heads x 788, V = 4, rows
-// of 16: 11.2 against 6.7 us; 16 x 2688, V = 8, rows of 54: 23.8 against 13.7; 8 x 2048, V = 4, rows of 102: 20.2 against 17.1 us), not taken
-// for 8 heads x 2048, V = 1, rows of 102 (43 against 47 us) and 2 heads x 1588, V = 2, width 128, rows of 381 (19.6 against 23 us).
+// One launch against the two it replaces as microseconds, fitted to 1920 masks (bands and random ones, 1..16 heads x 512..4096, head
+// widths of 64 and 128, rows of 10 to 490 nonzero vectors, every V; profiles/attention_rows_rule_survey.txt), the two to within 7 %, the
+// one to within 6 %: one launch costs 2 to 3 us less, and nothing per row beyond its gathers, which come by the same columns; the two gather
+// in wider waves, so that many long rows are theirs.  Taken for 2569 of 3840 layers, 1.44 times faster in the median (16 heads x 788, V =
+// 4, rows of 16: 11.2 against 6.7 us; 8 x 2048, V = 4, rows of 102: 17.9 against 14.8 us), slower for 32, by more than 3 % for 15 (8 x 2728, V
+// = 2, width 128, a band of 36: 27.0 against 31.6 us); of the others 145 would gain more than 5 %.  Not taken for 16 x 3928, V = 8, rows of
+// 393 (69 against 75 us) and 8 x 2048, V = 1, rows of 102 (43 against 47 us).
 int attention_rows_waves(bool keep, int heads, int m_vec, int n, int vec_length, int d_qk, int d_v, int nonzeros_vec, int longest_row_vec)
 {
     const Options &o = options();
@@ -335,17 +336,19 @@ int attention_rows_waves(bool keep, int heads, int m_vec, int n, int vec_length,
         return 0;   // (a launch shape of the other kernels is asked for)
     const int wide = d_v == 128, v = vec_length == 1 ? 0 : (vec_length == 2 ? 1 : (vec_length == 4 ? 2 : 3));
     const double rows = 1e-3 * m_vec * heads, gathers = 1e-6 * (double)nonzeros_vec * heads, mean = 1e-2 * nonzeros_vec / m_vec;
-    struct Two {
-        double launches, row, gather;
+    struct Cost {
+        double launch, row, gather, mean;
     };
-    static constexpr Two kTwo[2][2][4] = {{{{7.5, 0.26, 17.1}, {7.8, 0.69, 14.5}, {8.1, 0.64, 19.5}, {8.1, 1.27, 20.8}},
-                                           {{8.5, 0.70, 19.9}, {7.3, 1.08, 24.2}, {8.1, 0.91, 33.0}, {9.2, 0.43, 38.8}}},
-                                          {{{7.65, 0.32, 17.5}, {8.2, 0.71, 14.8}, {8.3, 0.79, 20.2}, {8.5, 1.41, 22.2}},
-                                           {{8.3, 0.83, 19.8}, {7.4, 1.32, 22.9}, {8.3, 1.14, 32.6}, {10.6, 0.01, 40.1}}}};
-    const Two &two = kTwo[keep][wide][v];
-    const double one = keep ? (wide ? 6.0 + 47.1 * gathers + 0.43 * mean : 5.4 + 0.19 * rows + 23.6 * gathers + 0.45 * mean)
-                            : (wide ? 5.75 + 39.8 * gathers + 0.6 * mean : 5.6 + 23.0 * gathers + 0.3 * mean);
-    if (one > 0.95 * (two.launches + two.row * rows + two.gather * gathers)) return 0;
+    static constexpr Cost kTwo[2][2][4] = {{{{5.5, 0.44, 13.02, 1.62}, {6.02, 0.49, 14.03, 1.09}, {6.42, 0.66, 16.21, 0.89}, {6.83, 0.92, 19.01, 1.06}},
+                                            {{5.39, 0.88, 15.75, 2.25}, {5.75, 0.91, 20.36, 1.89}, {6.41, 1.11, 26.43, 1.06}, {6.84, 1.56, 31.24, 1.21}}},
+                                           {{{5.95, 0.47, 13.31, 1.37}, {6.45, 0.56, 14.14, 0.85}, {6.6, 0.81, 16.72, 0.91}, {7.16, 1.17, 20.41, 1.11}},
+                                            {{5.84, 0.96, 14.94, 1.93}, {6.04, 1.08, 20.0, 1.45}, {6.91, 1.19, 26.75, 0.98}, {7.86, 1.36, 32.77, 1.25}}}};
+    static constexpr Cost kOne[2][2][4] = {{{{3.45, 0.12, 22.04, 0.74}, {3.72, 0.12, 22.46, 0.58}, {3.77, 0.13, 23.11, 0.61}, {3.98, 0.02, 24.86, 0.4}},
+                                            {{3.52, 0.23, 38.51, 0.73}, {3.85, 0.33, 38.78, 0.65}, {4.0, 0.34, 41.06, 0.61}, {4.24, 0.31, 43.76, 0.54}}},
+                                           {{{3.88, 0.17, 22.39, 0.3}, {4.07, 0.18, 22.48, 0.34}, {4.07, 0.19, 23.01, 0.42}, {4.17, 0.1, 25.62, 0.31}},
+                                            {{3.85, 0.19, 40.09, 0.9}, {4.16, 0.04, 49.08, 0.81}, {4.2, 0.09, 45.64, 0.68}, {4.36, 0.03, 47.67, 0.66}}}};
+    const auto us = [&](const Cost &c) { return c.launch + c.row * rows + c.gather * gathers + c.mean * mean; };
+    if (us(kOne[keep][wide][v]) > 0.95 * us(kTwo[keep][wide][v])) return 0;
     // as few waves as hold the row; twice as many where the chip has room for them
     const int steps = (longest_row_vec + kStep - 1) / kStep, held = d_v == 64 ? 4 : 2;
     int waves = 1;
