@@ -108,6 +108,18 @@ def test_nan_and_infinity_stay_in_their_row(gpu):
         assert torch.equal(bad, want)
 
 
+def test_a_wave_of_nan_is_the_whole_rows(gpu):
+    """A row longer than announced, with NaN wherever one of two waves looks: its probabilities are NaN at the other's nonzeros too."""
+    pat = _pattern(4, (300, 40), 400, 3)
+    prob = ops.DeviceProblem(pat)
+    q, k, v = (torch.randn((1, rows, 64), device="cuda").half() for rows in (pat.m, 400, 400))
+    k[0, torch.from_numpy(np.r_[pat.column_indices[:128], pat.column_indices[256:300]]).cuda().long()] = float("nan")
+    out, kept = torch.empty_like(q), torch.empty((1, pat.nnz_vec, 4), dtype=torch.float16, device="cuda")
+    with _lib.thread_options(attention_rows=3):
+        assert _rows(prob, q, k, v, out, kept, 0.1, longest=40) == 0
+    assert bool(torch.isnan(kept[0, :300]).all()) and bool(torch.isnan(out[0, :4]).all())
+
+
 def test_the_default_route(gpu):
     """8 heads x 1024, V = 8, 96 %: the operators that keep the probabilities and the default without a caller's scores run in one
     launch, other layers and scores that a caller asked for as they did; replays of a capture give the eager bits."""

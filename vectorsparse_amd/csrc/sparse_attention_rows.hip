@@ -230,11 +230,16 @@ attention_rows_kernel(int heads, int n, const int *__restrict__ row_indices, con
                 for (int t = 0; t < 2 * STEPS; ++t)
 #pragma unroll
                     for (int e = 0; e < 4; ++e) sum += __builtin_amdgcn_exp2f(score[t][e] - here);
+            } else {   // (nothing, or NaN alone: the row's)
+#pragma unroll
+                for (int t = 0; t < 2 * STEPS; ++t)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) sum += score[t][e] == score[t][e] ? 0.f : score[t][e];
             }
             peak = here;
         }
         const float highest = all_waves(most(peak), 0);
-        const float inverse = 1.f / all_waves(total(peak > -__builtin_inff() ? sum * __builtin_amdgcn_exp2f(peak - highest) : 0.f), 1);
+        const float inverse = 1.f / all_waves(total(peak > -__builtin_inff() ? sum * __builtin_amdgcn_exp2f(peak - highest) : sum), 1);
         for (int base = beg + wave * STEPS * kStep; base < end; base += W * STEPS * kStep) {
             columns_of(whole, column, base);
             scores_of(whole, column, score, base);
