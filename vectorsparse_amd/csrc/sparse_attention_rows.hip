@@ -10,8 +10,8 @@
 //   maximum and sum: over the wave's registers, the four groups, the waves; the probabilities are rounded to fp16 and it is
 //   those that are multiplied, as the operators do.
 //
-// What bounds it (8 heads x 2048, V = 4, width 64, rows of 102: 17.1 us with the probabilities, 15.5 us without; 20.2 us as two launches): the
-// gathers - 107 MB, of which a request asks sixteen half lines (k) or four lines (v) - behind a chain of five dependent loads that
+// What bounds it (8 heads x 2048, V = 4, width 64, rows of 102, HIP-graph replays: 15.1 us with the probabilities, 14.8 us without; 18.6 and 17.8 us
+// as two launches): the gathers - 107 MB, of which a request asks sixteen half lines (k) or four lines (v) - behind a chain of five dependent loads that
 // four waves per SIMD hide from each other in part.  Registers hold both gathers of a wave's two steps; of three and four steps k comes in
 // halves and v behind it (all of k at once spills: 8 heads x 648, width 128, rows of 65: 13.7 against 9.9 us).
 #include <type_traits>
@@ -148,15 +148,14 @@ attention_rows_kernel(int heads, int n, const int *__restrict__ row_indices, con
         }
         wave_lds_fence();
     };
-    auto probabilities = [&](float4_t (&score)[2 * STEPS], int s, float peak, float inverse, bool stage) __attribute__((always_inline)) {
+    auto probabilities = [&](const float4_t (&score)[2 * STEPS], int s, float inverse) __attribute__((always_inline)) {
         half8_t p;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             const int t = 2 * s + e / 4;
             p[e] = (half_t)(score[t][e % 4] * inverse);
-            if (KEEP && stage && c < V) mine[(16 * t + 4 * g + e % 4) * V + c] = p[e];
+            if (KEEP && c < V) mine[(16 * t + 4 * g + e % 4) * V + c] = p[e];
         }
-        (void)peak;
         return p;
     };
 
@@ -200,7 +199,7 @@ attention_rows_kernel(int heads, int n, const int *__restrict__ row_indices, con
                 }
             const float inverse = 1.f / all_waves(total(sum), 1);
 #pragma unroll
-            for (int s = 0; s < NS; ++s) multiply(rows[s], probabilities(score, s, peak, inverse, true));
+            for (int s = 0; s < NS; ++s) multiply(rows[s], probabilities(score, s, inverse));
             if constexpr (KEEP && NS > 0) keep(end - base < NS * kStep ? end - base : NS * kStep, base);
         };
         if (count <= 0) run(std::integral_constant<int, 0>());
@@ -251,7 +250,7 @@ attention_rows_kernel(int heads, int n, const int *__restrict__ row_indices, con
                 for (int t = 2 * s; t < 2 * s + 2; ++t)
 #pragma unroll
                     for (int e = 0; e < 4; ++e) score[t][e] = __builtin_amdgcn_exp2f(score[t][e] - highest);
-                multiply(rows, probabilities(score, s, highest, inverse, true));
+                multiply(rows, probabilities(score, s, inverse));
             }
             if constexpr (KEEP) keep(end - base < STEPS * kStep ? end - base : STEPS * kStep, base);
         }

@@ -36,8 +36,8 @@
 //      same order.  One more MFMA per step with an all-ones B operand yields the row sums of the rounded
 //      p in exactly the accumulator layout, so normalising needs no cross-lane traffic.
 // Planned launches of eight waves do not hold the union at once: sparse_attention_stream_kernel below runs
-// steps 2 (the copy) to C per sub-round of 128 ranks, the next sub-round's rows on their way meanwhile, with
-// the V rows transposed while they are copied (one transposition per workgroup instead of one per wave).
+// steps 2 (the copy) to C per sub-round of 128 ranks, the next sub-round's rows on their way to LDS meanwhile;
+// V rows are transposed by the instruction that reads them.
 #include "vs_common.hpp"
 
 namespace vs {
@@ -759,7 +759,6 @@ sparse_attention_union_kernel(int m_vec, int n, int d_qk, int d_v, int u_max,
 // exponentials) and the phases of a wave, one after the other.  Through registers, V transposed on its way to LDS, two barriers per
 // sub-round: 19.1 us; copied, with the start values and maxima as the compiler makes them of selects and fmaxf (three and two
 // instructions instead of two and one): 18.3 us.
-typedef int int2_t __attribute__((ext_vector_type(2)));
 
 // A row of K is 4 KS pieces of 16 bytes, piece p of row r at place p ^ stream_k_turn(r): sixteen lanes that read one piece of
 // sixteen rows touch every bank once.  A row of V is CPL pieces of 32 bytes, the same way for transposing reads of eight rows.

@@ -62,14 +62,6 @@ struct __align__(16) UnitInfo {
     int first, count, bad, unused;               // its steps in the lists; 1: rows that have to go nonzero by nonzero
 };
 
-// Orders LDS only: requests stay in flight across it.
-__device__ __forceinline__ void lds_only_barrier()
-{
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
-
 constexpr int kPackThreads = 1024, kPackSteps = 64;   // steps of a unit in LDS at once (64 KB)
 template <int V>
 constexpr int list_steps_in_lds() { return V == 1 ? 16 : 8; }
@@ -628,10 +620,11 @@ int launch_packed_shape(int m, int V, int k, int n, const PackedLayout &at, cons
 
 // Both launches as microseconds, fitted to 220 problems (256..4096 rows, 256..4608 columns, widths of 128..2048, 50..98 %, every V;
 // profiles/spmm_packed_rule_survey.txt) to within 6 % (tiles of 256 rows) and 9 %: a step of a tile takes its time whatever
-// else runs (LDS and the memory pipe of one CU), a listed nonzero of a unit a gather of its row for every tile.  Where the
-// rule takes them they are 1.1 to 2.3 times faster than what ran before.  The
-// line lies 15 % on this side of the others' estimate, which is low where tiles of either kind come in: at the line, 2248 x 2742 x 1488,
-// V = 1, 90 %: 44.3 against 33.7 us; 2672 x 2353 x 1224, V = 8, 80 %: 32.4 against 30.1 us.  Below 25 us the packing is
+// else runs (LDS and the memory pipe of one CU), a listed nonzero of a unit a gather of its row for every tile.  The rule
+// takes them for 20 of the survey's 440 choices: 18 are 1.14 to 2.3 times faster than what ran before, two level (3368 x 1801 x 992, V = 4,
+// 80 %: 0.99 and 1.01); of the others 30 would gain more than 5 %, up to 1.86 times, mostly where rhs no longer fits an XCD's L2, which the
+// others' estimate does not know.  The line lies 15 % on this side of that estimate: at the line, 2248 x 2742 x 1488, V = 1, 90 %: 44.3
+// against 33.7 us.  Below 25 us the packing is
 // too large a part of it: 1571 x 1116 x 1976, V = 1, 92 %: 20.8 against 22.5 us.
 //
 // The lists of uneven rows, or of columns in clusters, are many times those of even ones, and a wave goes through those of its units

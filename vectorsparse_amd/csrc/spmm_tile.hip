@@ -383,6 +383,14 @@ int launch_tile(int shape, int m_vec, int k, int n, const int *row_offsets, cons
 
 }  // namespace
 
+// Gathering, in the estimates of fastest_tile below.
+double spmm_gather_us(bool fine_grained, int vec_length, double nonzeros_vec, int k)
+{
+    const int v = vec_length == 1 ? 0 : (vec_length == 2 ? 1 : (vec_length == 4 ? 2 : 3));
+    static constexpr double kPerMega[2][4] = {{0.088, 0.089, 0.0925, 0.0995}, {0.076, 0.091, 0.134, 0.28}};
+    return (fine_grained ? 4.7 : 4.0) + kPerMega[fine_grained][v] * 1e-6 * nonzeros_vec * k;
+}
+
 // Both sides of the choice as microseconds per launch, fitted to 2500 problems (64..4096 rows, 64..4608 columns, widths of
 // 32..2048, 50..95 %, every V; device time).
 // Gathering: a launch, then a time per nonzero vector and dense column (the fine-grained kernel's grows with V).  Tiles: a
@@ -402,13 +410,6 @@ int launch_tile(int shape, int m_vec, int k, int n, const int *row_offsets, cons
 // 79 us (64 x 128); 2048 x 2304 x 256, V = 2, 50 %: 31 against 18 us (32 x 64); 2048 x 2304 x 512, V = 4, 90 %: 9.1 against
 // 18.5 us; at the line, 2048 x 2304 x 256, V = 1, 90 %: 13.4 (MFMA) and 12.6 us (fine-grained) against 12.9 us.
 // Only where the caller vouches for strictly ascending columns: a row in another order makes its workgroup go nonzero by nonzero.
-double spmm_gather_us(bool fine_grained, int vec_length, double nonzeros_vec, int k)
-{
-    const int v = vec_length == 1 ? 0 : (vec_length == 2 ? 1 : (vec_length == 4 ? 2 : 3));
-    static constexpr double kPerMega[2][4] = {{0.088, 0.089, 0.0925, 0.0995}, {0.076, 0.091, 0.134, 0.28}};
-    return (fine_grained ? 4.7 : 4.0) + kPerMega[fine_grained][v] * 1e-6 * nonzeros_vec * k;
-}
-
 // The fastest tile shape where one is expected to be ahead of gathering (0: none), and the time of what is then run.
 static int fastest_tile(bool fine_grained, int m_vec, int k, int n, int vec_length, double nonzeros_vec, int longest_vec, double &us)
 {
