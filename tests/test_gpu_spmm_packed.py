@@ -221,3 +221,23 @@ def test_uneven_rows_are_not_packed(gpu):
                 assert torch.equal(prob.spmm(B, kernel=kernel, row_length_hint=hint), got)
             with _lib.thread_options(spmm_packed=2):
                 assert not torch.equal(prob.spmm(B, kernel=kernel, row_length_hint=hint), got)
+
+
+def test_two_streams_pack_at_the_same_time(gpu):
+    """Every call packs into a workspace of its stream: two problems on two streams, without a wait between them, give the bits that
+    each gives alone."""
+    problems = []
+    for seed in (3, 4):
+        pat = cv.random_values(cv.binomial_pattern(2048, 4096, 0.95, seed=seed, vec_length=1), seed)
+        problems.append((ops.DeviceProblem(pat), torch.from_numpy(cv.dense_uniform(4096, 2048, seed=seed)).cuda()))
+    alone = [prob.spmm(B) for prob, B in problems]
+    outs = [[torch.empty_like(x) for _ in range(4)] for x in alone]
+    streams = [torch.cuda.Stream() for _ in problems]
+    torch.cuda.synchronize()
+    for turn in range(4):
+        for (prob, B), mine, stream in zip(problems, outs, streams):
+            with torch.cuda.stream(stream):
+                prob.spmm(B, out=mine[turn])
+    torch.cuda.synchronize()
+    for want, got in zip(alone, outs):
+        assert all(torch.equal(want, x) for x in got)

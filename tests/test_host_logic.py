@@ -511,6 +511,18 @@ def test_what_packed_rows_list_is_counted(V):
         assert ops.spmm_packed_lists(pat) == want, (kind, m_vec)
         assert ops.DeviceProblem(pat, device="cpu").packed_lists == want
     assert ops.spmm_packed_lists(cv.ColVecCSR(0, 8, V, np.zeros(1, dtype=np.int32), np.zeros(0, dtype=np.int32))) == (0, 0, 0)
+    assert ops.spmm_packed_lists(cv.ColVecCSR(2, 8, V, np.array([0, 2, 9], dtype=np.int32), np.zeros(2, dtype=np.int32))) is None
+    assert ops.DeviceProblem(cv.ColVecCSR(1, 8, 3, np.array([0, 2], dtype=np.int32), np.arange(2, dtype=np.int32)), device="cpu").packed_lists == (0, 0, 0)
+    rng = np.random.default_rng(V)
+    for lengths in ((0, 5, 1, 0, 2, 40), (3,), (2, 2), (1, 1, 1)):
+        good = cv.ColVecCSR(len(lengths), 64, V, *cv._pattern_from_lengths(rng, len(lengths), 64, np.array(lengths)))
+        assert ops.spmm_packed_lists(good) is not None
+        for at in range(1, good.nnz_vec):
+            for column in (good.column_indices[at - 1], good.column_indices[at - 1] - 1):
+                bad = cv.ColVecCSR(good.m_vec, 64, V, good.row_offsets, good.column_indices.copy())
+                bad.column_indices[at] = column
+                assert (ops.spmm_packed_lists(bad) is not None) == ops.columns_ascend(bad.row_offsets, bad.column_indices, strictly=True)
+                assert ops.DeviceProblem(bad, device="cpu").columns_distinct == (ops.spmm_packed_lists(bad) is not None)
 
 
 @pytest.mark.parametrize("V,n,k,density", [(1, 4096, 2048, 0.1), (2, 4096, 1024, 0.1), (2, 4096, 2048, 0.15), (4, 4096, 2048, 0.2)])

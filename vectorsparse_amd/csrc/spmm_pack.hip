@@ -676,22 +676,28 @@ int spmm_packed_choice(bool fine_grained, int m_vec, int k, int n, int vec_lengt
     return wide_us <= narrow_us ? 1 : 2;
 }
 
-PackedLists spmm_packed_lists(int m_vec, int vec_length, const int *row_offsets, const int *column_indices)
+bool spmm_packed_lists(int m_vec, int vec_length, const int *row_offsets, const int *column_indices, PackedLists &most)
 {
     const int unit_rows = kUnitRows / vec_length;
-    PackedLists most{0, 0, 0};
-    int two = 0, four = 0;
+    most = {0, 0, 0};
+    int two = 0, four = 0, falls = 0;
     for (int unit = 0; unit * (long long)unit_rows < m_vec; ++unit) {
         const int first = unit * unit_rows, behind = std::min(first + unit_rows, m_vec);
         int count = 0;
-        for (int r = first; r < behind; ++r)
-            for (int j = row_offsets[r] + 2; j < row_offsets[r + 1]; ++j) count += ((column_indices[j] ^ column_indices[j - 2]) & ~3) == 0;
+        for (int r = first; r < behind; ++r) {
+            const int beg = row_offsets[r], end = row_offsets[r + 1];
+            if (end - beg > 1) falls |= column_indices[beg + 1] <= column_indices[beg];
+            for (int j = beg + 2; j < end; ++j) {
+                falls |= column_indices[j] <= column_indices[j - 1];
+                count += ((column_indices[j] ^ column_indices[j - 2]) & ~3) == 0;
+            }
+        }
         const int steps = (count + kListed - 1) / kListed;
         two = (unit & 1 ? two : 0) + steps;
         four = (unit & 3 ? four : 0) + steps;
         most = {std::max(most.rows16, steps), std::max(most.rows32, two), std::max(most.rows64, four)};
     }
-    return most;
+    return !falls;
 }
 
 PackedLists spmm_packed_lists_bound(int m_vec, int n, int vec_length, int nonzeros_vec, int longest_row_vec)

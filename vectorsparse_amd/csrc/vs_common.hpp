@@ -376,8 +376,8 @@ struct PackedLists {
     int rows16, rows32, rows64;   // steps of 32 nonzeros, of the fullest 16, 32 and 64 scalar rows
 };
 int spmm_packed_choice(bool fine_grained, int m_vec, int k, int n, int vec_length, int nonzeros_vec, int longest_row_vec, const PackedLists *lists);
-// Host arrays, columns that ascend strictly in every row.
-PackedLists spmm_packed_lists(int m_vec, int vec_length, const int *row_offsets, const int *column_indices);
+// Host arrays; false where columns do not ascend strictly in every row.
+bool spmm_packed_lists(int m_vec, int vec_length, const int *row_offsets, const int *column_indices, PackedLists &most);
 // The same of a pattern of which only the longest row is known: the most that rows of random columns take (their number in a row
 // grows faster than the row).
 PackedLists spmm_packed_lists_bound(int m_vec, int n, int vec_length, int nonzeros_vec, int longest_row_vec);

@@ -450,7 +450,8 @@ int vs_spmm_packed_lists(int m_vec, int vec_length, const int *row_offsets, cons
 {
     if (m_vec < 0 || !vec_ok(vec_length) || !lists || (m_vec > 0 && !row_offsets)) return VS_ERROR_INVALID_VALUE;
     if (m_vec > 0 && row_offsets[m_vec] > row_offsets[0] && !column_indices) return VS_ERROR_INVALID_VALUE;
-    const vs::PackedLists most = vs::spmm_packed_lists(m_vec, vec_length, row_offsets, column_indices);
+    vs::PackedLists most;
+    if (!vs::spmm_packed_lists(m_vec, vec_length, row_offsets, column_indices, most)) return VS_ERROR_NOT_SUPPORTED;
     lists[0] = most.rows16;
     lists[1] = most.rows32;
     lists[2] = most.rows64;

@@ -188,18 +188,23 @@ def spmm_split_rows(m_vec, vec_length, k, n, nonzeros_vec, row_offsets, column_i
 def spmm_packed_workspace_bytes(m_vec, vec_length, k, n, nonzeros_vec, longest_row_vec, fine_grained=False, lists=None):
     """Workspace of the SpMM on packed rows (vs_spmm_f16_packed); 0 where other kernels are expected to be faster.  lists:
     the pattern's `spmm_packed_lists`, None for the worst that the counts allow."""
-    counted = None if lists is None else (ctypes.c_int * 3)(*lists)
+    counted = None if lists is None else _Counts(*lists)
     return int(_lib.lib().vs_spmm_packed_workspace_bytes_lists(int(fine_grained), m_vec, vec_length, k, n, nonzeros_vec, longest_row_vec, counted))
 
 
+_Counts = ctypes.c_int * 3
+
+
 def spmm_packed_lists(pattern):
-    """What the SpMM on packed rows lists of a pattern of strictly ascending columns: steps of 32 nonzeros of its fullest
-    16, 32 and 64 scalar rows."""
+    """What the SpMM on packed rows lists of a pattern: steps of 32 nonzeros of its fullest 16, 32 and 64 scalar rows; None
+    where the columns do not ascend strictly in every row, and for what no kernel takes."""
     ro = np.ascontiguousarray(pattern.row_offsets, dtype=np.int32)
     ci = np.ascontiguousarray(pattern.column_indices, dtype=np.int32)
-    counted = (ctypes.c_int * 3)()
-    _lib.check(_lib.lib().vs_spmm_packed_lists(pattern.m_vec, pattern.vec_length, ro.ctypes.data, ci.ctypes.data, counted), "vs_spmm_packed_lists")
-    return tuple(counted)
+    if ro.size <= pattern.m_vec or ro.min() < 0 or ro.max() > ci.size:   # (not a pattern: nothing to read)
+        return None
+    counted = _Counts()
+    st = _lib.lib().vs_spmm_packed_lists(pattern.m_vec, pattern.vec_length, ro.ctypes.data, ci.ctypes.data, counted)
+    return None if st else tuple(counted)
 
 
 def spmm_slab_workspace_bytes(m_vec, vec_length, k, n):
@@ -991,9 +996,10 @@ class DeviceProblem:
         self.row_offsets = torch.from_numpy(np.ascontiguousarray(pattern.row_offsets)).to(device)
         self.column_indices = torch.from_numpy(np.ascontiguousarray(pattern.column_indices)).to(device)
         # hints: SDDMM and SpMM run dense patterns of ascending columns on whole tiles
-        self.columns_distinct = columns_ascend(pattern.row_offsets, pattern.column_indices, strictly=True)
+        lists = spmm_packed_lists(pattern)
+        self.columns_distinct = lists is not None
         self.columns_sorted = self.columns_distinct or columns_ascend(pattern.row_offsets, pattern.column_indices)
-        self.packed_lists = spmm_packed_lists(pattern) if self.columns_distinct else (0, 0, 0)
+        self.packed_lists = lists or (0, 0, 0)
         self._workspace = None  # partial tiles of the split-row SpMM, allocated on first use
         self._parts = {}        # limit -> (RowParts, its list on the device, workspace), made on first use
         self._parts_need = {}
