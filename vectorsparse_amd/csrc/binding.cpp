@@ -64,6 +64,20 @@ struct Reader {
         if (!o || !PyBool_Check(o)) ok = false;
         return o == Py_True;
     }
+    // a tuple of three integers; None: false
+    bool counts(int (&to)[3])
+    {
+        PyObject *o = next();
+        if (o == Py_None) return false;
+        if (!o || !PyTuple_CheckExact(o) || PyTuple_GET_SIZE(o) != 3) {
+            ok = false;
+            return false;
+        }
+        Reader each(&PyTuple_GET_ITEM(o, 0), 3);
+        for (int &count : to) count = each.integer();
+        ok &= each.ok;
+        return ok;
+    }
     float number()
     {
         PyObject *o = next();
@@ -192,8 +206,8 @@ PyObject *spmm(PyObject *, PyObject *const *args, Py_ssize_t n_args)
 }
 
 // (fine_grained, m_vec, vec_length, k, n, nonzeros_vec, longest_row_vec, long_rows, row_length_hints, row_indices, row_offsets,
-// column_indices, values, rhs, out, stream, may_pack, and the three counts of vs_spmm_packed_lists), fp16 outputs; -2 - with nothing
-// launched - where spmm_packed is expected to be faster and the caller may make its workspace
+// column_indices, values, rhs, out, stream, lists), fp16 outputs; lists: the three counts of vs_spmm_packed_lists where the caller may
+// make a workspace, else None; -2 - with nothing launched - where spmm_packed is expected to be faster
 PyObject *spmm_ascending(PyObject *, PyObject *const *args, Py_ssize_t n_args)
 {
     Reader r(args, n_args);
@@ -204,9 +218,8 @@ PyObject *spmm_ascending(PyObject *, PyObject *const *args, Py_ssize_t n_args)
     const int *ri = (const int *)r.indices(), *ro = (const int *)r.indices(), *ci = (const int *)r.indices();
     const void *values = r.halves(), *rhs = r.halves();
     void *out = r.halves(), *stream = r.stream();
-    const bool may_pack = r.flag();
-    const int lists[3] = {r.integer(), r.integer(), r.integer()};
-    if (may_pack && r.done() && vs_spmm_packed_workspace_bytes_lists(fine_grained, m_vec, v, k, n, nnz, longest, lists) > 0) return PyLong_FromLong(-2);
+    int lists[3];
+    if (r.counts(lists) && r.done() && vs_spmm_packed_workspace_bytes_lists(fine_grained, m_vec, v, k, n, nnz, longest, lists) > 0) return PyLong_FromLong(-2);
     return status_of(r, [&] {
         return fine_grained ? vs_cuda_spmm_f16_ascending(m_vec, v, k, n, nnz, longest, hints, ri, ro, ci, values, rhs, out, stream)
                             : vs_wmma_spmm_f16_ascending(m_vec, v, k, n, nnz, longest, long_rows, hints, ri, ro, ci, values, rhs, out, stream);

@@ -1090,13 +1090,13 @@ class DeviceProblem:
         if self.columns_distinct and out.dtype == torch.float16:
             st = _native.spmm_ascending(kernel != "wmma", self.m_vec, self.vec_length, k, self.n, self.nnz_vec, self.longest_row_vec,
                                         self.long_rows, bool(row_length_hint), self.row_indices, self.row_offsets,
-                                        self.column_indices, self.values, rhs_matrix, out, stream, True, *self.packed_lists)
+                                        self.column_indices, self.values, rhs_matrix, out, stream, self.packed_lists)
             if st == -2:
                 st = self._spmm_packed(rhs_matrix, kernel != "wmma", out, stream)
                 if st is None:
                     st = _native.spmm_ascending(kernel != "wmma", self.m_vec, self.vec_length, k, self.n, self.nnz_vec, self.longest_row_vec,
                                                 self.long_rows, bool(row_length_hint), self.row_indices, self.row_offsets,
-                                                self.column_indices, self.values, rhs_matrix, out, stream, False, *self.packed_lists)
+                                                self.column_indices, self.values, rhs_matrix, out, stream, None)
             if st >= 0:
                 if st:
                     _lib.check(st, "vs_%s_spmm_f16%s" % ("wmma" if kernel == "wmma" else "cuda", "_batched" if row_length_hint else ""))
