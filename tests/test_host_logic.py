@@ -565,3 +565,13 @@ def test_attention_rows_is_for_layers_it_is_faster_on(heads, seq, V, d, mean, ke
     status = _lib.lib().vs_sparse_attention_rows_f16(heads, m_vec, V, seq, d, d, m_vec * mean, mean + mean // 3, 0, 0, 0, 0, seq * d, 0, seq * d, 0, seq * d,
                                                      0, seq * d, 16 if keep else 0, m_vec * mean * V, 1.0, 0)
     assert status == (1 if taken else 801)
+
+
+def test_attention_rows_refuses_more_rows_than_a_launch_has_threads_for():
+    """(without addresses, as above)"""
+    def status(heads, m_vec):
+        return _lib.lib().vs_sparse_attention_rows_f16(heads, m_vec, 1, 64, 64, 64, m_vec, 1, 0, 0, 0, 0, 64, 0, 64, 0, 64, 0, m_vec * 64, 0, 0, 1.0, 0)
+
+    for option in (0, 2, 5):
+        with _lib.thread_options(attention_rows=option):
+            assert status(7, 1 << 20) == 1 and status(8, 1 << 20) == status(1, 1 << 23) == status(4096, 1 << 12) == 801

@@ -332,8 +332,8 @@ int attention_rows_waves(bool keep, int heads, int m_vec, int n, int vec_length,
     const Options &o = options();
     if (o.attention_rows == 1) return 0;
     if (d_qk != d_v || (d_v != 64 && d_v != 128) || n <= 0 || m_vec <= 0 || heads <= 0 || (long long)n * d_v >= (1LL << 30) ||
-        (long long)m_vec * heads > 0x7fffffffLL)
-        return 0;
+        (long long)m_vec * heads >= (1LL << 32) / 512)
+        return 0;   // (a launch has fewer than 2^32 threads, eight waves for a row at most)
     if (o.attention_rows >= 2) return 1 << (o.attention_rows - 2);
     if (longest_row_vec < 0 || longest_row_vec > 512 || o.softmax_spmm || o.sddmm_slots || o.sddmm_block_waves || o.sddmm_group || o.sddmm_tile ||
         o.spmm_waves || o.spmm_cols_per_lane || o.spmm_steps)
