@@ -575,3 +575,12 @@ def test_attention_rows_refuses_more_rows_than_a_launch_has_threads_for():
     for option in (0, 2, 5):
         with _lib.thread_options(attention_rows=option):
             assert status(7, 1 << 20) == 1 and status(8, 1 << 20) == status(1, 1 << 23) == status(4096, 1 << 12) == 801
+
+
+def test_packed_rows_refuse_more_rows_than_a_launch_has_threads_for():
+    for option in (2, 3):
+        with _lib.thread_options(spmm_packed=option):
+            need = lambda m_vec, V, k: ops.spmm_packed_workspace_bytes(m_vec, V, k, 64, 4096, 64)
+            assert need(1 << 22, 8, 64) > 0 and need(1 << 25, 1, 64) > 0 and need(1 << 20, 8, 1 << 14) == 0
+            assert need((1 << 26) - 2048, 1, 64) > 0
+            assert need(1 << 23, 8, 64) == need((1 << 26) - 2047, 1, 64) == need(1 << 25, 2, 64) == need(1 << 24, 2, 1 << 19) == 0

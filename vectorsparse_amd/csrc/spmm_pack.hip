@@ -645,8 +645,10 @@ int spmm_packed_choice(bool fine_grained, int m_vec, int k, int n, int vec_lengt
     const Options &o = options();
     if (o.spmm_packed == 1) return 0;
     if (m_vec <= 0 || k <= 0 || k % 8 != 0 || n <= 0 || nonzeros_vec <= 0 || nonzeros_vec > (1 << 26) || ((long long)n + 1024) * k >= (1LL << 30) || k >= (1 << 24)) return 0;
-    // (a tile's packed operands are addressed with 32-bit offsets)
-    if ((long long)m_vec * vec_length > (1 << 30) || n > (1 << 22)) return 0;
+    // (a tile's packed operands are addressed with 32-bit offsets; a launch has fewer than 2^32 threads: 64 per row for the packing, 512 per
+    // tile of 128 x 128 for the product)
+    if ((long long)m_vec * vec_length > (1 << 26) - 2048 || n > (1 << 22)) return 0;
+    if (((long long)m_vec * vec_length / 128 + 2) * (k / 128 + 2) >= (1LL << 32) / 512) return 0;
     if (o.spmm_packed >= 2) return o.spmm_packed - 1;
     if (o.spmm_tile || o.spmm_waves || o.spmm_cols_per_lane || o.spmm_steps || o.spmm_pipe || o.spmm_gather || o.spmm_teams || o.spmm_blocks_per_wave || o.spmm_guard_waves)
         return 0;  // a launch shape of other kernels is asked for
