@@ -613,7 +613,8 @@ class SparseAttention:
     # tokens, random, every V; head widths to 32, 64 and 128).  Streamed workgroups: launch, per sub-round of the longest one,
     # launch under load, per workgroup and per sub-round in 512ths, merge, per tile of the longest merge.  Measured again over
     # 240 drawn masks (profiles/attention_split_rule_survey.txt) the estimates are high by 6 % (streamed with a merge; spread
-    # 9 %), 21 % (one workgroup per block; 11 %), 7 % (row parts; 9 %) and 19 % (two launches; 11 %).
+    # 9 %), 21 % (one workgroup per block; 11 %), 7 % (row parts; 9 %) and 19 % (two launches; 11 %); the streamed kernel has lost
+    # another 5 to 14 % since.
     _STREAM_US = ((3.47, 2.06, 5.15, 2.13, 4.21, 2.9, 0.5), (3.41, 2.47, 5.86, 4.21, 4.87, 3.12, 0.49),
                   (4.1, 3.64, 6.0, 10.63, 10.22, 3.98, 1.01))
     # The three operators on row parts: launches, per thousand vector rows of 16 heads, per thousand nonzero vectors of 16 heads
