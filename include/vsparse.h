@@ -308,7 +308,7 @@ int vs_cuda_spmm_f16_ascending(int m_vec, int vec_length, int k, int n, int nonz
  * vs_spmm_packed_workspace_bytes: what the call needs (16-byte aligned, uninitialised, used by one call at a time), 0 where
  * the entry points above are expected to be faster or have to take the call; the call returns VS_ERROR_NOT_SUPPORTED where they
  * would for even rows.  Uneven rows list more: vs_spmm_packed_workspace_bytes expects the worst that nonzeros_vec and longest_row_vec
- * allow, vs_spmm_packed_workspace_bytes_lists (NULL: the same) what vs_spmm_packed_lists has counted in the host's pattern, the steps
+ * allow where columns lie at random, vs_spmm_packed_workspace_bytes_lists (NULL: the same) what vs_spmm_packed_lists has counted in the host's pattern, the steps
  * of 32 nonzeros that the fullest 16, 32 and 64 scalar rows list (VS_ERROR_NOT_SUPPORTED: a row's columns do not ascend strictly).  Not more than 1 GiB, unless the option asks for the kernel.
  * No counterpart in the reference.
  */

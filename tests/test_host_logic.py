@@ -584,3 +584,23 @@ def test_packed_rows_refuse_more_rows_than_a_launch_has_threads_for():
             assert need(1 << 22, 8, 64) > 0 and need(1 << 25, 1, 64) > 0 and need(1 << 20, 8, 1 << 14) == 0
             assert need((1 << 26) - 2048, 1, 64) > 0
             assert need(1 << 23, 8, 64) == need((1 << 26) - 2047, 1, 64) == need(1 << 25, 2, 64) == need(1 << 24, 2, 1 << 19) == 0
+
+
+def test_the_packed_launch_takes_what_the_lists_allow():
+    """The entry point has no lists: whatever a workspace was asked for with them must not be refused there (without a workspace it is
+    an invalid value, before anything is read)."""
+    rng = np.random.default_rng(5)
+    taken = refused = 0
+    for _ in range(20000):
+        V, fine = int(rng.choice([1, 2, 4, 8])), bool(rng.integers(2))
+        m_vec, n, k = (int(round(np.exp(rng.uniform(np.log(lo), np.log(hi))) / step)) * step for lo, hi, step in ((500 / V, 8000 / V, 1), (500, 8000, 1), (200, 2048, 8)))
+        density = rng.uniform(0.02, 0.4)
+        nnz, longest = int(m_vec * n * density), int(n * min(1.0, density * np.exp(abs(rng.normal(0, 1)))))
+        lists = sorted(int(x) for x in rng.integers(0, 40, 3))
+        if ops.spmm_packed_workspace_bytes(m_vec, V, k, n, nnz, longest, fine, lists) == 0:
+            refused += 1
+            continue
+        taken += 1
+        st = _lib.lib().vs_spmm_f16_packed(int(fine), m_vec, V, k, n, nnz, longest, 4096, 4096, 4096, 4096, 4096, 0, 0, 0)
+        assert st == 1, (fine, m_vec, V, k, n, nnz, longest, lists)
+    assert taken > 1000 and refused > 1000

@@ -662,7 +662,8 @@ int spmm_packed_choice(bool fine_grained, int m_vec, int k, int n, int vec_lengt
     const double wide = std::ceil(m / 256) * std::ceil(k / 128.0) / 256, narrow = std::ceil(m / 128) * std::ceil(k / 128.0) / 256;
     double wide_us = 11.8 + (0.498 * steps + 0.116 * listed) * std::ceil(wide) + 9.4 * wide + 0.19e-3 * unit;
     double narrow_us = 6.6 + (0.417 * steps + 0.043 * listed) * std::ceil(narrow) + 7.1 * narrow + 0.57e-3 * unit;
-    if (lists) {
+    if (others >= gather) others += (fine_grained ? 0.03 : 0.005) * std::fmax(0.0, longest_row_vec - 2 * density * n);
+    if (lists) {   // (nothing here makes packing look faster: the launch, which has no lists, takes what was found with them)
         // (what the fullest of 64 even rows takes: a fourth more than the mean, half a step of padding per unit)
         const double even = 1.25 * 4 * (listed / kListed + 0.5);
         const auto turns = [&](double row) { return std::fmax(0.0, std::ceil(row / (64 * vec_length)) - (vec_length <= 2 ? 8 : 4)); };
@@ -672,7 +673,6 @@ int spmm_packed_choice(bool fine_grained, int m_vec, int k, int n, int vec_lengt
         const double packing = more_turns * (0.55 + 0.27 * passes);
         wide_us += kDoubt * (packing + 0.94 * std::fmax(0.0, lists->rows64 - even) * std::ceil(wide));
         narrow_us += kDoubt * (packing + 0.5 * std::fmax(0.0, lists->rows32 - even / 2) * std::ceil(narrow));
-        if (others >= gather) others += (fine_grained ? 0.03 : 0.005) * std::fmax(0.0, longest_row_vec - 2 * density * n);
     }
     if (std::fmin(wide_us, narrow_us) > 1.15 * others) return 0;
     return wide_us <= narrow_us ? 1 : 2;

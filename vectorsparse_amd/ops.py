@@ -187,7 +187,8 @@ def spmm_split_rows(m_vec, vec_length, k, n, nonzeros_vec, row_offsets, column_i
 
 def spmm_packed_workspace_bytes(m_vec, vec_length, k, n, nonzeros_vec, longest_row_vec, fine_grained=False, lists=None):
     """Workspace of the SpMM on packed rows (vs_spmm_f16_packed); 0 where other kernels are expected to be faster.  lists:
-    the pattern's `spmm_packed_lists`, None for the worst that the counts allow."""
+    the pattern's `spmm_packed_lists`, None for the worst that the counts allow where columns lie at
+    random."""
     counted = None if lists is None else _Counts(*lists)
     return int(_lib.lib().vs_spmm_packed_workspace_bytes_lists(int(fine_grained), m_vec, vec_length, k, n, nonzeros_vec, longest_row_vec, counted))
 
