@@ -631,7 +631,8 @@ int launch_packed_shape(int m, int V, int k, int n, const PackedLayout &at, cons
 // alone: 0.94 us per step of the fullest 64 rows (tiles of 256), 0.5 us of the fullest 32 (of 128), and packing a row beyond what a
 // wave keeps 0.55 us per turn of 64 nonzeros and 0.27 us more for every further pass over it, which its unit's list asks for.  Fitted
 // to 81 problems (4096 x 4096 x 2048 and less, even to Pareto rows) within 4 % (tiles of 256) and 6 %.  Gathering waits for its longest
-// row too: 0.03 us per nonzero vector beyond two mean rows on the fine-grained path, 0.005 us on the matrix cores.  4096 x 4096 x 2048, V = 4, 80 %:
+// row too: 0.005 us per nonzero vector beyond two mean rows, 0.03 us on the fine-grained path where it fills the chip (a dense row
+// among even ones, 4096 x 4096 x 2048, V = 4, 95 %: 187 us, 140 packed, 52 without it; 1148 x 4419 x 1808, V = 4, 90 %: 78 us, 125 packed).  4096 x 4096 x 2048, V = 4, 80 %:
 // 67 us for even rows, 171 us (and 118 us as they run now) for log-normal rows of width 0.5, 364 us (124 us) for Pareto rows.
 //
 // The workspace grows with the matrix, whatever its sparsity, and those who call the operators did not ask for one: none beyond
@@ -662,7 +663,8 @@ int spmm_packed_choice(bool fine_grained, int m_vec, int k, int n, int vec_lengt
     const double wide = std::ceil(m / 256) * std::ceil(k / 128.0) / 256, narrow = std::ceil(m / 128) * std::ceil(k / 128.0) / 256;
     double wide_us = 11.8 + (0.498 * steps + 0.116 * listed) * std::ceil(wide) + 9.4 * wide + 0.19e-3 * unit;
     double narrow_us = 6.6 + (0.417 * steps + 0.043 * listed) * std::ceil(narrow) + 7.1 * narrow + 0.57e-3 * unit;
-    if (others >= gather) others += (fine_grained ? 0.03 : 0.005) * std::fmax(0.0, longest_row_vec - 2 * density * n);
+    const bool full = fine_grained && m_vec * std::ceil(k / 128.0) >= 16384;
+    if (others >= gather) others += (full ? 0.03 : 0.005) * std::fmax(0.0, longest_row_vec - 2 * density * n);
     if (lists) {   // (nothing here makes packing look faster: the launch, which has no lists, takes what was found with them)
         // (what the fullest of 64 even rows takes: a fourth more than the mean, half a step of padding per unit)
         const double even = 1.25 * 4 * (listed / kListed + 0.5);
