@@ -630,7 +630,8 @@ int launch_packed_shape(int m, int V, int k, int n, const PackedLayout &at, cons
 // The lists of uneven rows, or of columns in clusters, are many times those of even ones, and a wave goes through those of its units
 // alone: 0.94 us per step of the fullest 64 rows (tiles of 256), 0.5 us of the fullest 32 (of 128), and packing a row beyond what a
 // wave keeps 0.55 us per turn of 64 nonzeros and 0.27 us more for every further pass over it, which its unit's list asks for.  Fitted
-// to 81 problems (4096 x 4096 x 2048 and less, even to Pareto rows) within 4 % (tiles of 256) and 6 %.  Gathering waits for its longest
+// to 81 problems (4096 x 4096 x 2048 and less, even to Pareto rows; profiles/spmm_packed_uneven_survey.txt) within 4 % (tiles of 256) and 6 %.
+// Of 320 choices drawn again 29 are packed, two of them slower (0.87 and 0.92 of the speed).  Gathering waits for its longest
 // row too: 0.005 us per nonzero vector beyond two mean rows, 0.03 us on the fine-grained path where it fills the chip (a dense row
 // among even ones, 4096 x 4096 x 2048, V = 4, 95 %: 187 us, 140 packed, 52 without it; 1148 x 4419 x 1808, V = 4, 90 %: 78 us, 125 packed).  4096 x 4096 x 2048, V = 4, 80 %:
 // 67 us for even rows, 171 us (and 118 us as they run now) for log-normal rows of width 0.5, 364 us (124 us) for Pareto rows.
